@@ -188,14 +188,11 @@ fp_status ensure_k(fp_ctx* ctx, int K) {
     // K-sized arrays grow only; a smaller K reuses them
     FP_TRY(dalloc(ctx, &ctx->sizes, (size_t)K));
     FP_TRY(dalloc(ctx, &ctx->sizes_frozen, (size_t)K));
-    FP_TRY(dalloc(ctx, &ctx->cand_tot, (size_t)K));
-    FP_TRY(dalloc(ctx, &ctx->over_idx, (size_t)K));
+    FP_TRY(dalloc(ctx, &ctx->over, (size_t)K));
     ctx->kcap = K;
   }
   if (ctx->K != K) {
-    // the BAL histogram is all zero between rounds whatever its shape; the
-    // candidate totals restart from zero
-    fill_async<long long>(ctx, ctx->cand_tot, (size_t)K, 0);
+    // the BAL histogram is all zero between rounds whatever its shape
     ctx->K = K;
     ctx->gen++;
   }
@@ -409,6 +406,8 @@ fp_status fp_upload(fp_ctx* ctx, int nov, int noe, const unsigned* net_ptr, cons
   ctx->rmax = 0;
   ctx->hist_cap = 0;
   ctx->compact_cap = 0;
+  ctx->masks = nullptr;
+  ctx->mask_cap = 0;
   ctx->cn.ready = false;
   ctx->cn.ops_cap = 0;
   ctx->vol.rmax = 0;
@@ -597,7 +596,6 @@ fp_status fp_upload(fp_ctx* ctx, int nov, int noe, const unsigned* net_ptr, cons
   FP_TRY(dalloc(ctx, &ctx->flags, 4));
   fill_async<int>(ctx, ctx->flags, 4, 0);
   FP_TRY(dalloc(ctx, &ctx->moves, 1));
-  FP_TRY(dalloc(ctx, &ctx->over_count, 1));
   fill_async<unsigned>(ctx, ctx->net_stamp, (size_t)std::max(noe, 1), 0u);
   FP_HIP_OK(hipGetLastError());
   FP_HIP_OK(hipStreamSynchronize(ctx->stream));

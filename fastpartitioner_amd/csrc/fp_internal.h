@@ -81,6 +81,15 @@ __device__ __forceinline__ T uniform_load(const T* p) {
   return *(const __attribute__((address_space(4))) T*)p;
 }
 
+// The same for element i of an array at a 32-bit byte offset from a
+// wave-uniform base: the offset is the scalar load's own, no 64-bit address is
+// computed, and consecutive elements are one load.
+template <typename T>
+__device__ __forceinline__ T uniform_load_at(const void* base, unsigned byte_off, int i) {
+  return ((const __attribute__((address_space(4))) T*)((const __attribute__((address_space(4))) char*)base +
+                                                       byte_off))[i];
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_sum(T x) {
   for (int off = WAVE / 2; off > 0; off >>= 1) x += __shfl_xor(x, off);
@@ -223,25 +232,6 @@ __device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long x)
   return ((unsigned long long)mh << 32) | ml;
 }
 
-// first index k in [lo, hi) with arr[k] >= key (arr ascending); wave-uniform result
-__device__ __forceinline__ unsigned wave_lower_bound(const int* __restrict__ arr, unsigned lo, unsigned hi, int key) {
-  const int lane = lane_id();
-  while (hi - lo > WAVE) {
-    const unsigned step = (hi - lo + WAVE - 1) / WAVE;
-    const unsigned k = lo + (unsigned)lane * step;
-    const bool lt = k < hi && arr[k] < key;
-    const int c = __popcll(__ballot(lt));
-    if (c == 0) return lo;
-    const unsigned nlo = lo + (unsigned)(c - 1) * step + 1;
-    const unsigned nhi = min(hi, lo + (unsigned)c * step);
-    lo = nlo;
-    hi = nhi;
-  }
-  const unsigned k = lo + (unsigned)lane;
-  const bool lt = k < hi && arr[k] < key;
-  return lo + (unsigned)__popcll(__ballot(lt));
-}
-
 // index of the entry of part p in list[0..L) or -1; wave-uniform
 __device__ __forceinline__ int wave_find(const unsigned* list, int L, int p, unsigned pmask) {
   const int lane = lane_id();
@@ -342,6 +332,35 @@ __device__ __forceinline__ void wave_ilist_move(unsigned* list, unsigned short* 
     L++;
   }
   wave_lds_sync();
+}
+
+// The leading moves of a window (bit l of m: lane l moves a pin from part own
+// to part d, in lane order) that neither empty nor add an entry change counts
+// only, in any order: they are made together. A move counts as such when d has
+// an entry and own's count outlasts all of the window's removals from it. The
+// rest, from the first other move on, is returned for wave_ilist_move.
+__device__ __forceinline__ unsigned long long wave_ilist_moves(unsigned* list, const unsigned short* at,
+                                                               unsigned long long m, int own, int d, int pb) {
+  const int lane = lane_id();
+  const unsigned inc = 1u << pb;
+  const bool mine = (m >> lane) & 1ull;
+  const int jp = mine && own >= 0 ? (int)at[own] : (int)LIST_NONE;
+  const int jq = mine ? (int)at[d] : (int)LIST_NONE;
+  const bool leaves = jp != (int)LIST_NONE;
+  const unsigned c0 = leaves ? list[jp] >> pb : 0u;
+  wave_lds_sync();
+  if (leaves) atomicSub(&list[jp], inc);
+  wave_lds_sync();
+  const unsigned c1 = leaves ? list[jp] >> pb : 0u;
+  const unsigned outs = (c0 - c1) & (~0u >> pb);  // the count field may have wrapped
+  const bool safe = jq != (int)LIST_NONE && (own < 0 || (leaves && outs < c0));
+  const unsigned long long other = __ballot(mine && !safe);
+  const int first = other ? __ffsll((long long)other) - 1 : WAVE;
+  wave_lds_sync();
+  if (leaves && lane >= first) atomicAdd(&list[jp], inc);  // taken back
+  if (mine && lane < first) atomicAdd(&list[jq], inc);
+  wave_lds_sync();
+  return first == WAVE ? 0ull : m & ~((1ull << first) - 1ull);
 }
 
 // First 64 words of net n's segment (seg = net_ptr[n] + n): the segment holds
@@ -472,6 +491,13 @@ __device__ __forceinline__ void wave_touch_nets(const unsigned* __restrict__ vn,
   }
 }
 
+// Stamps a vertex's nets with the round's tag. Called by the whole wavefront;
+// waves that stamp the same net write the same value.
+__device__ __forceinline__ void wave_stamp_nets(const unsigned* __restrict__ vn, int deg, unsigned tag,
+                                                unsigned* __restrict__ net_stamp) {
+  for (int i = lane_id(); i < deg; i += WAVE) net_stamp[vn[i]] = tag;
+}
+
 // A wave's newly touched nets, staged in its own LDS buffer of TOUCH_BUF
 // entries and appended to the round's touched list a buffer at a time: one
 // atomic on the list's counter per flush instead of one per vertex (atomics
@@ -564,32 +590,24 @@ __device__ __forceinline__ void wave_rank_window(const int* apply_pins, unsigned
     hi = e;
     return;
   }
-  lo = wave_lower_bound(apply_pins, s, e, r0);
-  hi = wave_lower_bound(apply_pins, lo, e, r1);
-}
-
-// Walks a wave's share of the touched nets (entries first, first + stride,
-// ... of touched): their ids and pin ranges are loaded 64 nets at a time,
-// one net per lane, then f(n, s, e) runs on every lane for each net in
-// order, with [s, e) the net's range in net_ptr.
-template <class F>
-__device__ __forceinline__ void wave_for_touched(const int* __restrict__ touched, int ntouched,
-                                                 const unsigned* __restrict__ net_ptr, int first, int stride, F f) {
+  // both bounds narrow 64-fold per step, their probes loaded together
   const int lane = lane_id();
-  for (long long b0 = first; b0 < ntouched; b0 += (long long)WAVE * stride) {
-    const long long ij = b0 + (long long)lane * stride;
-    int nj = 0;
-    unsigned sj = 0, ej = 0;
-    if (ij < ntouched) {
-      nj = touched[ij];
-      sj = net_ptr[nj];
-      ej = net_ptr[nj + 1];
-    }
-    const int cnt = (int)min((long long)WAVE, ((long long)ntouched - b0 + stride - 1) / stride);
-    for (int j = 0; j < cnt; j++)
-      f(__builtin_amdgcn_readlane(nj, j), (unsigned)__builtin_amdgcn_readlane((int)sj, j),
-        (unsigned)__builtin_amdgcn_readlane((int)ej, j));
+  unsigned a0 = s, a1 = e, b0 = s, b1 = e;
+  while (a1 - a0 > (unsigned)WAVE || b1 - b0 > (unsigned)WAVE) {
+    const unsigned sa = (a1 - a0 + WAVE - 1) / WAVE, sb = (b1 - b0 + WAVE - 1) / WAVE;
+    const unsigned ka = a0 + (unsigned)lane * sa, kb = b0 + (unsigned)lane * sb;
+    const int xa = ka < a1 ? apply_pins[ka] : INT_MAX, xb = kb < b1 ? apply_pins[kb] : INT_MAX;
+    const unsigned ca = (unsigned)__popcll(__ballot(ka < a1 && xa < r0)), cb = (unsigned)__popcll(__ballot(kb < b1 && xb < r1));
+    // the bound lies after the last probe below the key, up to the next one
+    a1 = ca == 0 ? a0 : min(a1, a0 + ca * sa);
+    a0 = ca == 0 ? a0 : a0 + (ca - 1) * sa + 1;
+    b1 = cb == 0 ? b0 : min(b1, b0 + cb * sb);
+    b0 = cb == 0 ? b0 : b0 + (cb - 1) * sb + 1;
   }
+  const unsigned ka = a0 + (unsigned)lane, kb = b0 + (unsigned)lane;
+  const int xa = ka < a1 ? apply_pins[ka] : INT_MAX, xb = kb < b1 ? apply_pins[kb] : INT_MAX;
+  lo = a0 + (unsigned)__popcll(__ballot(ka < a1 && xa < r0));
+  hi = b0 + (unsigned)__popcll(__ballot(kb < b1 && xb < r1));
 }
 
 // Writes a list back to both the packed segment and its evaluation view.
@@ -695,6 +713,9 @@ struct fp_ctx {
   unsigned* vtx_seg = nullptr;
   long long* sizes = nullptr;
   bool has_state = false;
+  unsigned long long* masks = nullptr;  // the nets' part masks of a running refinement (fp_masks.h)
+  size_t mask_cap = 0;                  // its capacity in words
+  bool use_masks = true;                // a server turns them off where its budget has no room for them
 
   // round scratch
   int rmax = 0;
@@ -702,10 +723,10 @@ struct fp_ctx {
   int* flags = nullptr;  // [0] CN edit list overflow: the size it needed (0 = none), [1] a repeated
                          // pin's net over CN_MAXOPS ops, [2] CN passes applied (counted by the commit)
   unsigned* net_stamp = nullptr;  // round tag of the last round that touched the net (cleared every pass)
-  long long *cand_tot = nullptr, *sizes_frozen = nullptr, *pref = nullptr;
+  long long *sizes_frozen = nullptr, *pref = nullptr;
   int* hist = nullptr;
   size_t hist_cap = 0;
-  int *over_idx = nullptr, *over_count = nullptr;
+  int* over = nullptr;  // BAL: parts whose candidates exceed their room this round
   unsigned long long* moves = nullptr;
   int2* compact_tiles = nullptr;  // per-tile move / event totals of a round's compaction
   int compact_cap = 0;
@@ -779,6 +800,7 @@ struct RefinePlan {
   int R = 0;
   int eval_waves = 0;
   int eval_grid = 0;
+  unsigned long long* masks = nullptr;  // evaluate through the nets' part masks (fp_masks.h); null: through the lists
 };
 
 // plan_*: checks, scratch, and the per-refinement initialisation kernels

@@ -23,7 +23,7 @@
 #include <thread>
 #include <unordered_map>
 
-#include "fp_internal.h"
+#include "fp_masks.h"
 
 struct fp_server {
   int device = 0;
@@ -51,6 +51,7 @@ struct fp_server {
     fp_schedule sched{};
     std::vector<int> part;
     long long footprint = 0;
+    bool masks = true;  // the footprint has room for the nets' part masks
     // results
     bool done = false;
     fp_status status = FP_OK;
@@ -107,6 +108,13 @@ long long scratch_bytes(const fp_server::Graph& g, fp_metric metric, int K, int 
   return b;
 }
 
+// The nets' part masks of a request whose objective uses them. They are
+// optional: a request that fits the budget only without them is evaluated
+// through the lists.
+long long mask_bytes(const fp_server::Graph& g, fp_metric metric, int K) {
+  return metric == FP_METRIC_TV ? 16ll * fpe::mask_words(K) * ((long long)g.noe + 1) : 0;
+}
+
 // a new context holding graph g's upload (the caller holds no lock)
 fp_status upload_replica(fp_server* s, const fp_server::Graph& g, fp_ctx** out) {
   fp_ctx* ctx = nullptr;
@@ -123,6 +131,7 @@ fp_status upload_replica(fp_server* s, const fp_server::Graph& g, fp_ctx** out) 
 }
 
 void run_request(fp_server* s, fp_server::Request& q, fp_ctx* ctx) {
+  ctx->use_masks = q.masks;
   fp_status st = fp_set_partition(ctx, q.K, q.part.data());
   fp_refine_stats stats{};
   if (st == FP_OK) st = fp_refine(ctx, q.metric, q.passes, q.has_sched ? &q.sched : nullptr, &stats);
@@ -303,6 +312,9 @@ fp_status fp_server_submit(fp_server* s, int graph_id, fp_metric metric, int K, 
     const fp_server::Graph& g = *s->graphs[(size_t)graph_id];
     q->part.assign(part, part + g.nov);
     q->footprint = g.bytes + scratch_bytes(g, metric, K, sched ? sched->round : 0);
+    const long long extra = mask_bytes(g, metric, K);
+    q->masks = q->footprint + extra <= s->budget;
+    if (q->masks) q->footprint += extra;
     if (q->footprint > s->budget)
       return sfail(s, FP_ERR_BUDGET, "request needs %lld bytes, the budget is %lld", q->footprint, s->budget);
   }

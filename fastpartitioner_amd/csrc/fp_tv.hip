@@ -2,29 +2,31 @@
 // TV/partition.cpp:669-896 round schedule).
 //
 // One pass = rounds of R consecutive ordering positions. A round is:
-//   k_tv_eval    one wavefront per vertex (grid-stride over the round,
-//                software-pipelined over the wave's vertices) sweeps the lists
-//                of the vertex's nets in their 16-bit evaluation view -- one
-//                128-byte read per net brings its lambda and first 63
+//   k_tv_eval_masks  (K <= 512) scores a vertex per wavefront from its nets'
+//                part masks (fp_masks.h): counts per part in registers, the
+//                LDG2 decision by a lexicographic wave reduction (parts that
+//                share the best score and size are told apart by where the
+//                reference's scan meets them), then the TV gain test
+//   k_tv_eval    (larger K) the same from the lists' 16-bit evaluation view:
+//                one 128-byte read per net brings its lambda and first 63
 //                entries, 3 nets in flight; the further windows of long
 //                lists follow as one task list over all of the vertex's long
-//                nets, 2 windows in flight -- into LDS histograms of pin
-//                counts per part, then picks the LDG2 decision by a
-//                lexicographic wave reduction (a vertex whose best score and
-//                size two parts share is swept again with the
-//                first-appearance ranks that break the tie) and applies the
-//                TV gain test. Candidates stamp their nets into the
-//                round's touched-net list; BAL also accumulates candidate
-//                weights per part and per (part, 64-slot tile).
-//   k_bal_scan   BAL: parts whose candidate weight exceeds cap - size get a
-//                dense index; for each, an exclusive scan over tiles
+//                nets, 2 windows in flight; pin counts per part in LDS
+//                Both write the slots' decisions and (BAL) the candidate
+//                weights per (part, 64-slot tile); REF candidates stamp
+//                their nets with the round's tag
+//   k_bal_scan   BAL: per part, whether its candidates exceed cap - size, and
+//                then an exclusive scan of its row of tile weights
 //   k_bal_admit  BAL: prefix admission per part in ordering order, commit of
-//                part vector and sizes
-//   k_apply      one wavefront per touched net (one lane per net of at most 8
-//                pins) replays the round's moves on its list in ordering
-//                order (plus, for REF, the commit of the part vector and the
-//                source-part sizes in extra blocks)
-#include "fp_internal.h"
+//                part vector and sizes; the admitted stamp their nets
+//   k_apply      replays the round's moves on the lists (and masks) of the
+//                stamped nets in ordering order: a lane per net of at most 8
+//                pins, a wavefront per larger one (plus, for REF, the commit of
+//                the part vector and the source-part sizes in extra blocks).
+//                A stamp is a plain store; a list of the touched nets took an
+//                atomic per workgroup on one counter, about 12 ns each one
+//                after another (a 16,384-slot evaluation: 56 -> 17 us without)
+#include "fp_masks.h"
 
 namespace fpe {
 namespace {
@@ -46,8 +48,11 @@ constexpr int LONG_TASKS = FP_LONG_TASKS;  // windows of long lists (any of the 
 constexpr int SCAN_RUN = 16;     // consecutive tiles per thread in the BAL scan
 constexpr int APPLY_BLOCK = 256;
 constexpr int SMALL_NET = 8;     // nets of at most this many pins are replayed one per lane
-constexpr int APPLY_NET_BLOCKS = 8192;
-constexpr int APPLY_GROUP = 4;   // 64-rank windows of a net whose loads the apply issues together
+constexpr int APPLY_NET_BLOCKS = 2048;  // all resident at 8 waves per SIMD (8,192 cost 8 to 18%)
+constexpr int APPLY_NETS = 512;    // nets per block of the apply at most
+constexpr unsigned HUGE_NET = 256;  // nets of at least this many pins are replayed first
+constexpr int APPLY_GROUP = 4;     // 64-rank windows of a net whose loads the apply issues together
+constexpr int APPLY_TOGETHER = 8;  // moves of a window tried together (wave_ilist_moves)
 
 struct EvalArgs {
   const unsigned* vtx_ptr;
@@ -68,18 +73,19 @@ struct EvalArgs {
   int* slot_dec;
   int* dec_out;   // nullable (fp_eval_moves)
   int* gain_out;  // nullable
-  // touched-net list of the round (nullable: no stamping)
+  // the round's tag goes to the stamps of the nets its candidates touch (nullable: no stamping)
   unsigned tag;
   unsigned* net_stamp;
-  int* touched;
-  int* tcount;
-  int* tcount_next;
-  // BAL (nullable): candidate weight per part, per (part, tile); frozen sizes copy
-  long long* cand_tot;
+  // BAL (nullable): candidate weight per (part, tile); frozen sizes copy
   int* hist;
   long long* sizes_frozen;
   // initial partition (nullable): the lowest-index part of minimum frozen size
   int* fb_out;
+  // the nets' part masks (k_tv_eval_masks)
+  const unsigned long long* masks;
+  int noe;
+  unsigned last_pin;  // the last element of vtx_nets
+  int per_wave;       // consecutive slots per wave (<= 64)
 };
 
 // slot decision of an unplaced vertex whose part the fallback assigns
@@ -163,15 +169,12 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
   unsigned* wbase = s_skey + K;
   __shared__ long long red_sz[EVAL_BLOCK / WAVE];
   __shared__ int red_ix[EVAL_BLOCK / WAVE];
-  __shared__ int s_tn[EVAL_BLOCK / WAVE + 1];
   const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
   // per wavefront: cnt[K] and first[K], each followed by 64 spare slots that
   // take the atomics of lanes past a list's end (no branch around them)
   unsigned* cnt = wbase + (size_t)wave * 2 * (size_t)(K + WAVE);
   unsigned* first = cnt + K + WAVE;
   const int spare = K + lane_id();
-  // per wavefront: the nets its accepted vertices touch, before they go to the touched list
-  WaveTouch tb{wbase + (size_t)nw * 2 * (size_t)(K + WAVE) + (size_t)wave * TOUCH_BUF, 0};
 
   // penalties of the frozen part sizes: penalty = 1 - (1.0 * size / C)  (TV/partition.cpp:103)
   long long bs = LLONG_MAX;
@@ -191,7 +194,6 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
     if (os < bs || (os == bs && oi < bi)) { bs = os; bi = oi; }
   }
   if (lane == 0) { red_sz[wave] = bs; red_ix[wave] = bi; }
-  if (blockIdx.x == 0 && threadIdx.x == 0 && a.tcount_next) *a.tcount_next = 0;
   __syncthreads();
   int fb = red_ix[0];
   {
@@ -425,77 +427,427 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
       a.slot_dec[slot] = dd;
       if (MODE == EVAL_REFINE && a.dec_out) a.dec_out[v] = d;
       if (MODE == EVAL_REFINE && a.gain_out) a.gain_out[v] = d == own ? INT_MIN : lg - (deg - (int)craw);
-      if (dd >= 0 && a.cand_tot) {
+      if (dd >= 0 && a.hist) {
         const int w = a.vwgt ? a.vwgt[v] : 1;
-        atomic_add_i64(&a.cand_tot[d], w);
         atomicAdd(&a.hist[(size_t)d * (size_t)a.ntiles + (size_t)(slot / TILE)], w);
       }
     }
-    if (accept && a.touched)
-      wave_touch_nets_staged(a.vtx_nets + vb, deg, a.tag, a.net_stamp, tb, a.touched, a.tcount);
+    if (accept && a.net_stamp) wave_stamp_nets(a.vtx_nets + vb, deg, a.tag, a.net_stamp);
     slot += stride;
     hv[0] = hv[1]; hown[0] = hown[1]; hvb[0] = hvb[1]; hdeg[0] = hdeg[1];
     hv[1] = hv[2]; hown[1] = hown[2]; hvb[1] = hvb[2]; hdeg[1] = hdeg[2];
     sg0 = sg1;
   }
-  if (a.touched) block_touch_flush(tb, a.touched, a.tcount, s_tn);
 }
 
-// BAL step 1: over-subscribed parts (candidate weight > cap - frozen size) get
-// a dense index; one block per such part scans its tile histogram (exclusive)
-// into pref and clears the histogram row.
-__global__ void __launch_bounds__(256) k_bal_scan(int* __restrict__ hist, long long* __restrict__ pref, int ntiles,
-                                                  int K, const long long* __restrict__ sizes_frozen,
-                                                  const long long* __restrict__ cand_tot, long long cap,
-                                                  int* __restrict__ over_idx, int* __restrict__ over_count) {
-  extern __shared__ __align__(16) unsigned char lds[];
-  int* s_list = reinterpret_cast<int*>(lds);  // K
-  __shared__ int s_wi[16];
-  __shared__ long long s_wl[16];
-  int base = 0;
-  for (int d0 = 0; d0 < K; d0 += (int)blockDim.x) {
-    const int d = d0 + (int)threadIdx.x;
-    const int f = (d < K && cand_tot[d] > cap - sizes_frozen[d]) ? 1 : 0;
-    int tot;
-    const int ex = block_excl_scan(f, s_wi, &tot);
-    if (d < K) {
-      if (f) s_list[base + ex] = d;
-      if (blockIdx.x == 0) over_idx[d] = f ? base + ex : -1;
-    }
-    base += tot;
+// The lowest-index part of minimum size (TV/partition.cpp:118-132), by the
+// whole wavefront.
+__device__ __forceinline__ int wave_lightest_part(const long long* __restrict__ sizes, int K) {
+  long long bs = LLONG_MAX;
+  int bi = INT_MAX;
+  for (int q = lane_id(); q < K; q += WAVE) {
+    const long long sz = sizes[q];
+    if (sz < bs || bi == INT_MAX) { bs = sz; bi = q; }
   }
-  const int nover = base;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *over_count = nover;
+  for (int off = WAVE / 2; off > 0; off >>= 1) {
+    const long long os = __shfl_xor(bs, off);
+    const int oi = __shfl_xor(bi, off);
+    if (os < bs || (os == bs && oi < bi)) { bs = os; bi = oi; }
+  }
+  return __builtin_amdgcn_readfirstlane(bi);
+}
+
+// A count as a double, by one full-rate addition: 2^52 + x has x in the low
+// word (the conversion instruction takes four times as long).
+__device__ __forceinline__ double exact_double(unsigned x) {
+  return __longlong_as_double((long long)((0x43300000ull << 32) | x)) - 4503599627370496.0;
+}
+
+// Records of nets in flight per wave: their words (2 P SGPRs each) have to fit
+// the scalar registers.
+template <int P>
+constexpr int mask_nets_in_flight() {
+  return P <= 2 ? 8 : (P <= 4 ? 4 : (P <= 6 ? 3 : 2));
+}
+
+// k_tv_eval through the nets' part masks (fp_masks.h), for K <= 64 P: lane l
+// counts parts l, l + 64, ... of the vertex in registers. Per net a record's
+// P present words come into scalar registers and are added with the lane's
+// bit as the carry-in; the penalties and counts of a lane's parts stay in
+// registers, so the sweep and the LDG scan touch no LDS. The single bit of the
+// vertex's own part comes from one word per net, a net per lane.
+// A wave takes per_wave consecutive slots: their headers are loaded a slot per
+// lane, their decisions written a slot per lane at the end. Both the vector
+// and the scalar unit are near their issue limit here, so addresses are 32-bit
+// offsets (the host checks the arrays' sizes) and everything per vertex that
+// a lane can hold is held by one.
+// The decision, the gain test and everything written are k_tv_eval's.
+template <int P, int MODE>
+__global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu(P <= 6 ? 7 : 6, P <= 6 ? 7 : 6))) k_tv_eval_masks(EvalArgs a) {
+  constexpr int NB = mask_nets_in_flight<P>();
+  constexpr int CH = (WAVE / NB) * NB;  // nets per chunk: no batch reaches past the wave's last lane
+  constexpr unsigned ROW = 16u * P;     // bytes of a record
+  __shared__ double s_pen[64 * P];
+  __shared__ unsigned s_skey[64 * P];
+  const int K = a.K;
+  const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
+  const int s0 = ((int)blockIdx.x * nw + wave) * a.per_wave;
+  const int ns = min(a.per_wave, a.nslots - s0);
+
+  // lane i: slot s0 + i's vertex, its part and its net range
+  int v_l = 0, own_l = 0;
+  unsigned vb_l = 0, ve_l = 0;
+  if (lane < ns) {
+    const int z = a.r0 + s0 + lane;
+    v_l = a.order ? a.order[z] : z;
+    own_l = a.part[v_l];
+    vb_l = a.vtx_ptr[v_l];
+    ve_l = a.vtx_ptr[v_l + 1];
+  }
+  // penalties of the frozen part sizes: penalty = 1 - (1.0 * size / C)  (TV/partition.cpp:103)
+  for (int q = (int)threadIdx.x; q < 64 * P; q += (int)blockDim.x) {
+    const long long sz = q < K ? a.sizes[q] : 0;
+    s_skey[q] = size_key(sz);
+    s_pen[q] = q < K ? 1.0 - ((double)sz / a.C) : 0.0;
+    if (blockIdx.x == 0 && a.sizes_frozen && q < K) a.sizes_frozen[q] = sz;
+  }
+  if (MODE != EVAL_REFINE && blockIdx.x == 0 && wave == 0) {
+    const int fb = wave_lightest_part(a.sizes, K);
+    if (lane == 0) *a.fb_out = fb;
+  }
   __syncthreads();
-  // each thread scans SCAN_RUN consecutive tiles, loaded together, so a
-  // 4096-tile row takes one round trip to memory and one block scan
-  for (int o = (int)blockIdx.x; o < nover; o += (int)gridDim.x) {
-    const int d = s_list[o];
+  // per part of the lane: penalty, size key, and the part's number with bit 16
+  // set where its size lies within the bands (compared as size keys, the same order)
+  double pen[P];
+  unsigned skey[P];
+  int pid[P];
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    pen[u] = s_pen[u * WAVE + lane];
+    skey[u] = s_skey[u * WAVE + lane];
+    const bool in = skey[u] <= size_key(a.max_pw) && (MODE != EVAL_REFINE || skey[u] >= size_key(a.min_pw));
+    pid[u] = (u * WAVE + lane) | (in ? 1 << 16 : 0);
+  }
+  auto load_row = [&](unsigned off, unsigned long long (&w)[P]) {
+#pragma unroll
+    for (int u = 0; u < P; u++) w[u] = uniform_load_at<unsigned long long>(a.masks, off, u);
+  };
+  auto votes = [&](unsigned long long (&w)[P]) {
+    if (MODE == EVAL_INIT_CN) {  // only nets of one part vote
+      int c = 0;
+#pragma unroll
+      for (int u = 0; u < P; u++) c += (int)__popcll(w[u]);
+#pragma unroll
+      for (int u = 0; u < P; u++) w[u] = c == 1 ? w[u] : 0ull;
+    }
+  };
+  const char* masks = reinterpret_cast<const char*>(a.masks);
+  // lane j: net j of slot s0 + i's vertex; past its last net some other net.
+  // Loaded a vertex ahead, by every lane (a load that a branch may skip could
+  // only be waited for together with the ones after it).
+  const char* nets = reinterpret_cast<const char*>(a.vtx_nets);
+  auto load_nets = [&](int i) -> unsigned {
+    const unsigned k = (unsigned)__builtin_amdgcn_readlane((int)vb_l, i) + (unsigned)lane;
+    return *reinterpret_cast<const unsigned*>(nets + min(k, a.last_pin) * 4u);
+  };
+
+  int dec_l = -1;  // lane i: slot s0 + i's decision: a part, -1 (none) or SLOT_FALLBACK
+  // the headers have arrived before the loop (else its first wait would take in the loads of every turn)
+  asm volatile("" ::"v"(own_l), "v"(vb_l), "v"(ve_l));
+  unsigned id = ns > 0 ? load_nets(0) : 0u;
+  for (int i = 0; i < ns; i++) {
+    const unsigned id_next = load_nets(min(i + 1, ns - 1));
+    const int own = __builtin_amdgcn_readlane(own_l, i);
+    const unsigned vb = (unsigned)__builtin_amdgcn_readlane((int)vb_l, i);
+    const int deg = (int)((unsigned)__builtin_amdgcn_readlane((int)ve_l, i) - vb);
+    const unsigned id0 = id;
+    id = id_next;
+    if (MODE != EVAL_REFINE && own >= 0) continue;  // already placed
+
+    unsigned cnt[P];
+#pragma unroll
+    for (int u = 0; u < P; u++) cnt[u] = 0;
+    int lg = 0;  // leave gain: nets where v is the only pin of its part (TV/partition.cpp:365-368)
+    // nn <= CH nets of the vertex, lane j's the one with id ids
+    auto count_nets = [&](unsigned ids, int nn) {
+      const unsigned off = (lane < nn ? ids : (unsigned)a.noe) * ROW;  // past the last net: the zero record
+      unsigned sw = 0;
+      if (MODE == EVAL_REFINE)
+        sw = *reinterpret_cast<const unsigned*>(masks + (8u * P + 4u * (unsigned)(own >> 5)) + off);
+      // a batch's loads are all issued before the first is waited for
+      auto batch = [&](int j0, int n) {
+        unsigned long long w[NB][P];
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+          if (j < n) load_row((unsigned)__builtin_amdgcn_readlane((int)off, j0 + j), w[j]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+          if (j < n) {
+            votes(w[j]);
+#pragma unroll
+            for (int u = 0; u < P; u++) add_lane_bit(cnt[u], w[j][u]);
+          }
+      };
+      int j0 = 0;
+      for (; j0 + NB <= nn; j0 += NB) batch(j0, NB);
+      if (j0 < nn) batch(j0, nn - j0);
+      if (MODE == EVAL_REFINE) lg += (int)__popcll(__ballot(((sw >> (own & 31)) & 1u) != 0u));
+    };
+    count_nets(id0, min(deg, CH));
+    for (int c0 = CH; c0 < deg; c0 += CH)
+      count_nets(*reinterpret_cast<const unsigned*>(nets + min(vb + (unsigned)(c0 + lane), a.last_pin) * 4u),
+                 min(deg - c0, CH));
+    // scores (TV/partition.cpp:98-116), scores[part_id]-- (:345). A part in
+    // none of the nets scores 0 (own is in all of them; a vertex without nets
+    // keeps its 0), which is no candidate.
+    double sc[P];
+    double best = 0;
+    const int mine = (deg > 0 ? own : -1) - lane;  // 64 u where own is this lane's part u
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      const unsigned adj = MODE == EVAL_REFINE ? sub_lane_bit(cnt[u], __ballot(mine == u * WAVE)) : cnt[u];
+      sc[u] = exact_double(adj) * pen[u];
+      best = fmax(best, sc[u]);
+    }
+    // the wave's best: positive doubles order like their bit patterns, the
+    // high words first and the low words only where several lanes share it
+    const unsigned long long bb = (unsigned long long)__double_as_longlong(best);
+    const unsigned hi = (unsigned)(bb >> 32);
+    const unsigned mh = wave_max_u32(hi);
+    int d = -1;
+    unsigned craw = 0;
+    bool in_band = false;
+    if (mh != 0 || __ballot(bb != 0ull) != 0ull) {
+      const unsigned long long hl = __ballot(hi == mh);
+      unsigned ml;
+      if (__popcll(hl) == 1)
+        ml = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)bb, __ffsll((long long)hl) - 1);
+      else
+        ml = wave_max_u32(hi == mh ? (unsigned)bb : 0u);
+      const double m1 = __longlong_as_double((long long)(((unsigned long long)mh << 32) | ml));
+      unsigned long long tie[P];
+      int ntie = 0;
+#pragma unroll
+      for (int u = 0; u < P; u++) {
+        tie[u] = __ballot(sc[u] == m1);
+        ntie += (int)__popcll(tie[u]);
+      }
+      if (ntie > 1) {
+        // equal scores: the lightest part
+        unsigned k2 = ~0u;
+#pragma unroll
+        for (int u = 0; u < P; u++) k2 = min(k2, sc[u] == m1 ? skey[u] : ~0u);
+        const unsigned m2 = wave_min_u32(k2);
+        ntie = 0;
+#pragma unroll
+        for (int u = 0; u < P; u++) {
+          tie[u] &= __ballot(skey[u] == m2);
+          ntie += (int)__popcll(tie[u]);
+        }
+        if (ntie > 1) {
+          // equal sizes too: the part the reference's scan meets first, i.e.
+          // of the first net that lists one of them, the earliest in its list
+          // (TV/partition.cpp:318-338)
+          for (int t = 0; t < deg; t++) {
+            unsigned long long w[P];
+            load_row(uniform_load(a.vtx_nets + (vb + (unsigned)t)) * ROW, w);
+            votes(w);
+            int c = 0;
+#pragma unroll
+            for (int u = 0; u < P; u++) {
+              w[u] &= tie[u];
+              c += (int)__popcll(w[u]);
+            }
+            if (c == 0) continue;
+            if (c > 1) {
+              const unsigned seg = uniform_load(a.vtx_seg + (vb + (unsigned)t));
+              const int L = (int)a.ev[seg];
+              for (int t0 = 0; t0 < L; t0 += WAVE) {
+                const int e = t0 + lane;
+                const int q = e < L ? (int)(a.ev[seg + 1u + (unsigned)e] & ~EV_SINGLE) : 0;
+                unsigned long long x = 0;
+#pragma unroll
+                for (int u = 0; u < P; u++) x = (q >> 6) == u ? w[u] : x;
+                const unsigned long long hit = __ballot(e < L && ((x >> (q & (WAVE - 1))) & 1ull));
+                if (hit) {
+                  const int f = __builtin_amdgcn_readlane(q, __ffsll((long long)hit) - 1);
+#pragma unroll
+                  for (int u = 0; u < P; u++) w[u] = (f >> 6) == u ? 1ull << (f & (WAVE - 1)) : 0ull;
+                  break;
+                }
+              }
+            }
+#pragma unroll
+            for (int u = 0; u < P; u++) tie[u] = w[u];
+            break;
+          }
+        }
+      }
+      // one bit is left: its part and count, from the lane that holds them
+      unsigned long long any = 0;
+      int px = 0;
+      unsigned cx = 0;
+#pragma unroll
+      for (int u = 0; u < P; u++) {
+        any |= tie[u];
+        const bool t = __builtin_amdgcn_inverse_ballot_w64(tie[u]);
+        px = t ? pid[u] : px;
+        cx = t ? cnt[u] : cx;
+      }
+      const int l = __ffsll((long long)any) - 1;
+      const int pl = __builtin_amdgcn_readlane(px, l);
+      craw = (unsigned)__builtin_amdgcn_readlane((int)cx, l);
+      d = pl & 0xFFFF;
+      in_band = (pl >> 16) != 0;
+    }
+    const bool none = d < 0;  // no part above score 0: the fallback
+    int dd;
+    if (MODE == EVAL_REFINE) {
+      if (none) {
+        d = wave_lightest_part(a.sizes, K);
+        int px = 0;
+        unsigned cx = 0;
+#pragma unroll
+        for (int u = 0; u < P; u++) {
+          px = (d >> 6) == u ? pid[u] : px;
+          cx = (d >> 6) == u ? cnt[u] : cx;
+        }
+        in_band = (__builtin_amdgcn_readlane(px, d & (WAVE - 1)) >> 16) != 0;
+        craw = (unsigned)__builtin_amdgcn_readlane((int)cx, d & (WAVE - 1));
+      }
+      // outside the bands the vertex stays (TV/partition.cpp:135-143)
+      const int al = deg - (int)craw;  // arrival loss: nets of v lacking d (TV/partition.cpp:369-377)
+      const bool accept = in_band && d != own && lg >= al;  // TV/partition.cpp:380
+      dd = accept ? d : -1;
+      if (accept && a.net_stamp) {
+        if (lane < min(deg, CH)) a.net_stamp[id0] = a.tag;
+        if (deg > CH) wave_stamp_nets(a.vtx_nets + (vb + (unsigned)CH), deg - CH, a.tag, a.net_stamp);
+      }
+    } else {
+      // an unplaced vertex with no part above score 0, or whose choice is
+      // above the band, takes its turn in the fallback
+      dd = none || !in_band ? SLOT_FALLBACK : d;
+    }
+    dec_l = lane == i ? dd : dec_l;
+  }
+  if (lane < ns) {
+    a.slot_own[s0 + lane] = own_l;
+    a.slot_dec[s0 + lane] = dec_l;
+    if (dec_l >= 0 && a.hist) {
+      const int w = a.vwgt ? a.vwgt[v_l] : 1;
+      atomicAdd(&a.hist[(size_t)dec_l * (size_t)a.ntiles + (size_t)((s0 + lane) / TILE)], w);
+    }
+  }
+}
+
+// the instance of k_tv_eval_masks for K parts
+template <int MODE>
+void (*eval_masks_kernel(int K))(EvalArgs) {
+  switch (mask_words(K)) {
+    case 1: return k_tv_eval_masks<1, MODE>;
+    case 2: return k_tv_eval_masks<2, MODE>;
+    case 3: return k_tv_eval_masks<3, MODE>;
+    case 4: return k_tv_eval_masks<4, MODE>;
+    case 5: return k_tv_eval_masks<5, MODE>;
+    case 6: return k_tv_eval_masks<6, MODE>;
+    case 7: return k_tv_eval_masks<7, MODE>;
+    default: return k_tv_eval_masks<8, MODE>;
+  }
+}
+
+// BAL step 1, per part: its candidates' weight is its row of the tile
+// histogram. A part whose candidates exceed cap - size is over-subscribed:
+// over[d] is set and pref's row d receives the exclusive prefix sums of the
+// tiles. The row is cleared for the next round. Rows of up to
+// SCAN_WAVE_TILES tiles are taken by one wavefront each, longer ones by a block,
+// whose threads load SCAN_RUN consecutive tiles together: a 4096-tile row
+// takes one round trip to memory and one block scan. Summing the rows here
+// spares the evaluation a 64-bit atomic per candidate on one of K words.
+constexpr int SCAN_WAVE_TILES = 16 * WAVE;
+
+template <bool WAVE_ROWS>
+__global__ void __launch_bounds__(256) k_bal_scan(int* __restrict__ hist, long long* __restrict__ pref, int ntiles,
+                                                  int K, const long long* __restrict__ sizes_frozen, long long cap,
+                                                  int* __restrict__ over) {
+  __shared__ long long s_wl[16];
+  const int lane = lane_id();
+  if (WAVE_ROWS) {
+    const int nw = (int)(blockDim.x / WAVE);
+    for (int d = (int)blockIdx.x * nw + wave_id(); d < K; d += (int)gridDim.x * nw) {
+      int* row = hist + (size_t)d * (size_t)ntiles;
+      int x[SCAN_WAVE_TILES / WAVE];
+      int sum = 0;  // total weights fit an int
+#pragma unroll
+      for (int p = 0; p < SCAN_WAVE_TILES / WAVE; p++) {
+        const int t = p * WAVE + lane;
+        x[p] = t < ntiles ? row[t] : 0;
+      }
+#pragma unroll
+      for (int p = 0; p < SCAN_WAVE_TILES / WAVE; p++) sum += x[p];
+      const int tot = wave_sum(sum);
+      const bool ov = tot > cap - sizes_frozen[d];
+      if (lane == 0) over[d] = ov ? 1 : 0;
+      if (tot == 0 && !ov) continue;
+      int acc = 0;
+#pragma unroll
+      for (int p = 0; p < SCAN_WAVE_TILES / WAVE; p++) {
+        const int t = p * WAVE + lane;
+        if (ov && p * WAVE < ntiles) {
+          const int incl = wave_incl_scan(x[p]);
+          if (t < ntiles) pref[(size_t)d * (size_t)ntiles + (size_t)t] = acc + (incl - x[p]);
+          acc += __builtin_amdgcn_readlane(incl, WAVE - 1);
+        }
+        if (t < ntiles && x[p]) row[t] = 0;
+      }
+    }
+    return;
+  }
+  const int step = (int)blockDim.x * SCAN_RUN;
+  for (int d = (int)blockIdx.x; d < K; d += (int)gridDim.x) {
     int* row = hist + (size_t)d * (size_t)ntiles;
-    long long* out = pref + (size_t)o * (size_t)ntiles;
-    long long carry = 0;
-    for (int t0 = 0; t0 < ntiles; t0 += (int)blockDim.x * SCAN_RUN) {
+    long long* out = pref + (size_t)d * (size_t)ntiles;
+    int x[SCAN_RUN];
+    auto load = [&](int t0) -> long long {
       const int tb = t0 + (int)threadIdx.x * SCAN_RUN;
-      int x[SCAN_RUN];
+      long long run = 0;
 #pragma unroll
       for (int p = 0; p < SCAN_RUN; p++) {
         const int v = row[min(tb + p, ntiles - 1)];
         x[p] = tb + p < ntiles ? v : 0;
       }
-      long long run = 0;
 #pragma unroll
       for (int p = 0; p < SCAN_RUN; p++) run += x[p];
-      long long tot;
-      long long acc = carry + block_excl_scan(run, s_wl, &tot);
+      return run;
+    };
+    long long sum = 0, first = 0;
+    for (int t0 = 0; t0 < ntiles; t0 += step) {
+      const long long r = load(t0);
+      if (t0 == 0) first = r;
+      sum += r;
+    }
+    long long tot;
+    (void)block_excl_scan(sum, s_wl, &tot);
+    const bool ov = tot > cap - sizes_frozen[d];
+    if (threadIdx.x == 0) over[d] = ov ? 1 : 0;
+    if (tot == 0 && !ov) continue;
+    long long carry = 0;
+    for (int t0 = 0; t0 < ntiles; t0 += step) {
+      const long long run = ntiles > step ? load(t0) : first;
+      const int tb = t0 + (int)threadIdx.x * SCAN_RUN;
+      if (ov) {
+        long long chunk;
+        long long acc = carry + block_excl_scan(run, s_wl, &chunk);
 #pragma unroll
-      for (int p = 0; p < SCAN_RUN; p++) {
-        if (tb + p < ntiles) {
-          out[tb + p] = acc;
-          row[tb + p] = 0;
+        for (int p = 0; p < SCAN_RUN; p++) {
+          if (tb + p < ntiles) out[tb + p] = acc;
+          acc += x[p];
         }
-        acc += x[p];
+        carry += chunk;
       }
-      carry += tot;
+#pragma unroll
+      for (int p = 0; p < SCAN_RUN; p++)
+        if (tb + p < ntiles && x[p]) row[tb + p] = 0;
     }
   }
 }
@@ -503,13 +855,12 @@ __global__ void __launch_bounds__(256) k_bal_scan(int* __restrict__ hist, long l
 // Initial partition, between the evaluation and the admission (one block):
 // the j-th fallback slot of the sub-round, in slot order, takes part
 // (fb + j) mod K, fb the lowest-index part of minimum frozen size, and its
-// weight joins the candidate totals and tile histogram.
+// weight joins the tile histogram.
 constexpr int FALLBACK_RUN = 16;  // consecutive slots per thread in k_init_fallback
 
 __global__ void __launch_bounds__(1024) k_init_fallback(int* __restrict__ slot_dec, const int* __restrict__ order,
                                                         const int* __restrict__ vwgt, int r0, int nslots, int ntiles,
-                                                        int K, const int* __restrict__ fb_in,
-                                                        long long* __restrict__ cand_tot, int* __restrict__ hist) {
+                                                        int K, const int* __restrict__ fb_in, int* __restrict__ hist) {
   __shared__ int s_wi[16];
   const int fb = *fb_in;
   int carry = 0;
@@ -535,7 +886,6 @@ __global__ void __launch_bounds__(1024) k_init_fallback(int* __restrict__ slot_d
         slot_dec[slot] = d;
         const int z = r0 + slot;
         const int w = vwgt ? vwgt[order ? order[z] : z] : 1;
-        atomic_add_i64(&cand_tot[d], w);
         atomicAdd(&hist[(size_t)d * (size_t)ntiles + (size_t)(slot / TILE)], w);
       }
     carry += tot;
@@ -546,24 +896,26 @@ __global__ void __launch_bounds__(1024) k_init_fallback(int* __restrict__ slot_d
 // d is admitted iff frozen_size[d] + (weight of earlier candidates into d) + w
 // <= cap (first_free: or it is the first candidate into d); every other
 // candidate is admitted. Commits part vector and sizes of admitted moves (a
-// vertex without a part, own -1, only adds to its new part's size); clears
-// the tile's histogram cells of non-over parts. AGG:
+// vertex without a part, own -1, only adds to its new part's size). AGG:
 // the block sums its size changes per part in LDS first, so that sizes takes
 // one atomic per part and block (same-address atomics from every wave would
-// queue at one L2 slice).
+// queue at one L2 slice: about 12 ns each, so the blocks are as large as they
+// can be).
+constexpr int ADMIT_BLOCK = 1024;
+
 template <bool AGG>
-__global__ void __launch_bounds__(256) k_bal_admit(int* __restrict__ slot_dec, const int* __restrict__ slot_own,
+__global__ void __launch_bounds__(ADMIT_BLOCK) k_bal_admit(int* __restrict__ slot_dec, const int* __restrict__ slot_own,
                                                    const int* __restrict__ order, const int* __restrict__ vwgt,
                                                    int r0, int nslots, int ntiles, int K,
                                                    const long long* __restrict__ sizes_frozen, long long cap,
-                                                   bool first_free, const int* __restrict__ over_idx,
-                                                   const int* __restrict__ over_count,
-                                                   const long long* __restrict__ pref, int* __restrict__ hist,
-                                                   int* __restrict__ part, long long* __restrict__ sizes,
-                                                   long long* __restrict__ cand_tot,
-                                                   unsigned long long* __restrict__ moves) {
+                                                   bool first_free, const int* __restrict__ over,
+                                                   const long long* __restrict__ pref, int* __restrict__ part,
+                                                   long long* __restrict__ sizes,
+                                                   unsigned long long* __restrict__ moves,
+                                                   const unsigned* __restrict__ vtx_ptr,
+                                                   const unsigned* __restrict__ vtx_nets, unsigned tag,
+                                                   unsigned* __restrict__ net_stamp) {
   const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
-  const int nover = *over_count;
   // the block's admitted moves, added to the global count once per block
   // (same-address atomics from every wave would queue at one L2 slice)
   __shared__ unsigned long long s_moves;
@@ -574,8 +926,6 @@ __global__ void __launch_bounds__(256) k_bal_admit(int* __restrict__ slot_dec, c
   if (AGG)
     for (int d = (int)threadIdx.x; d < K; d += (int)blockDim.x) s_dsz[d] = 0;
   __syncthreads();
-  if (blockIdx.x == 0)
-    for (int d = (int)threadIdx.x; d < K; d += (int)blockDim.x) cand_tot[d] = 0;
   for (int tile = (int)blockIdx.x * nw + wave; tile < ntiles; tile += (int)gridDim.x * nw) {
     const int slot = tile * TILE + lane;
     int d = -1, v = -1;
@@ -586,9 +936,9 @@ __global__ void __launch_bounds__(256) k_bal_admit(int* __restrict__ slot_dec, c
       v = order ? order[z] : z;
       w = vwgt ? vwgt[v] : 1;
     }
-    const int o = (d >= 0 && nover > 0) ? over_idx[d] : -1;
+    const bool o = d >= 0 && over[d] != 0;
     bool adm = d >= 0;
-    if (__ballot(o >= 0)) {
+    if (__ballot(o)) {
       // weight of earlier candidates into the same part within the tile
       long long pre = 0;
       const int wi = (int)w;  // vertex weights are int
@@ -596,15 +946,12 @@ __global__ void __launch_bounds__(256) k_bal_admit(int* __restrict__ slot_dec, c
         const int dj = __builtin_amdgcn_readlane(d, j), wj = __builtin_amdgcn_readlane(wi, j);
         if (j < lane && dj == d) pre += wj;
       }
-      if (o >= 0) {
-        const long long before = pref[(size_t)o * (size_t)ntiles + (size_t)tile] + pre;
+      if (o) {
+        const long long before = pref[(size_t)d * (size_t)ntiles + (size_t)tile] + pre;
         adm = sizes_frozen[d] + before + w <= cap || (first_free && before == 0);
       }
     }
-    if (d >= 0) {
-      if (o < 0) hist[(size_t)d * (size_t)ntiles + (size_t)tile] = 0;
-      if (!adm) slot_dec[slot] = -1;
-    }
+    if (d >= 0 && !adm) slot_dec[slot] = -1;
     if (adm) {
       part[v] = d;
       const int own = slot_own[slot];
@@ -615,6 +962,27 @@ __global__ void __launch_bounds__(256) k_bal_admit(int* __restrict__ slot_dec, c
         if (own >= 0) atomic_add_i64(&sizes[own], -w);
         atomic_add_i64(&sizes[d], w);
       }
+    }
+    // the admitted moves' nets get the round's tag: by the move's lane, four
+    // at a time, or by the wave for a vertex of more than 64 nets
+    unsigned vb = 0, ve = 0;
+    if (adm) {
+      vb = vtx_ptr[v];
+      ve = vtx_ptr[v + 1];
+    }
+    const bool hub = adm && ve - vb > (unsigned)WAVE;
+    if (adm && !hub)
+      for (unsigned j = vb; j < ve; j += 4) {
+        unsigned n[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) n[u] = vtx_nets[min(j + (unsigned)u, ve - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) net_stamp[n[u]] = tag;
+      }
+    for (unsigned long long hm = __ballot(hub); hm; hm &= hm - 1) {
+      const int l = __ffsll((long long)hm) - 1;
+      const unsigned b = (unsigned)__builtin_amdgcn_readlane((int)vb, l);
+      wave_stamp_nets(vtx_nets + b, (int)((unsigned)__builtin_amdgcn_readlane((int)ve, l) - b), tag, net_stamp);
     }
     const unsigned long long am = __ballot(adm);
     if (lane == 0 && am) atomicAdd(&s_moves, (unsigned long long)__popcll(am));
@@ -633,10 +1001,15 @@ struct ApplyArgs {
   const int* apply_pins;
   const int* slot_own;
   const int* slot_dec;
-  const int* touched;
-  const int* tcount;
+  const unsigned* net_stamp;  // the nets stamped with the round's tag are touched
+  unsigned tag;
+  int noe, per_block;         // each block takes per_block consecutive nets
+  int lane_words;             // LDS words per lane of the small nets' replay
+  int wave_bytes;             // LDS bytes per wave
   unsigned* ent;
   unsigned short* ev;
+  unsigned long long* masks;  // nullable: the nets' part masks, kept in step with the lists
+  int mask_words;
   int K, pb;
   unsigned pmask;
   int r0, r1;
@@ -655,19 +1028,13 @@ struct ApplyArgs {
 // (TV/partition.cpp:818-830: the destination's size is left unchanged).
 // INDEXED: each wave keeps a part -> position index of its list in LDS (2
 // bytes per part after the lists), for K where it fits.
-// bytes of the per-wave lists (and indexes) at the start of the apply's LDS
-template <bool INDEXED>
-__host__ __device__ __forceinline__ size_t apply_list_bytes(int K, int nw) {
-  return (size_t)nw * (size_t)K * (sizeof(unsigned) + (INDEXED ? sizeof(unsigned short) : 0));
-}
-
 // One lane replays the round's moves on a net of at most SMALL_NET pins, in
-// the rank order of its pins, on a copy of the list in the lane's own LDS
-// slots: the same edits, in the same order, as the wavefront replay (remove
-// = decrement or swap-with-last, add = increment or append). The list and the
-// ranks load together, then the moves of the ranked pins.
-__device__ __forceinline__ void lane_replay_small(const ApplyArgs& a, int n, unsigned s, unsigned e, unsigned* my) {
-  const unsigned np = e - s;
+// the rank order of its pins, on a copy of the list in its registers: the
+// same edits, in the same order, as the wavefront replay (remove = decrement
+// or swap-with-last, add = increment or append). The list and the ranks load
+// together, then the moves of the ranked pins. A list in the lane's LDS words
+// instead waited out an LDS read per entry looked at (13 to 25 us for 64 nets).
+__device__ __forceinline__ void lane_replay_small(const ApplyArgs& a, int n, unsigned s, unsigned np, unsigned* my) {
   const unsigned seg = s + (unsigned)n;
   int r[SMALL_NET];
   unsigned x[SMALL_NET + 1];
@@ -680,54 +1047,121 @@ __device__ __forceinline__ void lane_replay_small(const ApplyArgs& a, int n, uns
   for (int i = 0; i < SMALL_NET; i++) {
     const bool in = r[i] >= a.r0 && r[i] < a.r1;
     dd[i] = in ? a.slot_dec[r[i] - a.r0] : -1;
-    oo[i] = in ? a.slot_own[r[i] - a.r0] : 0;
+    oo[i] = in ? a.slot_own[r[i] - a.r0] : -1;
   }
   int L = (int)x[0];
+  int key[SMALL_NET];  // part of each entry, -1 past the list
+  int cnt[SMALL_NET];
 #pragma unroll
-  for (int t = 0; t < SMALL_NET; t++)
-    if (t < L) my[t] = x[t + 1];
+  for (int t = 0; t < SMALL_NET; t++) {
+    key[t] = t < L ? (int)(x[t + 1] & a.pmask) : -1;
+    cnt[t] = (int)(x[t + 1] >> a.pb);
+  }
   bool any = false;
-#pragma unroll
-  for (int i = 0; i < SMALL_NET; i++) any |= dd[i] >= 0;
-  if (!any) return;
-  const unsigned inc = 1u << a.pb;
 #pragma unroll
   for (int i = 0; i < SMALL_NET; i++) {
     if (dd[i] < 0) continue;
+    any = true;
     const int p = oo[i], q = dd[i];
-    int jp = -1;
-    for (int t = 0; t < L; t++)
-      if ((int)(my[t] & a.pmask) == p) jp = t;
-    if (jp >= 0) {
-      const unsigned y = my[jp];
-      if ((y >> a.pb) > 1u) {
-        my[jp] = y - inc;
-      } else {
-        my[jp] = my[L - 1];
-        L--;
-      }
+    // the last entry, should it have to fill p's place
+    int lk = -1, lc = 0;
+#pragma unroll
+    for (int t = 0; t < SMALL_NET; t++) {
+      lk = t == L - 1 ? key[t] : lk;
+      lc = t == L - 1 ? cnt[t] : lc;
     }
-    int jq = -1;
-    for (int t = 0; t < L; t++)
-      if ((int)(my[t] & a.pmask) == q) jq = t;
-    if (jq >= 0) {
-      my[jq] += inc;
-    } else {
-      my[L] = inc | (unsigned)q;
-      L++;
+    bool gone = false;
+#pragma unroll
+    for (int t = 0; t < SMALL_NET; t++) {
+      const bool hit = p >= 0 && key[t] == p;
+      const bool last = hit && cnt[t] == 1;
+      gone |= last;
+      key[t] = last ? lk : key[t];
+      cnt[t] = last ? lc : cnt[t] - (hit ? 1 : 0);
     }
+    L -= gone ? 1 : 0;
+    bool found = false;
+#pragma unroll
+    for (int t = 0; t < SMALL_NET; t++) {
+      key[t] = gone && t == L ? -1 : key[t];
+      const bool hit = key[t] == q;
+      found |= hit;
+      cnt[t] += hit ? 1 : 0;
+    }
+#pragma unroll
+    for (int t = 0; t < SMALL_NET; t++) {
+      key[t] = !found && t == L ? q : key[t];
+      cnt[t] = !found && t == L ? 1 : cnt[t];
+    }
+    L += found ? 0 : 1;
   }
-  for (int t = 0; t < L; t++) {
-    const unsigned y = my[t];
-    a.ent[seg + 1 + (unsigned)t] = y;
-    a.ev[seg + 1 + (unsigned)t] = ev_word(y, a.pb, a.pmask);
+  if (!any) return;
+  unsigned y[SMALL_NET];
+#pragma unroll
+  for (int t = 0; t < SMALL_NET; t++) {
+    y[t] = ((unsigned)cnt[t] << a.pb) | (unsigned)key[t];
+    if (t < L) {
+      a.ent[seg + 1 + (unsigned)t] = y[t];
+      a.ev[seg + 1 + (unsigned)t] = ev_word(y[t], a.pb, a.pmask);
+    }
   }
   a.ent[seg] = (unsigned)L;
   a.ev[seg] = (unsigned short)L;
+  if (a.masks) lane_store_masks(y, L, a.pb, a.pmask, a.mask_words, my, a.masks + (size_t)n * (size_t)(2 * a.mask_words));
+}
+
+// One wavefront replays the round's moves (lane l: dd >= 0, the part its pin
+// moves to, and oo, the part it leaves) on a net of at most 64 pins, lane t
+// holding entry t of the list: an edit is a few ballots and lane writes, with
+// no LDS.
+__device__ __forceinline__ void wave_replay_medium(const ApplyArgs& a, int n, unsigned s, int L0, unsigned x, int dd,
+                                                   int oo, unsigned* words) {
+  const int lane = lane_id();
+  const unsigned seg = s + (unsigned)n;
+  int L = L0;
+  int key = lane < L ? (int)(x & a.pmask) : -1;
+  unsigned cnt = x >> a.pb;
+  for (unsigned long long m = __ballot(dd >= 0); m; m &= m - 1) {
+    const int l = __ffsll((long long)m) - 1;
+    const int p = __builtin_amdgcn_readlane(oo, l), q = __builtin_amdgcn_readlane(dd, l);
+    const unsigned long long mp = __ballot(key == p && p >= 0);
+    if (mp) {
+      const int jp = __ffsll((long long)mp) - 1;
+      if (__builtin_amdgcn_readlane((int)cnt, jp) > 1) {
+        cnt = sub_lane_bit(cnt, mp);
+      } else {
+        // the last entry takes p's place
+        L--;
+        const int lk = __builtin_amdgcn_readlane(key, L), lc = __builtin_amdgcn_readlane((int)cnt, L);
+        key = lane == jp ? lk : key;
+        cnt = lane == jp ? (unsigned)lc : cnt;
+        key = lane == L ? -1 : key;
+      }
+    }
+    const unsigned long long mq = __ballot(key == q);
+    if (mq) {
+      add_lane_bit(cnt, mq);
+    } else {
+      key = lane == L ? q : key;
+      cnt = lane == L ? 1u : cnt;
+      L++;
+    }
+  }
+  const unsigned y = (cnt << a.pb) | (unsigned)key;
+  if (lane < L) {
+    a.ent[seg + 1 + (unsigned)lane] = y;
+    a.ev[seg + 1 + (unsigned)lane] = ev_word(y, a.pb, a.pmask);
+  }
+  if (lane == 0) {
+    a.ent[seg] = (unsigned)L;
+    a.ev[seg] = (unsigned short)L;
+  }
+  if (a.masks) wave_store_entry_masks(lane < L, (unsigned)key, cnt, a.mask_words, words,
+                                      a.masks + (size_t)n * (size_t)(2 * a.mask_words));
 }
 
 template <bool INDEXED>
-__global__ void __launch_bounds__(APPLY_BLOCK) k_apply(ApplyArgs a) {
+__global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) k_apply(ApplyArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
   if ((int)blockIdx.x >= a.net_blocks) {
@@ -745,30 +1179,115 @@ __global__ void __launch_bounds__(APPLY_BLOCK) k_apply(ApplyArgs a) {
     block_count_add(a.moves, mv);
     return;
   }
-  unsigned* list = reinterpret_cast<unsigned*>(lds) + (size_t)wave * (size_t)a.K;
-  unsigned short* at = reinterpret_cast<unsigned short*>(reinterpret_cast<unsigned*>(lds) + (size_t)nw * (size_t)a.K) +
-                       (size_t)wave * (size_t)a.K;
-  // per lane: SMALL_NET + 1 words (the odd stride keeps the lanes on distinct banks)
-  unsigned* my = reinterpret_cast<unsigned*>(lds + apply_list_bytes<INDEXED>(a.K, nw)) +
-                 (size_t)(wave * WAVE + lane) * (size_t)(SMALL_NET + 1);
+  // the wave's own region: first the lanes' words of their mask records (an
+  // odd number each, which keeps them on distinct banks), then a net's
+  unsigned char* mem = lds + (size_t)wave * (size_t)a.wave_bytes;
+  unsigned* my = reinterpret_cast<unsigned*>(mem) + (size_t)lane * (size_t)a.lane_words;
+  unsigned* list = reinterpret_cast<unsigned*>(mem);
+  unsigned short* at = reinterpret_cast<unsigned short*>(list + a.K);
+  __shared__ unsigned s_words[APPLY_BLOCK / WAVE][4 * MASK_PMAX];
+  unsigned* words = s_words[wave];
+  __shared__ int s_cnt[4];  // touched small nets, other nets, nets handed out, huge nets
+  __shared__ unsigned short s_net[APPLY_NETS];  // the small ones from the front, the others from the back
+  __shared__ unsigned s_start[APPLY_NETS], s_len[APPLY_NETS];
+  __shared__ unsigned short s_huge[APPLY_NETS];  // positions of the huge ones, which are replayed first
+
+  // the block's touched nets, the small ones and the others apart: a wave
+  // then replays 64 small nets at a time, a lane each, and the big ones go
+  // to whichever wave is free
+  const int n0 = (int)blockIdx.x * a.per_block;
+  const int nn = min(a.per_block, a.noe - n0);
+  if (threadIdx.x < 4) s_cnt[threadIdx.x] = 0;
+  __syncthreads();
+  for (int i0 = 0; i0 < nn; i0 += APPLY_BLOCK) {
+    const int i = i0 + (int)threadIdx.x;
+    const bool hit = i < nn && a.net_stamp[n0 + i] == a.tag;
+    unsigned st = 0, len = 0;
+    if (hit) {
+      st = a.net_ptr[n0 + i];
+      len = a.net_ptr[n0 + i + 1] - st;
+    }
+    const bool sm = hit && len <= (unsigned)SMALL_NET;
+    const unsigned long long ms = __ballot(sm), mb = __ballot(hit && !sm);
+    int bs = 0, bb = 0;
+    if (lane == 0) {
+      if (ms) bs = atomicAdd(&s_cnt[0], (int)__popcll(ms));
+      if (mb) bb = atomicAdd(&s_cnt[1], (int)__popcll(mb));
+    }
+    // lane 0's, read while every lane is active
+    bs = __builtin_amdgcn_readlane(bs, 0);
+    bb = __builtin_amdgcn_readlane(bb, 0);
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    const int k = sm ? bs + (int)__popcll(ms & lt) : APPLY_NETS - 1 - (bb + (int)__popcll(mb & lt));
+    if (hit) {
+      s_net[k] = (unsigned short)i;
+      s_start[k] = st;
+      s_len[k] = len;
+      if (len >= HUGE_NET) s_huge[atomicAdd(&s_cnt[3], 1)] = (unsigned short)k;
+    }
+  }
+  __syncthreads();
+  const int nsmall = __builtin_amdgcn_readfirstlane(s_cnt[0]), nbig = __builtin_amdgcn_readfirstlane(s_cnt[1]);
+  const int nhuge = __builtin_amdgcn_readfirstlane(s_cnt[3]);
+
+  for (int b = wave * WAVE; b < nsmall; b += nw * WAVE)
+    if (b + lane < nsmall) lane_replay_small(a, n0 + s_net[b + lane], s_start[b + lane], s_len[b + lane], my);
+  if (nbig == 0) return;
+  wave_lds_sync();
   if (INDEXED) wave_index_init(at, a.K);
-  const int ntouched = *a.tcount;
-  // a net's head: the first 64 words of its segment and, for a net of at
-  // most 64 pins, its ranks; loaded while the wave's previous net is replayed
+
+  // The others in three stages, so that a net of at most 64 pins waits for no
+  // load of its own: its head (its list and its ranks; of a larger net the
+  // first 64 words of its segment) loads while the net before the previous
+  // one is replayed, its ranks' decisions while the previous one is
   struct NetHead {
-    unsigned x;
-    int r;
+    int n, r, dd, oo, L;
+    unsigned s, e, x;
   };
-  auto head = [&](int n, unsigned s, unsigned e) -> NetHead {
-    NetHead h;
-    h.x = wave_list_head(a.ent, s + (unsigned)n, e - s);
-    h.r = e - s <= (unsigned)WAVE && (unsigned)lane < e - s ? a.apply_pins[s + (unsigned)lane] : INT_MAX;
+  auto next_head = [&]() -> NetHead {
+    NetHead h{-1, INT_MAX, -1, -1, 0, 0u, 0u, 0u};
+    int k = 0;
+    if (lane == 0) k = atomicAdd(&s_cnt[2], 1);
+    k = __builtin_amdgcn_readlane(k, 0);
+    for (;;) {
+      if (k >= nhuge + nbig) return h;
+      if (k < nhuge) {
+        k = __builtin_amdgcn_readfirstlane((int)s_huge[k]);
+        break;
+      }
+      k = APPLY_NETS - 1 - (k - nhuge);
+      if (nhuge == 0 || __builtin_amdgcn_readfirstlane((int)s_len[k]) < (int)HUGE_NET) break;
+      if (lane == 0) k = atomicAdd(&s_cnt[2], 1);  // a huge one again: the next
+      k = __builtin_amdgcn_readlane(k, 0);
+    }
+    h.n = n0 + __builtin_amdgcn_readfirstlane((int)s_net[k]);
+    h.s = (unsigned)__builtin_amdgcn_readfirstlane((int)s_start[k]);
+    const unsigned np = (unsigned)__builtin_amdgcn_readfirstlane((int)s_len[k]);
+    h.e = h.s + np;
+    const unsigned seg = h.s + (unsigned)h.n;
+    if (np <= (unsigned)WAVE) {
+      h.L = (int)a.ent[seg];
+      h.x = (unsigned)lane < np ? a.ent[seg + 1u + (unsigned)lane] : 0u;
+      h.r = (unsigned)lane < np ? a.apply_pins[h.s + (unsigned)lane] : INT_MAX;
+    } else {
+      h.x = wave_list_head(a.ent, seg, np);
+    }
     return h;
   };
-  auto replay_net = [&](int n, unsigned s, unsigned e, const NetHead& h) {
+  auto load_moves = [&](NetHead& h) {
+    if (h.r >= a.r0 && h.r < a.r1) {
+      h.dd = a.slot_dec[h.r - a.r0];
+      h.oo = a.slot_own[h.r - a.r0];
+    }
+  };
+  auto replay_net = [&](const NetHead& h) {
+    const int n = h.n;
+    const unsigned s = h.s, e = h.e;
     const unsigned seg = s + (unsigned)n;
-    const bool small = e - s <= (unsigned)WAVE;
-    const int r_small = h.r;
+    if (e - s <= (unsigned)WAVE) {
+      if (__ballot(h.dd >= 0)) wave_replay_medium(a, n, s, __builtin_amdgcn_readfirstlane(h.L), h.x, h.dd, h.oo, words);
+      return;
+    }
     unsigned lo, hi;
     wave_rank_window(a.apply_pins, s, e, a.r0, a.r1, lo, hi);
     int L = wave_list_stage(a.ent, seg, h.x, list);
@@ -783,7 +1302,7 @@ __global__ void __launch_bounds__(APPLY_BLOCK) k_apply(ApplyArgs a) {
 #pragma unroll
       for (int u = 0; u < APPLY_GROUP; u++) {
         const unsigned k = k0 + (unsigned)(u * WAVE + lane);
-        rr[u] = small ? (u == 0 ? r_small : INT_MAX) : (k < hi ? a.apply_pins[k] : INT_MAX);
+        rr[u] = k < hi ? a.apply_pins[k] : INT_MAX;
       }
 #pragma unroll
       for (int u = 0; u < APPLY_GROUP; u++) {
@@ -797,8 +1316,15 @@ __global__ void __launch_bounds__(APPLY_BLOCK) k_apply(ApplyArgs a) {
 #pragma unroll
       for (int u = 0; u < APPLY_GROUP; u++) {
         unsigned long long m = __ballot(dd[u] >= 0);
+        dirty |= m != 0;
+        bool together = INDEXED;  // worth trying in this window
         while (m) {
-          dirty = true;
+          if (together && __popcll(m) >= APPLY_TOGETHER) {
+            const int before = (int)__popcll(m);
+            m = wave_ilist_moves(list, at, m, oo[u], dd[u], a.pb);
+            together = before - (int)__popcll(m) >= APPLY_TOGETHER / 2;
+            if (!m) break;
+          }
           const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)m) - 1);
           m &= m - 1;
           const int o = __builtin_amdgcn_readlane(oo[u], l), d = __builtin_amdgcn_readlane(dd[u], l);
@@ -813,82 +1339,52 @@ __global__ void __launch_bounds__(APPLY_BLOCK) k_apply(ApplyArgs a) {
       }
     }
     if (dirty) wave_list_store(a.ent, a.ev, seg, list, L, a.pb, a.pmask);
+    if (INDEXED && dirty && a.masks)
+      wave_store_masks(list, at, a.K, a.pb, a.mask_words, a.masks + (size_t)n * (size_t)(2 * a.mask_words));
     if (INDEXED) wave_index_clear(list, L, at, a.pmask);
     wave_lds_sync();
   };
-  // the wave's share of the touched nets, 64 at a time, one per lane: nets of
-  // at most SMALL_NET pins are replayed by their lanes, the others by the
-  // whole wavefront one after another, the next one's head loading meanwhile
-  const int stride = a.net_blocks * nw;
-  for (long long b0 = (int)blockIdx.x * nw + wave; b0 < ntouched; b0 += (long long)WAVE * stride) {
-    const long long ij = b0 + (long long)lane * stride;
-    int nj = 0;
-    unsigned sj = 0, ej = 0;
-    if (ij < ntouched) {
-      nj = a.touched[ij];
-      sj = a.net_ptr[nj];
-      ej = a.net_ptr[nj + 1];
-    }
-    const bool sm = ij < ntouched && ej - sj <= (unsigned)SMALL_NET;
-    unsigned long long big = __ballot(ij < ntouched && !sm);
-    auto net_at = [&](int j, int& n, unsigned& s, unsigned& e) {
-      n = __builtin_amdgcn_readlane(nj, j);
-      s = (unsigned)__builtin_amdgcn_readlane((int)sj, j);
-      e = (unsigned)__builtin_amdgcn_readlane((int)ej, j);
-    };
-    int j = -1, n = 0;
-    unsigned s = 0, e = 0;
-    NetHead cur{0u, INT_MAX};
-    if (big) {
-      j = __builtin_amdgcn_readfirstlane(__ffsll((long long)big) - 1);
-      big &= big - 1;
-      net_at(j, n, s, e);
-      cur = head(n, s, e);
-    }
-    if (sm) lane_replay_small(a, nj, sj, ej, my);
-    while (j >= 0) {
-      int jn = -1, nn = 0;
-      unsigned sn = 0, en = 0;
-      NetHead nxt = cur;
-      if (big) {
-        jn = __builtin_amdgcn_readfirstlane(__ffsll((long long)big) - 1);
-        big &= big - 1;
-        net_at(jn, nn, sn, en);
-        nxt = head(nn, sn, en);
-      }
-      replay_net(n, s, e, cur);
-      j = jn;
-      n = nn;
-      s = sn;
-      e = en;
-      cur = nxt;
-    }
+  NetHead cur = next_head(), nxt = next_head();
+  load_moves(cur);
+  while (cur.n >= 0) {
+    const NetHead nn2 = next_head();
+    load_moves(nxt);
+    replay_net(cur);
+    cur = nxt;
+    nxt = nn2;
   }
 }
 
-// the apply's LDS: a K-entry list per wave, and the part -> position index
-// where it fits the budget
-// LDS of the apply: per wave a K-entry list and, where it fits the budget,
-// the part -> position index; then SMALL_NET + 1 words per lane
-constexpr size_t APPLY_SMALL_BYTES = (size_t)APPLY_BLOCK * (SMALL_NET + 1) * sizeof(unsigned);
+// LDS of the apply, per wave: a K-entry list and, where it fits the budget,
+// the part -> position index, or before that half a mask record per lane
+int apply_lane_words(int K) { return 2 * mask_words(K) + 1; }
+
+// the block's touched nets and its waves' mask words
+constexpr size_t APPLY_STATIC = (size_t)APPLY_NETS * 10 + (size_t)(APPLY_BLOCK / WAVE) * 4 * MASK_PMAX * sizeof(unsigned) + 64;
+
+size_t apply_wave_bytes(int K, bool indexed) {
+  const size_t list = (size_t)K * (sizeof(unsigned) + (indexed ? sizeof(unsigned short) : 0));
+  return (std::max(list, (size_t)WAVE * (size_t)apply_lane_words(K) * sizeof(unsigned)) + 15) & ~(size_t)15;
+}
 
 bool apply_indexed(int K) {
-  return apply_list_bytes<true>(K, APPLY_BLOCK / WAVE) + APPLY_SMALL_BYTES <= (size_t)LDS_BUDGET;
+  return (size_t)(APPLY_BLOCK / WAVE) * apply_wave_bytes(K, true) + APPLY_STATIC <= (size_t)LDS_BUDGET;
 }
 
-size_t apply_lds(int K) {
-  return (apply_indexed(K) ? apply_list_bytes<true>(K, APPLY_BLOCK / WAVE)
-                           : apply_list_bytes<false>(K, APPLY_BLOCK / WAVE)) +
-         APPLY_SMALL_BYTES;
-}
+size_t apply_lds(int K) { return (size_t)(APPLY_BLOCK / WAVE) * apply_wave_bytes(K, apply_indexed(K)); }
 
 size_t eval_lds(int K, int waves) {
-  return (size_t)K * 12 + (size_t)waves * (8 * (size_t)(K + WAVE) + 4 * (size_t)TOUCH_BUF);
+  return (size_t)K * 12 + (size_t)waves * 8 * (size_t)(K + WAVE);
 }
+
+// the largest K of the refinements with a schedule and of the device stream:
+// 12 + 8 bytes per part and 1.5 KiB in one workgroup of one wavefront
+constexpr int EVAL_KMAX = (LDS_BUDGET - 1536) / 20;
 
 int eval_waves(int K) {
   // LDS: 12 bytes per part shared by the block + 8 bytes per part (and per
-  // spare slot) and the touched-net buffer per wavefront
+  // spare slot) per wavefront
+  if (K > EVAL_KMAX) return 0;
   for (int w = EVAL_BLOCK / WAVE; w >= 1; w--)
     if (eval_lds(K, w) <= (size_t)LDS_BUDGET) return w;
   return 0;
@@ -915,6 +1411,53 @@ fp_status ensure_bal_scratch(fp_ctx* ctx, int R) {
     ctx->hist_cap = need;
   }
   return FP_OK;
+}
+
+// The slots per wave of k_tv_eval_masks, and its grid: as many waves as fit the
+// GPU at 7 per SIMD share the slots evenly. Twice as many cost a round of
+// 16,384 slots 9% (each wave sets itself up for one or two vertices) and gain
+// one of 262,144 1%.
+constexpr int MASK_EVAL_WAVES = 7168;
+
+int eval_masks_args(const fp_ctx* ctx, const unsigned long long* masks, int grid_cap, EvalArgs& a) {
+  constexpr int nw = EVAL_BLOCK / WAVE;
+  a.masks = masks;
+  a.noe = ctx->noe;
+  a.last_pin = (unsigned)std::max(ctx->pins - 1, 0ll);
+  const int waves = grid_cap > 0 ? std::min(MASK_EVAL_WAVES, grid_cap * nw) : MASK_EVAL_WAVES;
+  a.per_wave = std::max(1, std::min(WAVE, (a.nslots + waves - 1) / waves));
+  const int need = (a.nslots + a.per_wave - 1) / a.per_wave;
+  return std::max(1, (need + nw - 1) / nw);
+}
+
+// The apply's blocks and their nets: about APPLY_NET_BLOCKS blocks, of 16 to
+// APPLY_NETS nets each.
+int apply_blocks(const fp_ctx* ctx, int& per_block) {
+  per_block = std::max(16, std::min(APPLY_NETS, (ctx->noe + APPLY_NET_BLOCKS - 1) / APPLY_NET_BLOCKS));
+  return std::max(1, (ctx->noe + per_block - 1) / per_block);
+}
+
+// the scan and the admission of a BAL round (first_free: of a sub-round of the stream)
+void launch_admission(fp_ctx* ctx, int r0, int nslots, int ntiles, long long cap, bool first_free, unsigned tag) {
+  const int K = ctx->K;
+  if (ntiles <= SCAN_WAVE_TILES)
+    k_bal_scan<true><<<std::max(1, std::min((K + 3) / 4, 1024)), 256, 0, ctx->stream>>>(
+        ctx->hist, ctx->pref, ntiles, K, ctx->sizes_frozen, cap, ctx->over);
+  else
+    k_bal_scan<false><<<std::max(1, std::min(K, 1024)), 256, 0, ctx->stream>>>(ctx->hist, ctx->pref, ntiles, K,
+                                                                               ctx->sizes_frozen, cap, ctx->over);
+  // the size changes are summed per block in LDS where K parts fit
+  // large blocks where that still leaves many: every block adds to the K size
+  // words, one after another (rounds of 262,144 slots: 16.4 -> 14.2 us with 16
+  // waves; rounds of 16,384, whose blocks are few: 7.3 us with 4 waves, 13.4 with 16)
+  const int ablock = ntiles >= 2048 ? ADMIT_BLOCK : 256;
+  const int tiles = ablock / WAVE;  // per block
+  const int agrid = std::max(1, std::min((ntiles + tiles - 1) / tiles, 4096));
+  const size_t lds = (size_t)K * sizeof(long long);
+  const bool agg = lds <= (size_t)LDS_BUDGET;
+  (agg ? k_bal_admit<true> : k_bal_admit<false>)<<<agrid, ablock, agg ? lds : 0, ctx->stream>>>(
+      ctx->slot_dec, ctx->slot_own, ctx->order, ctx->vwgt, r0, nslots, ntiles, K, ctx->sizes_frozen, cap, first_free,
+      ctx->over, ctx->pref, ctx->part, ctx->sizes, ctx->moves, ctx->vtx_ptr, ctx->vtx_nets, tag, ctx->net_stamp);
 }
 
 fp_status check_sched(fp_ctx* ctx, const fp_schedule* s) {
@@ -963,10 +1506,13 @@ fp_status plan_tv(fp_ctx* ctx, RefinePlan& p) {
   const int waves = p.eval_waves > 0 ? std::min(p.eval_waves, eval_waves(K)) : eval_waves(K);
   if (waves == 0) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d needs more LDS than a workgroup has", K);
   p.eval_waves = waves;
-  if (apply_lds(K) > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
+  if (apply_lds(K) + APPLY_STATIC > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
   p.R = std::min(p.sched.round, ctx->nov);
   FP_TRY(ensure_round_scratch(ctx, p.R));
   if (p.sched.kind == FP_SCHED_BAL) FP_TRY(ensure_bal_scratch(ctx, p.R));
+  // the part masks of the resident lists, kept in step by the passes
+  p.masks = ensure_masks(ctx);
+  if (p.masks) build_masks(ctx, p.masks);
   return FP_OK;
 }
 
@@ -977,62 +1523,54 @@ fp_status pass_tv(fp_ctx* ctx, const RefinePlan& p) {
   const size_t lds_e = eval_lds(K, waves);
   const size_t lds_a = apply_lds(K);
   auto apply = apply_indexed(K) ? k_apply<true> : k_apply<false>;
-  const size_t lds_s = (size_t)K * sizeof(int);
-  // every pass restarts its round tags: clear the stamps and the touched counters
+  // every pass restarts its round tags: clear the stamps
   pass_begin(ctx, nullptr, 0, nullptr);
   unsigned tag = 0;
   for (int r0 = 0; r0 < nov; r0 += R) {
     const int nslots = std::min(R, nov - r0);
     const int ntiles = (nslots + TILE - 1) / TILE;
     tag++;
-    const int par = (int)(tag & 1u);
     EvalArgs a = make_eval_args(ctx, sched);
     a.r0 = r0;
     a.nslots = nslots;
     a.ntiles = ntiles;
     a.tag = tag;
-    a.net_stamp = ctx->net_stamp;
-    a.touched = ctx->touched;
-    a.tcount = ctx->counters + par;
-    a.tcount_next = ctx->counters + (par ^ 1);
+    if (!bal) a.net_stamp = ctx->net_stamp;  // BAL: k_bal_admit stamps the admitted moves' nets
     if (bal) {
-      a.cand_tot = ctx->cand_tot;
       a.hist = ctx->hist;
       a.sizes_frozen = ctx->sizes_frozen;
     }
-    int grid = eval_grid(nslots, waves);
-    if (p.eval_grid > 0) grid = std::min(grid, p.eval_grid);
-    FP_TRY(launch_timed(ctx, k_tv_eval<EVAL_REFINE>, grid, waves * WAVE, lds_e, a));
+    if (p.masks) {
+      const int grid = eval_masks_args(ctx, p.masks, p.eval_grid, a);
+      FP_TRY(launch_timed(ctx, eval_masks_kernel<EVAL_REFINE>(K), grid, EVAL_BLOCK, 0, a));
+    } else {
+      int grid = eval_grid(nslots, waves);
+      if (p.eval_grid > 0) grid = std::min(grid, p.eval_grid);
+      FP_TRY(launch_timed(ctx, k_tv_eval<EVAL_REFINE>, grid, waves * WAVE, lds_e, a));
+    }
     if (bal) {
-      k_bal_scan<<<std::max(1, std::min(K, 512)), 256, lds_s, ctx->stream>>>(
-          ctx->hist, ctx->pref, ntiles, K, ctx->sizes_frozen, ctx->cand_tot, sched->cap, ctx->over_idx,
-          ctx->over_count);
-      // the size changes are summed per block in LDS where K parts fit
-      const int agrid = std::max(1, std::min((ntiles + 3) / 4, 4096));
-      if ((size_t)K * sizeof(long long) <= (size_t)LDS_BUDGET)
-        k_bal_admit<true><<<agrid, 256, (size_t)K * sizeof(long long), ctx->stream>>>(
-            ctx->slot_dec, ctx->slot_own, ctx->order, ctx->vwgt, r0, nslots, ntiles, K, ctx->sizes_frozen, sched->cap,
-            false, ctx->over_idx, ctx->over_count, ctx->pref, ctx->hist, ctx->part, ctx->sizes, ctx->cand_tot, ctx->moves);
-      else
-        k_bal_admit<false><<<agrid, 256, 0, ctx->stream>>>(
-            ctx->slot_dec, ctx->slot_own, ctx->order, ctx->vwgt, r0, nslots, ntiles, K, ctx->sizes_frozen, sched->cap,
-            false, ctx->over_idx, ctx->over_count, ctx->pref, ctx->hist, ctx->part, ctx->sizes, ctx->cand_tot, ctx->moves);
+      launch_admission(ctx, r0, nslots, ntiles, sched->cap, false, tag);
     }
     ApplyArgs ap{};
     ap.net_ptr = ctx->net_ptr;
     ap.apply_pins = ctx->apply_pins;
     ap.slot_own = ctx->slot_own;
     ap.slot_dec = ctx->slot_dec;
-    ap.touched = ctx->touched;
-    ap.tcount = ctx->counters + par;
+    ap.net_stamp = ctx->net_stamp;
+    ap.tag = tag;
+    ap.noe = ctx->noe;
     ap.ent = ctx->ent;
     ap.ev = ctx->ev;
+    ap.masks = p.masks;
+    ap.mask_words = mask_words(K);
     ap.K = K;
     ap.pb = ctx->pb;
     ap.pmask = ctx->pmask;
     ap.r0 = r0;
     ap.r1 = r0 + nslots;
-    ap.net_blocks = net_grid(ctx, APPLY_NET_BLOCKS, APPLY_BLOCK / WAVE);
+    ap.net_blocks = apply_blocks(ctx, ap.per_block);
+    ap.lane_words = apply_lane_words(K);
+    ap.wave_bytes = (int)apply_wave_bytes(K, apply_indexed(K));
     int grid_a = ap.net_blocks;
     if (!bal) {
       ap.order = ctx->order;
@@ -1135,7 +1673,7 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
   FP_HIP_OK(hipSetDevice(ctx->device));
   FP_TRY(ensure_k(ctx, K));
   FP_TRY(check_envelope(ctx));
-  if (apply_lds(K) > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
+  if (apply_lds(K) + APPLY_STATIC > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
   const int nov = ctx->nov;
   const int R = std::max(1, std::min(round, nov));
   const int waves = eval_waves(K);
@@ -1146,8 +1684,9 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
   fill_async<int>(ctx, ctx->part, (size_t)std::max(nov, 1), -1);
   fill_async<unsigned>(ctx, ctx->ent, segs, 0u);
   fill_async<unsigned short>(ctx, ctx->ev, segs, (unsigned short)0);
+  unsigned long long* masks = ensure_masks(ctx);
+  if (masks) fill_async<unsigned long long>(ctx, masks, ((size_t)ctx->noe + 1) * (size_t)(2 * mask_words(K)), 0ull);
   fill_async<long long>(ctx, ctx->sizes, (size_t)K, 0);
-  fill_async<long long>(ctx, ctx->cand_tot, (size_t)K, 0);
   fill_async<unsigned long long>(ctx, ctx->moves, 1, 0ull);
   pass_begin(ctx, nullptr, 0, nullptr);
   hipEvent_t e0 = pooled_event(ctx, 0), e1 = pooled_event(ctx, 1);
@@ -1157,7 +1696,6 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
   const size_t lds_e = eval_lds(K, waves);
   const size_t lds_a = apply_lds(K);
   auto apply = apply_indexed(K) ? k_apply<true> : k_apply<false>;
-  const bool agg = (size_t)K * sizeof(long long) <= (size_t)LDS_BUDGET;
   int* fb = ctx->counters + 2;
   unsigned tag = 0;
   long long subrounds = 0, rounds = 0;
@@ -1165,7 +1703,6 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
   auto subround = [&](int r0, int nslots) -> fp_status {
     const int ntiles = (nslots + TILE - 1) / TILE;
     tag++;
-    const int par = (int)(tag & 1u);
     EvalArgs a{};
     a.pad_seg = (unsigned)((size_t)ctx->pins + (size_t)ctx->noe);
     a.vtx_ptr = ctx->vtx_ptr;
@@ -1188,47 +1725,40 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
     a.nslots = nslots;
     a.ntiles = ntiles;
     a.tag = tag;
-    a.net_stamp = ctx->net_stamp;
-    a.touched = ctx->touched;
-    a.tcount = ctx->counters + par;
-    a.tcount_next = ctx->counters + (par ^ 1);
-    a.cand_tot = ctx->cand_tot;
     a.hist = ctx->hist;
     a.sizes_frozen = ctx->sizes_frozen;
     a.fb_out = fb;
-    const int grid = eval_grid(nslots, waves);
-    if (eval_mode == EVAL_INIT_CN)
+    const int grid = masks ? eval_masks_args(ctx, masks, 0, a) : eval_grid(nslots, waves);
+    if (masks)
+      (eval_mode == EVAL_INIT_CN ? eval_masks_kernel<EVAL_INIT_CN>(K)
+                                 : eval_masks_kernel<EVAL_INIT>(K))<<<grid, EVAL_BLOCK, 0, ctx->stream>>>(a);
+    else if (eval_mode == EVAL_INIT_CN)
       k_tv_eval<EVAL_INIT_CN><<<grid, waves * WAVE, lds_e, ctx->stream>>>(a);
     else
       k_tv_eval<EVAL_INIT><<<grid, waves * WAVE, lds_e, ctx->stream>>>(a);
     k_init_fallback<<<1, 1024, 0, ctx->stream>>>(ctx->slot_dec, ctx->order, ctx->vwgt, r0, nslots, ntiles, K, fb,
-                                                 ctx->cand_tot, ctx->hist);
-    k_bal_scan<<<std::max(1, std::min(K, 512)), 256, (size_t)K * sizeof(int), ctx->stream>>>(
-        ctx->hist, ctx->pref, ntiles, K, ctx->sizes_frozen, ctx->cand_tot, cap, ctx->over_idx, ctx->over_count);
-    const int agrid = std::max(1, std::min((ntiles + 3) / 4, 4096));
-    if (agg)
-      k_bal_admit<true><<<agrid, 256, (size_t)K * sizeof(long long), ctx->stream>>>(
-          ctx->slot_dec, ctx->slot_own, ctx->order, ctx->vwgt, r0, nslots, ntiles, K, ctx->sizes_frozen, cap, true,
-          ctx->over_idx, ctx->over_count, ctx->pref, ctx->hist, ctx->part, ctx->sizes, ctx->cand_tot, ctx->moves);
-    else
-      k_bal_admit<false><<<agrid, 256, 0, ctx->stream>>>(
-          ctx->slot_dec, ctx->slot_own, ctx->order, ctx->vwgt, r0, nslots, ntiles, K, ctx->sizes_frozen, cap, true,
-          ctx->over_idx, ctx->over_count, ctx->pref, ctx->hist, ctx->part, ctx->sizes, ctx->cand_tot, ctx->moves);
+                                                 ctx->hist);
+    launch_admission(ctx, r0, nslots, ntiles, cap, true, tag);
     ApplyArgs ap{};
     ap.net_ptr = ctx->net_ptr;
     ap.apply_pins = ctx->apply_pins;
     ap.slot_own = ctx->slot_own;
     ap.slot_dec = ctx->slot_dec;
-    ap.touched = ctx->touched;
-    ap.tcount = ctx->counters + par;
+    ap.net_stamp = ctx->net_stamp;
+    ap.tag = tag;
+    ap.noe = ctx->noe;
     ap.ent = ctx->ent;
     ap.ev = ctx->ev;
+    ap.masks = masks;
+    ap.mask_words = mask_words(K);
     ap.K = K;
     ap.pb = ctx->pb;
     ap.pmask = ctx->pmask;
     ap.r0 = r0;
     ap.r1 = r0 + nslots;
-    ap.net_blocks = net_grid(ctx, APPLY_NET_BLOCKS, APPLY_BLOCK / WAVE);
+    ap.net_blocks = apply_blocks(ctx, ap.per_block);
+    ap.lane_words = apply_lane_words(K);
+    ap.wave_bytes = (int)apply_wave_bytes(K, apply_indexed(K));
     apply<<<ap.net_blocks, APPLY_BLOCK, lds_a, ctx->stream>>>(ap);
     FP_HIP_OK(hipGetLastError());
     subrounds++;

@@ -1,0 +1,104 @@
+"""The evaluation through the nets' part masks and the apply that keeps them:
+K at the edges of the 64-part words and of the masks' range, net sizes at the
+edges of the apply's classes (8 | 9, 64 | 65, 255 | 256 pins and thousands),
+vertex degrees past one chunk of nets. Bit-exact against the oracle."""
+import numpy as np
+import pytest
+
+from fastpartitioner_amd import hypergraph as H
+from fastpartitioner_amd.engine import SCHED_BAL, SCHED_REF, Engine, schedule
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _mixed(seed, nov=4000, hubs=(60, 63, 64, 65, 127, 129, 200)):
+    rng = np.random.default_rng(seed)
+    sizes = [1, 2, 7, 8, 9, 16, 17, 63, 64, 65, 128, 255, 256, 257] * 6 + [1500, 3000] * 3
+    sizes += list(rng.integers(2, 13, 3 * nov))
+    nets = [list(rng.choice(np.arange(len(hubs), nov), size=s, replace=False)) for s in sizes]
+    small = np.arange(14 * 6 + 6, len(nets))
+    for h, d in enumerate(hubs):
+        for i in rng.choice(small, size=d, replace=False):
+            nets[i].append(h)
+    net_ptr = np.zeros(len(nets) + 1, dtype=np.uint32)
+    net_ptr[1:] = np.cumsum([len(n) for n in nets])
+    pins = np.concatenate([np.array(n) for n in nets]).astype(np.uint32)
+    return H.Hypergraph.from_nets(nov, net_ptr, pins, np.array([n[0] for n in nets], np.int32),
+                                  rng.integers(1, 9, nov).astype(np.int32))
+
+
+def _same(got, st):
+    for k in ("part", "ep_ends", "ep_parts", "ep_cnt"):
+        assert np.array_equal(getattr(got, k), getattr(st, k)), k
+    assert np.array_equal(got.sizes, st.sizes.astype(np.int64))
+
+
+@pytest.mark.parametrize("permuted", [False, True])
+@pytest.mark.parametrize("K", [2, 63, 64, 65, 128, 129, 256, 257, 320, 448, 511, 512, 513])
+def test_tv_masks_at_word_and_size_edges(K, permuted):
+    hg = _mixed(K)
+    rng = np.random.default_rng(K + 1)
+    order = rng.permutation(hg.nov).astype(np.int32) if permuted else None
+    part = rng.integers(0, K, hg.nov).astype(np.int32)
+    W = hg.total_weight()
+    C, cap = 1.5 * W / K, int(1.3 * W / K) + 8
+    print(f"masks: K={K} permuted={permuted} pins={hg.pins}", flush=True)
+    with Engine(0) as eng:
+        eng.upload(hg, order)
+        for R in (500, hg.nov):
+            eng.set_partition(K, part)
+            moves = eng.refine("TV", 3, schedule(SCHED_BAL, R, C, cap, 0, cap)).moves
+            st = O.build_state(hg, K, part, order)
+            O.tv_refine_bal(hg, st, C, cap, 0, cap, 3, R, order)
+            assert moves > 0
+            _same(eng.get_state(), st)
+        # the reference's schedule counts vertices, not weights: unit weights
+        hg.vwgt = None
+        eng.upload(hg, order)
+        C = 1.5 * hg.nov / K
+        eng.set_partition(K, part)
+        moves = eng.refine("TV", 2, schedule(SCHED_REF, 700, C, hg.nov, 0)).moves
+        st = O.build_state(hg, K, part, order)
+        st.sizes = st.sizes.astype(np.int32)
+        O.tv_refine_par(hg, st, C, hg.nov, 0, 2, 700, ordering=order)
+        assert moves > 0
+        _same(eng.get_state(), st)
+
+
+@pytest.mark.parametrize("mode", ["ldg_bands", "ldg", "cn_ldg"])
+@pytest.mark.parametrize("K", [3, 64, 65, 512, 513])
+def test_stream_masks_at_word_edges(mode, K):
+    hg = _mixed(100 + K)
+    W = hg.total_weight()
+    C, max_pw, cap = 1.2 * W / K, int(1.4 * W / K), int(1.2 * W / K) + 8
+    num = {"ldg_bands": 0, "ldg": 1, "cn_ldg": 2}[mode]
+    print(f"stream masks: K={K} mode={mode}", flush=True)
+    with Engine(0) as eng:
+        eng.upload(hg)
+        for R in (1, 900):
+            eng.initial_partition(num, K, R, C, max_pw, cap)
+            st, _ = O.round_ldg(hg, K, mode, C, max_pw, R, cap)
+            _same(eng.get_state(), st)
+
+
+def test_masks_follow_every_change_of_the_lists():
+    # other objectives edit the lists between two TV refinements
+    hg = _mixed(9)
+    K = 96
+    part = np.random.default_rng(2).integers(0, K, hg.nov).astype(np.int32)
+    W = hg.total_weight()
+    C, cap = 1.5 * W / K, int(1.3 * W / K) + 8
+    sched = schedule(SCHED_BAL, 1000, C, cap, 0, cap)
+    st = O.build_state(hg, K, part)
+    with Engine(0) as eng:
+        eng.upload(hg)
+        eng.set_partition(K, part)
+        for _ in range(2):
+            eng.refine("TV", 1, sched)
+            O.tv_refine_bal(hg, st, C, cap, 0, cap, 1, 1000)
+            eng.refine("CN", 1)
+            st.sizes = st.sizes.astype(np.int32)
+            O.cn_refine(hg, st, 1, serial=False)
+            st.sizes = st.sizes.astype(np.int64)
+            _same(eng.get_state(), st)
