@@ -283,17 +283,15 @@ struct BfsScratch {
   int* counts = nullptr;  // [0] level nets, [1] candidates, [2] min
   void* temp = nullptr;
   size_t temp_bytes = 0;
-  std::vector<void*> all;
-  ~BfsScratch() {
-    for (void* p : all) (void)hipFree(p);
-  }
+  // one allocation for all arrays: the first call of every get only adds up
+  // their sizes, the second hands out their places
+  char* base = nullptr;
+  size_t total = 0;
+  ~BfsScratch() { (void)hipFree(base); }
   template <typename T>
-  bool get(T** p, size_t n) {
-    void* q = nullptr;
-    if (hipMalloc(&q, sizeof(T) * std::max<size_t>(n, 1)) != hipSuccess) return false;
-    all.push_back(q);
-    *p = static_cast<T*>(q);
-    return true;
+  void get(T** p, size_t n) {
+    if (base) *p = reinterpret_cast<T*>(base + total);
+    total += (sizeof(T) * std::max<size_t>(n, 1) + 255) / 256 * 256;
   }
 };
 
@@ -386,15 +384,34 @@ fp_status fp_bfs_ordering(fp_ctx* ctx, int start, int view, int* ordering, int* 
   FP_HIP_OK(hipSetDevice(ctx->device));
   BfsScratch s;
   const size_t nv = (size_t)nov, ne = (size_t)std::max(noe, 1);
-  if (!s.get(&s.dist, nv) || !s.get(&s.plev, nv) || !s.get(&s.pos, nv) || !s.get(&s.vkey, nv) || !s.get(&s.net_owner, ne) || !s.get(&s.net_done, ne) ||
-      !s.get(&s.level_nets, ne) || !s.get(&s.cand, nv) || !s.get(&s.keys, nv) || !s.get(&s.keys_out, nv) ||
-      !s.get(&s.vals, nv) || !s.get(&s.order, nv) || !s.get(&s.counts, 4))
-    return fail(ctx, FP_ERR_OOM, "BFS scratch allocation failed");
   if (hipcub::DeviceRadixSort::SortPairs(nullptr, s.temp_bytes, s.keys, s.keys_out, s.vals, s.order, nov, 0, 64,
                                          ctx->stream) != hipSuccess)
     return fail(ctx, FP_ERR_HIP, "BFS sort sizing failed");
-  if (!s.get(reinterpret_cast<unsigned char**>(&s.temp), s.temp_bytes))
-    return fail(ctx, FP_ERR_OOM, "BFS sort scratch allocation failed");
+  for (int turn = 0; turn < 2; turn++) {
+    s.get(&s.dist, nv);
+    s.get(&s.plev, nv);
+    s.get(&s.pos, nv);
+    s.get(&s.vkey, nv);
+    s.get(&s.net_owner, ne);
+    s.get(&s.net_done, ne);
+    s.get(&s.level_nets, ne);
+    s.get(&s.cand, nv);
+    s.get(&s.keys, nv);
+    s.get(&s.keys_out, nv);
+    s.get(&s.vals, nv);
+    s.get(&s.order, nv);
+    s.get(&s.counts, 4);
+    s.get(reinterpret_cast<unsigned char**>(&s.temp), s.temp_bytes);
+    if (turn == 0) {
+      void* q = nullptr;
+      if (hipMalloc(&q, s.total) != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(ctx, FP_ERR_OOM, "BFS scratch allocation failed");
+      }
+      s.base = static_cast<char*>(q);
+      s.total = 0;
+    }
+  }
   const unsigned* pins =
       view == FP_BFS_PINS_UPLOADED ? ctx->net_pins : reinterpret_cast<const unsigned*>(ctx->apply_pins);
   hipEvent_t e0 = pooled_event(ctx, 0), e1 = pooled_event(ctx, 1);

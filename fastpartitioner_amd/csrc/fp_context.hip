@@ -61,15 +61,38 @@ fp_status fail(fp_ctx* c, fp_status st, const char* fmt, ...) {
   return st;
 }
 
+// Arrays live until the next upload, so they are cut from slabs one after
+// another: a slab is one hipMalloc, rounded up to SLAB_BYTES, and its rest
+// serves the arrays to come. (A hipMalloc costs tens of microseconds, and one
+// that has to map new memory about two milliseconds, several times the
+// smallest request.) At most SLAB_BYTES per slab stay unused.
 fp_status dalloc_bytes(fp_ctx* ctx, void** p, size_t bytes) {
+  constexpr size_t SLAB_BYTES = size_t{2} << 20, ALIGN = 256;
   *p = nullptr;
-  void* q = nullptr;
-  hipError_t e = hipMalloc(&q, bytes);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(ctx, FP_ERR_OOM, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
+  const size_t need = std::max(bytes, size_t{1});
+  char* q = nullptr;
+  for (auto& s : ctx->slabs)
+    if (s.size - s.used >= need) {
+      q = static_cast<char*>(s.base) + s.used;
+      s.used = std::min(s.size, (s.used + need + ALIGN - 1) / ALIGN * ALIGN);
+      break;
+    }
+  if (!q) {
+    size_t size = (need + SLAB_BYTES - 1) / SLAB_BYTES * SLAB_BYTES;
+    void* base = nullptr;
+    hipError_t e = hipMalloc(&base, size);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      size = need;
+      e = hipMalloc(&base, size);
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(ctx, FP_ERR_OOM, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
+    }
+    q = static_cast<char*>(base);
+    ctx->slabs.push_back({base, size, std::min(size, (need + ALIGN - 1) / ALIGN * ALIGN)});
   }
-  ctx->owned.push_back(q);
   ctx->dev_bytes += (long long)bytes;
   ctx->gen++;
   *p = q;
@@ -77,8 +100,8 @@ fp_status dalloc_bytes(fp_ctx* ctx, void** p, size_t bytes) {
 }
 
 void dfree_all(fp_ctx* ctx) {
-  for (void* p : ctx->owned) (void)hipFree(p);
-  ctx->owned.clear();
+  for (auto& s : ctx->slabs) (void)hipFree(s.base);
+  ctx->slabs.clear();
   ctx->dev_bytes = 0;
   ctx->gen++;
 }

@@ -677,7 +677,11 @@ struct fp_ctx {
   hipStream_t stream = nullptr;
   char err[512] = {0};
   long long dev_bytes = 0;
-  std::vector<void*> owned;
+  struct Slab {
+    void* base;
+    size_t size, used;
+  };
+  std::vector<Slab> slabs;  // device memory, cut into arrays by dalloc_bytes
   // bumped by every change that can invalidate recorded kernel arguments
   // (device pointers, K, the list layout): allocation, freeing, a new K
   unsigned long long gen = 0;
