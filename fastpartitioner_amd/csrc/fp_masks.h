@@ -30,6 +30,20 @@ unsigned long long* ensure_masks(fp_ctx* ctx);
 // Every record from the resident lists, on the context's stream.
 void build_masks(fp_ctx* ctx, unsigned long long* masks);
 
+// Shape of the evaluations through the masks: each wave takes per_wave
+// consecutive slots (at most one per lane), as many waves as fit the GPU at 7
+// per SIMD, or as grid_cap > 0 blocks hold, sharing the slots evenly. Twice
+// as many waves cost a TV round of 16,384 slots 9% (each sets itself up for
+// one or two vertices) and gain one of 262,144 1%.
+inline int mask_eval_grid(int nslots, int grid_cap, int waves_per_block, int& per_wave) {
+  const int waves = grid_cap > 0 ? std::min(7168, grid_cap * waves_per_block) : 7168;
+  per_wave = std::max(1, std::min(WAVE, (nslots + waves - 1) / waves));
+  const int need = (nslots + per_wave - 1) / per_wave;
+  return std::max(1, (need + waves_per_block - 1) / waves_per_block);
+}
+// the last element of vtx_nets, which bounds its reads a vertex ahead
+inline unsigned mask_last_pin(const fp_ctx* ctx) { return (unsigned)std::max(ctx->pins - 1, 0ll); }
+
 #ifdef __HIPCC__
 // c += this lane's bit of m (m wave-uniform): the bit is the add's carry-in
 __device__ __forceinline__ void add_lane_bit(unsigned& c, unsigned long long m) {
@@ -40,6 +54,197 @@ __device__ __forceinline__ unsigned sub_lane_bit(unsigned c, unsigned long long 
   unsigned r;
   asm("v_subbrev_co_u32_e64 %0, vcc, 0, %1, %2" : "=v"(r) : "v"(c), "s"(m) : "vcc");
   return r;
+}
+
+// The counts start at MASK_BIAS: count_double turns a biased count, or one
+// less, into the signed number's double by one full-rate addition (2^52 + x has
+// x in the low word; the conversion instruction takes four times as long).
+constexpr unsigned MASK_BIAS = 0x80000000u;
+
+__device__ __forceinline__ double count_double(unsigned x) {
+  return __longlong_as_double((long long)((0x43300000ull << 32) | x)) - (4503599627370496.0 + 2147483648.0);
+}
+
+// Records of nets in flight per wave: their words (2 P SGPRs each) have to fit
+// the scalar registers.
+template <int P>
+constexpr int mask_nets_in_flight() {
+  return P <= 2 ? 8 : (P <= 4 ? 4 : (P <= 6 ? 3 : 2));
+}
+
+// nets per chunk of a vertex's nets: no batch reaches past the wave's last lane
+template <int P>
+constexpr int mask_chunk() {
+  return (WAVE / mask_nets_in_flight<P>()) * mask_nets_in_flight<P>();
+}
+
+// the present words of the record at byte offset off, into scalar registers
+template <int P>
+__device__ __forceinline__ void mask_load(const unsigned long long* masks, unsigned off, unsigned long long (&w)[P]) {
+#pragma unroll
+  for (int u = 0; u < P; u++) w[u] = uniform_load_at<unsigned long long>(masks, off, u);
+}
+
+// UNCUT: only a net of one part keeps its bit
+template <int P, bool UNCUT>
+__device__ __forceinline__ void mask_filter(unsigned long long (&w)[P]) {
+  if (!UNCUT) return;
+  int c = 0;
+#pragma unroll
+  for (int u = 0; u < P; u++) c += (int)__popcll(w[u]);
+#pragma unroll
+  for (int u = 0; u < P; u++) w[u] = c == 1 ? w[u] : 0ull;
+}
+
+// Adds nn <= mask_chunk nets to the counts of the lane's parts: lane j holds
+// the byte offset of net j's record. A batch's loads are all issued before the
+// first is waited for.
+template <int P, bool UNCUT>
+__device__ __forceinline__ void mask_count(const unsigned long long* masks, unsigned off, int nn, unsigned (&cnt)[P]) {
+  constexpr int NB = mask_nets_in_flight<P>();
+  auto batch = [&](int j0, int n) {
+    unsigned long long w[NB][P];
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+      if (j < n) mask_load<P>(masks, (unsigned)__builtin_amdgcn_readlane((int)off, j0 + j), w[j]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+      if (j < n) {
+        mask_filter<P, UNCUT>(w[j]);
+#pragma unroll
+        for (int u = 0; u < P; u++) add_lane_bit(cnt[u], w[j][u]);
+      }
+  };
+  int j0 = 0;
+  for (; j0 + NB <= nn; j0 += NB) batch(j0, NB);
+  if (j0 < nn) batch(j0, nn - j0);
+}
+
+// The LDG choice of a vertex (its nets vtx_nets[vb .. vb + deg)) from its
+// counts: the lexicographic max of (score, -size, -first appearance) over
+// score > 0, score = (count, less 1 for own) * penalty, which equals the
+// reference's scan over the parts it meets (TV/partition.cpp:98-116, :345).
+// pen holds the penalties, negative ones as 0 (which no more makes a candidate),
+// own is -1 for a vertex without a part. Returns pid of the part (lane l's
+// pid[u] for part 64 u + l) and its count, or -1 when no part scores above 0.
+template <int P, bool UNCUT>
+__device__ __forceinline__ int mask_ldg(const unsigned long long* masks, const unsigned* vtx_nets,
+                                        const unsigned* vtx_seg, const unsigned short* ev, unsigned vb, int deg,
+                                        int own, const unsigned (&cnt)[P], const double (&pen)[P],
+                                        const unsigned (&skey)[P], const int (&pid)[P], unsigned& craw) {
+  const int lane = lane_id();
+  double sc[P];
+  double best = 0;
+  const int mine = own - lane;  // 64 u where own is this lane's part u
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    // a part in none of the nets scores 0, or (own) no more, and is no candidate
+    sc[u] = count_double(sub_lane_bit(cnt[u], __ballot(mine == u * WAVE))) * pen[u];
+    best = fmax(best, sc[u]);
+  }
+  // the wave's best: positive doubles order like their bit patterns, the
+  // high words first and the low words only where several lanes share it
+  const unsigned long long bb = (unsigned long long)__double_as_longlong(best);
+  const unsigned hi = (unsigned)(bb >> 32);
+  const unsigned mh = wave_max_u32(hi);
+  if (mh == 0 && __ballot(bb != 0ull) == 0ull) return -1;
+  const unsigned long long hl = __ballot(hi == mh);
+  unsigned ml;
+  if (__popcll(hl) == 1)
+    ml = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)bb, __ffsll((long long)hl) - 1);
+  else
+    ml = wave_max_u32(hi == mh ? (unsigned)bb : 0u);
+  const double m1 = __longlong_as_double((long long)(((unsigned long long)mh << 32) | ml));
+  unsigned long long tie[P];
+  int ntie = 0;
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    tie[u] = __ballot(sc[u] == m1);
+    ntie += (int)__popcll(tie[u]);
+  }
+  if (ntie > 1) {
+    // equal scores: the lightest part
+    unsigned k2 = ~0u;
+#pragma unroll
+    for (int u = 0; u < P; u++) k2 = min(k2, sc[u] == m1 ? skey[u] : ~0u);
+    const unsigned m2 = wave_min_u32(k2);
+    ntie = 0;
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      tie[u] &= __ballot(skey[u] == m2);
+      ntie += (int)__popcll(tie[u]);
+    }
+    if (ntie > 1) {
+      // equal sizes too: the part the reference's scan meets first, i.e. of the
+      // first net that lists one of them, the earliest in its list
+      // (TV/partition.cpp:318-338)
+      for (int t = 0; t < deg; t++) {
+        unsigned long long w[P];
+        mask_load<P>(masks, uniform_load(vtx_nets + (vb + (unsigned)t)) * (16u * P), w);
+        mask_filter<P, UNCUT>(w);
+        int c = 0;
+#pragma unroll
+        for (int u = 0; u < P; u++) {
+          w[u] &= tie[u];
+          c += (int)__popcll(w[u]);
+        }
+        if (c == 0) continue;
+        if (c > 1) {
+          const unsigned seg = uniform_load(vtx_seg + (vb + (unsigned)t));
+          const int L = (int)ev[seg];
+          for (int t0 = 0; t0 < L; t0 += WAVE) {
+            const int e = t0 + lane;
+            const int q = e < L ? (int)(ev[seg + 1u + (unsigned)e] & ~EV_SINGLE) : 0;
+            unsigned long long x = 0;
+#pragma unroll
+            for (int u = 0; u < P; u++) x = (q >> 6) == u ? w[u] : x;
+            const unsigned long long hit = __ballot(e < L && ((x >> (q & (WAVE - 1))) & 1ull));
+            if (hit) {
+              const int f = __builtin_amdgcn_readlane(q, __ffsll((long long)hit) - 1);
+#pragma unroll
+              for (int u = 0; u < P; u++) w[u] = (f >> 6) == u ? 1ull << (f & (WAVE - 1)) : 0ull;
+              break;
+            }
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < P; u++) tie[u] = w[u];
+        break;
+      }
+    }
+  }
+  // one bit is left: its part and count, from the lane that holds them
+  unsigned long long any = 0;
+  int px = 0;
+  unsigned cx = 0;
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    any |= tie[u];
+    const bool t = __builtin_amdgcn_inverse_ballot_w64(tie[u]);
+    px = t ? pid[u] : px;
+    cx = t ? cnt[u] : cx;
+  }
+  const int l = __ffsll((long long)any) - 1;
+  craw = (unsigned)__builtin_amdgcn_readlane((int)cx, l) - MASK_BIAS;
+  return __builtin_amdgcn_readlane(px, l);
+}
+
+// The lowest-index part of minimum size (TV/partition.cpp:118-132), by the
+// whole wavefront.
+__device__ __forceinline__ int wave_lightest_part(const long long* __restrict__ sizes, int K) {
+  long long bs = LLONG_MAX;
+  int bi = INT_MAX;
+  for (int q = lane_id(); q < K; q += WAVE) {
+    const long long sz = sizes[q];
+    if (sz < bs || bi == INT_MAX) { bs = sz; bi = q; }
+  }
+  for (int off = WAVE / 2; off > 0; off >>= 1) {
+    const long long os = __shfl_xor(bs, off);
+    const int oi = __shfl_xor(bi, off);
+    if (os < bs || (os == bs && oi < bi)) { bs = os; bi = oi; }
+  }
+  return __builtin_amdgcn_readfirstlane(bi);
 }
 
 // One lane's record from a list of at most N entries x[0 .. L) in registers

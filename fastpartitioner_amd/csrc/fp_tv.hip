@@ -440,36 +440,6 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
   }
 }
 
-// The lowest-index part of minimum size (TV/partition.cpp:118-132), by the
-// whole wavefront.
-__device__ __forceinline__ int wave_lightest_part(const long long* __restrict__ sizes, int K) {
-  long long bs = LLONG_MAX;
-  int bi = INT_MAX;
-  for (int q = lane_id(); q < K; q += WAVE) {
-    const long long sz = sizes[q];
-    if (sz < bs || bi == INT_MAX) { bs = sz; bi = q; }
-  }
-  for (int off = WAVE / 2; off > 0; off >>= 1) {
-    const long long os = __shfl_xor(bs, off);
-    const int oi = __shfl_xor(bi, off);
-    if (os < bs || (os == bs && oi < bi)) { bs = os; bi = oi; }
-  }
-  return __builtin_amdgcn_readfirstlane(bi);
-}
-
-// A count as a double, by one full-rate addition: 2^52 + x has x in the low
-// word (the conversion instruction takes four times as long).
-__device__ __forceinline__ double exact_double(unsigned x) {
-  return __longlong_as_double((long long)((0x43300000ull << 32) | x)) - 4503599627370496.0;
-}
-
-// Records of nets in flight per wave: their words (2 P SGPRs each) have to fit
-// the scalar registers.
-template <int P>
-constexpr int mask_nets_in_flight() {
-  return P <= 2 ? 8 : (P <= 4 ? 4 : (P <= 6 ? 3 : 2));
-}
-
 // k_tv_eval through the nets' part masks (fp_masks.h), for K <= 64 P: lane l
 // counts parts l, l + 64, ... of the vertex in registers. Per net a record's
 // P present words come into scalar registers and are added with the lane's
@@ -484,9 +454,8 @@ constexpr int mask_nets_in_flight() {
 // The decision, the gain test and everything written are k_tv_eval's.
 template <int P, int MODE>
 __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu(P <= 6 ? 7 : 6, P <= 6 ? 7 : 6))) k_tv_eval_masks(EvalArgs a) {
-  constexpr int NB = mask_nets_in_flight<P>();
-  constexpr int CH = (WAVE / NB) * NB;  // nets per chunk: no batch reaches past the wave's last lane
-  constexpr unsigned ROW = 16u * P;     // bytes of a record
+  constexpr int CH = mask_chunk<P>();
+  constexpr unsigned ROW = 16u * P;  // bytes of a record
   __shared__ double s_pen[64 * P];
   __shared__ unsigned s_skey[64 * P];
   const int K = a.K;
@@ -508,7 +477,7 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
   for (int q = (int)threadIdx.x; q < 64 * P; q += (int)blockDim.x) {
     const long long sz = q < K ? a.sizes[q] : 0;
     s_skey[q] = size_key(sz);
-    s_pen[q] = q < K ? 1.0 - ((double)sz / a.C) : 0.0;
+    s_pen[q] = q < K ? fmax(1.0 - ((double)sz / a.C), 0.0) : 0.0;
     if (blockIdx.x == 0 && a.sizes_frozen && q < K) a.sizes_frozen[q] = sz;
   }
   if (MODE != EVAL_REFINE && blockIdx.x == 0 && wave == 0) {
@@ -528,19 +497,6 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
     const bool in = skey[u] <= size_key(a.max_pw) && (MODE != EVAL_REFINE || skey[u] >= size_key(a.min_pw));
     pid[u] = (u * WAVE + lane) | (in ? 1 << 16 : 0);
   }
-  auto load_row = [&](unsigned off, unsigned long long (&w)[P]) {
-#pragma unroll
-    for (int u = 0; u < P; u++) w[u] = uniform_load_at<unsigned long long>(a.masks, off, u);
-  };
-  auto votes = [&](unsigned long long (&w)[P]) {
-    if (MODE == EVAL_INIT_CN) {  // only nets of one part vote
-      int c = 0;
-#pragma unroll
-      for (int u = 0; u < P; u++) c += (int)__popcll(w[u]);
-#pragma unroll
-      for (int u = 0; u < P; u++) w[u] = c == 1 ? w[u] : 0ull;
-    }
-  };
   const char* masks = reinterpret_cast<const char*>(a.masks);
   // lane j: net j of slot s0 + i's vertex; past its last net some other net.
   // Loaded a vertex ahead, by every lane (a load that a branch may skip could
@@ -566,7 +522,7 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
 
     unsigned cnt[P];
 #pragma unroll
-    for (int u = 0; u < P; u++) cnt[u] = 0;
+    for (int u = 0; u < P; u++) cnt[u] = MASK_BIAS;
     int lg = 0;  // leave gain: nets where v is the only pin of its part (TV/partition.cpp:365-368)
     // nn <= CH nets of the vertex, lane j's the one with id ids
     auto count_nets = [&](unsigned ids, int nn) {
@@ -574,133 +530,18 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
       unsigned sw = 0;
       if (MODE == EVAL_REFINE)
         sw = *reinterpret_cast<const unsigned*>(masks + (8u * P + 4u * (unsigned)(own >> 5)) + off);
-      // a batch's loads are all issued before the first is waited for
-      auto batch = [&](int j0, int n) {
-        unsigned long long w[NB][P];
-#pragma unroll
-        for (int j = 0; j < NB; j++)
-          if (j < n) load_row((unsigned)__builtin_amdgcn_readlane((int)off, j0 + j), w[j]);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < NB; j++)
-          if (j < n) {
-            votes(w[j]);
-#pragma unroll
-            for (int u = 0; u < P; u++) add_lane_bit(cnt[u], w[j][u]);
-          }
-      };
-      int j0 = 0;
-      for (; j0 + NB <= nn; j0 += NB) batch(j0, NB);
-      if (j0 < nn) batch(j0, nn - j0);
+      mask_count<P, MODE == EVAL_INIT_CN>(a.masks, off, nn, cnt);
       if (MODE == EVAL_REFINE) lg += (int)__popcll(__ballot(((sw >> (own & 31)) & 1u) != 0u));
     };
     count_nets(id0, min(deg, CH));
     for (int c0 = CH; c0 < deg; c0 += CH)
       count_nets(*reinterpret_cast<const unsigned*>(nets + min(vb + (unsigned)(c0 + lane), a.last_pin) * 4u),
                  min(deg - c0, CH));
-    // scores (TV/partition.cpp:98-116), scores[part_id]-- (:345). A part in
-    // none of the nets scores 0 (own is in all of them; a vertex without nets
-    // keeps its 0), which is no candidate.
-    double sc[P];
-    double best = 0;
-    const int mine = (deg > 0 ? own : -1) - lane;  // 64 u where own is this lane's part u
-#pragma unroll
-    for (int u = 0; u < P; u++) {
-      const unsigned adj = MODE == EVAL_REFINE ? sub_lane_bit(cnt[u], __ballot(mine == u * WAVE)) : cnt[u];
-      sc[u] = exact_double(adj) * pen[u];
-      best = fmax(best, sc[u]);
-    }
-    // the wave's best: positive doubles order like their bit patterns, the
-    // high words first and the low words only where several lanes share it
-    const unsigned long long bb = (unsigned long long)__double_as_longlong(best);
-    const unsigned hi = (unsigned)(bb >> 32);
-    const unsigned mh = wave_max_u32(hi);
-    int d = -1;
     unsigned craw = 0;
-    bool in_band = false;
-    if (mh != 0 || __ballot(bb != 0ull) != 0ull) {
-      const unsigned long long hl = __ballot(hi == mh);
-      unsigned ml;
-      if (__popcll(hl) == 1)
-        ml = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)bb, __ffsll((long long)hl) - 1);
-      else
-        ml = wave_max_u32(hi == mh ? (unsigned)bb : 0u);
-      const double m1 = __longlong_as_double((long long)(((unsigned long long)mh << 32) | ml));
-      unsigned long long tie[P];
-      int ntie = 0;
-#pragma unroll
-      for (int u = 0; u < P; u++) {
-        tie[u] = __ballot(sc[u] == m1);
-        ntie += (int)__popcll(tie[u]);
-      }
-      if (ntie > 1) {
-        // equal scores: the lightest part
-        unsigned k2 = ~0u;
-#pragma unroll
-        for (int u = 0; u < P; u++) k2 = min(k2, sc[u] == m1 ? skey[u] : ~0u);
-        const unsigned m2 = wave_min_u32(k2);
-        ntie = 0;
-#pragma unroll
-        for (int u = 0; u < P; u++) {
-          tie[u] &= __ballot(skey[u] == m2);
-          ntie += (int)__popcll(tie[u]);
-        }
-        if (ntie > 1) {
-          // equal sizes too: the part the reference's scan meets first, i.e.
-          // of the first net that lists one of them, the earliest in its list
-          // (TV/partition.cpp:318-338)
-          for (int t = 0; t < deg; t++) {
-            unsigned long long w[P];
-            load_row(uniform_load(a.vtx_nets + (vb + (unsigned)t)) * ROW, w);
-            votes(w);
-            int c = 0;
-#pragma unroll
-            for (int u = 0; u < P; u++) {
-              w[u] &= tie[u];
-              c += (int)__popcll(w[u]);
-            }
-            if (c == 0) continue;
-            if (c > 1) {
-              const unsigned seg = uniform_load(a.vtx_seg + (vb + (unsigned)t));
-              const int L = (int)a.ev[seg];
-              for (int t0 = 0; t0 < L; t0 += WAVE) {
-                const int e = t0 + lane;
-                const int q = e < L ? (int)(a.ev[seg + 1u + (unsigned)e] & ~EV_SINGLE) : 0;
-                unsigned long long x = 0;
-#pragma unroll
-                for (int u = 0; u < P; u++) x = (q >> 6) == u ? w[u] : x;
-                const unsigned long long hit = __ballot(e < L && ((x >> (q & (WAVE - 1))) & 1ull));
-                if (hit) {
-                  const int f = __builtin_amdgcn_readlane(q, __ffsll((long long)hit) - 1);
-#pragma unroll
-                  for (int u = 0; u < P; u++) w[u] = (f >> 6) == u ? 1ull << (f & (WAVE - 1)) : 0ull;
-                  break;
-                }
-              }
-            }
-#pragma unroll
-            for (int u = 0; u < P; u++) tie[u] = w[u];
-            break;
-          }
-        }
-      }
-      // one bit is left: its part and count, from the lane that holds them
-      unsigned long long any = 0;
-      int px = 0;
-      unsigned cx = 0;
-#pragma unroll
-      for (int u = 0; u < P; u++) {
-        any |= tie[u];
-        const bool t = __builtin_amdgcn_inverse_ballot_w64(tie[u]);
-        px = t ? pid[u] : px;
-        cx = t ? cnt[u] : cx;
-      }
-      const int l = __ffsll((long long)any) - 1;
-      const int pl = __builtin_amdgcn_readlane(px, l);
-      craw = (unsigned)__builtin_amdgcn_readlane((int)cx, l);
-      d = pl & 0xFFFF;
-      in_band = (pl >> 16) != 0;
-    }
+    const int pl = mask_ldg<P, MODE == EVAL_INIT_CN>(a.masks, a.vtx_nets, a.vtx_seg, a.ev, vb, deg,
+                                                     MODE == EVAL_REFINE ? own : -1, cnt, pen, skey, pid, craw);
+    int d = pl < 0 ? -1 : pl & 0xFFFF;
+    bool in_band = pl >= 0 && (pl >> 16) != 0;
     const bool none = d < 0;  // no part above score 0: the fallback
     int dd;
     if (MODE == EVAL_REFINE) {
@@ -714,7 +555,7 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
           cx = (d >> 6) == u ? cnt[u] : cx;
         }
         in_band = (__builtin_amdgcn_readlane(px, d & (WAVE - 1)) >> 16) != 0;
-        craw = (unsigned)__builtin_amdgcn_readlane((int)cx, d & (WAVE - 1));
+        craw = (unsigned)__builtin_amdgcn_readlane((int)cx, d & (WAVE - 1)) - MASK_BIAS;
       }
       // outside the bands the vertex stays (TV/partition.cpp:135-143)
       const int al = deg - (int)craw;  // arrival loss: nets of v lacking d (TV/partition.cpp:369-377)
@@ -1413,23 +1254,6 @@ fp_status ensure_bal_scratch(fp_ctx* ctx, int R) {
   return FP_OK;
 }
 
-// The slots per wave of k_tv_eval_masks, and its grid: as many waves as fit the
-// GPU at 7 per SIMD share the slots evenly. Twice as many cost a round of
-// 16,384 slots 9% (each wave sets itself up for one or two vertices) and gain
-// one of 262,144 1%.
-constexpr int MASK_EVAL_WAVES = 7168;
-
-int eval_masks_args(const fp_ctx* ctx, const unsigned long long* masks, int grid_cap, EvalArgs& a) {
-  constexpr int nw = EVAL_BLOCK / WAVE;
-  a.masks = masks;
-  a.noe = ctx->noe;
-  a.last_pin = (unsigned)std::max(ctx->pins - 1, 0ll);
-  const int waves = grid_cap > 0 ? std::min(MASK_EVAL_WAVES, grid_cap * nw) : MASK_EVAL_WAVES;
-  a.per_wave = std::max(1, std::min(WAVE, (a.nslots + waves - 1) / waves));
-  const int need = (a.nslots + a.per_wave - 1) / a.per_wave;
-  return std::max(1, (need + nw - 1) / nw);
-}
-
 // The apply's blocks and their nets: about APPLY_NET_BLOCKS blocks, of 16 to
 // APPLY_NETS nets each.
 int apply_blocks(const fp_ctx* ctx, int& per_block) {
@@ -1541,7 +1365,10 @@ fp_status pass_tv(fp_ctx* ctx, const RefinePlan& p) {
       a.sizes_frozen = ctx->sizes_frozen;
     }
     if (p.masks) {
-      const int grid = eval_masks_args(ctx, p.masks, p.eval_grid, a);
+      a.masks = p.masks;
+      a.noe = ctx->noe;
+      a.last_pin = mask_last_pin(ctx);
+      const int grid = mask_eval_grid(nslots, p.eval_grid, EVAL_BLOCK / WAVE, a.per_wave);
       FP_TRY(launch_timed(ctx, eval_masks_kernel<EVAL_REFINE>(K), grid, EVAL_BLOCK, 0, a));
     } else {
       int grid = eval_grid(nslots, waves);
@@ -1728,7 +1555,10 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
     a.hist = ctx->hist;
     a.sizes_frozen = ctx->sizes_frozen;
     a.fb_out = fb;
-    const int grid = masks ? eval_masks_args(ctx, masks, 0, a) : eval_grid(nslots, waves);
+    a.masks = masks;
+    a.noe = ctx->noe;
+    a.last_pin = mask_last_pin(ctx);
+    const int grid = masks ? mask_eval_grid(nslots, 0, EVAL_BLOCK / WAVE, a.per_wave) : eval_grid(nslots, waves);
     if (masks)
       (eval_mode == EVAL_INIT_CN ? eval_masks_kernel<EVAL_INIT_CN>(K)
                                  : eval_masks_kernel<EVAL_INIT>(K))<<<grid, EVAL_BLOCK, 0, ctx->stream>>>(a);

@@ -22,6 +22,7 @@
 //                  decided together where bounds allow
 //   k_vol_replay   (commit) list edits, part vector and both part sizes of the
 //                  moves up to the stop
+#include "fp_masks.h"
 #include "fp_round.h"
 
 namespace fpe {
@@ -82,6 +83,11 @@ struct VolEvalArgs {
   int* touched;
   int* tcount;
   int* tcount_next;
+  // k_vol_eval_masks
+  const unsigned long long* masks;
+  int noe;
+  unsigned last_pin;
+  int per_wave;
 };
 
 // The first-appearance rank of the LDG tie-break (MGV/partition.cpp:765-790)
@@ -368,6 +374,213 @@ __global__ void __launch_bounds__(VOL_BLOCK) k_vol_eval(VolEvalArgs a) {
   }
 }
 
+// k_vol_eval through the nets' part masks (fp_masks.h), for K <= 64 P, the
+// slots shared out and the counts kept as in k_tv_eval_masks. The gain and loss
+// terms need three facts per net, a net per lane: whether v is own's only pin
+// there and whether the chosen part is listed are one bit each of the net's
+// record, and lambda (v's own source nets) is the record's bit count; sweeping
+// the lists a second time for them took as long as the first sweep.
+constexpr int VOL_MASK_BLOCK = 256;
+
+template <int P>
+__global__ void __launch_bounds__(VOL_MASK_BLOCK) __attribute__((amdgpu_waves_per_eu(P <= 6 ? 7 : 6, P <= 6 ? 7 : 6)))
+k_vol_eval_masks(VolEvalArgs a) {
+  constexpr int CH = mask_chunk<P>();
+  constexpr unsigned ROW = 16u * P;  // bytes of a record
+  __shared__ double s_pen[64 * P];
+  __shared__ unsigned s_skey[64 * P];
+  __shared__ int s_delta[VOL_MASK_BLOCK / WAVE][64 * P];    // losses - gains per part
+  __shared__ unsigned s_hit[VOL_MASK_BLOCK / WAVE][2 * P];  // max parts the move affects (MSRV), one bit per part
+  const int K = a.K;
+  const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
+  int* delta = s_delta[wave];
+  unsigned* hitb = s_hit[wave];
+  const int s0 = ((int)blockIdx.x * nw + wave) * a.per_wave;
+  const int ns = min(a.per_wave, a.nslots - s0);
+
+  // lane i: slot s0 + i's vertex, its part and its net range
+  int v_l = 0, own_l = 0;
+  unsigned vb_l = 0, ve_l = 0;
+  if (lane < ns) {
+    const int z = a.r0 + s0 + lane;
+    v_l = a.order ? a.order[z] : z;
+    own_l = a.part[v_l];
+    vb_l = a.vtx_ptr[v_l];
+    ve_l = a.vtx_ptr[v_l + 1];
+  }
+  // penalty = 1 - (1.0 * size / C) (MGV/partition.cpp:36)
+  for (int q = (int)threadIdx.x; q < 64 * P; q += (int)blockDim.x) {
+    const long long sz = q < K ? a.sizes[q] : 0;
+    s_skey[q] = size_key(sz);
+    s_pen[q] = q < K ? fmax(1.0 - ((double)sz / a.C), 0.0) : 0.0;
+  }
+  for (int q = lane; q < 64 * P; q += WAVE) delta[q] = 0;
+  if (lane < 2 * P) hitb[lane] = 0u;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && a.tcount_next) *a.tcount_next = 0;
+  __syncthreads();
+  double pen[P];
+  unsigned skey[P];
+  int pid[P];
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    pen[u] = s_pen[u * WAVE + lane];
+    skey[u] = s_skey[u * WAVE + lane];
+    pid[u] = u * WAVE + lane;
+  }
+  const int M = a.mstat[0], cntM = a.mstat[1];
+  const char* masks = reinterpret_cast<const char*>(a.masks);
+  const char* nets = reinterpret_cast<const char*>(a.vtx_nets);
+  // lane j: net j of slot s0 + i's vertex; past its last net some other net
+  auto load_nets = [&](int i) -> unsigned {
+    const unsigned k = (unsigned)__builtin_amdgcn_readlane((int)vb_l, i) + (unsigned)lane;
+    return *reinterpret_cast<const unsigned*>(nets + min(k, a.last_pin) * 4u);
+  };
+
+  int dec_l = -1;  // lane i: slot s0 + i's decision
+  // the headers have arrived before the loop (else its first wait would take in the loads of every turn)
+  asm volatile("" ::"v"(v_l), "v"(own_l), "v"(vb_l), "v"(ve_l));
+  unsigned id = ns > 0 ? load_nets(0) : 0u;
+  for (int i = 0; i < ns; i++) {
+    const unsigned id_next = load_nets(min(i + 1, ns - 1));
+    const int v = __builtin_amdgcn_readlane(v_l, i);
+    const int own = __builtin_amdgcn_readlane(own_l, i);
+    const unsigned vb = (unsigned)__builtin_amdgcn_readlane((int)vb_l, i);
+    const int deg = (int)((unsigned)__builtin_amdgcn_readlane((int)ve_l, i) - vb);
+    // one chunk of v's nets, a net per lane: its record's offset, whether v is
+    // own's only pin in it, its source part (own for v's own source nets)
+    struct Chunk {
+      unsigned off;
+      unsigned sw;
+      int s, ip;
+    };
+    auto load_chunk = [&](unsigned ids, int nn) -> Chunk {
+      Chunk c;
+      c.off = (lane < nn ? ids : (unsigned)a.noe) * ROW;  // past the last net: the zero record
+      c.sw = *reinterpret_cast<const unsigned*>(masks + (8u * P + 4u * (unsigned)(own >> 5)) + c.off);
+      c.s = lane < nn ? a.src[ids] : -1;
+      return c;
+    };
+    auto net_ids = [&](int c0) -> unsigned {
+      return *reinterpret_cast<const unsigned*>(nets + min(vb + (unsigned)(c0 + lane), a.last_pin) * 4u);
+    };
+    auto source_part = [&](Chunk& c) { c.ip = c.s < 0 ? -1 : (c.s == v ? own : a.part[c.s]); };
+    const unsigned id0 = id;
+    id = id_next;
+    unsigned cnt[P];
+#pragma unroll
+    for (int u = 0; u < P; u++) cnt[u] = MASK_BIAS;
+    Chunk c0 = load_chunk(id0, min(deg, CH));
+    mask_count<P, false>(a.masks, c0.off, min(deg, CH), cnt);
+    source_part(c0);
+    for (int b = CH; b < deg; b += CH) {
+      const int nn = min(deg - b, CH);
+      mask_count<P, false>(a.masks, (lane < nn ? net_ids(b) : (unsigned)a.noe) * ROW, nn, cnt);
+    }
+    unsigned craw = 0;
+    int d = mask_ldg<P, false>(a.masks, a.vtx_nets, a.vtx_seg, a.ev, vb, deg, own, cnt, pen, skey, pid, craw);
+    if (d < 0) d = wave_lightest_part(a.sizes, K);  // MGV/partition.cpp:48-60
+    if (d == own) continue;
+    // gains / losses (MGV/partition.cpp:800-840; MSRV/partition.cpp:852-897),
+    // accumulated as delta[p] = losses[p] - gains[p]
+    int d_own = 0, d_dec = 0;
+    for (int b = 0; b < deg; b += CH) {
+      const int nn = min(deg - b, CH);
+      Chunk c = c0;
+      if (b > 0) {
+        c = load_chunk(net_ids(b), nn);
+        source_part(c);
+      }
+      const unsigned fw = *reinterpret_cast<const unsigned*>(masks + 4u * (unsigned)(d >> 5) + c.off);
+      if (lane < nn) {
+        const bool single = (c.sw >> (own & 31)) & 1u, found = (fw >> (d & 31)) & 1u;
+        if (c.s == v) {
+          int L = 0;
+#pragma unroll
+          for (int u = 0; u < P; u++)
+            L += (int)__popcll(*reinterpret_cast<const unsigned long long*>(masks + 8u * u + c.off));
+          d_own -= L - 1;  // gains[part_id] += end_cnt - 1
+          d_dec += L - 1;  // losses[decision] += end_cnt - 1
+          if (single) d_dec -= 1;
+          if (!found) d_dec += 1;
+        } else {
+          const int dl = (found ? 0 : 1) - (single ? 1 : 0);
+          if (dl) atomicAdd(&delta[c.ip], dl);
+          if (a.msrv) {
+            if (single) d_own -= 1;
+            if (!found) d_dec += 1;
+          }
+        }
+      }
+    }
+    d_own = wave_sum(d_own);
+    d_dec = wave_sum(d_dec);
+    if (lane == 0) {
+      atomicAdd(&delta[own], d_own);
+      atomicAdd(&delta[d], d_dec);
+    }
+    wave_lds_sync();
+    // the affected parts: own, d and every net's source part; every other part
+    // has gains = losses = 0. g(part) runs for every one of them
+    auto for_items = [&](auto g) {
+      if (lane < 2) g(lane == 0 ? own : d);
+      if (c0.ip >= 0) g(c0.ip);
+      for (int b = CH; b < deg; b += CH) {
+        const int nn = min(deg - b, CH);
+        if (lane < nn) {
+          const int s = a.src[net_ids(b)];
+          g(s == v ? own : a.part[s]);
+        }
+      }
+    };
+    // MSRV: max parts untouched by the move have gains = losses = 0 and fail
+    // the strict test, so every max part must be affected: maxhit counts the
+    // distinct max parts among the items
+    bool bad = false;
+    int maxhit = 0;
+    for_items([&](int p) {
+      const int dl = delta[p];
+      const int vv = a.vol[p];
+      if (vv == M) {
+        if (a.msrv ? dl >= 0 : dl > 0) bad = true;  // a max part must gain (MSRV: strictly)
+        const unsigned bit = 1u << (p & 31);
+        if (!(atomicOr(&hitb[p >> 5], bit) & bit)) maxhit++;
+      } else if (vv + dl >= M) {
+        bad = true;  // no other part may reach the max
+      }
+    });
+    bad = __ballot(bad) != 0;
+    maxhit = wave_sum(maxhit);
+    wave_lds_sync();
+    for_items([&](int p) {
+      delta[p] = 0;
+      hitb[p >> 5] = 0u;
+    });
+    wave_lds_sync();
+    if (!bad && (!a.msrv || maxhit == cntM)) {
+      dec_l = lane == i ? d : dec_l;
+      wave_touch_nets(a.vtx_nets + vb, deg, a.tag, a.net_stamp, a.touched, a.tcount);
+    }
+  }
+  if (lane < ns) {
+    a.slot_own[s0 + lane] = own_l;
+    a.slot_dec[s0 + lane] = dec_l;
+  }
+}
+
+// the instance of k_vol_eval_masks for K parts
+void (*vol_masks_kernel(int K))(VolEvalArgs) {
+  switch (mask_words(K)) {
+    case 1: return k_vol_eval_masks<1>;
+    case 2: return k_vol_eval_masks<2>;
+    case 3: return k_vol_eval_masks<3>;
+    case 4: return k_vol_eval_masks<4>;
+    case 5: return k_vol_eval_masks<5>;
+    case 6: return k_vol_eval_masks<6>;
+    case 7: return k_vol_eval_masks<7>;
+    default: return k_vol_eval_masks<8>;
+  }
+}
+
 // First word of a volume event: the net's source part (or -1) and its change
 // (-1, 0 or +1) in one int.
 __device__ __forceinline__ int vol_event_word(int sp, int dsp) { return ((sp + 1) << 2) | (dsp + 1); }
@@ -392,6 +605,8 @@ struct VolReplayArgs {
   long long* sizes;
   unsigned long long* moves;
   int4* evbuf;
+  unsigned long long* masks;  // nullable: the nets' part masks, kept in step with the lists
+  int mask_words;
   int K, pb;
   unsigned pmask;
   int r0, r1, msrv, commit, net_blocks;
@@ -516,7 +731,11 @@ __global__ void __launch_bounds__(REPLAY_BLOCK) k_vol_replay(VolReplayArgs a) {
         dirty = true;
       }
     }
-    if (a.commit && dirty) wave_list_store(a.ent, a.ev, seg, list, L, a.pb, a.pmask);
+    if (a.commit && dirty) {
+      wave_list_store(a.ent, a.ev, seg, list, L, a.pb, a.pmask);
+      if (INDEXED && a.masks)
+        wave_store_masks(list, at, a.K, a.pb, a.mask_words, a.masks + (size_t)n * (size_t)(2 * a.mask_words));
+    }
     if (INDEXED) wave_index_clear(list, L, at, a.pmask);
     wave_lds_sync();
   }
@@ -881,6 +1100,9 @@ fp_status plan_vol(fp_ctx* ctx, RefinePlan& p) {
   const int ngrid = std::max(1, std::min((ctx->noe + 255) / 256, 4096));
   k_vol_init<<<std::min(ngrid * 8, 1024), 256, (size_t)K * sizeof(int), ctx->stream>>>(
       ctx->net_ptr, ctx->ent, ctx->src, ctx->part, ctx->noe, ctx->pmask, K, msrv ? 1 : 0, vs.vol);
+  // the part masks of the resident lists, kept in step by the passes
+  p.masks = ensure_masks(ctx);
+  if (p.masks) build_masks(ctx, p.masks);
   FP_HIP_OK(hipGetLastError());
   return FP_OK;
 }
@@ -930,9 +1152,17 @@ fp_status pass_vol(fp_ctx* ctx, const RefinePlan& p) {
     a.touched = ctx->touched;
     a.tcount = ctx->counters + par;
     a.tcount_next = ctx->counters + (par ^ 1);
-    int egrid = std::max(1, std::min((nslots + waves - 1) / waves, 8192));
-    if (p.eval_grid > 0) egrid = std::min(egrid, p.eval_grid);
-    FP_TRY(launch_timed(ctx, k_vol_eval, egrid, waves * WAVE, lds_e, a));
+    if (p.masks) {
+      a.masks = p.masks;
+      a.noe = ctx->noe;
+      a.last_pin = mask_last_pin(ctx);
+      const int egrid = mask_eval_grid(nslots, p.eval_grid, VOL_MASK_BLOCK / WAVE, a.per_wave);
+      FP_TRY(launch_timed(ctx, vol_masks_kernel(K), egrid, VOL_MASK_BLOCK, 0, a));
+    } else {
+      int egrid = std::max(1, std::min((nslots + waves - 1) / waves, 8192));
+      if (p.eval_grid > 0) egrid = std::min(egrid, p.eval_grid);
+      FP_TRY(launch_timed(ctx, k_vol_eval, egrid, waves * WAVE, lds_e, a));
+    }
     launch_round_compact<false>(ctx, ctx->order, r0, nslots, vs.slot_mi, vs.mv, vs.mstat);
     VolReplayArgs ra{};
     ra.net_ptr = ctx->net_ptr;
@@ -952,6 +1182,8 @@ fp_status pass_vol(fp_ctx* ctx, const RefinePlan& p) {
     ra.sizes = ctx->sizes;
     ra.moves = ctx->moves;
     ra.evbuf = vs.evbuf;
+    ra.masks = p.masks;
+    ra.mask_words = mask_words(K);
     ra.K = K;
     ra.pb = ctx->pb;
     ra.pmask = ctx->pmask;
