@@ -7,11 +7,16 @@
 // pc[a][b] > 0. Besides pc (int, K x K) the engine keeps its nonzero pattern
 // as two bitmaps, B (rows a) and BT (rows b), so that the loss terms of a
 // candidate part k -- "receiver r with pc[k][r] == 0" and "sender s with
-// pc[s][k] == 0" -- are one bit of a 64-bit word per (r or s, 64 parts k).
+// pc[s][k] == 0" -- are one bit of a 64-bit word per (r or s, 64 parts k), and
+// the bitmap of its ones, which the gain terms test. The diagonals of B and BT
+// are set: the loss terms skip k == r and k == s.
 //
 // A TM round (the reference runs a whole pass as one round):
-//   k_conn_eval   one wavefront per vertex: receivers, senders and gain on the
-//                 frozen state, then the best part over all k (lanes = k)
+//   k_conn_eval_masks (K <= 512) receivers, senders and gain on the frozen
+//                 state from the nets' part masks (fp_masks.h), the nets of
+//                 several vertices gathered together, then the best part over
+//                 all k (lanes = k)
+//   k_conn_eval   (larger K) the same from the lists, one wavefront per vertex
 //   k_round_compact the candidates in vertex order, with their weights
 //   k_tm_admit    one wavefront: candidates in vertex order, skipping a
 //                 destination whose size reached C * 1.02 (TM/partition.cpp:
@@ -20,9 +25,9 @@
 //   k_conn_apply  (mode 0) one wavefront per touched net replays the admitted
 //                 moves on its list and adds each move's pc changes (atomics:
 //                 pc's final value does not depend on their order)
-//   k_conn_bits   B, BT and msg from pc
+//   k_conn_bits   B, BT, the ones and msg from pc
 // An MSM round:
-//   k_conn_eval, k_round_compact
+//   the evaluation, k_round_compact
 //   k_conn_apply  (mode 1, dry) per touched net and move, the pc changes the
 //                 reference's apply makes, into per-incidence event slots
 //   k_msm_scan    one wavefront applies the moves' pc changes in order, counts
@@ -30,6 +35,7 @@
 //                 after the first move whose max-message set gains a part
 //   k_conn_apply  (mode 2, commit) list edits, part vector and sizes up to the stop
 //   k_conn_bits
+#include "fp_masks.h"
 #include "fp_round.h"
 
 namespace fpe {
@@ -60,38 +66,53 @@ __global__ void __launch_bounds__(256) k_conn_init(const unsigned* __restrict__ 
   }
 }
 
-// One block (four wavefronts) per 64 x 64 tile of pc: the tile's words of B
-// (wavefront 0) and BT (wavefront 1), and the popcounts of its B words into
-// msg (zeroed before; msg null: left as it is).
+// One block (four wavefronts) per 64 x 64 tile of pc: the tile's words of B,
+// BT and the ones, and the popcounts of its B words without the diagonal into
+// msg (zeroed before; msg null: left as it is). A wavefront takes 16 rows, a
+// lane per column, so that a row's word is the ballot of its comparisons; the
+// words of BT are ballots over the tile's columns in LDS. The launch is bound
+// by latency, one load of 16 rows and one exchange through LDS.
+constexpr int BITS_ROWS = 16;
+
 __global__ void __launch_bounds__(256) k_conn_bits(const int* __restrict__ pc, int K, int W,
                                                     unsigned long long* __restrict__ B,
-                                                    unsigned long long* __restrict__ BT, int* __restrict__ msg) {
+                                                    unsigned long long* __restrict__ BT,
+                                                    unsigned long long* __restrict__ ones, int* __restrict__ msg) {
   __shared__ int tile[WAVE][WAVE + 1];
-  const int lane = lane_id(), wave = (int)(threadIdx.x / WAVE);
+  const int lane = lane_id(), r0 = wave_id() * BITS_ROWS;
   const int ta = (int)blockIdx.y, tb = (int)blockIdx.x;
-  for (int r = wave; r < WAVE; r += (int)(blockDim.x / WAVE)) {
-    const int a = ta * WAVE + r, b = tb * WAVE + lane;
-    tile[r][lane] = (a < K && b < K) ? pc[(size_t)a * (size_t)K + (size_t)b] : 0;
+  const int b = tb * WAVE + lane;
+  int x[BITS_ROWS];
+#pragma unroll
+  for (int r = 0; r < BITS_ROWS; r++) {
+    const int a = ta * WAVE + r0 + r;
+    x[r] = a < K && b < K ? pc[(size_t)a * (size_t)K + (size_t)b] : 0;
+  }
+  // lane r < BITS_ROWS: the words of row, and then of column, r0 + r
+  unsigned long long row = 0, one = 0, col = 0;
+#pragma unroll
+  for (int r = 0; r < BITS_ROWS; r++) {
+    tile[r0 + r][lane] = x[r];
+    const unsigned long long rb = __ballot(x[r] > 0), ob = __ballot(x[r] == 1);
+    row = lane == r ? rb : row;
+    one = lane == r ? ob : one;
   }
   __syncthreads();
-  if (wave == 0) {
-    // row a = ta*64 + lane, columns b = tb*64 + c
-    unsigned long long row = 0;
-    for (int c = 0; c < WAVE; c++)
-      if (tile[lane][c] > 0 && ta * WAVE + lane != tb * WAVE + c) row |= 1ull << c;
-    const int a = ta * WAVE + lane;
-    if (a < K) {
-      B[(size_t)a * (size_t)W + (size_t)tb] = row;
-      if (row && msg) atomicAdd(&msg[a], __popcll(row));
-    }
-  } else if (wave == 1) {
-    // row b = tb*64 + lane of the transpose, columns a = ta*64 + c
-    unsigned long long col = 0;
-    for (int c = 0; c < WAVE; c++)
-      if (tile[c][lane] > 0 && ta * WAVE + c != tb * WAVE + lane) col |= 1ull << c;
-    const int b = tb * WAVE + lane;
-    if (b < K) BT[(size_t)b * (size_t)W + (size_t)ta] = col;
+#pragma unroll
+  for (int r = 0; r < BITS_ROWS; r++) {
+    const unsigned long long cb = __ballot(tile[lane][r0 + r] > 0);
+    col = lane == r ? cb : col;
   }
+  if (lane >= BITS_ROWS) return;
+  const unsigned long long diag = ta == tb ? 1ull << (r0 + lane) : 0ull;
+  const int a = ta * WAVE + r0 + lane, c = tb * WAVE + r0 + lane;
+  if (a < K) {
+    B[(size_t)a * (size_t)W + (size_t)tb] = row | diag;
+    ones[(size_t)a * (size_t)W + (size_t)tb] = one;
+    row &= ~diag;
+    if (row && msg) atomicAdd(&msg[a], __popcll(row));
+  }
+  if (c < K) BT[(size_t)c * (size_t)W + (size_t)ta] = col | diag;
 }
 
 struct ConnEvalArgs {
@@ -118,6 +139,10 @@ struct ConnEvalArgs {
   int* touched;
   int* tcount;
   int* tcount_next;
+  // k_conn_eval_masks
+  const unsigned long long* ones;
+  const unsigned long long* masks;
+  int per_wave;  // consecutive slots per wave (<= 64)
 };
 
 __device__ __forceinline__ bool bit_of(const unsigned* m, int p) { return (m[p >> 5] >> (p & 31)) & 1u; }
@@ -256,16 +281,12 @@ __global__ void __launch_bounds__(CONN_BLOCK) __attribute__((amdgpu_waves_per_eu
         // k on ties. A part connected to every receiver and every sender has
         // loss 0, so improvement = gain, the largest possible: the first such
         // candidate is found by ANDing their bitmap words, 64 parts at a time
-        // (an item's own bit counts as connected: its loss term skips k ==
-        // the item)
         auto and_rows = [&](const int* items, int nitems, const unsigned long long* rows, int w) {
           unsigned long long all = ~0ull;
           for (int i0 = 0; i0 < nitems; i0 += WAVE) {
             unsigned long long x = ~0ull;
             if (i0 + lane < nitems) {
-              const int it = items[i0 + lane];
-              x = rows[(size_t)it * (size_t)a.W + (size_t)w];
-              if ((it >> 6) == w) x |= 1ull << (it & 63);
+              x = rows[(size_t)items[i0 + lane] * (size_t)a.W + (size_t)w];
             }
             all &= wave_and_u64(x);
           }
@@ -305,9 +326,9 @@ __global__ void __launch_bounds__(CONN_BLOCK) __attribute__((amdgpu_waves_per_eu
       } else {
         // MSM: every max part must gain strictly more than it loses, no other
         // part may reach the max; improvement = sum over the max parts.
-        // The max parts among the items number X (own and the senders) plus
-        // one if k is a max part outside them, and must be all cntM of them:
-        // with X + 1 < cntM no k passes
+        // The max parts among the items (own and the senders) number X and must
+        // be all cntM of them: a max part k outside the items gains nothing,
+        // so with X < cntM no k passes
         const bool own_s = bit_of(smark, own);
         const int g_own = gain_own + ((own_s && bit_of(sgain, own)) ? 1 : 0);
         int X = 0;
@@ -318,7 +339,7 @@ __global__ void __launch_bounds__(CONN_BLOCK) __attribute__((amdgpu_waves_per_eu
         X = wave_sum(X) + (a.msg[own] == M ? 1 : 0);
         const int m_own = a.msg[own];
         int bimp = -1, bk = INT_MAX;
-        for (int k0 = 0; X + 1 >= cntM && k0 < K; k0 += WAVE) {
+        for (int k0 = 0; X == cntM && k0 < K; k0 += WAVE) {
           const int k = k0 + lane, w = k0 / WAVE;
           const bool valid = k < K && k != own;
           const int kc = valid ? k : own;
@@ -390,6 +411,305 @@ __global__ void __launch_bounds__(CONN_BLOCK) __attribute__((amdgpu_waves_per_eu
     wave_lds_sync();
   }
   block_touch_flush(tb, a.touched, a.tcount, s_tn);
+}
+
+// k_conn_eval through the nets' part masks (fp_masks.h), for K <= 64 P. A wave
+// takes per_wave consecutive vertices, whose nets are consecutive too: as many
+// whole vertices as have 64 nets together are gathered at once, a net per lane
+// (source, source part, the single bit of the vertex's part, pc's bits and the
+// messages), so that the chain of four dependent reads is paid per 64 nets and
+// not per vertex. Per vertex the rest is scalar masks over those lanes: the
+// receivers are the present words of its source nets' records, the senders the
+// first lane of each source part, the gains popcounts against the ones bitmap.
+//   TM: the rows of BT (receivers) and B (senders) are counted like records
+//   (mask_count): loss(k) = items - count(k), so the best part is the largest
+//   count over the parts lighter than C, the lowest k on ties.
+//   MSM: with m the messages, M their maximum and l_s(k) = 1 where pc[s][k] is
+//   0, a part k passes when all cntM max parts are among own and the senders
+//   and each gains more than it loses, and no other item reaches M:
+//     a max sender needs its gain bit and l_s(k) = 0 (unless it is k);
+//     a sender of M - 1 messages without a gain needs l_s(k) = 0 (unless it is k);
+//     own, if a sender, needs l_own(k) = 0 where one more would break its rule;
+//     k needs receiver losses(k) < gain bit(k) + M - m_k.
+//   The improvement differs between the parts that pass only by l_own(k) of a
+//   max own. Most vertices end at the first condition, before any row is read.
+template <int P, bool MSM>
+__global__ void __launch_bounds__(CONN_BLOCK) __attribute__((amdgpu_waves_per_eu(P <= 6 ? 7 : 6, P <= 6 ? 7 : 6)))
+k_conn_eval_masks(ConnEvalArgs a) {
+  constexpr int NW = CONN_BLOCK / WAVE;
+  constexpr unsigned ROW = 16u * P, BROW = 8u * P;  // bytes of a record and of a bitmap row
+  __shared__ unsigned s_items[NW][WAVE];  // byte offsets (from B) of rows to count
+  __shared__ unsigned s_seen[NW][2 * P];  // a vertex of several chunks: its senders so far
+  __shared__ unsigned s_gain[NW][2 * P];  // MSM: the vertex's senders with a gain
+  __shared__ unsigned s_touch[NW][TOUCH_BUF];
+  __shared__ int s_tn[NW + 1];
+  const int K = a.K;
+  const int lane = lane_id(), wave = wave_id();
+  unsigned* items = s_items[wave];
+  unsigned* seen = s_seen[wave];
+  unsigned* sgain = s_gain[wave];
+  WaveTouch tb{s_touch[wave], 0};
+  const int s0 = ((int)blockIdx.x * NW + wave) * a.per_wave;
+  const int ns = min(a.per_wave, a.nslots - s0);
+  if (blockIdx.x == 0 && threadIdx.x == 0 && a.tcount_next) *a.tcount_next = 0;
+
+  // lane i: slot s0 + i's part and net range
+  int own_l = 0, m_l = 0;
+  unsigned vb_l = 0, ve_l = 0;
+  if (lane < ns) {
+    const int v = a.r0 + s0 + lane;
+    own_l = a.part[v];
+    vb_l = a.vtx_ptr[v];
+    ve_l = a.vtx_ptr[v + 1];
+    if (MSM) m_l = a.msg[own_l];
+  }
+  if (lane < 2 * P) {
+    seen[lane] = 0u;
+    sgain[lane] = 0u;
+  }
+  unsigned light = 0;  // TM, bit u: part 64 u + lane is lighter than C
+  if (!MSM) {
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      const int k = u * WAVE + lane;
+      light |= k < K && (double)a.sizes[min(k, K - 1)] < a.C ? 1u << u : 0u;
+    }
+  }
+  const int M = MSM ? uniform_load(a.mstat) : 0, cntM = MSM ? uniform_load(a.mstat + 1) : 0;
+  const unsigned bt = (unsigned)K * BROW;  // BT's rows follow B's
+  const unsigned long long lt = (1ull << lane) - 1ull;
+  wave_lds_sync();
+
+  int dec_l = -1;  // lane i: slot s0 + i's decision
+  for (int i = 0; i < ns;) {
+    // vertices i .. i1 - 1: the ones whose nets fit 64 lanes, or one larger vertex by itself
+    const unsigned cb = (unsigned)__builtin_amdgcn_readlane((int)vb_l, i);
+    const unsigned long long fit = __ballot(lane >= i && lane < ns && ve_l - cb <= (unsigned)WAVE);
+    const bool big = fit == 0ull;
+    const int i1 = big ? i + 1 : WAVE - __builtin_clzll(fit);
+    const unsigned ce = (unsigned)__builtin_amdgcn_readlane((int)ve_l, i1 - 1);
+    unsigned cnt[P];
+    int gain_s = 0, nit = 0, nitems = 0, X = 0, own_s = 0, own_g = 0;
+    bool bad = false;
+    auto flush = [&]() {
+      if (nit == 0) return;
+      wave_lds_sync();
+      const unsigned off = items[lane];
+      mask_count<P, false>(a.B, off, nit, cnt);
+      nitems += nit;
+      nit = 0;
+      wave_lds_sync();
+    };
+    int j = i;
+    for (unsigned c0 = cb; j < i1; c0 += (unsigned)WAVE) {
+      // lane: one net of vertex i + vi
+      const int nn = (int)min((unsigned)WAVE, ce - c0);
+      int vi = i;
+      for (int t = i + 1; t < i1; t++) vi += (unsigned)__builtin_amdgcn_readlane((int)vb_l, t) - c0 <= (unsigned)lane ? 1 : 0;
+      const int own_n = __shfl(own_l, vi);
+      unsigned net = 0;
+      int ps = -1, m_s = -1;
+      bool isrc = false, sgl = false, one = false;
+      if (lane < nn) {
+        net = a.vtx_nets[c0 + (unsigned)lane];
+        const int s = a.src[net];
+        const unsigned* rec = reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(a.masks) + net * ROW);
+        sgl = (rec[2 * P + (own_n >> 5)] >> (own_n & 31)) & 1u;
+        isrc = s == a.r0 + s0 + vi;
+        ps = a.part[s];
+        const unsigned* orow = reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(a.ones) + (unsigned)ps * BROW);
+        one = (orow[own_n >> 5] >> (own_n & 31)) & 1u;
+        if (MSM) m_s = a.msg[ps];
+      }
+      const unsigned long long SRC = __ballot(isrc), SGL = __ballot(sgl), GAIN = __ballot(sgl && one && !isrc);
+      const unsigned long long MAXM = MSM ? __ballot(m_s == M) : 0ull, M1 = MSM ? __ballot(m_s == M - 1) : 0ull;
+
+      for (; j < i1; j++) {
+        const int own = __builtin_amdgcn_readlane(own_l, j);
+        const unsigned vb = (unsigned)__builtin_amdgcn_readlane((int)vb_l, j);
+        const unsigned ve = (unsigned)__builtin_amdgcn_readlane((int)ve_l, j);
+        if (vb >= c0) {
+#pragma unroll
+          for (int u = 0; u < P; u++) cnt[u] = 0;
+          gain_s = nit = nitems = X = own_s = own_g = 0;
+          bad = false;
+        }
+        // the vertex's lanes of this chunk
+        const int b = big ? 0 : (int)(vb - c0), e = (int)min(ve - c0, (unsigned)WAVE);
+        const unsigned long long range = (e == WAVE ? ~0ull : (1ull << e) - 1ull) & (b == WAVE ? 0ull : ~0ull << b);
+        // senders: the first net of each source part in the vertex's net order
+        unsigned long long m = range & ~SRC, fm = 0;
+        if (big) m &= ~__ballot(((m >> lane) & 1ull) && bit_of(seen, ps));
+        while (m) {
+          const unsigned long long bit = m & (0ull - m);
+          fm |= bit;
+          m &= ~__ballot(ps == __builtin_amdgcn_readlane(ps, __builtin_ctzll(m)));
+        }
+        const bool first = (fm >> lane) & 1ull;
+        gain_s += (int)__popcll(fm & GAIN);
+        unsigned long long rows = fm;  // the senders whose rows the decision needs
+        if (MSM) {
+          const unsigned long long ownm = fm & __ballot(ps == own);
+          own_s |= ownm != 0ull;
+          own_g |= (ownm & GAIN) != 0ull;
+          X += (int)__popcll(fm & MAXM & ~ownm);
+          bad |= (fm & MAXM & ~ownm & ~GAIN) != 0ull;
+          rows &= ~ownm & (MAXM | (M1 & ~GAIN));
+          if (fm & GAIN) {
+            if (first && ((GAIN >> lane) & 1ull)) atomicOr(&sgain[ps >> 5], 1u << (ps & 31));
+          }
+        }
+        if (big) {
+          if (first) atomicOr(&seen[ps >> 5], 1u << (ps & 31));
+          if (nit + (int)__popcll(rows) > WAVE) flush();
+          wave_lds_sync();
+        }
+        if ((rows >> lane) & 1ull) items[nit + (int)__popcll(rows & lt)] = (unsigned)ps * BROW;
+        nit += (int)__popcll(rows);
+        if (ve - c0 > (unsigned)WAVE) break;  // the vertex goes on in the next chunk
+
+        // the vertex's receivers, what its source nets list after it left, and its gain there
+        auto receivers = [&](unsigned long long(&recv)[P]) -> int {
+          int gain = 0;
+#pragma unroll
+          for (int u = 0; u < P; u++) recv[u] = 0;
+          for (unsigned c = big ? vb : c0; c <= c0; c += (unsigned)WAVE) {
+            unsigned n = net;
+            unsigned long long sm = range & SRC, alone = SGL;
+            if (c < c0) {  // an earlier chunk of a larger vertex
+              n = a.vtx_nets[c + (unsigned)lane];
+              sm = __ballot(a.src[n] == a.r0 + s0 + j);
+              const unsigned* rec = reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(a.masks) + n * ROW);
+              alone = __ballot((rec[2 * P + (own >> 5)] >> (own & 31)) & 1u);
+            }
+            for (; sm; sm &= sm - 1) {
+              const int jn = __builtin_ctzll(sm);
+              unsigned long long w[P], o1[P];
+              mask_load<P>(a.masks, (unsigned)__builtin_amdgcn_readlane((int)n, jn) * ROW, w);
+              mask_load<P>(a.ones, (unsigned)own * BROW, o1);
+              const unsigned long long left = 1ull << (own & 63), kept = (alone >> jn) & 1ull ? 0ull : left;
+#pragma unroll
+              for (int u = 0; u < P; u++) {
+                const bool mine = (own >> 6) == u;
+                gain += (int)__popcll(w[u] & o1[u] & (mine ? ~left : ~0ull));
+                recv[u] |= w[u] & (mine ? ~left | kept : ~0ull);
+              }
+            }
+          }
+          return gain;
+        };
+        // counts the receivers' rows
+        auto count_rows = [&](const unsigned long long(&recv)[P]) {
+          int nr = 0;
+#pragma unroll
+          for (int u = 0; u < P; u++) nr += (int)__popcll(recv[u]);
+          const bool fits = nit + nr <= WAVE;
+#pragma unroll
+          for (int u = 0; u < P; u++) {
+            if (recv[u] == 0ull) continue;
+            if (!fits) flush();
+            if ((recv[u] >> lane) & 1ull)
+              items[nit + (int)__popcll(recv[u] & lt)] = bt + (unsigned)(u * WAVE + lane) * BROW;
+            nit += (int)__popcll(recv[u]);
+          }
+          flush();
+        };
+        int dec = -1;
+        if (!MSM) {
+          unsigned long long recv[P];
+          const int gain = gain_s + receivers(recv);
+          if (gain > 0) {
+            count_rows(recv);
+            unsigned key = 0;  // 8 * (count + 1) + 7 - u
+#pragma unroll
+            for (int u = 0; u < P; u++) {
+              const bool ok = ((light >> u) & 1u) && u * WAVE + lane != own;
+              key = max(key, ok ? 8u * cnt[u] + (15u - (unsigned)u) : 0u);
+            }
+            const unsigned mk = wave_max_u32(key);
+            if (mk != 0u && gain - nitems + (int)(mk >> 3) - 1 > 0)
+              dec = (int)(7u - (mk & 7u)) * WAVE + __builtin_ctzll(__ballot(key == mk));
+          }
+        } else {
+          const int m_own = __builtin_amdgcn_readlane(m_l, j);
+          const bool own_max = m_own == M;
+          unsigned long long recv[P];
+          int gain_own = 0;
+          bool go = !bad && X + (own_max ? 1 : 0) == cntM;
+          if (go) {
+            gain_own = receivers(recv);
+            go = gain_own + gain_s > 0 && (!own_max || gain_own + own_g > 0);
+          }
+          if (go) {
+            const int g_own = gain_own + own_g;
+            if (own_s && (own_max ? g_own == 1 : m_own + 1 - g_own >= M)) {
+              if (nit == WAVE) flush();
+              if (lane == 0) items[nit] = (unsigned)own * BROW;
+              nit++;
+            }
+            flush();
+            unsigned good = 0;
+#pragma unroll
+            for (int u = 0; u < P; u++) {
+              good |= cnt[u] == (unsigned)nitems && u * WAVE + lane < K && u * WAVE + lane != own ? 1u << u : 0u;
+              cnt[u] = 0;
+            }
+            if (__ballot(good != 0u)) {
+              nitems = 0;
+              (void)receivers(recv);
+              count_rows(recv);
+              unsigned key = ~0u;  // l_own(k), then k
+#pragma unroll
+              for (int u = 0; u < P; u++) {
+                const int k = u * WAVE + lane;
+                const int gk = (int)((sgain[k >> 5] >> (k & 31)) & 1u);
+                const int l = own_max && own_s
+                                  ? (int)!((a.B[(size_t)own * (size_t)P + (size_t)u] >> lane) & 1ull)
+                                  : 0;
+                const bool ok = ((good >> u) & 1u) && nitems - (int)cnt[u] < gk + M - a.msg[min(k, K - 1)];
+                key = min(key, ok ? ((unsigned)l << 16) | (unsigned)k : ~0u);
+              }
+              const unsigned mk = wave_min_u32(key);
+              if (mk != ~0u) dec = (int)(mk & 0xFFFFu);
+            }
+          }
+          if (gain_s > 0) {
+            wave_lds_sync();
+            if (lane < 2 * P) sgain[lane] = 0u;
+            wave_lds_sync();
+          }
+        }
+        if (big) {
+          wave_lds_sync();
+          if (lane < 2 * P) seen[lane] = 0u;
+          wave_lds_sync();
+        }
+        dec_l = lane == j ? dec : dec_l;
+        if (dec >= 0) wave_touch_nets_staged(a.vtx_nets + vb, (int)(ve - vb), a.tag, a.net_stamp, tb, a.touched, a.tcount);
+      }
+    }
+    i = i1;
+  }
+  if (lane < ns) {
+    a.slot_own[s0 + lane] = own_l;
+    a.slot_dec[s0 + lane] = dec_l;
+  }
+  block_touch_flush(tb, a.touched, a.tcount, s_tn);
+}
+
+// the instance of k_conn_eval_masks for K parts
+template <bool MSM>
+void (*conn_masks_kernel(int K))(ConnEvalArgs) {
+  switch (mask_words(K)) {
+    case 1: return k_conn_eval_masks<1, MSM>;
+    case 2: return k_conn_eval_masks<2, MSM>;
+    case 3: return k_conn_eval_masks<3, MSM>;
+    case 4: return k_conn_eval_masks<4, MSM>;
+    case 5: return k_conn_eval_masks<5, MSM>;
+    case 6: return k_conn_eval_masks<6, MSM>;
+    case 7: return k_conn_eval_masks<7, MSM>;
+    default: return k_conn_eval_masks<8, MSM>;
+  }
 }
 
 // TM apply order (TM/partition.cpp:1111-1125): the round's candidates (the
@@ -550,6 +870,8 @@ struct ConnApplyArgs {
   int* pc;
   int2* evbuf;
   unsigned long long* moves;
+  unsigned long long* masks;  // nullable: the nets' part masks, kept in step with the lists
+  int mask_words;
   int K, pb;
   unsigned pmask;
   int r0, r1;
@@ -609,6 +931,7 @@ __global__ void __launch_bounds__(REPLAY_BLOCK) k_conn_apply(ConnApplyArgs a) {
     return;
   }
   unsigned* list = reinterpret_cast<unsigned*>(lds) + (size_t)wave * (size_t)a.K;
+  unsigned* mask_lds = reinterpret_cast<unsigned*>(lds) + (size_t)nw * (size_t)a.K + (size_t)(wave * 4 * a.mask_words);
   const int ntouched = *a.tcount;
   for (int i = (int)blockIdx.x * nw + wave; i < ntouched; i += a.net_blocks * nw) {
     const int n = a.touched[i];
@@ -682,7 +1005,12 @@ __global__ void __launch_bounds__(REPLAY_BLOCK) k_conn_apply(ConnApplyArgs a) {
         if (is_src) sp = d;
       }
     }
-    if (a.mode != 1 && dirty) wave_list_store(a.ent, a.ev, seg, list, L, a.pb, a.pmask);
+    if (a.mode != 1 && dirty) {
+      wave_list_store(a.ent, a.ev, seg, list, L, a.pb, a.pmask);
+      if (a.masks)
+        wave_store_list_masks(list, L, a.pb, a.pmask, a.mask_words, mask_lds,
+                              a.masks + (size_t)n * (size_t)(2 * a.mask_words));
+    }
     wave_lds_sync();
   }
 }
@@ -800,8 +1128,7 @@ fp_status ensure_conn_scratch(fp_ctx* ctx, int R) {
   if (K > c.kcap) {
     FP_TRY(dalloc(ctx, &c.pc, (size_t)K * (size_t)K));
     FP_TRY(dalloc(ctx, &c.msg, (size_t)K));
-    FP_TRY(dalloc(ctx, &c.B, (size_t)K * (size_t)W));
-    FP_TRY(dalloc(ctx, &c.BT, (size_t)K * (size_t)W));
+    FP_TRY(dalloc(ctx, &c.B, 3 * (size_t)K * (size_t)W));
     FP_TRY(dalloc(ctx, &c.mstat, 8));
     c.kcap = K;
   }
@@ -819,13 +1146,14 @@ fp_status ensure_conn_scratch(fp_ctx* ctx, int R) {
   return FP_OK;
 }
 
-// B and BT from pc, and msg recounted unless the caller has it (an MSM round's
+// B, BT and the ones from pc, and msg recounted unless the caller has it (an MSM round's
 // scan leaves the exact counts)
 void launch_bits(fp_ctx* ctx, bool recount_msg = true) {
   auto& c = ctx->conn;
   const int K = ctx->K, W = (K + 63) / 64;
   if (recount_msg) fill_async<int>(ctx, c.msg, (size_t)K, 0);
-  k_conn_bits<<<dim3((unsigned)W, (unsigned)W), 256, 0, ctx->stream>>>(c.pc, K, W, c.B, c.BT,
+  const size_t n = (size_t)K * (size_t)W;
+  k_conn_bits<<<dim3((unsigned)W, (unsigned)W), 256, 0, ctx->stream>>>(c.pc, K, W, c.B, c.B + n, c.B + 2 * n,
                                                                        recount_msg ? c.msg : nullptr);
 }
 
@@ -856,6 +1184,9 @@ fp_status plan_conn(fp_ctx* ctx, RefinePlan& p) {
   k_conn_init<<<std::min(ngrid * 8, 4096), 256, 0, ctx->stream>>>(ctx->net_ptr, ctx->ent, ctx->src, ctx->part, ctx->noe, ctx->pmask, K,
                                                c.pc);
   launch_bits(ctx);
+  // the part masks of the resident lists, kept in step by the passes
+  p.masks = ensure_masks(ctx);
+  if (p.masks) build_masks(ctx, p.masks);
   FP_HIP_OK(hipGetLastError());
   return FP_OK;
 }
@@ -865,7 +1196,8 @@ fp_status pass_conn(fp_ctx* ctx, const RefinePlan& p) {
   const int nov = ctx->nov, K = ctx->K, W = (K + 63) / 64, R = p.R, waves = p.eval_waves;
   const int rcap = conn_rcap(ctx), scap = conn_scap(ctx);
   const size_t lds_e = conn_eval_lds(K, waves, rcap, scap);
-  const size_t lds_r = (size_t)(REPLAY_BLOCK / WAVE) * (size_t)K * sizeof(unsigned);
+  const int P = p.masks ? mask_words(K) : 0;
+  const size_t lds_r = (size_t)(REPLAY_BLOCK / WAVE) * (size_t)(K + 4 * P) * sizeof(unsigned);
   auto& c = ctx->conn;
   const double thr = p.sched.ldg_C * (1.02);
   pass_begin(ctx, msm ? c.msg : nullptr, K, c.mstat);
@@ -884,7 +1216,7 @@ fp_status pass_conn(fp_ctx* ctx, const RefinePlan& p) {
     a.sizes = ctx->sizes;
     a.pc = c.pc;
     a.B = c.B;
-    a.BT = c.BT;
+    a.BT = c.B + (size_t)K * (size_t)W;
     a.msg = c.msg;
     a.mstat = c.mstat;
     a.K = K;
@@ -902,9 +1234,16 @@ fp_status pass_conn(fp_ctx* ctx, const RefinePlan& p) {
     a.touched = ctx->touched;
     a.tcount = ctx->counters + par;
     a.tcount_next = ctx->counters + (par ^ 1);
-    int egrid = std::max(1, std::min((nslots + waves - 1) / waves, 8192));
-    if (p.eval_grid > 0) egrid = std::min(egrid, p.eval_grid);
-    FP_TRY(launch_timed(ctx, k_conn_eval, egrid, waves * WAVE, lds_e, a));
+    if (p.masks) {
+      a.ones = c.B + 2 * (size_t)K * (size_t)W;
+      a.masks = p.masks;
+      const int egrid = mask_eval_grid(nslots, p.eval_grid, CONN_BLOCK / WAVE, a.per_wave);
+      FP_TRY(launch_timed(ctx, msm ? conn_masks_kernel<true>(K) : conn_masks_kernel<false>(K), egrid, CONN_BLOCK, 0, a));
+    } else {
+      int egrid = std::max(1, std::min((nslots + waves - 1) / waves, 8192));
+      if (p.eval_grid > 0) egrid = std::min(egrid, p.eval_grid);
+      FP_TRY(launch_timed(ctx, k_conn_eval, egrid, waves * WAVE, lds_e, a));
+    }
     ConnApplyArgs ap{};
     ap.net_ptr = ctx->net_ptr;
     ap.apply_pins = ctx->apply_pins;
@@ -927,6 +1266,8 @@ fp_status pass_conn(fp_ctx* ctx, const RefinePlan& p) {
     ap.pc = c.pc;
     ap.evbuf = c.evbuf;
     ap.moves = ctx->moves;
+    ap.masks = p.masks;
+    ap.mask_words = P;
     ap.K = K;
     ap.pb = ctx->pb;
     ap.pmask = ctx->pmask;

@@ -765,8 +765,9 @@ struct fp_ctx {
   struct {
     int* pc = nullptr;                 // K*K: nets with source in part a and pins in part b
     int* msg = nullptr;                // K: parts each part sends to
-    unsigned long long* B = nullptr;   // K rows of ceil(K/64) words: bit (a, b) = pc[a][b] > 0
-    unsigned long long* BT = nullptr;  // transpose of B
+    // K rows of ceil(K/64) words: bit (a, b) = pc[a][b] > 0 or a == b; then its
+    // transpose, then the bits pc[a][b] == 1
+    unsigned long long* B = nullptr;
     int* mstat = nullptr;              // as vol.mstat, over msg
     int* slot_mi = nullptr;
     int4* mv = nullptr;

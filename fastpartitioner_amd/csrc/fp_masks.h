@@ -280,6 +280,24 @@ __device__ __forceinline__ void wave_store_entry_masks(bool in, unsigned key, un
   wave_lds_sync();
 }
 
+// One wavefront's record from a list in LDS, assembled in 4 P LDS words of the
+// wave's own.
+__device__ __forceinline__ void wave_store_list_masks(const unsigned* list, int L, int pb, unsigned pmask, int P,
+                                                      unsigned* words, unsigned long long* __restrict__ out) {
+  const int lane = lane_id();
+  if (lane < 4 * P) words[lane] = 0u;
+  wave_lds_sync();
+  for (int t = lane; t < L; t += WAVE) {
+    const unsigned x = list[t];
+    const unsigned q = x & pmask, bit = 1u << (q & 31u);
+    atomicOr(&words[q >> 5], bit);
+    if ((x >> pb) == 1u) atomicOr(&words[2 * P + (int)(q >> 5)], bit);
+  }
+  wave_lds_sync();
+  if (lane < 4 * P) reinterpret_cast<unsigned*>(out)[lane] = words[lane];
+  wave_lds_sync();
+}
+
 // One wavefront's record from a list in LDS with its part -> position index
 // (wave_index_set): lane l looks up parts l, l + 64, ...
 __device__ __forceinline__ void wave_store_masks(const unsigned* list, const unsigned short* at, int K, int pb, int P,

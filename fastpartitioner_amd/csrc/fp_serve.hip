@@ -112,7 +112,7 @@ long long scratch_bytes(const fp_server::Graph& g, fp_metric metric, int K, int 
 // optional: a request that fits the budget only without them is evaluated
 // through the lists.
 long long mask_bytes(const fp_server::Graph& g, fp_metric metric, int K) {
-  return metric == FP_METRIC_TV || metric == FP_METRIC_MSV || metric == FP_METRIC_MSRV ? 16ll * fpe::mask_words(K) * ((long long)g.noe + 1) : 0;
+  return metric == FP_METRIC_CN ? 0 : 16ll * fpe::mask_words(K) * ((long long)g.noe + 1);
 }
 
 // a new context holding graph g's upload (the caller holds no lock)

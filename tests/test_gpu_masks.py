@@ -102,3 +102,40 @@ def test_masks_follow_every_change_of_the_lists():
             O.cn_refine(hg, st, 1, serial=False)
             st.sizes = st.sizes.astype(np.int64)
             _same(eng.get_state(), st)
+
+
+def _sparse(seed, nov=3000, hubs=(60, 63, 64, 65, 127, 129, 200)):
+    # short nets, so that single connections between parts (what a message gain
+    # needs) exist, a few long ones, random sources, and hub vertices
+    rng = np.random.default_rng(seed)
+    sizes = [65, 130, 700] + list(rng.integers(1, 4, nov))
+    nets = [list(rng.choice(np.arange(len(hubs), nov), size=s, replace=False)) for s in sizes]
+    for h, d in enumerate(hubs):
+        for i in rng.choice(np.arange(3, len(nets)), size=d, replace=False):
+            nets[i].append(h)
+    net_ptr = np.zeros(len(nets) + 1, dtype=np.uint32)
+    net_ptr[1:] = np.cumsum([len(n) for n in nets])
+    pins = np.concatenate([np.array(n) for n in nets]).astype(np.uint32)
+    return H.Hypergraph.from_nets(nov, net_ptr, pins, np.array([n[rng.integers(len(n))] for n in nets], np.int32))
+
+
+@pytest.mark.parametrize("metric", ["TM", "MSM"])
+@pytest.mark.parametrize("K", [2, 63, 64, 65, 129, 192, 257, 320, 449, 512, 513])
+def test_message_masks_at_word_edges(metric, K):
+    hg = _sparse(K)
+    C, max_pw, min_pw = H.ref_constants(hg.nov, K)
+    for R in ((700, 1 << 30) if metric == "TM" else (100, 900)):
+        st = O.tm_init(hg, K, C) if metric == "TM" else O.msm_init(hg, K, C)
+        print(f"message masks: {metric} K={K} R={R} pins={hg.pins}", flush=True)
+        with Engine(0) as eng:
+            eng.upload(hg)
+            eng.set_state(K, st.part, st.ep_ends, st.ep_parts, st.ep_cnt, st.sizes)
+            stats = eng.refine(metric, 4, schedule(SCHED_REF, R, C, max_pw, min_pw))
+            got = eng.get_state()
+            pc, msg = eng.connections()
+        moves = O.tm_refine_par(hg, st, C, 4, R) if metric == "TM" else O.msm_refine_par(hg, st, 4, R)
+        assert stats.moves == moves
+        _same(got, st)
+        want = st.pc.reshape(K, K).copy()
+        np.fill_diagonal(want, 0)
+        assert np.array_equal(pc, want) and np.array_equal(msg, st.msg)
