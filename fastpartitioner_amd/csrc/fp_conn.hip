@@ -477,6 +477,10 @@ k_conn_eval_masks(ConnEvalArgs a) {
   }
   const int M = MSM ? uniform_load(a.mstat) : 0, cntM = MSM ? uniform_load(a.mstat + 1) : 0;
   const unsigned bt = (unsigned)K * BROW;  // BT's rows follow B's
+  // lane l < 2 P: word l of the row at byte offset off (the others: the last word)
+  auto row_word = [&](const unsigned long long* rows, unsigned off) -> unsigned {
+    return *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(rows) + (off + 4u * (unsigned)min(lane, 2 * P - 1)));
+  };
   const unsigned long long lt = (1ull << lane) - 1ull;
   wave_lds_sync();
 
@@ -488,6 +492,7 @@ k_conn_eval_masks(ConnEvalArgs a) {
     const bool big = fit == 0ull;
     const int i1 = big ? i + 1 : WAVE - __builtin_clzll(fit);
     const unsigned ce = (unsigned)__builtin_amdgcn_readlane((int)ve_l, i1 - 1);
+    const int dmax = big ? WAVE : (int)wave_max_u32((fit >> lane) & 1ull ? ve_l - vb_l : 0u);
     unsigned cnt[P];
     int gain_s = 0, nit = 0, nitems = 0, X = 0, own_s = 0, own_g = 0;
     bool bad = false;
@@ -522,6 +527,18 @@ k_conn_eval_masks(ConnEvalArgs a) {
         if (MSM) m_s = a.msg[ps];
       }
       const unsigned long long SRC = __ballot(isrc), SGL = __ballot(sgl), GAIN = __ballot(sgl && one && !isrc);
+      // the first net of each source part among each vertex's: no earlier lane
+      // of the vertex has the same part (all vertices of the chunk together,
+      // the lanes shifted one further at a time)
+      unsigned long long FIRST = ~SRC & (nn == WAVE ? ~0ull : (1ull << nn) - 1ull);
+      {
+        const int key = lane < nn && !isrc ? (vi << 16) | ps : -1;
+        int x = key;
+        for (int d = 1; d < dmax; d++) {
+          x = wave_shift_up(x);
+          FIRST &= ~__ballot(x == key);
+        }
+      }
       const unsigned long long MAXM = MSM ? __ballot(m_s == M) : 0ull, M1 = MSM ? __ballot(m_s == M - 1) : 0ull;
 
       for (; j < i1; j++) {
@@ -538,41 +555,23 @@ k_conn_eval_masks(ConnEvalArgs a) {
         const int b = big ? 0 : (int)(vb - c0), e = (int)min(ve - c0, (unsigned)WAVE);
         const unsigned long long range = (e == WAVE ? ~0ull : (1ull << e) - 1ull) & (b == WAVE ? 0ull : ~0ull << b);
         // senders: the first net of each source part in the vertex's net order
-        unsigned long long m = range & ~SRC, fm = 0;
-        if (big) m &= ~__ballot(((m >> lane) & 1ull) && bit_of(seen, ps));
-        while (m) {
-          const unsigned long long bit = m & (0ull - m);
-          fm |= bit;
-          m &= ~__ballot(ps == __builtin_amdgcn_readlane(ps, __builtin_ctzll(m)));
-        }
-        const bool first = (fm >> lane) & 1ull;
-        gain_s += (int)__popcll(fm & GAIN);
-        unsigned long long rows = fm;  // the senders whose rows the decision needs
-        if (MSM) {
-          const unsigned long long ownm = fm & __ballot(ps == own);
-          own_s |= ownm != 0ull;
-          own_g |= (ownm & GAIN) != 0ull;
-          X += (int)__popcll(fm & MAXM & ~ownm);
-          bad |= (fm & MAXM & ~ownm & ~GAIN) != 0ull;
-          rows &= ~ownm & (MAXM | (M1 & ~GAIN));
-          if (fm & GAIN) {
-            if (first && ((GAIN >> lane) & 1ull)) atomicOr(&sgain[ps >> 5], 1u << (ps & 31));
-          }
-        }
+        unsigned long long fm = range & FIRST;
         if (big) {
-          if (first) atomicOr(&seen[ps >> 5], 1u << (ps & 31));
-          if (nit + (int)__popcll(rows) > WAVE) flush();
-          wave_lds_sync();
+          fm &= ~__ballot(((fm >> lane) & 1ull) && bit_of(seen, ps));
+          if ((fm >> lane) & 1ull) atomicOr(&seen[ps >> 5], 1u << (ps & 31));
         }
-        if ((rows >> lane) & 1ull) items[nit + (int)__popcll(rows & lt)] = (unsigned)ps * BROW;
-        nit += (int)__popcll(rows);
-        if (ve - c0 > (unsigned)WAVE) break;  // the vertex goes on in the next chunk
+        gain_s += (int)__popcll(fm & GAIN);
+        const bool last = ve - c0 <= (unsigned)WAVE;  // the vertex ends in this chunk
 
-        // the vertex's receivers, what its source nets list after it left, and its gain there
-        auto receivers = [&](unsigned long long(&recv)[P]) -> int {
-          int gain = 0;
-#pragma unroll
-          for (int u = 0; u < P; u++) recv[u] = 0;
+        // Receivers: what the vertex's source nets list after it left, and its
+        // gain there. Lane l < 2 P takes words l of the rows.
+        unsigned rw = 0;
+        auto receivers = [&]() -> int {
+          if (!big && (range & SRC) == 0ull) return 0;
+          const unsigned left = lane == (own >> 5) ? 1u << (own & 31) : 0u;
+          const unsigned o1 = row_word(a.ones, (unsigned)own * BROW) & ~left;
+          int g = 0;
+          rw = 0;
           for (unsigned c = big ? vb : c0; c <= c0; c += (unsigned)WAVE) {
             unsigned n = net;
             unsigned long long sm = range & SRC, alone = SGL;
@@ -584,42 +583,53 @@ k_conn_eval_masks(ConnEvalArgs a) {
             }
             for (; sm; sm &= sm - 1) {
               const int jn = __builtin_ctzll(sm);
-              unsigned long long w[P], o1[P];
-              mask_load<P>(a.masks, (unsigned)__builtin_amdgcn_readlane((int)n, jn) * ROW, w);
-              mask_load<P>(a.ones, (unsigned)own * BROW, o1);
-              const unsigned long long left = 1ull << (own & 63), kept = (alone >> jn) & 1ull ? 0ull : left;
-#pragma unroll
-              for (int u = 0; u < P; u++) {
-                const bool mine = (own >> 6) == u;
-                gain += (int)__popcll(w[u] & o1[u] & (mine ? ~left : ~0ull));
-                recv[u] |= w[u] & (mine ? ~left | kept : ~0ull);
-              }
+              const unsigned w = row_word(a.masks, (unsigned)__builtin_amdgcn_readlane((int)n, jn) * ROW);
+              g += (int)__popc(w & o1);
+              rw |= (alone >> jn) & 1ull ? w & ~left : w;
             }
           }
-          return gain;
+          return wave_sum(lane < 2 * P ? g : 0);
         };
-        // counts the receivers' rows
-        auto count_rows = [&](const unsigned long long(&recv)[P]) {
-          int nr = 0;
-#pragma unroll
-          for (int u = 0; u < P; u++) nr += (int)__popcll(recv[u]);
-          const bool fits = nit + nr <= WAVE;
-#pragma unroll
-          for (int u = 0; u < P; u++) {
-            if (recv[u] == 0ull) continue;
-            if (!fits) flush();
-            if ((recv[u] >> lane) & 1ull)
-              items[nit + (int)__popcll(recv[u] & lt)] = bt + (unsigned)(u * WAVE + lane) * BROW;
-            nit += (int)__popcll(recv[u]);
+        // counts the rows of the items and of the receivers
+        auto count_rows = [&]() {
+          for (unsigned long long m = __ballot(lane < 2 * P && rw != 0u); m; m &= m - 1) {
+            const int q = __builtin_ctzll(m);
+            const unsigned x = (unsigned)__builtin_amdgcn_readlane((int)rw, q);
+            if (nit + (int)__popc(x) > WAVE) flush();
+            if (lane < 32 && ((x >> (lane & 31)) & 1u))
+              items[nit + (int)__popc(x & (unsigned)lt)] = bt + (unsigned)(32 * q + lane) * BROW;
+            nit += (int)__popc(x);
           }
           flush();
         };
+        int gain = 0;
+        if (!MSM) {
+          if (last) gain = gain_s + receivers();
+          if (!big && gain <= 0) continue;
+        }
+        unsigned long long rows = fm;  // the senders whose rows the decision needs
+        if (MSM) {
+          const unsigned long long ownm = fm & __ballot(ps == own);
+          own_s |= ownm != 0ull;
+          own_g |= (ownm & GAIN) != 0ull;
+          X += (int)__popcll(fm & MAXM & ~ownm);
+          bad |= (fm & MAXM & ~ownm & ~GAIN) != 0ull;
+          rows &= ~ownm & (MAXM | (M1 & ~GAIN));
+          if (fm & GAIN) {
+            if ((fm & GAIN) >> lane & 1ull) atomicOr(&sgain[ps >> 5], 1u << (ps & 31));
+          }
+        }
+        if (big) {
+          if (nit + (int)__popcll(rows) > WAVE) flush();
+          wave_lds_sync();
+        }
+        if ((rows >> lane) & 1ull) items[nit + (int)__popcll(rows & lt)] = (unsigned)ps * BROW;
+        nit += (int)__popcll(rows);
+        if (!last) break;  // the vertex goes on in the next chunk
         int dec = -1;
         if (!MSM) {
-          unsigned long long recv[P];
-          const int gain = gain_s + receivers(recv);
           if (gain > 0) {
-            count_rows(recv);
+            count_rows();
             unsigned key = 0;  // 8 * (count + 1) + 7 - u
 #pragma unroll
             for (int u = 0; u < P; u++) {
@@ -633,11 +643,10 @@ k_conn_eval_masks(ConnEvalArgs a) {
         } else {
           const int m_own = __builtin_amdgcn_readlane(m_l, j);
           const bool own_max = m_own == M;
-          unsigned long long recv[P];
           int gain_own = 0;
           bool go = !bad && X + (own_max ? 1 : 0) == cntM;
           if (go) {
-            gain_own = receivers(recv);
+            gain_own = receivers();
             go = gain_own + gain_s > 0 && (!own_max || gain_own + own_g > 0);
           }
           if (go) {
@@ -656,8 +665,7 @@ k_conn_eval_masks(ConnEvalArgs a) {
             }
             if (__ballot(good != 0u)) {
               nitems = 0;
-              (void)receivers(recv);
-              count_rows(recv);
+              count_rows();
               unsigned key = ~0u;  // l_own(k), then k
 #pragma unroll
               for (int u = 0; u < P; u++) {
@@ -877,6 +885,9 @@ struct ConnApplyArgs {
   int r0, r1;
   int mode;  // 0: TM apply, 1: MSM dry, 2: MSM commit
   int net_blocks;
+  // k_tm_apply
+  int lane_words;  // LDS words per lane of the small nets' replay
+  int wave_bytes;  // LDS bytes per wave
 };
 
 // The pc changes of one move v: own -> d on one net, from its list after the
@@ -1012,6 +1023,216 @@ __global__ void __launch_bounds__(REPLAY_BLOCK) k_conn_apply(ConnApplyArgs a) {
                               a.masks + (size_t)n * (size_t)(2 * a.mask_words));
     }
     wave_lds_sync();
+  }
+}
+
+// k_conn_apply's mode 0 for K <= MASK_KMAX. A wave takes a run of touched nets, as
+// many as give every wave one: the ones of at most TM_SMALL pins a lane each,
+// the list in the lane's registers, then the others one after another, the list
+// in LDS with a part -> position index. Their pins come TM_GROUP windows of 64
+// at a time, and moves that only change counts, which change no connection
+// either, are made together (wave_ilist_moves). A wave per net and a scan of
+// the list per move took 124 us for the nets that 200,000 vertices' moves touch
+// (K = 512): a dozen dependent reads per net, and on the largest net
+// (thousands of pins) a window at a time.
+constexpr int TM_SMALL = 8;
+constexpr int TM_GROUP = 8;
+constexpr int TM_TOGETHER = 8;
+constexpr int TM_APPLY_BLOCKS = 1536;  // all resident at 6 waves per SIMD
+
+// One lane replays the moves on a net of at most TM_SMALL pins, in the rank
+// order of its pins, and adds each move's pc changes (conn_changes).
+__device__ __forceinline__ void lane_tm_apply(const ConnApplyArgs& a, int n, unsigned s, unsigned np, unsigned* my) {
+  const unsigned seg = s + (unsigned)n;
+  int r[TM_SMALL];
+  unsigned x[TM_SMALL + 1];
+#pragma unroll
+  for (int i = 0; i < TM_SMALL; i++) r[i] = (unsigned)i < np ? a.apply_pins[s + (unsigned)i] : INT_MAX;
+#pragma unroll
+  for (int t = 0; t <= TM_SMALL; t++) x[t] = (unsigned)t <= np ? a.ent[seg + (unsigned)t] : 0u;
+  const int srcv = a.src[n];
+  int dd[TM_SMALL], oo[TM_SMALL];
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < TM_SMALL; i++) {
+    const bool in = r[i] >= a.r0 && r[i] < a.r1;
+    dd[i] = in ? a.slot_dec[r[i] - a.r0] : -1;
+    oo[i] = in ? a.slot_own[r[i] - a.r0] : -1;
+    any |= dd[i] >= 0;
+  }
+  if (!any) return;
+  int sp = frozen_part(srcv, a.part, a.slot_own, a.r0, a.r1);
+  int L = (int)x[0];
+  int key[TM_SMALL];  // part of each entry, -1 past the list
+  int cnt[TM_SMALL];
+#pragma unroll
+  for (int t = 0; t < TM_SMALL; t++) {
+    key[t] = t < L ? (int)(x[t + 1] & a.pmask) : -1;
+    cnt[t] = (int)(x[t + 1] >> a.pb);
+  }
+#pragma unroll 1
+  for (int i = 0; i < TM_SMALL; i++) {
+    int p = -1, q = -1, ri = -1;
+#pragma unroll
+    for (int t = 0; t < TM_SMALL; t++) {
+      p = t == i ? oo[t] : p;
+      q = t == i ? dd[t] : q;
+      ri = t == i ? r[t] : ri;
+    }
+    if (q < 0) continue;
+    // the last entry, should it have to fill p's place
+    int lk = -1, lc = 0;
+#pragma unroll
+    for (int t = 0; t < TM_SMALL; t++) {
+      lk = t == L - 1 ? key[t] : lk;
+      lc = t == L - 1 ? cnt[t] : lc;
+    }
+    bool gone = false, has = false;
+#pragma unroll
+    for (int t = 0; t < TM_SMALL; t++) {
+      const bool hit = key[t] == p;
+      const bool last = hit && cnt[t] == 1;
+      has |= hit;
+      gone |= last;
+      key[t] = last ? lk : key[t];
+      cnt[t] = last ? lc : cnt[t] - (hit ? 1 : 0);
+    }
+    L -= gone ? 1 : 0;
+    bool found = false;
+#pragma unroll
+    for (int t = 0; t < TM_SMALL; t++) {
+      key[t] = gone && t == L ? -1 : key[t];
+      const bool hit = key[t] == q;
+      found |= hit;
+      cnt[t] += hit ? 1 : 0;
+    }
+#pragma unroll
+    for (int t = 0; t < TM_SMALL; t++) {
+      key[t] = !found && t == L ? q : key[t];
+      cnt[t] = !found && t == L ? 1 : cnt[t];
+    }
+    L += found ? 0 : 1;
+    if (ri == srcv) {
+#pragma unroll
+      for (int t = 0; t < TM_SMALL; t++) {
+        if (t >= L) continue;
+        if (key[t] != q) atomicAdd(&a.pc[q * a.K + key[t]], 1);
+        if ((key[t] != p && key[t] != q) || (key[t] == q && cnt[t] > 1)) atomicAdd(&a.pc[p * a.K + key[t]], -1);
+      }
+      sp = q;
+    } else {
+      if (!found) atomicAdd(&a.pc[sp * a.K + q], 1);
+      if (gone || !has) atomicAdd(&a.pc[sp * a.K + p], -1);
+    }
+  }
+  unsigned y[TM_SMALL];
+#pragma unroll
+  for (int t = 0; t < TM_SMALL; t++) {
+    y[t] = ((unsigned)cnt[t] << a.pb) | (unsigned)key[t];
+    if (t < L) {
+      a.ent[seg + 1 + (unsigned)t] = y[t];
+      a.ev[seg + 1 + (unsigned)t] = ev_word(y[t], a.pb, a.pmask);
+    }
+  }
+  a.ent[seg] = (unsigned)L;
+  a.ev[seg] = (unsigned short)L;
+  lane_store_masks(y, L, a.pb, a.pmask, a.mask_words, my, a.masks + (size_t)n * (size_t)(2 * a.mask_words));
+}
+
+__global__ void __launch_bounds__(REPLAY_BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) k_tm_apply(ConnApplyArgs a) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
+  // the wave's own region: the lanes' words of their mask records, then a net's list and index
+  unsigned char* mem = lds + (size_t)wave * (size_t)a.wave_bytes;
+  unsigned* my = reinterpret_cast<unsigned*>(mem) + (size_t)lane * (size_t)a.lane_words;
+  unsigned* list = reinterpret_cast<unsigned*>(mem);
+  unsigned short* at = reinterpret_cast<unsigned short*>(list + a.K);
+  const int ntouched = uniform_load(a.tcount);
+  const int waves = (int)gridDim.x * nw;
+  const int run = min(WAVE, (ntouched + waves - 1) / waves);
+  for (int b = ((int)blockIdx.x * nw + wave) * run; b < ntouched; b += waves * run) {
+    int net = 0;
+    unsigned ns = 0, ne = 0;
+    const bool mine = lane < run && b + lane < ntouched;
+    if (mine) {
+      net = a.touched[b + lane];
+      ns = a.net_ptr[net];
+      ne = a.net_ptr[net + 1];
+    }
+    const bool small = mine && ne - ns <= (unsigned)TM_SMALL;
+    if (small) lane_tm_apply(a, net, ns, ne - ns, my);
+    unsigned long long big = __ballot(mine && !small);
+    if (big == 0ull) continue;
+    wave_lds_sync();
+    wave_index_init(at, a.K);
+    for (; big; big &= big - 1) {
+      const int j = __ffsll((long long)big) - 1;
+      const int n = __builtin_amdgcn_readlane(net, j);
+      const unsigned s = (unsigned)__builtin_amdgcn_readlane((int)ns, j), e = (unsigned)__builtin_amdgcn_readlane((int)ne, j);
+      const unsigned seg = s + (unsigned)n;
+      const unsigned head = wave_list_head(a.ent, seg, e - s);
+      const int srcv = a.src[n];
+      unsigned lo, hi;
+      wave_rank_window(a.apply_pins, s, e, a.r0, a.r1, lo, hi);
+      int L = wave_list_stage(a.ent, seg, head, list);
+      wave_index_set(list, L, at, a.pmask);
+      int sp = frozen_part(srcv, a.part, a.slot_own, a.r0, a.r1);
+      bool dirty = false;
+      for (unsigned k0 = lo; k0 < hi; k0 += TM_GROUP * WAVE) {
+        int rr[TM_GROUP], dd[TM_GROUP], oo[TM_GROUP];
+#pragma unroll
+        for (int u = 0; u < TM_GROUP; u++) {
+          const unsigned k = k0 + (unsigned)(u * WAVE + lane);
+          rr[u] = k < hi ? a.apply_pins[k] : INT_MAX;
+        }
+#pragma unroll
+        for (int u = 0; u < TM_GROUP; u++) {
+          dd[u] = -1;
+          oo[u] = -1;
+          if (rr[u] >= a.r0 && rr[u] < a.r1) {
+            dd[u] = a.slot_dec[rr[u] - a.r0];
+            oo[u] = a.slot_own[rr[u] - a.r0];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < TM_GROUP; u++) {
+          unsigned long long m = __ballot(dd[u] >= 0);
+          const unsigned long long sm = m & __ballot(rr[u] == srcv);
+          dirty |= m != 0ull;
+          bool together = true;  // worth trying in this window
+          while (m) {
+            // the moves before the source's
+            const unsigned long long mt = (m & sm) ? m & (sm - 1ull) : m;
+            if (together && __popcll(mt) >= TM_TOGETHER) {
+              const unsigned long long rest = wave_ilist_moves(list, at, mt, oo[u], dd[u], a.pb);
+              together = __popcll(mt) - __popcll(rest) >= TM_TOGETHER / 2;
+              m = (m & ~mt) | rest;
+              if (!m) break;
+            }
+            const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)m) - 1);
+            m &= m - 1;
+            const int own = __builtin_amdgcn_readlane(oo[u], l), d = __builtin_amdgcn_readlane(dd[u], l);
+            unsigned co;
+            bool found;
+            wave_ilist_move(list, at, L, own, d, a.pb, a.pmask, co, found);
+            if ((sm >> l) & 1ull) {
+              conn_changes(list, L, own, d, true, sp, a.K, a.pb, a.pmask, [&](int, int cell, int dl) {
+                if (cell >= 0) atomicAdd(&a.pc[cell], dl);
+              });
+              sp = d;
+            } else if (lane == 0) {
+              if (!found) atomicAdd(&a.pc[sp * a.K + d], 1);
+              if (co <= 1u) atomicAdd(&a.pc[sp * a.K + own], -1);
+            }
+          }
+        }
+      }
+      if (dirty) {
+        wave_list_store(a.ent, a.ev, seg, list, L, a.pb, a.pmask);
+        wave_store_masks(list, at, a.K, a.pb, a.mask_words, a.masks + (size_t)n * (size_t)(2 * a.mask_words));
+      }
+      wave_index_clear(list, L, at, a.pmask);
+    }
   }
 }
 
@@ -1279,7 +1500,13 @@ fp_status pass_conn(fp_ctx* ctx, const RefinePlan& p) {
       k_tm_admit<<<1, WAVE, (size_t)K * (sizeof(long long) + 2 * sizeof(int)), ctx->stream>>>(
           ctx->slot_dec, c.mv, c.mstat, r0, K, thr, ctx->sizes, ctx->part, ctx->moves);
       ap.mode = 0;
-      k_conn_apply<<<ap.net_blocks, REPLAY_BLOCK, lds_r, ctx->stream>>>(ap);
+      if (p.masks) {
+        ap.lane_words = 2 * P + 1;
+        ap.wave_bytes = std::max(4 * WAVE * ap.lane_words, (6 * K + 15) & ~15);
+        k_tm_apply<<<TM_APPLY_BLOCKS, REPLAY_BLOCK, (size_t)(REPLAY_BLOCK / WAVE) * (size_t)ap.wave_bytes, ctx->stream>>>(ap);
+      } else {
+        k_conn_apply<<<ap.net_blocks, REPLAY_BLOCK, lds_r, ctx->stream>>>(ap);
+      }
     } else {
       launch_round_compact<false>(ctx, nullptr, r0, nslots, c.slot_mi, c.mv, c.mstat);
       ap.mode = 1;

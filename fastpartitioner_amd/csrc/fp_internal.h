@@ -129,6 +129,9 @@ __device__ __forceinline__ int wave_max(int x) {
   return __builtin_amdgcn_readlane(x, WAVE - 1);
 }
 
+// lane l: x of lane l - 1, and -1 for lane 0 (wave_shr:1)
+__device__ __forceinline__ int wave_shift_up(int x) { return dpp_i32<0x138>(-1, x); }
+
 // The same for unsigned max (identity 0) and min (identity ~0).
 __device__ __forceinline__ unsigned wave_max_u32(unsigned x) {
   x = max(x, (unsigned)dpp_i32<0xB1>(0, (int)x));
