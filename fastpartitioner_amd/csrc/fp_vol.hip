@@ -24,10 +24,12 @@
 //                  moves up to the stop
 #include "fp_masks.h"
 #include "fp_round.h"
+#include "fp_short.h"
 
 namespace fpe {
 namespace {
 
+constexpr int VOL_CU_WAVES = 24;  // resident wavefronts of k_vol_eval per CU
 constexpr int VOL_BLOCK = 512;  // at most 8 wavefronts; vol_eval_waves picks the count
 constexpr int VOL_KMAX = 4096;  // k_vol_scan: one lane of the max-set tracking holds at most 64 parts
 constexpr int REPLAY_BLOCK = 256;
@@ -83,11 +85,14 @@ struct VolEvalArgs {
   int* touched;
   int* tcount;
   int* tcount_next;
+  unsigned last_pin;  // the last element of vtx_nets and vtx_seg
+  int per_wave;       // consecutive slots per wave (<= 64)
+  // k_vol_eval
+  int shorts;        // the LDS has room for the short lists' rows
+  unsigned pad_seg;  // the 64 zero words after the last segment: a list of length 0
   // k_vol_eval_masks
   const unsigned long long* masks;
   int noe;
-  unsigned last_pin;
-  int per_wave;
 };
 
 // The first-appearance rank of the LDG tie-break (MGV/partition.cpp:765-790)
@@ -141,7 +146,90 @@ __device__ __forceinline__ int vol_tie_decision(const VolEvalArgs& a, unsigned v
   return __builtin_amdgcn_readlane(bq, wl);
 }
 
-__global__ void __launch_bounds__(VOL_BLOCK) k_vol_eval(VolEvalArgs a) {
+// LDS of k_vol_eval: 12 bytes per part shared by the workgroup, per wavefront
+// a count per part and a bit per part, then, where they fit too, per wavefront
+// the short lists' rows and two bytes per net.
+constexpr int VOL_SHORT_BYTES = SHORT_ROWS * (int)sizeof(uint2) + 2 * WAVE;
+
+__host__ __device__ __forceinline__ size_t vol_short_at(int K, int waves) {
+  return ((size_t)K * 12 + (size_t)waves * 4 * ((size_t)K + (size_t)((K + 31) / 32)) + 7) & ~(size_t)7;
+}
+
+// The LDG choice of a vertex with long lists or many nets, from K counts.
+__device__ int vol_long_choice(const VolEvalArgs& a, unsigned vb, int deg, int own, unsigned sg0, unsigned* cnt,
+                               const double* s_pen, const unsigned* s_skey, int fb) {
+  const int lane = lane_id(), K = a.K;
+  // scores: pin counts per part over v's nets (MGV/partition.cpp:765-790)
+  for (int c0 = 0; c0 < deg; c0 += WAVE) {
+    const int nn = min(WAVE, deg - c0);
+    const unsigned sg = c0 == 0 ? sg0 : (lane < nn ? a.vtx_seg[vb + (unsigned)(c0 + lane)] : 0u);
+    wave_sweep_lists<8, SWEEP_LONG_TASKS>(a.ev, sg, nn, [&](int, int, int, bool ok, unsigned x) {
+      if (ok) atomicAdd(&cnt[(int)(x & ~EV_SINGLE)], 1u);
+    });
+  }
+  wave_lds_sync();
+  // LDG: lexicographic max of (score, -size, -first rank) over score > 0.
+  // Scores are positive doubles, so their bit patterns order like the
+  // values: key1 = score bits (max), key2 = size_key(size) (min among key1
+  // ties); ltie: this lane met its best keys twice. The first-appearance
+  // rank only matters between parts tied on both keys (vol_tie_decision).
+  // Four 64-part chunks per step, without branches: their LDS reads issue
+  // together; every slot is cleared for the next vertex
+  unsigned long long b1 = 0;
+  unsigned b2 = ~0u;
+  int bq = -1;
+  bool ltie = false;
+  for (int q0 = 0; q0 < K; q0 += 4 * WAVE) {
+    unsigned cv[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int q = min(q0 + u * WAVE + lane, K - 1);
+      cv[u] = q0 + u * WAVE + lane < K ? cnt[q] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int q = q0 + u * WAVE + lane;
+      const int qc = min(q, K - 1);
+      if (q < K) cnt[q] = 0;
+      const int adj = (int)cv[u] - (q == own ? 1 : 0);  // scores[part_id]-- (MGV/partition.cpp:792-796)
+      const double sc = (double)adj * s_pen[qc];
+      const bool ok = cv[u] != 0 && sc > 0;
+      const unsigned long long k1 = ok ? (unsigned long long)__double_as_longlong(sc) : 0ull;
+      const unsigned k2 = s_skey[qc];
+      const bool better = ok && (k1 > b1 || (k1 == b1 && k2 < b2));
+      const bool same = ok && k1 == b1 && k2 == b2;
+      ltie = better ? false : (ltie || same);
+      b1 = better ? k1 : b1;
+      b2 = better ? k2 : b2;
+      bq = better ? q : bq;
+    }
+  }
+  const unsigned long long m1 = wave_max_u64(b1);
+  const unsigned m2 = wave_min_u32(b1 == m1 ? b2 : ~0u);
+  wave_lds_sync();
+  int d = fb;
+  if (m1 != 0) {
+    const unsigned long long cand = __ballot(b1 == m1 && b2 == m2);
+    if (__popcll(cand) > 1 || __ballot(b1 == m1 && b2 == m2 && ltie) != 0ull) {
+      d = vol_tie_decision(a, vb, deg, own, cnt, s_pen, s_skey, m1, m2);
+    } else {
+      d = __builtin_amdgcn_readlane(bq, __ffsll((long long)cand) - 1);
+    }
+  }
+  return d;
+}
+
+// K past the part masks' range, a wavefront per vertex. A vertex of few entries
+// takes its counts, its choice and the facts per net from the entries
+// themselves (fp_short.h); any other sweeps its lists into K counts, scans
+// them, and sweeps again for the facts.
+// 262,144 vertices of 13 nets of 13 pins, K = 1024: 130 us, 100 of them vector
+// issue (375 us with a sweep and a scan of K counts for every vertex; 230 us
+// with the sources' parts gathered for every vertex).
+// A wave takes per_wave consecutive slots, their headers a slot per lane; a
+// vertex's nets, segments and the sources' parts load while the one before it
+// is decided.
+__global__ void __launch_bounds__(VOL_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) k_vol_eval(VolEvalArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   const int K = a.K;
   double* s_pen = reinterpret_cast<double*>(lds);
@@ -151,6 +239,15 @@ __global__ void __launch_bounds__(VOL_BLOCK) k_vol_eval(VolEvalArgs a) {
   __shared__ int red_ix[VOL_BLOCK / WAVE];
   const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
   const int KW = (K + 31) / 32;
+  // the wave's rows (fp_short.h) and, a byte per net, whether v is own's only
+  // pin there and whether the chosen part is listed
+  uint2* rows = reinterpret_cast<uint2*>(lds + vol_short_at(K, nw)) + (size_t)wave * (VOL_SHORT_BYTES / sizeof(uint2));
+  unsigned char* single_b = reinterpret_cast<unsigned char*>(rows + SHORT_ROWS);
+  unsigned char* found_b = single_b + WAVE;
+  if (a.shorts) {
+    single_b[lane] = 0;
+    found_b[lane] = 0;
+  }
   unsigned* cnt = wbase + (size_t)wave * (size_t)(K + KW);
   unsigned* hitb = cnt + K;                  // max parts the move affects (MSRV), one bit per part
   int* delta = reinterpret_cast<int*>(cnt);  // reused once the decision is made (cnt is all 0 again)
@@ -194,83 +291,71 @@ __global__ void __launch_bounds__(VOL_BLOCK) k_vol_eval(VolEvalArgs a) {
   }
   const int M = a.mstat[0], cntM = a.mstat[1];
 
-  for (int slot = (int)blockIdx.x * nw + wave; slot < a.nslots; slot += (int)gridDim.x * nw) {
-    const int z = a.r0 + slot;
-    const int v = a.order ? a.order[z] : z;
-    const int own = a.part[v];
-    const unsigned vb = a.vtx_ptr[v];
-    const int deg = (int)(a.vtx_ptr[v + 1] - vb);
-    // this lane's net of the first chunk: segment offset and source part
-    // (own for v's own source nets), kept for the later passes
-    const unsigned sg0 = lane < deg ? a.vtx_seg[vb + (unsigned)lane] : 0u;
-    int ip0 = -1;
-    bool isrc0 = false;
-    if (lane < deg) {
-      const int s = a.src[a.vtx_nets[vb + (unsigned)lane]];
-      isrc0 = s == v;
-      ip0 = isrc0 ? own : a.part[s];
+  const int s0 = ((int)blockIdx.x * nw + wave) * a.per_wave;
+  const int ns = min(a.per_wave, a.nslots - s0);
+  // lane i: slot s0 + i's vertex, its part and its net range
+  int v_l = 0, own_l = 0, dec_l = -1;
+  unsigned vb_l = 0, ve_l = 0;
+  if (lane < ns) {
+    const int z = a.r0 + s0 + lane;
+    v_l = a.order ? a.order[z] : z;
+    own_l = a.part[v_l];
+    vb_l = a.vtx_ptr[v_l];
+    ve_l = a.vtx_ptr[v_l + 1];
+  }
+  // lane j: net j of slot s0 + i's vertex (past its last net that one again,
+  // which costs no cache line) and its segment offset, two vertices ahead; the
+  // net's length, one. The sources and their parts are two gathers more, of a
+  // cache line per net, and wait for a vertex whose choice is another part.
+  struct Net {
+    unsigned id, seg;
+  };
+  struct Head {
+    unsigned id, seg, len;
+  };
+  auto load_net = [&](int i) -> Net {
+    const unsigned b = (unsigned)__builtin_amdgcn_readlane((int)vb_l, i);
+    const unsigned e = (unsigned)__builtin_amdgcn_readlane((int)ve_l, i);
+    const unsigned k = min(min(b + (unsigned)lane, max(e, b + 1u) - 1u), a.last_pin);
+    return Net{a.vtx_nets[k], a.vtx_seg[k]};
+  };
+  auto load_head = [&](Net n) -> Head { return Head{n.id, n.seg, a.ev[n.seg]}; };
+  // the headers have arrived before the loop (else its first wait would take in the loads of every turn)
+  asm volatile("" ::"v"(v_l), "v"(own_l), "v"(vb_l), "v"(ve_l));
+  Net net{0u, 0u};
+  Head head{0u, 0u, 0u};
+  if (ns > 0) {
+    head = load_head(load_net(0));
+    net = load_net(min(1, ns - 1));
+  }
+  for (int i = 0; i < ns; i++) {
+    const int v = __builtin_amdgcn_readlane(v_l, i);
+    const int own = __builtin_amdgcn_readlane(own_l, i);
+    const unsigned vb = (unsigned)__builtin_amdgcn_readlane((int)vb_l, i);
+    const int deg = (int)((unsigned)__builtin_amdgcn_readlane((int)ve_l, i) - vb);
+    // this lane's net of the first chunk, kept for the later passes
+    const unsigned id0 = head.id;
+    const unsigned sg0 = lane < deg ? head.seg : a.pad_seg, len0 = lane < deg ? head.len : 0u;
+    ShortLists sl;
+    const bool shrt = a.shorts && short_load(a.ev, sg0, len0, deg, a.pad_seg, rows, sl);
+    head = load_head(net);
+    net = load_net(min(i + 2, ns - 1));
+    int d;
+    if (shrt) {
+      unsigned craw;
+      d = short_ldg(sl, cnt, s_pen, s_skey, own, craw);
+      if (d < 0) d = fb;
+    } else {
+      d = vol_long_choice(a, vb, deg, own, sg0, cnt, s_pen, s_skey, fb);
     }
 
-    // scores: pin counts per part over v's nets (MGV/partition.cpp:765-790)
-    for (int c0 = 0; c0 < deg; c0 += WAVE) {
-      const int nn = min(WAVE, deg - c0);
-      const unsigned sg = c0 == 0 ? sg0 : (lane < nn ? a.vtx_seg[vb + (unsigned)(c0 + lane)] : 0u);
-      wave_sweep_lists<8, SWEEP_LONG_TASKS>(a.ev, sg, nn, [&](int, int, int, bool ok, unsigned x) {
-        if (ok) atomicAdd(&cnt[(int)(x & ~EV_SINGLE)], 1u);
-      });
-    }
-    wave_lds_sync();
-    // LDG: lexicographic max of (score, -size, -first rank) over score > 0.
-    // Scores are positive doubles, so their bit patterns order like the
-    // values: key1 = score bits (max), key2 = size_key(size) (min among key1
-    // ties); ltie: this lane met its best keys twice. The first-appearance
-    // rank only matters between parts tied on both keys (vol_tie_decision).
-    // Four 64-part chunks per step, without branches: their LDS reads issue
-    // together; every slot is cleared for the next vertex
-    unsigned long long b1 = 0;
-    unsigned b2 = ~0u;
-    int bq = -1;
-    bool ltie = false;
-    for (int q0 = 0; q0 < K; q0 += 4 * WAVE) {
-      unsigned cv[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int q = min(q0 + u * WAVE + lane, K - 1);
-        cv[u] = q0 + u * WAVE + lane < K ? cnt[q] : 0u;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int q = q0 + u * WAVE + lane;
-        const int qc = min(q, K - 1);
-        if (q < K) cnt[q] = 0;
-        const int adj = (int)cv[u] - (q == own ? 1 : 0);  // scores[part_id]-- (MGV/partition.cpp:792-796)
-        const double sc = (double)adj * s_pen[qc];
-        const bool ok = cv[u] != 0 && sc > 0;
-        const unsigned long long k1 = ok ? (unsigned long long)__double_as_longlong(sc) : 0ull;
-        const unsigned k2 = s_skey[qc];
-        const bool better = ok && (k1 > b1 || (k1 == b1 && k2 < b2));
-        const bool same = ok && k1 == b1 && k2 == b2;
-        ltie = better ? false : (ltie || same);
-        b1 = better ? k1 : b1;
-        b2 = better ? k2 : b2;
-        bq = better ? q : bq;
-      }
-    }
-    const unsigned long long m1 = wave_max_u64(b1);
-    const unsigned m2 = wave_min_u32(b1 == m1 ? b2 : ~0u);
-    wave_lds_sync();
-    int d = fb;
-    if (m1 != 0) {
-      const unsigned long long cand = __ballot(b1 == m1 && b2 == m2);
-      if (__popcll(cand) > 1 || __ballot(b1 == m1 && b2 == m2 && ltie) != 0ull) {
-        d = vol_tie_decision(a, vb, deg, own, cnt, s_pen, s_skey, m1, m2);
-      } else {
-        d = __builtin_amdgcn_readlane(bq, __ffsll((long long)cand) - 1);
-      }
-    }
-
+    if (d == own) continue;
+    const int src0 = a.src[id0];
+    const bool isrc0 = lane < deg && src0 == v;
+    int ip0 = a.part[src0];  // the net's source part, own for v's own source nets
+    ip0 = lane < deg ? (isrc0 ? own : ip0) : -1;
     int dec = -1;
-    if (d != own) {
+    {
       // gains / losses (MGV/partition.cpp:800-840; MSRV/partition.cpp:852-897),
       // accumulated as delta[p] = losses[p] - gains[p]; lane j takes net j of
       // each chunk: whether v is own's only pin there (single), whether d is
@@ -290,17 +375,32 @@ __global__ void __launch_bounds__(VOL_BLOCK) k_vol_eval(VolEvalArgs a) {
             ip = isrc ? own : a.part[s];
           }
         }
-        unsigned long long smask = 0, fmask = 0;
+        bool single = false, found = false;
         int myL = 0;
-        wave_sweep_lists<8, SWEEP_LONG_TASKS>(a.ev, sg, nn, [&](int j, int L, int t, bool ok, unsigned x) {
-          const int q = (int)(x & ~EV_SINGLE);
-          if (__ballot(ok && q == own && (x & EV_SINGLE))) smask |= 1ull << j;
-          if (__ballot(ok && q == d)) fmask |= 1ull << j;
-          if (lane == j) myL = L;
-          (void)t;
-        });
+        if (shrt) {
+          // an entry of own with one pin, or of d, marks its net
+          short_each(sl, [&](int w, unsigned x) {
+            if (x == ((unsigned)own | EV_SINGLE)) single_b[short_net(rows, w)] = 1;
+            if ((x & ~EV_SINGLE) == (unsigned)d) found_b[short_net(rows, w)] = 1;
+          });
+          wave_lds_sync();
+          single = single_b[lane] != 0;
+          found = found_b[lane] != 0;
+          myL = (int)len0;
+          single_b[lane] = 0;
+          found_b[lane] = 0;
+        } else {
+          unsigned long long smask = 0, fmask = 0;
+          wave_sweep_lists<8, SWEEP_LONG_TASKS>(a.ev, sg, nn, [&](int j, int L, int, bool ok, unsigned x) {
+            const int q = (int)(x & ~EV_SINGLE);
+            if (__ballot(ok && q == own && (x & EV_SINGLE))) smask |= 1ull << j;
+            if (__ballot(ok && q == d)) fmask |= 1ull << j;
+            if (lane == j) myL = L;
+          });
+          single = (smask >> lane) & 1ull;
+          found = (fmask >> lane) & 1ull;
+        }
         if (lane < nn) {
-          const bool single = (smask >> lane) & 1ull, found = (fmask >> lane) & 1ull;
           if (isrc) {
             d_own -= myL - 1;  // gains[part_id] += end_cnt - 1
             d_dec += myL - 1;  // losses[decision] += end_cnt - 1
@@ -366,11 +466,12 @@ __global__ void __launch_bounds__(VOL_BLOCK) k_vol_eval(VolEvalArgs a) {
       wave_lds_sync();
       if (!bad && (!a.msrv || maxhit == cntM)) dec = d;
     }
-    if (lane == 0) {
-      a.slot_own[slot] = own;
-      a.slot_dec[slot] = dec;
-    }
+    dec_l = lane == i ? dec : dec_l;
     if (dec >= 0) wave_touch_nets(a.vtx_nets + vb, deg, a.tag, a.net_stamp, a.touched, a.tcount);
+  }
+  if (lane < ns) {
+    a.slot_own[s0 + lane] = own_l;
+    a.slot_dec[s0 + lane] = dec_l;
   }
 }
 
@@ -1025,27 +1126,28 @@ __global__ void __launch_bounds__(WAVE) k_vol_scan(int* __restrict__ vol_g, int 
   }
 }
 
-// LDS of an evaluation workgroup: 12 bytes per part shared by the workgroup,
-// per wavefront a count per part and a bit per part
-size_t vol_eval_lds(int K, int waves) {
-  return (size_t)K * 12 + (size_t)waves * 4 * ((size_t)K + (size_t)((K + 31) / 32));
+size_t vol_eval_lds(int K, int waves, bool shorts) {
+  return vol_short_at(K, waves) + (shorts ? (size_t)waves * VOL_SHORT_BYTES : 0);
 }
+
+// workgroups of that shape a CU holds (k_vol_eval's registers allow 6 waves per SIMD)
+int vol_eval_per_cu(int waves, size_t lds) { return std::min((int)((size_t)LDS_PER_CU / lds), VOL_CU_WAVES / waves); }
 
 // Wavefronts per evaluation workgroup: the count that keeps the most
 // wavefronts resident on a CU (K = 1024: 8 per workgroup, 3 workgroups, 24
-// wavefronts), the larger on ties.
+// wavefronts), the larger on ties. The largest K leaves no room for the rows.
 int vol_eval_waves(int K) {
   int best = 0, bw = 0;
   for (int w = 1; w <= VOL_BLOCK / WAVE; w++) {
-    const size_t lds = vol_eval_lds(K, w);
+    const size_t lds = vol_eval_lds(K, w, true);
     if (lds > (size_t)LDS_BUDGET) break;
-    const int per_cu = w * std::min((int)((size_t)LDS_PER_CU / lds), MAX_WAVES_PER_CU / w);
+    const int per_cu = w * vol_eval_per_cu(w, lds);
     if (per_cu >= best) {
       best = per_cu;
       bw = w;
     }
   }
-  return bw;
+  return bw == 0 && vol_eval_lds(K, 1, false) <= (size_t)LDS_BUDGET ? 1 : bw;
 }
 
 fp_status ensure_vol_scratch(fp_ctx* ctx, int R) {
@@ -1110,7 +1212,8 @@ fp_status plan_vol(fp_ctx* ctx, RefinePlan& p) {
 fp_status pass_vol(fp_ctx* ctx, const RefinePlan& p) {
   const bool msrv = p.metric == FP_METRIC_MSRV;
   const int nov = ctx->nov, K = ctx->K, R = p.R, waves = p.eval_waves;
-  const size_t lds_e = vol_eval_lds(K, waves);
+  const bool shorts = vol_eval_lds(K, waves, true) <= (size_t)LDS_BUDGET;
+  const size_t lds_e = vol_eval_lds(K, waves, shorts);
   // the replay's part -> position index where it fits the LDS budget
   const bool indexed = (size_t)(REPLAY_BLOCK / WAVE) * (size_t)K * (sizeof(unsigned) + sizeof(unsigned short)) <=
                        (size_t)LDS_BUDGET;
@@ -1152,15 +1255,25 @@ fp_status pass_vol(fp_ctx* ctx, const RefinePlan& p) {
     a.touched = ctx->touched;
     a.tcount = ctx->counters + par;
     a.tcount_next = ctx->counters + (par ^ 1);
+    a.last_pin = mask_last_pin(ctx);
     if (p.masks) {
       a.masks = p.masks;
       a.noe = ctx->noe;
-      a.last_pin = mask_last_pin(ctx);
       const int egrid = mask_eval_grid(nslots, p.eval_grid, VOL_MASK_BLOCK / WAVE, a.per_wave);
       FP_TRY(launch_timed(ctx, vol_masks_kernel(K), egrid, VOL_MASK_BLOCK, 0, a));
     } else {
-      int egrid = std::max(1, std::min((nslots + waves - 1) / waves, 8192));
-      if (p.eval_grid > 0) egrid = std::min(egrid, p.eval_grid);
+      a.pad_seg = (unsigned)((size_t)ctx->pins + (size_t)ctx->noe);
+      if (ctx->pins == 0) {
+        // the loads that every lane makes find net 0 and vertex 0 in the zero padding
+        const unsigned short* zeros = ctx->ev + a.pad_seg;
+        a.vtx_nets = a.vtx_seg = reinterpret_cast<const unsigned*>(zeros + (a.pad_seg & 1u));
+        a.src = reinterpret_cast<const int*>(a.vtx_nets);
+      }
+      a.shorts = shorts ? 1 : 0;
+      // as many blocks as the 256 CUs hold: a few more would run alone at the end
+      const int resident = 256 * std::max(1, vol_eval_per_cu(waves, lds_e));
+      const int egrid = mask_eval_grid(nslots, p.eval_grid > 0 ? std::min(p.eval_grid, resident) : resident, waves,
+                                       a.per_wave);
       FP_TRY(launch_timed(ctx, k_vol_eval, egrid, waves * WAVE, lds_e, a));
     }
     launch_round_compact<false>(ctx, ctx->order, r0, nslots, vs.slot_mi, vs.mv, vs.mstat);
