@@ -227,7 +227,7 @@ fp_status ensure_k(fp_ctx* ctx, int K) {
 
 namespace {
 
-constexpr int BUILD_KMAX = 4096;  // k_build_lists keeps four K-int arrays per wavefront in LDS
+constexpr int BUILD_KMAX = 4096;  // k_build_lists keeps two K-int arrays per wavefront in LDS
 
 // Per incidence of the vertex view: the segment of its net in the packed
 // connectivity layout (the net's list starts at net_ptr[n] + n).
@@ -240,69 +240,173 @@ __global__ void __launch_bounds__(256) k_vtx_seg(const unsigned* __restrict__ ne
   }
 }
 
-// One wavefront per net: the net's connectivity list from the part vector,
-// in first-appearance order along the ordering (the state the reference's
-// streaming initial partition leaves, TV/partition.cpp:240-263). The pins are
-// visited in rank order (apply_pins holds each net's pin ranks ascending), 64
-// at a time: the first lane of each part not yet listed appends it, then every
-// lane counts its pin. Writes the packed segment and its evaluation view.
-__global__ void __launch_bounds__(256) k_build_lists(const unsigned* __restrict__ net_ptr,
+// The nets' connectivity lists from the part vector, in first-appearance order
+// along the ordering (the state the reference's streaming initial partition
+// leaves, TV/partition.cpp:240-263): the pins are visited in rank order
+// (apply_pins holds each net's pin ranks ascending). Writes the packed segments
+// and their evaluation view.
+// Wavefronts take per_wave consecutive nets. Whole nets of at most 64 pins
+// share a window of 64 lanes, a pin per lane: the lanes' (net, part) keys
+// shifted past each other one lane at a time find every pin's later equals, so
+// a pin with no earlier one is a list entry and has counted its part. A longer
+// net goes 64 pins at a time through a slot per part in LDS: the first lane of
+// each part not yet listed appends it, then every lane counts its pin.
+// BUILD_GROUP windows' pins, then their parts, load together.
+// Bound by the part gathers, a cache line per pin. A wavefront per net, four
+// words of LDS per part and a load round per window took 233 us for 1,000,000
+// Zipf nets at K = 256 and 1,296 us for 2,000,000 of 13 pins at K = 1024; now
+// 150 us, much of it the largest nets' 79 windows, and 281 us.
+constexpr int BUILD_BLOCK = 256;
+constexpr int BUILD_GROUP = 4;
+constexpr int BUILD_BLOCKS = 2048;  // all resident at 8 waves per SIMD where the LDS allows
+constexpr unsigned SLOT_NONE = ~0u;
+constexpr size_t BUILD_STATIC = BUILD_BLOCK / WAVE * WAVE * sizeof(int);
+
+__global__ void __launch_bounds__(BUILD_BLOCK) k_build_lists(const unsigned* __restrict__ net_ptr,
                                                      const int* __restrict__ apply_pins, const int* __restrict__ order,
-                                                     const int* __restrict__ part, int noe, int K, int pb,
+                                                     const int* __restrict__ part, int noe, int per_wave, int K, int pb,
                                                      unsigned pmask, unsigned* __restrict__ ent,
                                                      unsigned short* __restrict__ ev) {
   extern __shared__ __align__(16) unsigned char lds[];
+  __shared__ int s_win[BUILD_BLOCK / WAVE][WAVE];
   const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
-  int* slot = reinterpret_cast<int*>(lds) + (size_t)wave * 4 * (size_t)K;  // list position of a part, -1
-  int* claim = slot + K;                                                   // first lane of a new part, 64
-  int* lcnt = claim + K;                                                   // pin count per list position
-  int* lq = lcnt + K;                                                      // part per list position
-  for (int q = lane; q < K; q += WAVE) {
-    slot[q] = -1;
-    claim[q] = WAVE;
-  }
+  int* winbuf = s_win[wave];                                                    // net starting at each window lane
+  unsigned* slot = reinterpret_cast<unsigned*>(lds) + (size_t)wave * 2 * (size_t)K;  // list position of a part
+  unsigned* list = slot + K;                                                    // the list: pins << pb | part
+  const unsigned inc = 1u << pb;
+  for (int q = lane; q < K; q += WAVE) slot[q] = SLOT_NONE;
   wave_lds_sync();
   const unsigned long long lt = (1ull << lane) - 1ull;
-  for (int n = (int)blockIdx.x * nw + wave; n < noe; n += (int)gridDim.x * nw) {
-    const unsigned s = net_ptr[n], e = net_ptr[n + 1];
-    int L = 0;
-    for (unsigned k0 = s; k0 < e; k0 += WAVE) {
-      const unsigned k = k0 + (unsigned)lane;
-      const bool ok = k < e;
-      int q = 0;
-      if (ok) {
-        const int r = apply_pins[k];
-        q = part[order ? order[r] : r];
+  auto part_at = [&](int r) -> int { return part[order ? order[r] : r]; };
+  auto store = [&](unsigned at, unsigned x) {
+    ent[at] = x;
+    ev[at] = ev_word(x, pb, pmask);
+  };
+  const int stride = (int)gridDim.x * nw * per_wave;
+  for (int c = ((int)blockIdx.x * nw + wave) * per_wave; c < noe; c += stride) {
+    const int nc = min(per_wave, noe - c);
+    // lane j: net c + j
+    unsigned start = 0, end = 0;
+    if (lane < nc) {
+      start = net_ptr[c + lane];
+      end = net_ptr[c + lane + 1];
+    }
+    const int len = (int)(end - start);
+    for (int i = 0; i < nc;) {
+      // up to BUILD_GROUP windows of whole nets of at most 64 pins, from net i on
+      int wi[BUILD_GROUP], wc[BUILD_GROUP], rr[BUILD_GROUP], qq[BUILD_GROUP];
+      unsigned wbase[BUILD_GROUP];
+      int ng = 0;
+#pragma unroll
+      for (int u = 0; u < BUILD_GROUP; u++) {
+        wi[u] = i;
+        wc[u] = 0;
+        wbase[u] = 0;
+        rr[u] = -1;
+        if (ng == u && i < nc) {
+          const unsigned base = (unsigned)__builtin_amdgcn_readlane((int)start, i);
+          const unsigned long long fit = __ballot(lane >= i && lane < nc && end - base <= (unsigned)WAVE);
+          const int cnt = (int)__popcll(fit);
+          if (cnt > 0) {
+            const unsigned np = (unsigned)__builtin_amdgcn_readlane((int)end, i + cnt - 1) - base;
+            wbase[u] = base;
+            wc[u] = cnt;
+            if ((unsigned)lane < np) rr[u] = apply_pins[base + (unsigned)lane];
+            i += cnt;
+            ng++;
+          }
+        }
       }
-      const bool fresh = ok && slot[q] < 0;
-      if (fresh) atomicMin(&claim[q], lane);
-      wave_lds_sync();
-      const bool first = fresh && claim[q] == lane;
-      const unsigned long long bm = __ballot(first);
-      if (first) {
-        const int pos = L + __popcll(bm & lt);
-        slot[q] = pos;
-        lcnt[pos] = 0;
-        lq[pos] = q;
-        claim[q] = WAVE;
+#pragma unroll
+      for (int u = 0; u < BUILD_GROUP; u++) qq[u] = rr[u] >= 0 ? part_at(rr[u]) : 0;
+#pragma unroll
+      for (int u = 0; u < BUILD_GROUP; u++) {
+        if (u >= ng) break;
+        const int i0 = wi[u];
+        const bool in_win = lane >= i0 && lane < i0 + wc[u];
+        winbuf[lane] = -1;
+        wave_lds_sync();
+        if (in_win && len > 0) winbuf[start - wbase[u]] = lane;
+        wave_lds_sync();
+        const int owner = max(wave_incl_max(winbuf[lane]), 0);  // net (lane of the chunk) of this lane's pin
+        const int key = rr[u] >= 0 ? (owner << 16) | qq[u] : -1;
+        const int dmax = (int)wave_max_u32(in_win ? (unsigned)len : 0u);
+        unsigned cnt = 1;
+        unsigned long long dup = 0;
+        int y = key;
+        for (int d = 1; d < dmax; d++) {
+          y = wave_shift_down(y);
+          const unsigned long long m = __ballot(y == key);
+          cnt += (m >> lane) & 1ull ? 1u : 0u;
+          dup |= m << d;
+        }
+        const unsigned long long first = __ballot(key >= 0) & ~dup;
+        const unsigned ostart = (unsigned)__shfl((int)start, owner);
+        const unsigned seg = ostart + (unsigned)(c + owner);
+        const unsigned long long before = lt & ~((1ull << ((ostart - wbase[u]) & (WAVE - 1u))) - 1ull);
+        if ((first >> lane) & 1ull)
+          store(seg + 1u + (unsigned)__popcll(first & before), (cnt << pb) | (unsigned)qq[u]);
+        if (in_win) {
+          const unsigned o = start - wbase[u];
+          const unsigned long long lanes = len >= WAVE ? ~0ull : ((1ull << len) - 1ull) << (o & (WAVE - 1u));
+          const unsigned L = len ? (unsigned)__popcll(first & lanes) : 0u;
+          ent[start + (unsigned)(c + lane)] = L;
+          ev[start + (unsigned)(c + lane)] = (unsigned short)L;
+        }
+        wave_lds_sync();
       }
-      L += __popcll(bm);
-      wave_lds_sync();
-      if (ok) atomicAdd(&lcnt[slot[q]], 1);
-      wave_lds_sync();
+      if (ng < BUILD_GROUP && i < nc) {
+        const unsigned s = (unsigned)__builtin_amdgcn_readlane((int)start, i);
+        const unsigned e = (unsigned)__builtin_amdgcn_readlane((int)end, i);
+        const unsigned seg = s + (unsigned)(c + i);
+        int L = 0;
+        for (unsigned k0 = s; k0 < e; k0 += 2 * BUILD_GROUP * WAVE) {
+          int r[2 * BUILD_GROUP], q[2 * BUILD_GROUP];
+#pragma unroll
+          for (int u = 0; u < 2 * BUILD_GROUP; u++) {
+            const unsigned k = k0 + (unsigned)(u * WAVE + lane);
+            r[u] = k < e ? apply_pins[k] : -1;
+          }
+#pragma unroll
+          for (int u = 0; u < 2 * BUILD_GROUP; u++) q[u] = r[u] >= 0 ? part_at(r[u]) : 0;
+#pragma unroll
+          for (int u = 0; u < 2 * BUILD_GROUP; u++) {
+            if (k0 + (unsigned)(u * WAVE) >= e) break;
+            const bool ok = r[u] >= 0;
+            const bool fresh = ok && slot[q[u]] == SLOT_NONE;
+            const unsigned claim = 0x80000000u | (unsigned)lane;
+            if (__ballot(fresh)) {
+              wave_lds_sync();
+              if (fresh) atomicMin(&slot[q[u]], claim);
+              wave_lds_sync();
+              const bool first = fresh && slot[q[u]] == claim;
+              const unsigned long long bm = __ballot(first);
+              wave_lds_sync();
+              if (first) {
+                const int pos = L + (int)__popcll(bm & lt);
+                slot[q[u]] = (unsigned)pos;
+                list[pos] = (unsigned)q[u];
+              }
+              L += (int)__popcll(bm);
+              wave_lds_sync();
+            }
+            if (ok) atomicAdd(&list[slot[q[u]]], inc);
+          }
+        }
+        wave_lds_sync();
+        for (int t = lane; t < L; t += WAVE) {
+          const unsigned x = list[t];
+          store(seg + 1u + (unsigned)t, x);
+          slot[x & pmask] = SLOT_NONE;
+        }
+        if (lane == 0) {
+          ent[seg] = (unsigned)L;
+          ev[seg] = (unsigned short)L;
+        }
+        wave_lds_sync();
+        i++;
+      }
     }
-    const unsigned seg = s + (unsigned)n;
-    for (int t = lane; t < L; t += WAVE) {
-      const unsigned x = ((unsigned)lcnt[t] << pb) | (unsigned)lq[t];
-      ent[seg + 1 + (unsigned)t] = x;
-      ev[seg + 1 + (unsigned)t] = ev_word(x, pb, pmask);
-      slot[lq[t]] = -1;
-    }
-    if (lane == 0) {
-      ent[seg] = (unsigned)L;
-      ev[seg] = (unsigned short)L;
-    }
-    wave_lds_sync();
   }
 }
 
@@ -642,10 +746,11 @@ fp_status fp_set_partition(fp_ctx* ctx, int K, const int* part) {
     FP_TRY(h2d(ctx, ctx->part, part, (size_t)ctx->nov));
     FP_TRY(h2d(ctx, ctx->sizes, sz.data(), (size_t)K));
     int waves = 4;
-    while (waves > 1 && (size_t)waves * 16 * (size_t)K > (size_t)LDS_BUDGET) waves--;
-    const int grid = std::max(1, std::min((noe + waves - 1) / waves, 8192));
-    k_build_lists<<<grid, waves * WAVE, (size_t)waves * 16 * (size_t)K, ctx->stream>>>(
-        ctx->net_ptr, ctx->apply_pins, ctx->order, ctx->part, noe, K, ctx->pb, ctx->pmask, ctx->ent, ctx->ev);
+    while (waves > 1 && (size_t)waves * 8 * (size_t)K + BUILD_STATIC > (size_t)LDS_BUDGET) waves--;
+    const int per_wave = std::max(1, std::min((noe + BUILD_BLOCKS * waves - 1) / (BUILD_BLOCKS * waves), WAVE));
+    const int grid = std::max(1, std::min((noe + per_wave * waves - 1) / (per_wave * waves), BUILD_BLOCKS));
+    k_build_lists<<<grid, waves * WAVE, (size_t)waves * 8 * (size_t)K, ctx->stream>>>(
+        ctx->net_ptr, ctx->apply_pins, ctx->order, ctx->part, noe, per_wave, K, ctx->pb, ctx->pmask, ctx->ent, ctx->ev);
     FP_HIP_OK(hipGetLastError());
     FP_HIP_OK(hipStreamSynchronize(ctx->stream));
     ctx->has_state = true;

@@ -129,8 +129,22 @@ __device__ __forceinline__ int wave_max(int x) {
   return __builtin_amdgcn_readlane(x, WAVE - 1);
 }
 
-// lane l: x of lane l - 1, and -1 for lane 0 (wave_shr:1)
+// lane l: x of lane l - 1, and -1 for lane 0 (wave_shr:1); x of lane l + 1, and
+// -1 for the last lane (wave_shl:1)
 __device__ __forceinline__ int wave_shift_up(int x) { return dpp_i32<0x138>(-1, x); }
+__device__ __forceinline__ int wave_shift_down(int x) { return dpp_i32<0x130>(-1, x); }
+
+// Inclusive max-scan over the wave (values >= -1); the DPP steps move -1 into
+// lanes they do not reach.
+__device__ __forceinline__ int wave_incl_max(int x) {
+  x = max(x, dpp_i32<0x111>(-1, x));
+  x = max(x, dpp_i32<0x112>(-1, x));
+  x = max(x, dpp_i32<0x114>(-1, x));
+  x = max(x, dpp_i32<0x118>(-1, x));
+  x = max(x, dpp_i32<0x142, 0xA>(-1, x));
+  x = max(x, dpp_i32<0x143, 0xC>(-1, x));
+  return x;
+}
 
 // The same for unsigned max (identity 0) and min (identity ~0).
 __device__ __forceinline__ unsigned wave_max_u32(unsigned x) {

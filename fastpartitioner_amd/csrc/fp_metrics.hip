@@ -76,18 +76,6 @@ struct MetricArgs {
   unsigned* partial;    // gridDim.x rows of PR words
 };
 
-// Inclusive max-scan over the wave (values >= -1); the DPP steps move -1 into
-// lanes they do not reach.
-__device__ __forceinline__ int wave_incl_max(int x) {
-  x = max(x, dpp_i32<0x111>(-1, x));
-  x = max(x, dpp_i32<0x112>(-1, x));
-  x = max(x, dpp_i32<0x114>(-1, x));
-  x = max(x, dpp_i32<0x118>(-1, x));
-  x = max(x, dpp_i32<0x142, 0xA>(-1, x));
-  x = max(x, dpp_i32<0x143, 0xC>(-1, x));
-  return x;
-}
-
 // Ascending bitonic sort of one key per lane across the wavefront.
 __device__ __forceinline__ unsigned wave_sort_u32(unsigned key) {
   const int lane = lane_id();

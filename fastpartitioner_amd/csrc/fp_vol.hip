@@ -36,8 +36,13 @@ constexpr int REPLAY_BLOCK = 256;
 constexpr int REPLAY_NET_BLOCKS = 2048;
 
 // per part: volume of every net whose source is in the part, lambda - 1 (plus,
-// for MSRV, one per other part of the net: what it receives); one wavefront
-// per net, block-private sums in LDS
+// for MSRV, one per other part of the net: what it receives); block-private
+// sums in LDS. A lane per net, so that 64 nets' dependent reads (offset, length
+// and source, the source's part) go together; MSRV's lists of more than
+// VOL_INIT_SMALL entries are taken by the wavefront. A wavefront per net took
+// 582 us for 2,000,000 nets (MSV) and 77 us for 200,000 (MSRV).
+constexpr int VOL_INIT_SMALL = 16;
+
 __global__ void __launch_bounds__(256) k_vol_init(const unsigned* __restrict__ net_ptr,
                                                   const unsigned* __restrict__ ent, const int* __restrict__ src,
                                                   const int* __restrict__ part, int noe, unsigned pmask, int K,
@@ -47,17 +52,33 @@ __global__ void __launch_bounds__(256) k_vol_init(const unsigned* __restrict__ n
   for (int q = (int)threadIdx.x; q < K; q += (int)blockDim.x) s_vol[q] = 0;
   __syncthreads();
   const int nw = (int)(gridDim.x * blockDim.x / WAVE);
-  for (int n = (int)((blockIdx.x * blockDim.x + threadIdx.x) / WAVE); n < noe; n += nw) {
-    const unsigned seg = net_ptr[n] + (unsigned)n;
-    const int L = (int)ent[seg];
-    if (L == 0) continue;
-    const int sp = part[src[n]];
-    if (L > 1 && lane == 0) atomicAdd(&s_vol[sp], L - 1);
-    if (msrv)
-      for (int t = lane; t < L; t += WAVE) {
+  for (int n0 = (int)((blockIdx.x * blockDim.x + threadIdx.x) / WAVE) * WAVE; n0 < noe; n0 += nw * WAVE) {
+    const int n = n0 + lane;
+    unsigned seg = 0;
+    int L = 0, sp = 0;
+    if (n < noe) {
+      seg = net_ptr[n] + (unsigned)n;
+      L = (int)ent[seg];
+      if (L > 0) sp = part[src[n]];
+    }
+    if (L > 1) atomicAdd(&s_vol[sp], L - 1);
+    if (!msrv) continue;
+    if (L <= VOL_INIT_SMALL) {
+#pragma unroll 4
+      for (int t = 0; t < L; t++) {
         const int q = (int)(ent[seg + 1 + (unsigned)t] & pmask);
         if (q != sp) atomicAdd(&s_vol[q], 1);
       }
+    }
+    for (unsigned long long m = __ballot(L > VOL_INIT_SMALL); m; m &= m - 1) {
+      const int j = __ffsll((long long)m) - 1;
+      const unsigned sj = (unsigned)__builtin_amdgcn_readlane((int)seg, j);
+      const int Lj = __builtin_amdgcn_readlane(L, j), spj = __builtin_amdgcn_readlane(sp, j);
+      for (int t = lane; t < Lj; t += WAVE) {
+        const int q = (int)(ent[sj + 1 + (unsigned)t] & pmask);
+        if (q != spj) atomicAdd(&s_vol[q], 1);
+      }
+    }
   }
   __syncthreads();
   for (int q = (int)threadIdx.x; q < K; q += (int)blockDim.x)
