@@ -4,8 +4,8 @@
 // reference's partition_par with one thread (CN/partition.cpp:436-836).
 //
 // A pass:
-//   k_cn_eval     one wavefront filters 64 nets at a time; every lambda = 2
-//                 net picks old = the part with the smaller pin count (ties:
+//   k_cn_eval     the lambda = 2 nets of up to 64 consecutive nets, their pins
+//                 packed into 64-lane windows; each picks old = the part with the smaller pin count (ties:
 //                 the second entry) and is accepted iff none of its old-side
 //                 pins lies on an uncut net (CN/partition.cpp:650-690)
 //   scan          push offsets: exclusive scan of the accepted nets' old-side
@@ -30,6 +30,7 @@ namespace {
 
 constexpr int CN_MAXOPS = 4096;  // ops per net and pass sorted in LDS; more go through k_cn_bigsort
 constexpr int SCAN_BLOCK = 1024;
+constexpr int CN_EVAL_WAVES = 8192;
 constexpr int CN_EVAL_GROUP = 4;  // a pin's nets whose lambdas k_cn_eval loads together
 
 struct CnEvalArgs {
@@ -42,30 +43,95 @@ struct CnEvalArgs {
   const int* part;
   int noe, pb;
   unsigned pmask;
+  int per_wave;  // consecutive nets per wave (<= 64)
   int* cn_old;  // accepted: old part; else -1
   int* cn_new;
   int* npush;
 };
 
+// A wavefront takes per_wave consecutive nets, a net per lane, and of these the
+// lambda = 2 nets of at most 64 pins together: whole nets share a window of 64
+// pins, a pin per lane, and a net's verdict is a mask over its lanes. Longer
+// ones go 64 pins at a time. Bound by the dependent gathers of an old-side pin
+// (its part, its net range, its nets' offsets and lambdas); most such nets have
+// 2 or 3 pins, and a wavefront for each left 61 lanes idle through that chain:
+// 120 us for 1,000,000 Zipf nets at K = 256, now 39 us.
 __global__ void __launch_bounds__(256) k_cn_eval(CnEvalArgs a) {
+  __shared__ int s_win[256 / WAVE][WAVE];
   const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
-  for (int n0 = ((int)blockIdx.x * nw + wave) * WAVE; n0 < a.noe; n0 += (int)gridDim.x * nw * WAVE) {
-    const int n = n0 + lane;
-    bool two = false;
-    if (n < a.noe) {
-      two = a.ev[a.net_ptr[n] + (unsigned)n] == 2;
-      if (!two) { a.cn_old[n] = -1; a.npush[n] = 0; }
+  int* winbuf = s_win[wave];  // net starting at each window lane
+  // whether one of v's nets is uncut: CN_EVAL_GROUP nets at a time, their
+  // segment offsets, then their lambdas
+  auto on_uncut = [&](int v) -> bool {
+    bool b = false;
+    const unsigned jb = a.vtx_ptr[v], je = a.vtx_ptr[v + 1];
+    for (unsigned j = jb; j < je && !b; j += CN_EVAL_GROUP) {
+      unsigned sg[CN_EVAL_GROUP];
+#pragma unroll
+      for (int u = 0; u < CN_EVAL_GROUP; u++) sg[u] = a.vtx_seg[min(j + (unsigned)u, je - 1)];
+#pragma unroll
+      for (int u = 0; u < CN_EVAL_GROUP; u++) b |= a.ev[sg[u]] == 1;
     }
-    unsigned long long m = __ballot(two);
-    while (m) {
-      const int nn = n0 + __ffsll((long long)m) - 1;
-      m &= m - 1;
-      const unsigned s = a.net_ptr[nn], e = a.net_ptr[nn + 1];
-      const unsigned seg = s + (unsigned)nn;
-      const unsigned x1 = a.ent[seg + 1], x2 = a.ent[seg + 2];
-      const int p1 = (int)(x1 & a.pmask), c1 = (int)(x1 >> a.pb);
-      const int p2 = (int)(x2 & a.pmask), c2 = (int)(x2 >> a.pb);
-      const int oldp = c1 < c2 ? p1 : p2, newp = c1 < c2 ? p2 : p1;
+    return b;
+  };
+  for (int n0 = ((int)blockIdx.x * nw + wave) * a.per_wave; n0 < a.noe; n0 += (int)gridDim.x * nw * a.per_wave) {
+    const int n = n0 + lane;
+    const bool in = lane < a.per_wave && n < a.noe;
+    unsigned start = 0, end = 0;
+    bool two = false;
+    int oldp = -1, newp = -1;
+    if (in) {
+      start = a.net_ptr[n];
+      end = a.net_ptr[n + 1];
+      const unsigned seg = start + (unsigned)n;
+      two = a.ev[seg] == 2;
+      if (!two) {
+        a.cn_old[n] = -1;
+        a.npush[n] = 0;
+      } else {
+        const unsigned x1 = a.ent[seg + 1], x2 = a.ent[seg + 2];
+        const bool second = (int)(x1 >> a.pb) < (int)(x2 >> a.pb);
+        oldp = (int)((second ? x1 : x2) & a.pmask);
+        newp = (int)((second ? x2 : x1) & a.pmask);
+      }
+    }
+    const int len = (int)(end - start);
+    const bool sel = two && len <= WAVE;
+    const int incl = wave_incl_scan(sel ? len : 0), excl = incl - (sel ? len : 0);
+    const int total = __builtin_amdgcn_readlane(incl, WAVE - 1);
+    for (int base = 0; base < total;) {
+      // the nets from pin base on that fit 64 lanes
+      const bool fit = sel && excl >= base && incl - base <= WAVE;
+      const int np = __builtin_amdgcn_readlane(incl, WAVE - 1 - __builtin_clzll(__ballot(fit))) - base;
+      winbuf[lane] = -1;
+      wave_lds_sync();
+      if (fit) winbuf[excl - base] = lane;
+      wave_lds_sync();
+      const int owner = max(wave_incl_max(winbuf[lane]), 0);
+      const unsigned first = (unsigned)__shfl((int)start - excl, owner) + (unsigned)base;
+      const int op = __shfl(oldp, owner);
+      bool isold = false, b = false;
+      if (lane < np) {
+        const int v = (int)a.net_pins[first + (unsigned)lane];
+        isold = a.part[v] == op;
+        if (isold) b = on_uncut(v);
+      }
+      const unsigned long long om = __ballot(isold), bm = __ballot(b);
+      if (fit) {
+        const unsigned long long lanes = len >= WAVE ? ~0ull : ((1ull << len) - 1ull) << (excl - base);
+        const bool bad = (bm & lanes) != 0ull;
+        a.cn_old[n] = bad ? -1 : oldp;
+        a.cn_new[n] = newp;
+        a.npush[n] = bad ? 0 : (int)__popcll(om & lanes);
+      }
+      base += np;
+      wave_lds_sync();
+    }
+    for (unsigned long long m = __ballot(two && !sel); m; m &= m - 1) {
+      const int j = __ffsll((long long)m) - 1;
+      const unsigned s = (unsigned)__builtin_amdgcn_readlane((int)start, j);
+      const unsigned e = (unsigned)__builtin_amdgcn_readlane((int)end, j);
+      const int op = __builtin_amdgcn_readlane(oldp, j);
       bool bad = false;
       int cnt = 0;
       for (unsigned k0 = s; k0 < e && !bad; k0 += WAVE) {
@@ -73,28 +139,16 @@ __global__ void __launch_bounds__(256) k_cn_eval(CnEvalArgs a) {
         bool isold = false, b = false;
         if (k < e) {
           const int v = (int)a.net_pins[k];
-          isold = a.part[v] == oldp;
-          if (isold) {
-            // v's nets CN_EVAL_GROUP at a time: their segment offsets load
-            // together, then their lambdas, instead of one dependent pair of
-            // loads per net
-            const unsigned jb = a.vtx_ptr[v], je = a.vtx_ptr[v + 1];
-            for (unsigned j = jb; j < je && !b; j += CN_EVAL_GROUP) {
-              unsigned sg[CN_EVAL_GROUP];
-#pragma unroll
-              for (int u = 0; u < CN_EVAL_GROUP; u++) sg[u] = a.vtx_seg[min(j + (unsigned)u, je - 1)];
-#pragma unroll
-              for (int u = 0; u < CN_EVAL_GROUP; u++) b |= a.ev[sg[u]] == 1;
-            }
-          }
+          isold = a.part[v] == op;
+          if (isold) b = on_uncut(v);
         }
-        cnt += __popcll(__ballot(isold));
-        bad = __ballot(b) != 0;
+        cnt += (int)__popcll(__ballot(isold));
+        bad = __ballot(b) != 0ull;
       }
-      if (lane == 0) {
-        a.cn_old[nn] = bad ? -1 : oldp;
-        a.cn_new[nn] = newp;
-        a.npush[nn] = bad ? 0 : cnt;
+      if (lane == j) {
+        a.cn_old[n] = bad ? -1 : oldp;
+        a.cn_new[n] = newp;
+        a.npush[n] = bad ? 0 : cnt;
       }
     }
   }
@@ -500,48 +554,55 @@ __global__ void __launch_bounds__(WAVE) k_cn_apply(CnApplyArgs a) {
   if (INDEXED) wave_index_init(at, a.K);
   const int nt = *a.tcount;
   if ((a.flags[0] | a.flags[1]) != 0) return;  // k_cn_apply_small reset the op counts
-  for (int i = (int)blockIdx.x; i < nt; i += (int)gridDim.x) {
-    const int t = a.touched[i];
-    const int c = a.opcnt[t];
-    if (c <= WAVE) continue;  // k_cn_apply_small's (reset to 0 there)
-    const long long off = a.opoff[t];
-    // up to CN_MAXOPS ops are sorted here; a big net's ops come in order
-    // from k_cn_bigsort and are read straight from the op list
-    const bool small = c <= CN_MAXOPS;
-    if (small) {
-      int P = 1;
-      while (P < c) P <<= 1;
-      for (int j = lane; j < P; j += WAVE) keys[j] = j < c ? (unsigned)a.ops[off + j] : 0xFFFFFFFFu;
-      wave_lds_sync();
-      if (c > 1) wave_bitonic_sort(keys, P);
-    }
-    const unsigned s0 = a.net_ptr[t], seg = s0 + (unsigned)t;
-    int L = wave_list_load(a.ent, seg, a.net_ptr[t + 1] - s0, list);
-    if (INDEXED) wave_index_set(list, L, at, a.pmask);
-    for (int j0 = 0; j0 < c; j0 += WAVE) {
-      // 64 moves at a time: each lane loads one move's old and new part
-      int from_l = 0, to_l = 0;
-      if (j0 + lane < c) {
-        const int m = small ? (int)keys[j0 + lane] : a.ops[off + j0 + lane];
-        from_l = a.mv_from[m];
-        to_l = a.cn_new[a.mv_net[m]];
+  // the block's touched nets (every gridDim-th: the ones with many ops stand
+  // together on the list), a net per lane: the few with more than 64 ops (the
+  // others are k_cn_apply_small's, their counts reset to 0 there)
+  for (long long i0 = (long long)blockIdx.x; i0 < nt; i0 += (long long)gridDim.x * WAVE) {
+    const long long i = i0 + (long long)lane * gridDim.x;
+    const int t_l = i < nt ? a.touched[i] : 0;
+    const int c_l = i < nt ? a.opcnt[t_l] : 0;
+    for (unsigned long long m = __ballot(c_l > WAVE); m; m &= m - 1) {
+      const int j = __ffsll((long long)m) - 1;
+      const int t = __builtin_amdgcn_readlane(t_l, j), c = __builtin_amdgcn_readlane(c_l, j);
+      const long long off = a.opoff[t];
+      // up to CN_MAXOPS ops are sorted here; a big net's ops come in order
+      // from k_cn_bigsort and are read straight from the op list
+      const bool small = c <= CN_MAXOPS;
+      if (small) {
+        int P = 1;
+        while (P < c) P <<= 1;
+        for (int k = lane; k < P; k += WAVE) keys[k] = k < c ? (unsigned)a.ops[off + k] : 0xFFFFFFFFu;
+        wave_lds_sync();
+        if (c > 1) wave_bitonic_sort(keys, P);
       }
-      const int nj = min(WAVE, c - j0);
-      for (int l = 0; l < nj; l++) {
-        const int p = __builtin_amdgcn_readlane(from_l, l), q = __builtin_amdgcn_readlane(to_l, l);
-        if (INDEXED) {
-          unsigned co;
-          bool found;
-          wave_ilist_move(list, at, L, p, q, a.pb, a.pmask, co, found);
-        } else {
-          wave_list_move(list, L, p, q, a.pb, a.pmask);
+      const unsigned s0 = a.net_ptr[t], seg = s0 + (unsigned)t;
+      int L = wave_list_load(a.ent, seg, a.net_ptr[t + 1] - s0, list);
+      if (INDEXED) wave_index_set(list, L, at, a.pmask);
+      for (int j0 = 0; j0 < c; j0 += WAVE) {
+        // 64 moves at a time: each lane loads one move's old and new part
+        int from_l = 0, to_l = 0;
+        if (j0 + lane < c) {
+          const int m = small ? (int)keys[j0 + lane] : a.ops[off + j0 + lane];
+          from_l = a.mv_from[m];
+          to_l = a.cn_new[a.mv_net[m]];
+        }
+        const int nj = min(WAVE, c - j0);
+        for (int l = 0; l < nj; l++) {
+          const int p = __builtin_amdgcn_readlane(from_l, l), q = __builtin_amdgcn_readlane(to_l, l);
+          if (INDEXED) {
+            unsigned co;
+            bool found;
+            wave_ilist_move(list, at, L, p, q, a.pb, a.pmask, co, found);
+          } else {
+            wave_list_move(list, L, p, q, a.pb, a.pmask);
+          }
         }
       }
+      wave_list_store(a.ent, a.ev, seg, list, L, a.pb, a.pmask);
+      if (INDEXED) wave_index_clear(list, L, at, a.pmask);
+      if (lane == 0) a.opcnt_reset[t] = 0;
+      wave_lds_sync();
     }
-    wave_list_store(a.ent, a.ev, seg, list, L, a.pb, a.pmask);
-    if (INDEXED) wave_index_clear(list, L, at, a.pmask);
-    if (lane == 0) a.opcnt_reset[t] = 0;
-    wave_lds_sync();
   }
 }
 
@@ -670,10 +731,13 @@ fp_status pass_cn(fp_ctx* ctx, const RefinePlan&) {
   // one round per pass: the touched-net counters start at 0
   pass_begin(ctx, nullptr, 0, nullptr);
   fill_async<unsigned long long>(ctx, s.totals, 5, 0ull);
+  // as many nets per wave as give the 8,192 resident waves a share
+  const int per_wave = std::max(1, std::min((noe + CN_EVAL_WAVES - 1) / CN_EVAL_WAVES, WAVE));
   CnEvalArgs ea{ctx->net_ptr, ctx->net_pins, ctx->vtx_ptr, ctx->vtx_seg, ctx->ent, ctx->ev, ctx->part,
-                noe, ctx->pb, ctx->pmask, s.old_part, s.new_part, s.npush};
+                noe, ctx->pb, ctx->pmask, per_wave, s.old_part, s.new_part, s.npush};
   const int waves_needed = (noe + WAVE - 1) / WAVE;
-  k_cn_eval<<<std::max(1, std::min((waves_needed + 3) / 4, 8192)), 256, 0, ctx->stream>>>(ea);
+  k_cn_eval<<<std::max(1, std::min((noe + 4 * per_wave - 1) / (4 * per_wave), CN_EVAL_WAVES / 4)), 256, 0,
+              ctx->stream>>>(ea);
   k_scan_sums<<<std::max(nblk, 1), SCAN_BLOCK, 0, ctx->stream>>>(s.npush, noe, s.sums);
   k_scan_top<<<1, SCAN_BLOCK, 0, ctx->stream>>>(s.sums, nblk, reinterpret_cast<long long*>(s.totals + 3));
   k_scan_apply<<<std::max(nblk, 1), SCAN_BLOCK, 0, ctx->stream>>>(s.npush, noe, s.sums, s.pbase);
