@@ -12,15 +12,15 @@
 //                  max part gains at least (MSV) / more than (MSRV) it loses
 //                  and no other part reaches the max
 //   k_round_compact accepted moves in visiting order, with event offsets
-//   k_vol_replay   (dry) one wavefront per touched net replays the round's
-//                  moves on its list in order and records, per (move, net),
+//   k_vol_events   one wavefront per touched net takes the round's moves of
+//                  its pins, 64 pins at a time, and records, per (move, net),
 //                  the volume changes the reference's apply makes
 //   k_vol_scan     one wavefront applies the moves' volume changes in order,
 //                  tracks the max set, and stops after the first move whose
 //                  max set holds a part the previous one did not
 //                  (MGV/partition.cpp:977-1003); batches of 64 moves are
 //                  decided together where bounds allow
-//   k_vol_replay   (commit) list edits, part vector and both part sizes of the
+//   k_vol_commit   list edits, part vector and both part sizes of the
 //                  moves up to the stop
 #include "fp_masks.h"
 #include "fp_round.h"
@@ -731,20 +731,189 @@ struct VolReplayArgs {
   int mask_words;
   int K, pb;
   unsigned pmask;
-  int r0, r1, msrv, commit, net_blocks;
+  int r0, r1, msrv, net_blocks;
 };
 
-// dry (commit = 0): per (move, net) volume changes of the reference's apply
-//   (MGV/partition.cpp:897-975; MSRV/partition.cpp:952-1052), recorded as
-//   (source part and its change, change of own part, change of new part,
-//   move index) at event slot mv.evoff + (position of the net in the move's
-//   vertex->nets list); the list edits stay in LDS
-// commit (commit = 1): list edits of the moves before the stop; blocks past
-//   net_blocks commit part vector and both part sizes
+// Per (move, net) the volume changes of the reference's apply
+// (MGV/partition.cpp:897-975; MSRV/partition.cpp:952-1052), recorded as (source
+// part and its change, change of own part, change of new part, move index) at
+// event slot mv.evoff + (position of the net in the move's vertex->nets list).
+// They depend on how many of the net's pins the two parts hold when the move
+// comes, on the list's length and on the source's part, but not on the list's
+// order: a wavefront per touched net takes the counts from the list into a word
+// per part, and 64 pins' moves together. A lane's counts are those at the
+// window's start corrected by each earlier move of the window (a readlane and a
+// few compares a move), the length and the source's part follow from ballots.
+// Bound by the dependent loads of the largest nets, VOL_EVENT_GROUP windows to
+// a round of them (eight windows in 130 registers leave 3 waves per SIMD; four
+// take 70). Replaying the list a move at a time, five dependent LDS accesses
+// each, took 103 us on average over the rounds of MSV and MSRV requests on Zipf
+// hypergraphs of 5,000 to 200,000 vertices sharing the GPU, up to 1.9 ms for a
+// net of 5,000 pins; now 20 us, up to 0.28 ms. Following all moves of a window,
+// not those of its open parts alone, took 30 us.
+constexpr int VOL_EVENT_GROUP = 4;   // windows of a net whose loads are issued together
+constexpr int VOL_COMMIT_GROUP = 4;  // the same in k_vol_commit
+constexpr int VOL_TOGETHER = 8;      // moves of a window worth trying together
+
+// LDS words a wavefront of k_vol_events needs: a count per part, cleared 16 bytes a lane
+__host__ __device__ constexpr int vol_event_words(int K) { return (K + 3) & ~3; }
+
+__global__ void __launch_bounds__(REPLAY_BLOCK) k_vol_events(VolReplayArgs a) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
+  const int words = vol_event_words(a.K);
+  int* cnt = reinterpret_cast<int*>(lds) + (size_t)wave * (size_t)words;
+  auto clear = [&] {
+    for (int t = 4 * lane; t < words; t += 4 * WAVE) *reinterpret_cast<int4*>(cnt + t) = make_int4(0, 0, 0, 0);
+  };
+  clear();
+  const unsigned long long lt = (1ull << lane) - 1ull;
+  const int ntouched = *a.tcount;
+  for (int i = (int)blockIdx.x * nw + wave; i < ntouched; i += a.net_blocks * nw) {
+    const int n = a.touched[i];
+    const unsigned s = a.net_ptr[n], e = a.net_ptr[n + 1];
+    const unsigned seg = s + (unsigned)n;
+    const unsigned head = wave_list_head(a.ent, seg, e - s);
+    const int srcv = a.src[n];
+    unsigned lo, hi;
+    wave_rank_window(a.apply_pins, s, e, a.r0, a.r1, lo, hi);
+    int sp_cur = a.part[srcv];  // the source's part as the moves go
+    int L = __builtin_amdgcn_readfirstlane((int)head);
+    wave_lds_sync();
+    if (lane >= 1 && lane <= L) cnt[head & a.pmask] = (int)(head >> a.pb);
+    for (int t = WAVE - 1 + lane; t < L; t += WAVE) {
+      const unsigned x = a.ent[seg + 1 + (unsigned)t];
+      cnt[x & a.pmask] = (int)(x >> a.pb);
+    }
+    wave_lds_sync();
+    for (unsigned k0 = lo; k0 < hi; k0 += VOL_EVENT_GROUP * WAVE) {
+      // per window: move index, own and new part, event offset less the start of
+      // the vertex's list, the bounds of the search for the net in it
+      int mi[VOL_EVENT_GROUP], oo[VOL_EVENT_GROUP], dd[VOL_EVENT_GROUP];
+      unsigned base[VOL_EVENT_GROUP], l0[VOL_EVENT_GROUP], l1[VOL_EVENT_GROUP];
+      unsigned from_src = 0;  // bit u: the window's move is the source's
+#pragma unroll
+      for (int u = 0; u < VOL_EVENT_GROUP; u++) {
+        const unsigned k = k0 + (unsigned)(u * WAVE + lane);
+        mi[u] = k < hi ? a.apply_pins[k] : INT_MAX;
+      }
+#pragma unroll
+      for (int u = 0; u < VOL_EVENT_GROUP; u++) mi[u] = mi[u] >= a.r0 && mi[u] < a.r1 ? a.slot_mi[mi[u] - a.r0] : -1;
+      int vv[VOL_EVENT_GROUP];
+#pragma unroll
+      for (int u = 0; u < VOL_EVENT_GROUP; u++) {
+        vv[u] = oo[u] = dd[u] = -1;
+        base[u] = 0;
+        if (mi[u] >= 0) {
+          const int4 m = a.mv[mi[u]];
+          vv[u] = m.x;
+          oo[u] = m.y;
+          dd[u] = m.z;
+          base[u] = (unsigned)m.w;
+        }
+      }
+      bool open = false;
+#pragma unroll
+      for (int u = 0; u < VOL_EVENT_GROUP; u++) {
+        l0[u] = l1[u] = 0;
+        if (mi[u] >= 0) {
+          l0[u] = a.vtx_ptr[vv[u]];
+          l1[u] = a.vtx_ptr[vv[u] + 1];
+        }
+        base[u] -= l0[u];
+        from_src |= vv[u] == srcv ? 1u << u : 0u;
+        open |= l0[u] < l1[u];
+      }
+      // the net's position in each moved vertex's list: the windows' searches in step
+      while (open) {
+        unsigned x[VOL_EVENT_GROUP];
+#pragma unroll
+        for (int u = 0; u < VOL_EVENT_GROUP; u++) x[u] = l0[u] < l1[u] ? a.vtx_nets[(l0[u] + l1[u]) >> 1] : 0u;
+        open = false;
+#pragma unroll
+        for (int u = 0; u < VOL_EVENT_GROUP; u++) {
+          const unsigned mid = (l0[u] + l1[u]) >> 1;
+          if (l0[u] < l1[u]) {
+            if (x[u] < (unsigned)n) l0[u] = mid + 1;
+            else l1[u] = mid;
+          }
+          open |= l0[u] < l1[u];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < VOL_EVENT_GROUP; u++) {
+        const bool act = mi[u] >= 0;
+        const unsigned long long m = __ballot(act);
+        if (m == 0ull) continue;
+        const int own = oo[u], d = dd[u];
+        int co = act ? cnt[own] : 0, cd = act ? cnt[d] : 0;
+        wave_lds_sync();
+        if (act) atomicSub(&cnt[own], 1);
+        wave_lds_sync();
+        // a part that keeps a pin whatever the order of the window's moves is
+        // never left and never new: only the other parts' moves are followed
+        const bool open_part = act && (cnt[own] < 1 || cnt[d] < 1);
+        for (unsigned long long b = __ballot(open_part); b & (b - 1); b &= b - 1) {  // the last comes before no other
+          const int l = __builtin_ctzll(b);
+          const int o = __builtin_amdgcn_readlane(own, l), q = __builtin_amdgcn_readlane(d, l);
+          if (lane > l) {
+            co += (q == own ? 1 : 0) - (o == own ? 1 : 0);
+            cd += (q == d ? 1 : 0) - (o == d ? 1 : 0);
+          }
+        }
+        const bool isrc = (from_src >> u) & 1u;
+        const bool gone = open_part && co == 1, found = !open_part || cd > 0;
+        const unsigned long long gm = __ballot(gone), nm = __ballot(act && !found), sm = __ballot(isrc);
+        const int lam_b = L + (int)__popcll(nm & lt) - (int)__popcll(gm & lt);
+        const int lam_mid = gone ? lam_b - 1 : lam_b;
+        // a net has one source among its pins: at most one move of the net is the source's
+        const int d_src = sm ? __builtin_amdgcn_readlane(d, __builtin_ctzll(sm)) : sp_cur;
+        const int sp = (sm & lt) ? d_src : sp_cur;
+        int e_own = 0, e_dec = 0, e_sp = 0, spx = -1;
+        if (isrc) e_own -= lam_b - 1;                       // send_volumes[part_id] -= end_cnt - 1
+        if (gone) {
+          if (!isrc) {
+            spx = sp;
+            e_sp -= 1;                                      // send_volumes[net_src_part]--
+            if (a.msrv) e_own -= 1;                         // received_volumes[part_id]--
+          }
+        } else if (isrc && a.msrv) {
+          e_own += 1;                                       // received_volumes[part_id]++
+        }
+        if (isrc) e_dec += lam_mid - 1;                     // send_volumes[net_src_part] += end_cnt - 1
+        if (found) {
+          if (isrc && a.msrv) e_dec -= 1;                   // received_volumes[decision]--
+        } else if (isrc) {
+          e_dec += 1;                                       // send_volumes[net_src_part]++ (source part = d)
+        } else {
+          spx = sp;
+          e_sp += 1;                                        // send_volumes[net_src_part]++
+          if (a.msrv) e_dec += 1;                           // received_volumes[decision]++
+        }
+        if (act)
+          a.evbuf[base[u] + l0[u]] = make_int4(vol_event_word(spx, e_sp), e_own, e_dec, mi[u]);
+        L += (int)__popcll(nm) - (int)__popcll(gm);
+        sp_cur = d_src;
+        wave_lds_sync();
+        if (act) atomicAdd(&cnt[d], 1);
+        wave_lds_sync();
+      }
+    }
+    wave_lds_sync();
+    clear();
+  }
+}
+
+// The list edits of the moves before the stop, a wavefront per touched net.
+// Moves that only change counts are made together (wave_ilist_moves), the
+// others one after another, in the visiting order; a net without a move before
+// the stop ends before its list is staged (13.8 -> 10.0 us on average over the
+// rounds that k_vol_events names);
+// blocks past net_blocks commit part vector and both part sizes.
 // INDEXED: each wave keeps a part -> position index of its list in LDS
 //   (2 bytes per part after the lists), for K where it fits
 template <bool INDEXED>
-__global__ void __launch_bounds__(REPLAY_BLOCK) k_vol_replay(VolReplayArgs a) {
+__global__ void __launch_bounds__(REPLAY_BLOCK) k_vol_commit(VolReplayArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
   const int nstop = a.mstat[3];
@@ -770,96 +939,68 @@ __global__ void __launch_bounds__(REPLAY_BLOCK) k_vol_replay(VolReplayArgs a) {
     const int n = a.touched[i];
     const unsigned s = a.net_ptr[n], e = a.net_ptr[n + 1];
     const unsigned seg = s + (unsigned)n;
+    const unsigned head = wave_list_head(a.ent, seg, e - s);
     unsigned lo, hi;
-    // a net of at most 64 pins: its ranks (and its source) are read together with its list
-    const bool small = e - s <= (unsigned)WAVE;
-    const int r_small = small && (unsigned)lane < e - s ? a.apply_pins[s + (unsigned)lane] : INT_MAX;
-    const int srcv = a.src[n];
     wave_rank_window(a.apply_pins, s, e, a.r0, a.r1, lo, hi);
-    int L = wave_list_load(a.ent, seg, e - s, list);
-    if (INDEXED) wave_index_set(list, L, at, a.pmask);
-    int sp_cur = a.commit ? 0 : a.part[srcv];  // the source's part as the replay goes
+    int L = 0;
     bool dirty = false;
-    for (unsigned k0 = lo; k0 < hi; k0 += WAVE) {
-      const unsigned k = k0 + (unsigned)lane;
-      int mi = -1;
-      const int r = small ? r_small : (k < hi ? a.apply_pins[k] : INT_MAX);
-      if (r >= a.r0 && r < a.r1) mi = a.slot_mi[r - a.r0];
-      if (a.commit && mi >= nstop) mi = -1;
-      // each lane fetches its own move (v, own, d, evoff) and, for the dry
-      // replay, the event slot of (move, n); the ordered replay below reads
-      // them from the lanes
-      int4 mm = make_int4(0, 0, 0, 0);
-      unsigned evslot = 0;
-      if (mi >= 0) {
-        mm = a.mv[mi];
-        if (!a.commit) {
-          const unsigned vb = a.vtx_ptr[mm.x], ve = a.vtx_ptr[mm.x + 1];
-          evslot = (unsigned)mm.w + (lane_lower_bound(a.vtx_nets, vb, ve, (unsigned)n) - vb);
+    for (unsigned k0 = lo; k0 < hi; k0 += VOL_COMMIT_GROUP * WAVE) {
+      int mi[VOL_COMMIT_GROUP], oo[VOL_COMMIT_GROUP], dd[VOL_COMMIT_GROUP];
+#pragma unroll
+      for (int u = 0; u < VOL_COMMIT_GROUP; u++) {
+        const unsigned k = k0 + (unsigned)(u * WAVE + lane);
+        mi[u] = k < hi ? a.apply_pins[k] : INT_MAX;
+      }
+#pragma unroll
+      for (int u = 0; u < VOL_COMMIT_GROUP; u++)
+        mi[u] = mi[u] >= a.r0 && mi[u] < a.r1 ? a.slot_mi[mi[u] - a.r0] : -1;
+#pragma unroll
+      for (int u = 0; u < VOL_COMMIT_GROUP; u++) {
+        oo[u] = dd[u] = 0;
+        if (mi[u] >= nstop) mi[u] = -1;
+        if (mi[u] >= 0) {
+          const int4 m = a.mv[mi[u]];
+          oo[u] = m.y;
+          dd[u] = m.z;
         }
       }
-      unsigned long long bm = __ballot(mi >= 0);
-      while (bm) {
-        const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)bm) - 1);
-        bm &= bm - 1;
-        const int v = __builtin_amdgcn_readlane(mm.x, l), own = __builtin_amdgcn_readlane(mm.y, l),
-                  d = __builtin_amdgcn_readlane(mm.z, l);
-        if (!a.commit) {
-          const bool isrc = srcv == v;
-          const int lam_b = L;
-          unsigned co;
-          bool found;
+#pragma unroll
+      for (int u = 0; u < VOL_COMMIT_GROUP; u++) {
+        unsigned long long m = __ballot(mi[u] >= 0);
+        if (m && !dirty) {
+          // the first move: the list is staged
+          dirty = true;
+          L = wave_list_stage(a.ent, seg, head, list);
+          if (INDEXED) wave_index_set(list, L, at, a.pmask);
+        }
+        bool together = INDEXED;  // worth trying in this window
+        while (m) {
+          if (together && __popcll(m) >= VOL_TOGETHER) {
+            const unsigned long long rest = wave_ilist_moves(list, at, m, oo[u], dd[u], a.pb);
+            together = __popcll(m) - __popcll(rest) >= VOL_TOGETHER / 2;
+            m = rest;
+            if (!m) break;
+          }
+          const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)m) - 1);
+          m &= m - 1;
+          const int own = __builtin_amdgcn_readlane(oo[u], l), d = __builtin_amdgcn_readlane(dd[u], l);
           if (INDEXED) {
+            unsigned co;
+            bool found;
             wave_ilist_move(list, at, L, own, d, a.pb, a.pmask, co, found);
           } else {
-            const int jo = wave_find(list, L, own, a.pmask);
-            co = jo >= 0 ? (list[jo] >> a.pb) : 0u;
-            found = wave_find(list, L, d, a.pmask) >= 0;
             wave_list_move(list, L, own, d, a.pb, a.pmask);
           }
-          const int lam_mid = co == 1u ? lam_b - 1 : lam_b;
-          int e_own = 0, e_dec = 0, e_sp = 0, spx = -1;
-          if (isrc) e_own -= lam_b - 1;                       // send_volumes[part_id] -= end_cnt - 1
-          if (co == 1u) {
-            if (!isrc) {
-              spx = sp_cur;
-              e_sp -= 1;                                      // send_volumes[net_src_part]--
-              if (a.msrv) e_own -= 1;                         // received_volumes[part_id]--
-            }
-          } else if (isrc && a.msrv) {
-            e_own += 1;                                       // received_volumes[part_id]++
-          }
-          if (isrc) e_dec += lam_mid - 1;                     // send_volumes[net_src_part] += end_cnt - 1
-          if (found) {
-            if (isrc && a.msrv) e_dec -= 1;                   // received_volumes[decision]--
-          } else if (isrc) {
-            e_dec += 1;                                       // send_volumes[net_src_part]++ (source part = d)
-          } else {
-            spx = sp_cur;
-            e_sp += 1;                                        // send_volumes[net_src_part]++
-            if (a.msrv) e_dec += 1;                           // received_volumes[decision]++
-          }
-          if (lane == 0)
-            a.evbuf[(unsigned)__builtin_amdgcn_readlane((int)evslot, l)] =
-                make_int4(vol_event_word(spx, e_sp), e_own, e_dec, __builtin_amdgcn_readlane(mi, l));
-          if (isrc) sp_cur = d;
-        } else if (INDEXED) {
-          unsigned co;
-          bool found;
-          wave_ilist_move(list, at, L, own, d, a.pb, a.pmask, co, found);
-        } else {
-          wave_list_move(list, L, own, d, a.pb, a.pmask);
         }
-        dirty = true;
       }
     }
-    if (a.commit && dirty) {
+    if (dirty) {
       wave_list_store(a.ent, a.ev, seg, list, L, a.pb, a.pmask);
       if (INDEXED && a.masks)
         wave_store_masks(list, at, a.K, a.pb, a.mask_words, a.masks + (size_t)n * (size_t)(2 * a.mask_words));
+      if (INDEXED) wave_index_clear(list, L, at, a.pmask);
+      wave_lds_sync();
     }
-    if (INDEXED) wave_index_clear(list, L, at, a.pmask);
-    wave_lds_sync();
   }
 }
 
@@ -1235,12 +1376,13 @@ fp_status pass_vol(fp_ctx* ctx, const RefinePlan& p) {
   const int nov = ctx->nov, K = ctx->K, R = p.R, waves = p.eval_waves;
   const bool shorts = vol_eval_lds(K, waves, true) <= (size_t)LDS_BUDGET;
   const size_t lds_e = vol_eval_lds(K, waves, shorts);
-  // the replay's part -> position index where it fits the LDS budget
+  // the commit's part -> position index where it fits the LDS budget
   const bool indexed = (size_t)(REPLAY_BLOCK / WAVE) * (size_t)K * (sizeof(unsigned) + sizeof(unsigned short)) <=
                        (size_t)LDS_BUDGET;
   const size_t lds_r = (size_t)(REPLAY_BLOCK / WAVE) * (size_t)K *
                        (sizeof(unsigned) + (indexed ? sizeof(unsigned short) : 0));
-  auto replay = indexed ? k_vol_replay<true> : k_vol_replay<false>;
+  auto commit = indexed ? k_vol_commit<true> : k_vol_commit<false>;
+  const size_t lds_d = (size_t)(REPLAY_BLOCK / WAVE) * (size_t)vol_event_words(K) * sizeof(int);
   const int batched = K <= VOL_BATCH_KMAX ? 1 : 0;
   const size_t lds_vol = ((size_t)K + WAVE + (batched ? vol_batch_ints(K) : 0)) * sizeof(int);
   const int stage_cap = (int)std::min<size_t>(4096, ((size_t)LDS_BUDGET - lds_vol) / sizeof(int4));
@@ -1325,11 +1467,9 @@ fp_status pass_vol(fp_ctx* ctx, const RefinePlan& p) {
     ra.r1 = r0 + nslots;
     ra.msrv = msrv ? 1 : 0;
     ra.net_blocks = net_grid(ctx, REPLAY_NET_BLOCKS, REPLAY_BLOCK / WAVE);
-    ra.commit = 0;
-    replay<<<ra.net_blocks, REPLAY_BLOCK, lds_r, ctx->stream>>>(ra);
+    k_vol_events<<<ra.net_blocks, REPLAY_BLOCK, lds_d, ctx->stream>>>(ra);
     k_vol_scan<<<1, WAVE, lds_s, ctx->stream>>>(vs.vol, K, vs.mv, vs.evbuf, vs.mstat, stage_cap, batched);
-    ra.commit = 1;
-    replay<<<ra.net_blocks + (nslots + REPLAY_BLOCK - 1) / REPLAY_BLOCK, REPLAY_BLOCK, lds_r, ctx->stream>>>(ra);
+    commit<<<ra.net_blocks + (nslots + REPLAY_BLOCK - 1) / REPLAY_BLOCK, REPLAY_BLOCK, lds_r, ctx->stream>>>(ra);
   }
   return FP_OK;
 }
