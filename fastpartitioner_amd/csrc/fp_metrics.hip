@@ -31,7 +31,13 @@ namespace {
 
 constexpr int MET_WAVES = 8;             // wavefronts per block
 constexpr int MET_BLOCK = MET_WAVES * WAVE;
-constexpr int MET_CHUNK = 64;            // nets per work item
+// Nets per work item: a wavefront's windows follow one another (offsets, pins,
+// parts, a sort of 64 keys), so an instance too small to give every wavefront 64
+// nets is cut finer, for MET_FILL_WAVES wavefronts (a block a CU; more blocks are
+// more partial rows to add up), down to a window of MET_CHUNK_MIN short nets.
+constexpr int MET_CHUNK = 64;
+constexpr int MET_CHUNK_MIN = 8;
+constexpr int MET_FILL_WAVES = 2048;
 constexpr int MET_GRID_MAX = 1024;       // blocks at most (rows of partial sums)
 constexpr int MET_LDS_KMAX = 4096;      // per-part counters in LDS up to here, in HBM above
 constexpr int MET_KMAX = 16384;
@@ -44,7 +50,7 @@ constexpr int MET_LDS_MSG_KMAX = 512;   // per-block message bitmaps in LDS up t
 // counters (send as int, receive, MGV send, TV, CN), then, with per-block
 // message bitmaps, the block's K x W bitmap.
 struct MetLayout {
-  int K, W, PS, PR, grid;
+  int K, W, PS, PR, grid, chunk;
   bool lds_acc, lds_msg;
   size_t bitmap_off, partial_off, words;
 };
@@ -57,7 +63,8 @@ MetLayout met_layout(int K, int noe, int grid_max) {
   L.lds_acc = K <= MET_LDS_KMAX;
   L.lds_msg = K <= MET_LDS_MSG_KMAX;
   L.PR = L.PS + (L.lds_msg ? K * L.W : 0);
-  const int chunks = std::max(1, (noe + MET_CHUNK - 1) / MET_CHUNK);
+  L.chunk = std::max(MET_CHUNK_MIN, std::min(MET_CHUNK, (noe + MET_FILL_WAVES - 1) / MET_FILL_WAVES));
+  const int chunks = std::max(1, (noe + L.chunk - 1) / L.chunk);
   L.grid = std::max(1, std::min(grid_max, (chunks + MET_WAVES - 1) / MET_WAVES));
   L.bitmap_off = 0;
   L.partial_off = L.bitmap_off + (size_t)K * (size_t)L.W;
@@ -70,7 +77,7 @@ struct MetricArgs {
   const unsigned* net_pins;
   const int* part;
   const int* src;
-  int noe, K, nov, pb, W, PS, PR;
+  int noe, K, nov, pb, W, PS, PR, chunk;
   int* lam;             // noe, nullable
   unsigned* bitmap;     // K x W words, zeroed
   unsigned* partial;    // gridDim.x rows of PR words
@@ -176,9 +183,9 @@ __global__ void __launch_bounds__(MET_BLOCK) __attribute__((amdgpu_waves_per_eu(
   // wavefront took its next chunk from serialised those atomics at one
   // address and cost the kernel half its time
   const int waves_total = (int)gridDim.x * MET_WAVES;
-  for (int chunk = (int)blockIdx.x * MET_WAVES + wave; (long long)chunk * MET_CHUNK < a.noe; chunk += waves_total) {
-    const int c = chunk * MET_CHUNK;
-    const int nc = min(MET_CHUNK, a.noe - c);
+  for (int chunk = (int)blockIdx.x * MET_WAVES + wave; (long long)chunk * a.chunk < a.noe; chunk += waves_total) {
+    const int c = chunk * a.chunk;
+    const int nc = min(a.chunk, a.noe - c);
     // lane j: net c + j
     unsigned start = 0, end = 0;
     int sj = -1, spj = -1;
@@ -495,6 +502,7 @@ fp_status met_launch(fp_ctx* ctx, const MetLayout& L, unsigned* scratch, long lo
   m.W = L.W;
   m.PS = L.PS;
   m.PR = L.PR;
+  m.chunk = L.chunk;
   m.lam = lam;
   m.bitmap = scratch + L.bitmap_off;
   m.partial = scratch + L.partial_off;
