@@ -28,7 +28,7 @@ constexpr int COMPACT_TILE = COMPACT_BLOCK * COMPACT_RUN;
 // vertices and weights are loaded here, all loads of the run issued
 // together, the indexes of the slots without a move clamped to the run's
 // first slot so that every load stays in bounds. Otherwise (few moves per
-// round) vertices and degrees are loaded per set bit where they are used.
+// round) compact_next loads them, a few moves together.
 struct CompactRun {
   unsigned acc;
   int dec[COMPACT_RUN], v[COMPACT_RUN], w[COMPACT_RUN];
@@ -71,19 +71,66 @@ __device__ __forceinline__ void compact_load(const int* __restrict__ slot_dec, c
   for (int j = 0; j < COMPACT_RUN; j++) r.w[j] = vwgt ? vwgt[r.v[j]] : 1;
 }
 
-// events of the run's moves (their vertices' degrees); none for WEIGHTS
-template <bool WEIGHTS>
-__device__ __forceinline__ int compact_events(const CompactRun& r, const int* __restrict__ order,
-                                              const unsigned* __restrict__ vtx_ptr, int r0, int first) {
-  int d = 0;
-  if (!WEIGHTS) {
-    for (unsigned m = r.acc; m; m &= m - 1) {
-      const int s = first + __builtin_ctz(m);
-      const int v = order ? order[r0 + s] : r0 + s;
-      d += (int)(vtx_ptr[v + 1] - vtx_ptr[v]);
+// The run's next moves, COMPACT_MOVES at a time, with their vertices, degrees
+// and, with `parts`, both parts: all loads of a step issued together (past the
+// last move they repeat it). A load of each move after another's had the
+// threads of many moves wait out up to 16 dependent rounds twice (rounds of
+// 16,384 slots in a batch of mixed objectives: 7.1 -> 6.5 us on average).
+constexpr int COMPACT_MOVES = 4;
+
+struct CompactMoves {
+  int n;
+  int s[COMPACT_MOVES], v[COMPACT_MOVES], deg[COMPACT_MOVES], own[COMPACT_MOVES], dec[COMPACT_MOVES];
+};
+
+// takes the moves it returns off the mask m (not 0)
+__device__ __forceinline__ void compact_next(unsigned& m, const int* __restrict__ slot_own,
+                                             const int* __restrict__ slot_dec, const int* __restrict__ order,
+                                             const unsigned* __restrict__ vtx_ptr, int r0, int first, bool parts,
+                                             CompactMoves& c) {
+  c.n = min((int)__popc(m), COMPACT_MOVES);
+  int last = first;
+#pragma unroll
+  for (int u = 0; u < COMPACT_MOVES; u++) {
+    last = m ? first + __builtin_ctz(m) : last;
+    c.s[u] = last;
+    m &= m - 1;  // 0 stays 0
+  }
+#pragma unroll
+  for (int u = 0; u < COMPACT_MOVES; u++) c.v[u] = order ? order[r0 + c.s[u]] : r0 + c.s[u];
+  if (parts) {
+#pragma unroll
+    for (int u = 0; u < COMPACT_MOVES; u++) {
+      c.own[u] = slot_own[c.s[u]];
+      c.dec[u] = slot_dec[c.s[u]];
     }
   }
-  return d;
+  unsigned lo[COMPACT_MOVES], hi[COMPACT_MOVES];
+#pragma unroll
+  for (int u = 0; u < COMPACT_MOVES; u++) {
+    lo[u] = vtx_ptr[c.v[u]];
+    hi[u] = vtx_ptr[c.v[u] + 1];
+  }
+#pragma unroll
+  for (int u = 0; u < COMPACT_MOVES; u++) c.deg[u] = (int)(hi[u] - lo[u]);
+}
+
+// Exclusive prefixes of x and y over the block and their totals, with one
+// barrier: every wave adds up the waves' sums itself. Each use has a scratch of
+// its own. Two scans of two barriers each made a round of 16,384 slots 6.0 us,
+// now 5.0 us (batch: 6.5 -> 5.6 us).
+__device__ __forceinline__ int2 compact_scan(int x, int y, int2* scratch, int2* total) {
+  const int lane = lane_id(), wave = (int)threadIdx.x / WAVE;
+  const int ix = wave_incl_scan(x), iy = wave_incl_scan(y);
+  if (lane == WAVE - 1) scratch[wave] = make_int2(ix, iy);
+  __syncthreads();
+  const int2 s = lane < COMPACT_BLOCK / WAVE ? scratch[lane] : make_int2(0, 0);
+  const int sx = wave_incl_scan(s.x), sy = wave_incl_scan(s.y);
+  const int w = __builtin_amdgcn_readfirstlane(wave);
+  const int bx = w ? __builtin_amdgcn_readlane(sx, max(w - 1, 0)) : 0;
+  const int by = w ? __builtin_amdgcn_readlane(sy, max(w - 1, 0)) : 0;
+  *total = make_int2(__builtin_amdgcn_readlane(sx, WAVE - 1), __builtin_amdgcn_readlane(sy, WAVE - 1));
+  return make_int2(bx + ix - x, by + iy - y);
 }
 
 template <bool WEIGHTS>
@@ -91,14 +138,22 @@ __global__ void __launch_bounds__(COMPACT_BLOCK) k_compact_count(const int* __re
                                                                  const int* __restrict__ order,
                                                                  const unsigned* __restrict__ vtx_ptr, int r0,
                                                                  int nslots, int2* __restrict__ tiles) {
-  __shared__ int s_w[COMPACT_BLOCK / WAVE];
+  __shared__ int2 s_w[COMPACT_BLOCK / WAVE];
   const int first = (int)blockIdx.x * COMPACT_TILE + (int)threadIdx.x * COMPACT_RUN;
   CompactRun r;
   compact_load<false>(slot_dec, order, nullptr, r0, nslots, first, r);
-  int tot, totd;
-  block_excl_scan((int)__popc(r.acc), s_w, &tot);
-  block_excl_scan(compact_events<WEIGHTS>(r, order, vtx_ptr, r0, first), s_w, &totd);
-  if (threadIdx.x == 0) tiles[blockIdx.x] = make_int2(tot, totd);
+  int events = 0;  // the run's moves' degrees; none for WEIGHTS
+  if (!WEIGHTS) {
+    CompactMoves c;
+    for (unsigned m = r.acc; m;) {
+      compact_next(m, nullptr, nullptr, order, vtx_ptr, r0, first, false, c);
+#pragma unroll
+      for (int u = 0; u < COMPACT_MOVES; u++) events += u < c.n ? c.deg[u] : 0;
+    }
+  }
+  int2 tot;
+  compact_scan((int)__popc(r.acc), events, s_w, &tot);
+  if (threadIdx.x == 0) tiles[blockIdx.x] = tot;
 }
 
 // tiles: the per-tile totals of k_compact_count, or null for a single tile
@@ -111,8 +166,8 @@ __global__ void __launch_bounds__(COMPACT_BLOCK) k_round_compact(const int* __re
                                                                  const int2* __restrict__ tiles,
                                                                  int* __restrict__ slot_mi, int4* __restrict__ mv,
                                                                  int* __restrict__ mstat) {
-  __shared__ int s_w[COMPACT_BLOCK / WAVE];
-  int base = 0, ebase = 0;
+  __shared__ int2 s_w[COMPACT_BLOCK / WAVE], s_t[COMPACT_BLOCK / WAVE];
+  int2 base = make_int2(0, 0);  // moves and events of the tiles before
   if (tiles) {
     int a = 0, e = 0;
     for (int t = (int)threadIdx.x; t < (int)blockIdx.x; t += COMPACT_BLOCK) {
@@ -120,15 +175,29 @@ __global__ void __launch_bounds__(COMPACT_BLOCK) k_round_compact(const int* __re
       a += x.x;
       e += x.y;
     }
-    block_excl_scan(a, s_w, &base);
-    block_excl_scan(e, s_w, &ebase);
+    compact_scan(a, e, s_t, &base);
   }
   const int first = (int)blockIdx.x * COMPACT_TILE + (int)threadIdx.x * COMPACT_RUN;
   CompactRun r;
   compact_load<WEIGHTS>(slot_dec, order, vwgt, r0, nslots, first, r);
-  int tot, totd;
-  const int ex = block_excl_scan((int)__popc(r.acc), s_w, &tot);
-  const int exd = block_excl_scan(compact_events<WEIGHTS>(r, order, vtx_ptr, r0, first), s_w, &totd);
+  // the first moves stay in registers from their count to their place
+  CompactMoves c0{};
+  int events = 0;
+  unsigned more = r.acc;
+  if (!WEIGHTS && more) {
+    compact_next(more, slot_own, slot_dec, order, vtx_ptr, r0, first, true, c0);
+#pragma unroll
+    for (int u = 0; u < COMPACT_MOVES; u++) events += u < c0.n ? c0.deg[u] : 0;
+    CompactMoves c;
+    for (unsigned m = more; m;) {
+      compact_next(m, slot_own, slot_dec, order, vtx_ptr, r0, first, false, c);
+#pragma unroll
+      for (int u = 0; u < COMPACT_MOVES; u++) events += u < c.n ? c.deg[u] : 0;
+    }
+  }
+  int2 tot;
+  const int2 ex = compact_scan((int)__popc(r.acc), events, s_w, &tot);
+  const int i0 = base.x + ex.x;
   const unsigned acc = r.acc;
   if (first + COMPACT_RUN <= nslots) {
     int4* q4 = reinterpret_cast<int4*>(slot_mi + first);
@@ -138,36 +207,41 @@ __global__ void __launch_bounds__(COMPACT_BLOCK) k_round_compact(const int* __re
 #pragma unroll
       for (int t = 0; t < 4; t++) {
         const int j = 4 * q + t;
-        w[t] = (acc >> j) & 1u ? base + ex + __popc(acc & ((1u << j) - 1u)) : -1;
+        w[t] = (acc >> j) & 1u ? i0 + __popc(acc & ((1u << j) - 1u)) : -1;
       }
       q4[q] = make_int4(w[0], w[1], w[2], w[3]);
     }
   } else {
     for (int j = 0; j < COMPACT_RUN && first + j < nslots; j++)
-      slot_mi[first + j] = (acc >> j) & 1u ? base + ex + __popc(acc & ((1u << j) - 1u)) : -1;
+      slot_mi[first + j] = (acc >> j) & 1u ? i0 + __popc(acc & ((1u << j) - 1u)) : -1;
   }
   if (WEIGHTS && acc) {
     int own[COMPACT_RUN];
 #pragma unroll
     for (int j = 0; j < COMPACT_RUN; j++) own[j] = slot_own[(acc >> j) & 1u ? first + j : first];
-    int i = base + ex;
+    int i = i0;
 #pragma unroll
     for (int j = 0; j < COMPACT_RUN; j++) {
       if ((acc >> j) & 1u) mv[i++] = make_int4(r.v[j], own[j], r.dec[j], r.w[j]);
     }
-  } else if (!WEIGHTS) {
-    int i = base + ex, e = ebase + exd;
-    for (unsigned m = acc; m; m &= m - 1) {
-      const int s = first + __builtin_ctz(m);
-      const int v = order ? order[r0 + s] : r0 + s;
-      mv[i++] = make_int4(v, slot_own[s], slot_dec[s], e);
-      e += (int)(vtx_ptr[v + 1] - vtx_ptr[v]);
+  } else if (!WEIGHTS && acc) {
+    int i = i0, e = base.y + ex.y;
+    while (true) {
+#pragma unroll
+      for (int u = 0; u < COMPACT_MOVES; u++) {
+        if (u < c0.n) {
+          mv[i++] = make_int4(c0.v[u], c0.own[u], c0.dec[u], e);
+          e += c0.deg[u];
+        }
+      }
+      if (!more) break;
+      compact_next(more, slot_own, slot_dec, order, vtx_ptr, r0, first, true, c0);
     }
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
-    mstat[2] = base + tot;
-    mstat[3] = base + tot;
-    mv[base + tot] = make_int4(-1, -1, -1, ebase + totd);  // end sentinel: move i has mv[i + 1].w - mv[i].w events
+    mstat[2] = base.x + tot.x;
+    mstat[3] = base.x + tot.x;
+    mv[base.x + tot.x] = make_int4(-1, -1, -1, base.y + tot.y);  // end sentinel: move i has mv[i + 1].w - mv[i].w events
   }
 }
 
