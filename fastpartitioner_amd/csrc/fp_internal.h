@@ -318,7 +318,7 @@ __device__ __forceinline__ void wave_ilist_move(unsigned* list, unsigned short* 
                                                 unsigned pmask, unsigned& co, bool& found) {
   const int lane = lane_id();
   const unsigned inc = 1u << pb;
-  const int jp = p < 0 ? (int)LIST_NONE : __builtin_amdgcn_readfirstlane((int)at[p]);  // p -1: no part yet
+  const int jp = __builtin_amdgcn_readfirstlane((int)at[p]);
   int jq = __builtin_amdgcn_readfirstlane((int)at[q]);
   const bool hasp = jp != (int)LIST_NONE;
   const unsigned x = (unsigned)__builtin_amdgcn_readfirstlane((int)list[hasp ? jp : 0]);
@@ -361,7 +361,7 @@ __device__ __forceinline__ unsigned long long wave_ilist_moves(unsigned* list, c
   const int lane = lane_id();
   const unsigned inc = 1u << pb;
   const bool mine = (m >> lane) & 1ull;
-  const int jp = mine && own >= 0 ? (int)at[own] : (int)LIST_NONE;
+  const int jp = mine ? (int)at[own] : (int)LIST_NONE;
   const int jq = mine ? (int)at[d] : (int)LIST_NONE;
   const bool leaves = jp != (int)LIST_NONE;
   const unsigned c0 = leaves ? list[jp] >> pb : 0u;
@@ -370,7 +370,7 @@ __device__ __forceinline__ unsigned long long wave_ilist_moves(unsigned* list, c
   wave_lds_sync();
   const unsigned c1 = leaves ? list[jp] >> pb : 0u;
   const unsigned outs = (c0 - c1) & (~0u >> pb);  // the count field may have wrapped
-  const bool safe = jq != (int)LIST_NONE && (own < 0 || (leaves && outs < c0));
+  const bool safe = jq != (int)LIST_NONE && leaves && outs < c0;
   const unsigned long long other = __ballot(mine && !safe);
   const int first = other ? __ffsll((long long)other) - 1 : WAVE;
   wave_lds_sync();
@@ -378,6 +378,33 @@ __device__ __forceinline__ unsigned long long wave_ilist_moves(unsigned* list, c
   if (mine && lane < first) atomicAdd(&list[jq], inc);
   wave_lds_sync();
   return first == WAVE ? 0ull : m & ~((1ull << first) - 1ull);
+}
+
+// A window of pins that had no part (the streaming partition: bit l of m set,
+// lane l's pin goes to part d): the parts not listed yet are appended in the
+// order of their first pins, a readlane and a ballot each, then every pin is
+// counted. The list comes out as after one wave_ilist_move a pin, which waits
+// out five dependent LDS accesses.
+__device__ __forceinline__ void wave_ilist_places(unsigned* list, unsigned short* at, int& L, unsigned long long m,
+                                                  int d, int pb) {
+  const int lane = lane_id();
+  const bool mine = (m >> lane) & 1ull;
+  int jq = mine ? (int)at[d] : 0;
+  for (unsigned long long b = __ballot(mine && jq == (int)LIST_NONE); b;) {
+    const int l = __builtin_ctzll(b);
+    const int q = __builtin_amdgcn_readlane(d, l);
+    const unsigned long long same = __ballot(mine && d == q);
+    jq = (same >> lane) & 1ull ? L : jq;
+    if (lane == l) {
+      list[L] = (unsigned)q;
+      at[q] = (unsigned short)L;
+    }
+    L++;
+    b &= ~same;
+  }
+  wave_lds_sync();
+  if (mine) atomicAdd(&list[jq], 1u << pb);
+  wave_lds_sync();
 }
 
 // First 64 words of net n's segment (seg = net_ptr[n] + n): the segment holds

@@ -1158,6 +1158,10 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
       for (int u = 0; u < APPLY_GROUP; u++) {
         unsigned long long m = __ballot(dd[u] >= 0);
         dirty |= m != 0;
+        if (INDEXED && m && __ballot(dd[u] >= 0 && oo[u] >= 0) == 0ull) {
+          wave_ilist_places(list, at, L, m, dd[u], a.pb);
+          continue;
+        }
         bool together = INDEXED;  // worth trying in this window
         while (m) {
           if (together && __popcll(m) >= APPLY_TOGETHER) {
