@@ -12,7 +12,7 @@ Metric: pin-visits/s = steps * pins / seconds (a pin-visit is one (vertex,
 incident net) incidence scored in a pass).
 
 Also reported on the same JSON line:
-  roofline      the evaluation kernel (k_tv_eval), timed live with HIP events
+  roofline      the evaluation kernel (k_tv_eval_masks), timed live with HIP events
                 on the engine's stream, against the 8 TB/s HBM peak
   cpu_baseline  the reference's own OpenMP refinement (partition_par,
                 TV/partition.cpp:512-981, built from its sources in oracle/_ref)
@@ -573,20 +573,24 @@ def run_tv1m(args):
     secs = t1 - t0
     value = args.steps * hg.pins / secs
 
-    # algorithmic bytes per pass of the evaluation step, per-unit model of the
-    # refinement's data in the reference layout (int32 part + int32 count per
-    # list entry), each byte counted once per use, no cache credit:
-    # 12 B per vertex, 12 B per (vertex, net) incidence, 8 B per list entry
-    # visited (Lambda = sum over nets of |n| * lambda(n))
+    # algorithmic bytes per pass of the evaluation step, each byte counted once
+    # per use, no cache credit: 12 B per vertex and, per (vertex, net)
+    # incidence, the net's id and the words of its part mask that are read, one
+    # per 64 parts and the own part's (K <= 512); past that, in the reference
+    # layout, 12 B per incidence and 8 B per list entry visited (Lambda = sum
+    # over nets of |n| * lambda(n))
     lam_avg = 0.5 * (lam0 + lam1)
-    bytes_pass = 12 * hg.nov + 12 * hg.pins + 8 * lam_avg
+    if K <= 512:
+        bytes_pass = 12 * hg.nov + (4 + 8 * ((K + 63) // 64 + 1)) * hg.pins
+    else:
+        bytes_pass = 12 * hg.nov + 12 * hg.pins + 8 * lam_avg
     avg_launch_ms = eval_ms / max(launches, 1)
     bytes_launch = bytes_pass * args.steps / max(launches, 1)
     achieved = bytes_launch / (avg_launch_ms * 1e-3) / 1e9
     traffic, traffic_detail = (None, {"skipped": "--no-traffic"}) if args.no_traffic else measure_traffic(args)
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-            "kernel": "k_tv_eval", "launches": launches, "avg_launch_us": round(avg_launch_ms * 1e3, 2),
+            "kernel": "k_tv_eval_masks" if K <= 512 else "k_tv_eval", "launches": launches, "avg_launch_us": round(avg_launch_ms * 1e3, 2),
             "bytes_per_launch": int(bytes_launch), "traffic_counters": traffic_detail,
             "pass_frac": round(bytes_pass / (secs / args.steps) / 1e9 / HBM_PEAK_GBS, 4)}
 
