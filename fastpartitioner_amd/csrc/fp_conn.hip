@@ -1313,10 +1313,11 @@ int conn_eval_waves(int K, int rcap, int scap) {
 }
 
 // MSM event slots per incidence (v, n): 2 * min(|n|, K) when v is n's source,
-// else 2 (the bounds of conn_changes). Built once per upload on the host.
+// else 2 (the bounds of conn_changes). Built on the host; they serve every K up
+// to the one they were built for, and any K once no net has more pins than that.
 fp_status ensure_incoff(fp_ctx* ctx) {
   auto& c = ctx->conn;
-  if (c.incoff_ready) return FP_OK;
+  if (c.incoff && std::min((unsigned)ctx->K, ctx->max_net) <= c.inc_k) return FP_OK;
   const int nov = ctx->nov, noe = ctx->noe;
   std::vector<unsigned> vptr((size_t)nov + 1), vnets((size_t)std::max(ctx->pins, 1ll));
   std::vector<int> srcs((size_t)std::max(noe, 1));
@@ -1335,11 +1336,15 @@ fp_status ensure_incoff(fp_ctx* ctx) {
     }
   if (acc >= (1ull << 32)) return fail(ctx, FP_ERR_UNSUPPORTED, "MSM event slots exceed 2^32");
   off[(size_t)ctx->pins] = (unsigned)acc;
-  FP_TRY(dalloc(ctx, &c.incoff, (size_t)ctx->pins + 1));
+  const long long cap = (long long)std::max(acc, 1ull);
+  if (cap > c.evcap) {
+    FP_TRY(dalloc(ctx, &c.evbuf, (size_t)cap));
+    c.evcap = cap;
+  }
+  if (!c.incoff) FP_TRY(dalloc(ctx, &c.incoff, (size_t)ctx->pins + 1));
+  c.inc_k = 0;
   FP_TRY(h2d(ctx, c.incoff, off.data(), (size_t)ctx->pins + 1));
-  FP_TRY(dalloc(ctx, &c.evbuf, (size_t)std::max(acc, 1ull)));
-  c.evcap = (long long)std::max(acc, 1ull);
-  c.incoff_ready = true;
+  c.inc_k = std::min((unsigned)ctx->K, ctx->max_net);
   return FP_OK;
 }
 

@@ -546,7 +546,8 @@ fp_status fp_upload(fp_ctx* ctx, int nov, int noe, const unsigned* net_ptr, cons
   ctx->conn.kcap = 0;
   ctx->conn.rmax = 0;
   ctx->conn.evcap = 0;
-  ctx->conn.incoff_ready = false;
+  ctx->conn.incoff = nullptr;
+  ctx->conn.inc_k = 0;
   ctx->lam = nullptr;
   ctx->met_scratch = nullptr;
   ctx->met_words = 0;

@@ -817,9 +817,9 @@ struct fp_ctx {
     int4* mv = nullptr;
     int2* evbuf = nullptr;             // MSM: per incidence, pc changes (cell, +-1)
     unsigned* incoff = nullptr;        // MSM: first event slot of each incidence (pins + 1)
+    unsigned inc_k = 0;                // the longest list that incoff has room for
     int kcap = 0, rmax = 0;
     long long evcap = 0;
-    bool incoff_ready = false;
   } conn;
 
   // metric scratch (grown on demand by fp_eval)
