@@ -862,13 +862,6 @@ struct ApplyArgs {
   unsigned long long* moves;
 };
 
-// Replays the round's moves on every touched net in ordering order
-// (TV/partition.cpp:846-890: remove = decrement or swap-with-last, add =
-// increment or append); one wavefront per net, the list staged in LDS.
-// Blocks past net_blocks commit the REF part vector and source-part sizes
-// (TV/partition.cpp:818-830: the destination's size is left unchanged).
-// INDEXED: each wave keeps a part -> position index of its list in LDS (2
-// bytes per part after the lists), for K where it fits.
 // One lane replays the round's moves on a net of at most SMALL_NET pins, in
 // the rank order of its pins, on a copy of the list in its registers: the
 // same edits, in the same order, as the wavefront replay (remove = decrement
@@ -1001,6 +994,23 @@ __device__ __forceinline__ void wave_replay_medium(const ApplyArgs& a, int n, un
                                       a.masks + (size_t)n * (size_t)(2 * a.mask_words));
 }
 
+// The apply's LDS that does not depend on K: the block's touched nets (the
+// small ones from the front, the others from the back), the positions of the
+// huge ones, which are replayed first, and the waves' mask words.
+struct ApplyNets {
+  int cnt[4];  // touched small nets, other nets, nets handed out, huge nets
+  unsigned words[APPLY_BLOCK / WAVE][4 * MASK_PMAX];
+  unsigned start[APPLY_NETS], len[APPLY_NETS];
+  unsigned short net[APPLY_NETS], huge[APPLY_NETS];
+};
+
+// Replays the round's moves on every touched net in ordering order
+// (TV/partition.cpp:846-890: remove = decrement or swap-with-last, add =
+// increment or append): a lane per small net, a wavefront per other one.
+// Blocks past net_blocks commit the REF part vector and source-part sizes
+// (TV/partition.cpp:818-830: the destination's size is left unchanged).
+// INDEXED: each wave keeps a part -> position index of its list in LDS (2
+// bytes per part after the list), for K where it fits.
 template <bool INDEXED>
 __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) k_apply(ApplyArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
@@ -1026,19 +1036,15 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
   unsigned* my = reinterpret_cast<unsigned*>(mem) + (size_t)lane * (size_t)a.lane_words;
   unsigned* list = reinterpret_cast<unsigned*>(mem);
   unsigned short* at = reinterpret_cast<unsigned short*>(list + a.K);
-  __shared__ unsigned s_words[APPLY_BLOCK / WAVE][4 * MASK_PMAX];
-  unsigned* words = s_words[wave];
-  __shared__ int s_cnt[4];  // touched small nets, other nets, nets handed out, huge nets
-  __shared__ unsigned short s_net[APPLY_NETS];  // the small ones from the front, the others from the back
-  __shared__ unsigned s_start[APPLY_NETS], s_len[APPLY_NETS];
-  __shared__ unsigned short s_huge[APPLY_NETS];  // positions of the huge ones, which are replayed first
+  __shared__ ApplyNets s;
+  unsigned* words = s.words[wave];
 
   // the block's touched nets, the small ones and the others apart: a wave
   // then replays 64 small nets at a time, a lane each, and the big ones go
   // to whichever wave is free
   const int n0 = (int)blockIdx.x * a.per_block;
   const int nn = min(a.per_block, a.noe - n0);
-  if (threadIdx.x < 4) s_cnt[threadIdx.x] = 0;
+  if (threadIdx.x < 4) s.cnt[threadIdx.x] = 0;
   __syncthreads();
   for (int i0 = 0; i0 < nn; i0 += APPLY_BLOCK) {
     const int i = i0 + (int)threadIdx.x;
@@ -1052,8 +1058,8 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
     const unsigned long long ms = __ballot(sm), mb = __ballot(hit && !sm);
     int bs = 0, bb = 0;
     if (lane == 0) {
-      if (ms) bs = atomicAdd(&s_cnt[0], (int)__popcll(ms));
-      if (mb) bb = atomicAdd(&s_cnt[1], (int)__popcll(mb));
+      if (ms) bs = atomicAdd(&s.cnt[0], (int)__popcll(ms));
+      if (mb) bb = atomicAdd(&s.cnt[1], (int)__popcll(mb));
     }
     // lane 0's, read while every lane is active
     bs = __builtin_amdgcn_readlane(bs, 0);
@@ -1061,18 +1067,18 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
     const unsigned long long lt = (1ull << lane) - 1ull;
     const int k = sm ? bs + (int)__popcll(ms & lt) : APPLY_NETS - 1 - (bb + (int)__popcll(mb & lt));
     if (hit) {
-      s_net[k] = (unsigned short)i;
-      s_start[k] = st;
-      s_len[k] = len;
-      if (len >= HUGE_NET) s_huge[atomicAdd(&s_cnt[3], 1)] = (unsigned short)k;
+      s.net[k] = (unsigned short)i;
+      s.start[k] = st;
+      s.len[k] = len;
+      if (len >= HUGE_NET) s.huge[atomicAdd(&s.cnt[3], 1)] = (unsigned short)k;
     }
   }
   __syncthreads();
-  const int nsmall = __builtin_amdgcn_readfirstlane(s_cnt[0]), nbig = __builtin_amdgcn_readfirstlane(s_cnt[1]);
-  const int nhuge = __builtin_amdgcn_readfirstlane(s_cnt[3]);
+  const int nsmall = __builtin_amdgcn_readfirstlane(s.cnt[0]), nbig = __builtin_amdgcn_readfirstlane(s.cnt[1]);
+  const int nhuge = __builtin_amdgcn_readfirstlane(s.cnt[3]);
 
   for (int b = wave * WAVE; b < nsmall; b += nw * WAVE)
-    if (b + lane < nsmall) lane_replay_small(a, n0 + s_net[b + lane], s_start[b + lane], s_len[b + lane], my);
+    if (b + lane < nsmall) lane_replay_small(a, n0 + s.net[b + lane], s.start[b + lane], s.len[b + lane], my);
   if (nbig == 0) return;
   wave_lds_sync();
   if (INDEXED) wave_index_init(at, a.K);
@@ -1088,22 +1094,22 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
   auto next_head = [&]() -> NetHead {
     NetHead h{-1, INT_MAX, -1, -1, 0, 0u, 0u, 0u};
     int k = 0;
-    if (lane == 0) k = atomicAdd(&s_cnt[2], 1);
+    if (lane == 0) k = atomicAdd(&s.cnt[2], 1);
     k = __builtin_amdgcn_readlane(k, 0);
     for (;;) {
       if (k >= nhuge + nbig) return h;
       if (k < nhuge) {
-        k = __builtin_amdgcn_readfirstlane((int)s_huge[k]);
+        k = __builtin_amdgcn_readfirstlane((int)s.huge[k]);
         break;
       }
       k = APPLY_NETS - 1 - (k - nhuge);
-      if (nhuge == 0 || __builtin_amdgcn_readfirstlane((int)s_len[k]) < (int)HUGE_NET) break;
-      if (lane == 0) k = atomicAdd(&s_cnt[2], 1);  // a huge one again: the next
+      if (nhuge == 0 || __builtin_amdgcn_readfirstlane((int)s.len[k]) < (int)HUGE_NET) break;
+      if (lane == 0) k = atomicAdd(&s.cnt[2], 1);  // a huge one again: the next
       k = __builtin_amdgcn_readlane(k, 0);
     }
-    h.n = n0 + __builtin_amdgcn_readfirstlane((int)s_net[k]);
-    h.s = (unsigned)__builtin_amdgcn_readfirstlane((int)s_start[k]);
-    const unsigned np = (unsigned)__builtin_amdgcn_readfirstlane((int)s_len[k]);
+    h.n = n0 + __builtin_amdgcn_readfirstlane((int)s.net[k]);
+    h.s = (unsigned)__builtin_amdgcn_readfirstlane((int)s.start[k]);
+    const unsigned np = (unsigned)__builtin_amdgcn_readfirstlane((int)s.len[k]);
     h.e = h.s + np;
     const unsigned seg = h.s + (unsigned)h.n;
     if (np <= (unsigned)WAVE) {
@@ -1123,14 +1129,14 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
   };
   auto replay_net = [&](const NetHead& h) {
     const int n = h.n;
-    const unsigned s = h.s, e = h.e;
-    const unsigned seg = s + (unsigned)n;
-    if (e - s <= (unsigned)WAVE) {
-      if (__ballot(h.dd >= 0)) wave_replay_medium(a, n, s, __builtin_amdgcn_readfirstlane(h.L), h.x, h.dd, h.oo, words);
+    const unsigned b = h.s, e = h.e;
+    const unsigned seg = b + (unsigned)n;
+    if (e - b <= (unsigned)WAVE) {
+      if (__ballot(h.dd >= 0)) wave_replay_medium(a, n, b, __builtin_amdgcn_readfirstlane(h.L), h.x, h.dd, h.oo, words);
       return;
     }
     unsigned lo, hi;
-    wave_rank_window(a.apply_pins, s, e, a.r0, a.r1, lo, hi);
+    wave_rank_window(a.apply_pins, b, e, a.r0, a.r1, lo, hi);
     int L = wave_list_stage(a.ent, seg, h.x, list);
     if (INDEXED) wave_index_set(list, L, at, a.pmask);
     bool dirty = false;
@@ -1204,16 +1210,13 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
 // the part -> position index, or before that half a mask record per lane
 int apply_lane_words(int K) { return 2 * mask_words(K) + 1; }
 
-// the block's touched nets and its waves' mask words
-constexpr size_t APPLY_STATIC = (size_t)APPLY_NETS * 10 + (size_t)(APPLY_BLOCK / WAVE) * 4 * MASK_PMAX * sizeof(unsigned) + 64;
-
 size_t apply_wave_bytes(int K, bool indexed) {
   const size_t list = (size_t)K * (sizeof(unsigned) + (indexed ? sizeof(unsigned short) : 0));
   return (std::max(list, (size_t)WAVE * (size_t)apply_lane_words(K) * sizeof(unsigned)) + 15) & ~(size_t)15;
 }
 
 bool apply_indexed(int K) {
-  return (size_t)(APPLY_BLOCK / WAVE) * apply_wave_bytes(K, true) + APPLY_STATIC <= (size_t)LDS_BUDGET;
+  return (size_t)(APPLY_BLOCK / WAVE) * apply_wave_bytes(K, true) + sizeof(ApplyNets) <= (size_t)LDS_BUDGET;
 }
 
 size_t apply_lds(int K) { return (size_t)(APPLY_BLOCK / WAVE) * apply_wave_bytes(K, apply_indexed(K)); }
@@ -1334,7 +1337,7 @@ fp_status plan_tv(fp_ctx* ctx, RefinePlan& p) {
   const int waves = p.eval_waves > 0 ? std::min(p.eval_waves, eval_waves(K)) : eval_waves(K);
   if (waves == 0) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d needs more LDS than a workgroup has", K);
   p.eval_waves = waves;
-  if (apply_lds(K) + APPLY_STATIC > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
+  if (apply_lds(K) + sizeof(ApplyNets) > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
   p.R = std::min(p.sched.round, ctx->nov);
   FP_TRY(ensure_round_scratch(ctx, p.R));
   if (p.sched.kind == FP_SCHED_BAL) FP_TRY(ensure_bal_scratch(ctx, p.R));
@@ -1504,7 +1507,7 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
   FP_HIP_OK(hipSetDevice(ctx->device));
   FP_TRY(ensure_k(ctx, K));
   FP_TRY(check_envelope(ctx));
-  if (apply_lds(K) + APPLY_STATIC > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
+  if (apply_lds(K) + sizeof(ApplyNets) > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
   const int nov = ctx->nov;
   const int R = std::max(1, std::min(round, nov));
   const int waves = eval_waves(K);
