@@ -679,6 +679,15 @@ __global__ void __launch_bounds__(256) k_cn_commit(const int* __restrict__ mv_v,
 
 }  // namespace
 
+// the edit list for `need` entries, at least twice what it held
+static fp_status cn_grow_ops(fp_ctx* ctx, long long need) {
+  auto& s = ctx->cn;
+  const long long cap = std::max(need, 2 * s.ops_cap);
+  FP_TRY(dgrow(ctx, &s.ops, (size_t)cap));
+  s.ops_cap = cap;
+  return FP_OK;
+}
+
 fp_status plan_cn(fp_ctx* ctx, RefinePlan& p) {
   const int noe = ctx->noe;
   const long long pins = ctx->pins;
@@ -716,6 +725,7 @@ fp_status plan_cn(fp_ctx* ctx, RefinePlan& p) {
     s.ops_cap = cap;
     s.ready = true;
   }
+  if (!s.ops) FP_TRY(cn_grow_ops(ctx, 0));  // a growth that failed
   fill_async<int>(ctx, ctx->flags, 4, 0);
   p.R = ctx->nov;
   return FP_OK;
@@ -786,9 +796,7 @@ fp_status cn_passes(fp_ctx* ctx, const RefinePlan& p, int passes) {
     if (f[2] < 0 || f[2] > run) return fail(ctx, FP_ERR_HIP, "CN pass count %d out of [0, %d]", f[2], run);
     done += f[2];
     if (f[0]) {
-      auto& s = ctx->cn;
-      s.ops_cap = std::max<long long>((long long)f[0], 2 * s.ops_cap);
-      FP_TRY(dalloc(ctx, &s.ops, (size_t)s.ops_cap));
+      FP_TRY(cn_grow_ops(ctx, f[0]));
       fill_async<int>(ctx, ctx->flags, 4, 0);
     } else if (f[2] != run) {
       return fail(ctx, FP_ERR_HIP, "CN passes: %d of %d applied without an overflow", f[2], run);
@@ -807,9 +815,7 @@ fp_status cn_after_pass(fp_ctx* ctx, int* redo) {
                 "a net with a repeated pin receives more than %d moves in one CN pass; that pass was not applied",
                 CN_MAXOPS);
   if (f[0]) {
-    auto& s = ctx->cn;
-    s.ops_cap = std::max<long long>((long long)f[0], 2 * s.ops_cap);
-    FP_TRY(dalloc(ctx, &s.ops, (size_t)s.ops_cap));
+    FP_TRY(cn_grow_ops(ctx, f[0]));
     fill_async<int>(ctx, ctx->flags, 4, 0);
     *redo = 1;
   }

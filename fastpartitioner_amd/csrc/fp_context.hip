@@ -75,7 +75,7 @@ fp_status dalloc_bytes(fp_ctx* ctx, void** p, size_t bytes) {
   const size_t need = std::max(bytes, size_t{1});
   char* q = nullptr;
   for (auto& s : ctx->slabs)
-    if (s.size - s.used >= need) {
+    if (!s.own && s.size - s.used >= need) {
       q = static_cast<char*>(s.base) + s.used;
       s.used = std::min(s.size, (s.used + need + ALIGN - 1) / ALIGN * ALIGN);
       break;
@@ -94,10 +94,33 @@ fp_status dalloc_bytes(fp_ctx* ctx, void** p, size_t bytes) {
       return fail(ctx, FP_ERR_OOM, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
     }
     q = static_cast<char*>(base);
-    ctx->slabs.push_back({base, size, std::min(size, (need + ALIGN - 1) / ALIGN * ALIGN)});
+    ctx->slabs.push_back({base, size, std::min(size, (need + ALIGN - 1) / ALIGN * ALIGN), false});
   }
   ctx->dev_bytes += (long long)bytes;
   ctx->gen++;
+  *p = q;
+  return FP_OK;
+}
+
+fp_status dgrow_bytes(fp_ctx* ctx, void** p, size_t bytes) {
+  const auto old = std::find_if(ctx->slabs.begin(), ctx->slabs.end(),
+                                [&](const fp_ctx::Slab& s) { return s.own && s.base == *p; });
+  *p = nullptr;
+  ctx->gen++;
+  if (old != ctx->slabs.end()) {
+    FP_HIP_OK(hipStreamSynchronize(ctx->stream));
+    (void)hipFree(old->base);
+    ctx->dev_bytes -= (long long)old->size;
+    ctx->slabs.erase(old);
+  }
+  void* q = nullptr;
+  const hipError_t e = hipMalloc(&q, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(ctx, FP_ERR_OOM, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
+  }
+  ctx->slabs.push_back({q, bytes, bytes, true});
+  ctx->dev_bytes += (long long)bytes;
   *p = q;
   return FP_OK;
 }

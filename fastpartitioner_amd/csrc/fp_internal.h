@@ -724,6 +724,7 @@ struct fp_ctx {
   struct Slab {
     void* base;
     size_t size, used;
+    bool own;  // one array's own allocation (dgrow_bytes)
   };
   std::vector<Slab> slabs;  // device memory, cut into arrays by dalloc_bytes
   // bumped by every change that can invalidate recorded kernel arguments
@@ -878,6 +879,9 @@ fp_status cn_after_pass(fp_ctx* ctx, int* redo);
 // has grown.
 fp_status cn_passes(fp_ctx* ctx, const RefinePlan& p, int passes);
 fp_status dalloc_bytes(fp_ctx* ctx, void** p, size_t bytes);
+// A larger array in the place of *p (nullable), whose contents are given up: an
+// allocation of its own, freed in its turn when it is replaced. On failure *p is null.
+fp_status dgrow_bytes(fp_ctx* ctx, void** p, size_t bytes);
 void dfree_all(fp_ctx* ctx);
 hipEvent_t pooled_event(fp_ctx* ctx, size_t i);
 
@@ -885,6 +889,13 @@ template <typename T>
 fp_status dalloc(fp_ctx* ctx, T** p, size_t count) {
   void* q = nullptr;
   fp_status s = dalloc_bytes(ctx, &q, (count ? count : 1) * sizeof(T));
+  *p = static_cast<T*>(q);
+  return s;
+}
+template <typename T>
+fp_status dgrow(fp_ctx* ctx, T** p, size_t count) {
+  void* q = *p;
+  fp_status s = dgrow_bytes(ctx, &q, (count ? count : 1) * sizeof(T));
   *p = static_cast<T*>(q);
   return s;
 }

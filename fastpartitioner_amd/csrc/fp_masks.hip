@@ -64,9 +64,9 @@ unsigned long long* ensure_masks(fp_ctx* ctx) {
   // the evaluation reads records and net ids at 32-bit byte offsets
   if (need * sizeof(unsigned long long) >= (size_t{1} << 32) || ctx->pins >= (1ll << 30)) return nullptr;
   if (need > ctx->mask_cap) {
-    unsigned long long* q = nullptr;
-    if (dalloc(ctx, &q, need) != FP_OK) return nullptr;
-    ctx->masks = q;
+    // a refinement rebuilds them: those of a smaller K are given back
+    ctx->mask_cap = 0;
+    if ((ctx->masks ? dgrow(ctx, &ctx->masks, need) : dalloc(ctx, &ctx->masks, need)) != FP_OK) return nullptr;
     ctx->mask_cap = need;
   }
   return ctx->masks;

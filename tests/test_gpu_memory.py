@@ -1,0 +1,35 @@
+"""What a context holds of the device's memory, and what it says it holds."""
+import numpy as np
+import pytest
+
+from fastpartitioner_amd import hypergraph as H
+from fastpartitioner_amd.engine import SCHED_REF, Engine, schedule
+
+pytestmark = pytest.mark.gpu
+
+
+def _refine(eng, hg, metric, K):
+    C, max_pw, min_pw = H.ref_constants(hg.nov, K)
+    eng.set_partition(K, (np.arange(hg.nov) * K // hg.nov).astype(np.int32))
+    eng.refine(metric, 1, schedule(SCHED_REF, 4096, C, max_pw, min_pw))
+
+
+def test_part_masks_of_a_smaller_k_are_given_back():
+    hg = H.colnet(40_000, H.DEG_FIXED, 4, seed=3)
+    with Engine(0) as eng:
+        eng.upload(hg)
+        _refine(eng, hg, "TV", 512)
+        direct = eng.device_bytes()
+    with Engine(0) as eng:
+        eng.upload(hg)
+        for K in range(64, 513, 64):
+            _refine(eng, hg, "TV", K)
+        stepwise = eng.device_bytes()
+        state = eng.get_state()
+        eng.upload(hg)
+        _refine(eng, hg, "TV", 512)
+        assert eng.device_bytes() <= stepwise
+        again = eng.get_state()
+    # 16 bytes a net and 64 parts: all eight arrays together are 23 MB, the last one 5.1 MB
+    assert stepwise - direct < 2 * 16 * 8 * hg.noe
+    assert np.array_equal(state.part, again.part) and np.array_equal(state.ep_parts, again.ep_parts)
