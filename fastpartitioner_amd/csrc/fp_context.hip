@@ -62,44 +62,44 @@ fp_status fail(fp_ctx* c, fp_status st, const char* fmt, ...) {
 }
 
 // Arrays live until the next upload, so they are cut from slabs one after
-// another: a slab is one hipMalloc, rounded up to SLAB_BYTES, and its rest
-// serves the arrays to come. (A hipMalloc costs tens of microseconds, and one
-// that has to map new memory about two milliseconds, several times the
-// smallest request.) At most SLAB_BYTES per slab stay unused. With 2 MiB the
-// arrays of an instance of 10,000 vertices and 80,000 pins ended at a slab's
-// end, and its first refinement opened another: 2.2 ms for the first pass on a
-// new context, 0.9 ms with 8.
-fp_status dalloc_bytes(fp_ctx* ctx, void** p, size_t bytes) {
-  constexpr size_t SLAB_BYTES = size_t{8} << 20, ALIGN = 256;
+// another: a slab is one hipMalloc of ctx->slab_bytes, whose rest serves the
+// arrays to come. (A hipMalloc past 1 MiB costs 13 us, one that has to map new
+// memory 0.3 to 0.8 ms, a multiple of the smallest request.) fp_upload sizes
+// the slabs by the instance (slab_size). An array of half a slab or more is an
+// allocation of its own, so less than half of a slab stays unused when the
+// next one opens. slab_bytes 0: every array is, and the context holds what its
+// arrays need, no more.
+constexpr size_t SLAB_MAX = size_t{8} << 20, SLAB_MIN = size_t{64} << 10;
+
+size_t dalign(size_t bytes) { return (std::max(bytes, size_t{1}) + 255) / 256 * 256; }
+
+fp_status device_block(fp_ctx* ctx, size_t size, size_t used, bool own, void** p) {
   *p = nullptr;
-  const size_t need = std::max(bytes, size_t{1});
-  char* q = nullptr;
-  for (auto& s : ctx->slabs)
-    if (!s.own && s.size - s.used >= need) {
-      q = static_cast<char*>(s.base) + s.used;
-      s.used = std::min(s.size, (s.used + need + ALIGN - 1) / ALIGN * ALIGN);
-      break;
-    }
-  if (!q) {
-    size_t size = (need + SLAB_BYTES - 1) / SLAB_BYTES * SLAB_BYTES;
-    void* base = nullptr;
-    hipError_t e = hipMalloc(&base, size);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      size = need;
-      e = hipMalloc(&base, size);
-    }
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      return fail(ctx, FP_ERR_OOM, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
-    }
-    q = static_cast<char*>(base);
-    ctx->slabs.push_back({base, size, std::min(size, (need + ALIGN - 1) / ALIGN * ALIGN), false});
+  void* base = nullptr;
+  const hipError_t e = hipMalloc(&base, size);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(ctx, FP_ERR_OOM, "hipMalloc(%zu bytes) failed: %s", size, hipGetErrorString(e));
   }
-  ctx->dev_bytes += (long long)bytes;
-  ctx->gen++;
-  *p = q;
+  ctx->slabs.push_back({base, size, used, own});
+  ctx->dev_bytes += (long long)size;
+  *p = base;
   return FP_OK;
+}
+
+fp_status dalloc_bytes(fp_ctx* ctx, void** p, size_t bytes) {
+  const size_t need = dalign(bytes);
+  ctx->gen++;
+  if (need < ctx->slab_bytes / 2) {
+    for (auto& s : ctx->slabs)
+      if (!s.own && s.size - s.used >= need) {
+        *p = static_cast<char*>(s.base) + s.used;
+        s.used += need;
+        return FP_OK;
+      }
+    if (device_block(ctx, ctx->slab_bytes, need, false, p) == FP_OK) return FP_OK;
+  }
+  return device_block(ctx, need, need, true, p);
 }
 
 fp_status dgrow_bytes(fp_ctx* ctx, void** p, size_t bytes) {
@@ -113,16 +113,21 @@ fp_status dgrow_bytes(fp_ctx* ctx, void** p, size_t bytes) {
     ctx->dev_bytes -= (long long)old->size;
     ctx->slabs.erase(old);
   }
-  void* q = nullptr;
-  const hipError_t e = hipMalloc(&q, bytes);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(ctx, FP_ERR_OOM, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
-  }
-  ctx->slabs.push_back({q, bytes, bytes, true});
-  ctx->dev_bytes += (long long)bytes;
-  *p = q;
-  return FP_OK;
+  const size_t need = dalign(bytes);
+  return device_block(ctx, need, need, true, p);
+}
+
+// The slabs of an instance: four times the upload's arrays, which holds them
+// and the scratch of a first refinement of most objectives, at most SLAB_MAX.
+// Upload, state, two TV passes and metrics on a new context (fixed degree 8),
+// in a process that has made others: 0.94 ms at 60,000 vertices, 1.33 at
+// 100,000, 1.0 at 300. An allocation per array takes 1.08, 1.52 and 0.3 to 1.6;
+// 8 MiB for every instance, larger arrays rounded up to it, takes 0.96 to 4.1,
+// 1.3 to 7 (memory mapped anew in most uploads) and 1.0 to 1.9, and has a
+// context of 100 KB hold 8 MiB.
+size_t slab_size(long long nov, long long noe, long long pins) {
+  const size_t arrays = (size_t)(22 * (pins + noe) + 16 * nov);
+  return (std::min(SLAB_MAX, std::max(SLAB_MIN, 4 * arrays)) + 4095) / 4096 * 4096;
 }
 
 void dfree_all(fp_ctx* ctx) {
@@ -553,6 +558,7 @@ fp_status fp_upload(fp_ctx* ctx, int nov, int noe, const unsigned* net_ptr, cons
   FP_HIP_OK(hipSetDevice(ctx->device));
   FP_HIP_OK(hipStreamSynchronize(ctx->stream));
   dfree_all(ctx);
+  if (!ctx->exact_memory) ctx->slab_bytes = slab_size(nov, noe, pins);
   ctx->has_graph = ctx->has_state = false;
   ctx->K = 0;
   ctx->kcap = 0;

@@ -724,9 +724,11 @@ struct fp_ctx {
   struct Slab {
     void* base;
     size_t size, used;
-    bool own;  // one array's own allocation (dgrow_bytes)
+    bool own;  // one array's own allocation
   };
-  std::vector<Slab> slabs;  // device memory, cut into arrays by dalloc_bytes
+  std::vector<Slab> slabs;    // device memory, cut into arrays by dalloc_bytes
+  size_t slab_bytes = 0;      // what a slab takes; 0: every array is an allocation of its own
+  bool exact_memory = false;  // a server's contexts: no slabs
   // bumped by every change that can invalidate recorded kernel arguments
   // (device pointers, K, the list layout): allocation, freeing, a new K
   unsigned long long gen = 0;

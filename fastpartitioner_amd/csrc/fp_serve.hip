@@ -115,10 +115,18 @@ long long mask_bytes(const fp_server::Graph& g, fp_metric metric, int K) {
   return metric == FP_METRIC_CN ? 0 : 16ll * fpe::mask_words(K) * ((long long)g.noe + 1);
 }
 
+// A new context whose memory is what its arrays need, no more: the admission
+// counts it.
+fp_status create_ctx(fp_server* s, fp_ctx** out) {
+  const fp_status st = fp_ctx_create(out, s->device);
+  if (st == FP_OK) (*out)->exact_memory = true;
+  return st;
+}
+
 // a new context holding graph g's upload (the caller holds no lock)
 fp_status upload_replica(fp_server* s, const fp_server::Graph& g, fp_ctx** out) {
   fp_ctx* ctx = nullptr;
-  fp_status st = fp_ctx_create(&ctx, s->device);
+  fp_status st = create_ctx(s, &ctx);
   if (st) return st;
   st = fp_upload(ctx, g.nov, g.noe, g.net_ptr.data(), g.net_pins.data(), nullptr, nullptr,
                  g.src.empty() ? nullptr : g.src.data(), g.vwgt.empty() ? nullptr : g.vwgt.data(), nullptr);
@@ -275,7 +283,7 @@ fp_status fp_server_add_graph(fp_server* s, int nov, int noe, const unsigned* ne
                               const int* src, const int* vwgt, int* graph_id) {
   if (!s || !graph_id) return FP_ERR_ARG;
   fp_ctx* ctx = nullptr;
-  fp_status st = fp_ctx_create(&ctx, s->device);
+  fp_status st = create_ctx(s, &ctx);
   if (st) return sfail(s, st, "fp_ctx_create failed");
   st = fp_upload(ctx, nov, noe, net_ptr, net_pins, nullptr, nullptr, src, vwgt, nullptr);
   if (st) {

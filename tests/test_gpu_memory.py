@@ -33,3 +33,19 @@ def test_part_masks_of_a_smaller_k_are_given_back():
     # 16 bytes a net and 64 parts: all eight arrays together are 23 MB, the last one 5.1 MB
     assert stepwise - direct < 2 * 16 * 8 * hg.noe
     assert np.array_equal(state.part, again.part) and np.array_equal(state.ep_parts, again.ep_parts)
+
+
+@pytest.mark.parametrize("nov", [1, 300, 1_000, 20_000])
+def test_a_context_says_what_it_holds(nov):
+    # its slabs: a few times its arrays, and no more once a refinement's
+    # scratch is cut from what they have left
+    hg = H.colnet(nov, H.DEG_FIXED, min(4, nov - 1), seed=3)
+    arrays = 22 * (hg.pins + hg.noe) + 16 * hg.nov
+    with Engine(0) as eng:
+        eng.upload(hg)
+        held = eng.device_bytes()
+        assert arrays <= held <= 4 * arrays + (64 << 10)
+        if nov > 1:
+            _refine(eng, hg, "TV", 16)
+            eng.metrics()
+            assert eng.device_bytes() == held
