@@ -679,6 +679,29 @@ __global__ void __launch_bounds__(256) k_cn_commit(const int* __restrict__ mv_v,
 
 }  // namespace
 
+// the first size of the edit list: a pass edits the lists of a pushed vertex's
+// nets, and a vertex is pushed by at most its degree many nets, so the sum of
+// degree^2 bounds it
+static long long cn_first_ops(const fp_ctx* ctx) {
+  return (long long)std::max<unsigned long long>(
+      1ull, std::min<unsigned long long>(ctx->sum_deg2, 4ull * (unsigned long long)std::max(ctx->pins, 1ll)));
+}
+
+static long long cn_big_cap(const fp_ctx* ctx) {
+  return (long long)(std::max<unsigned long long>(ctx->sum_deg2, 1ull) / (unsigned long long)CN_MAXOPS + 1);
+}
+
+long long cn_scratch_bytes(const fp_ctx* ctx) {
+  const auto& s = ctx->cn;
+  const long long ne = std::max(ctx->noe, 1), np = std::max(ctx->pins, 1ll);
+  const long long per_net = sizeof(*s.old_part) + sizeof(*s.new_part) + sizeof(*s.npush) + sizeof(*s.pbase) +
+                            sizeof(*s.opoff) + sizeof(*s.opcnt) + sizeof(*s.opfill);
+  return array_bytes(per_net * ne, 7) + array_bytes((long long)sizeof(*s.sums) * (ne / SCAN_BLOCK + 1)) +
+         array_bytes(16 * np, 4) + array_bytes(8 * (long long)sizeof(*s.totals)) + array_bytes(np / 8 + 4) +
+         array_bytes((long long)sizeof(*s.big) * cn_big_cap(ctx)) +
+         array_bytes((long long)sizeof(*s.ops) * cn_first_ops(ctx));
+}
+
 // the edit list for `need` entries, at least twice what it held
 static fp_status cn_grow_ops(fp_ctx* ctx, long long need) {
   auto& s = ctx->cn;
@@ -714,13 +737,10 @@ fp_status plan_cn(fp_ctx* ctx, RefinePlan& p) {
     // nets' bitmap; its ops at most sum of degree^2 (below): the big list, a
     // big net holding more than CN_MAXOPS of them
     FP_TRY(dalloc(ctx, &s.bigbits, (size_t)(np / 32 + 1)));
-    s.big_cap = (long long)(std::max<unsigned long long>(ctx->sum_deg2, 1ull) / (unsigned long long)CN_MAXOPS + 1);
+    s.big_cap = cn_big_cap(ctx);
     FP_TRY(dalloc(ctx, &s.big, (size_t)s.big_cap));
     fill_async<int>(ctx, s.opcnt, ne, 0);
-    // a pass edits the lists of a pushed vertex's nets, and a vertex is pushed
-    // by at most its degree many nets: sum of degree^2 bounds the edit list
-    const long long cap = (long long)std::max<unsigned long long>(
-        1ull, std::min<unsigned long long>(ctx->sum_deg2, 4ull * (unsigned long long)np));
+    const long long cap = cn_first_ops(ctx);
     FP_TRY(dalloc(ctx, &s.ops, (size_t)cap));
     s.ops_cap = cap;
     s.ready = true;

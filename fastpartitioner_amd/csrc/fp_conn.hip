@@ -1385,6 +1385,15 @@ void launch_bits(fp_ctx* ctx, bool recount_msg = true) {
 
 }  // namespace
 
+long long conn_scratch_bytes(const fp_ctx* ctx, int K, int R, bool msm) {
+  const long long W = (K + 63) / 64;
+  long long b = array_bytes(4ll * K * K + 24 * K * W + 4ll * K + 32, 4) + array_bytes(8ll * R + 20ll * (R + 1), 4) +
+                compact_tile_bytes(R);
+  // the events: two per incidence, two per entry of its net for the source's
+  if (msm) b += array_bytes(4 * (ctx->pins + 1) + (long long)sizeof(int2) * 4 * std::max(ctx->pins, 1ll), 2);
+  return b;
+}
+
 fp_status plan_conn(fp_ctx* ctx, RefinePlan& p) {
   const bool msm = p.metric == FP_METRIC_MSM;
   const int nov = ctx->nov, K = ctx->K;

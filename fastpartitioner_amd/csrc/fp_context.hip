@@ -231,6 +231,8 @@ fp_status h2d_bulk(fp_ctx* ctx, void* d, const void* h, size_t bytes) {
 }
 
 // K-sized arrays and the packed-entry layout for K parts
+long long k_scratch_bytes(int K) { return array_bytes(20ll * K, 3); }
+
 fp_status ensure_k(fp_ctx* ctx, int K) {
   if (K < 1) return fail(ctx, FP_ERR_ARG, "K must be >= 1");
   if (K > 16384) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d above 16384", K);  // parts fit the 15-bit view

@@ -871,6 +871,18 @@ fp_status pass_conn(fp_ctx* ctx, const RefinePlan& p);
 // dispatch on p.metric
 fp_status plan_refine(fp_ctx* ctx, fp_metric metric, const fp_schedule* sched, RefinePlan& p);
 fp_status record_pass(fp_ctx* ctx, const RefinePlan& p);
+// Device bytes that a request's calls allocate beyond the upload's arrays, on a
+// context without slabs: what every set of a part vector with K parts takes,
+// what a refinement plans (the part masks apart, which are optional) and what
+// fp_eval takes. CN's edit list counts at its first size.
+long long k_scratch_bytes(int K);
+long long tv_scratch_bytes(int K, int R, bool bal);
+long long cn_scratch_bytes(const fp_ctx* ctx);
+long long vol_scratch_bytes(const fp_ctx* ctx, int K, int R);
+long long conn_scratch_bytes(const fp_ctx* ctx, int K, int R, bool msm);
+long long eval_scratch_bytes(int K, int noe);
+// n arrays of `bytes` bytes together, each rounded up as dalloc does
+inline long long array_bytes(long long bytes, int n = 1) { return bytes + 256ll * n; }
 // CN only: after a pass, grows the edit list if the pass overflowed it (the
 // pass then left the state unchanged); *redo = 1 when it must run again
 fp_status cn_after_pass(fp_ctx* ctx, int* redo);

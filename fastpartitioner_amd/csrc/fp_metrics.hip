@@ -571,6 +571,14 @@ fp_status noalloc_scratch(fp_ctx* ctx, unsigned** out) {
 }
 
 }  // namespace
+
+long long eval_scratch_bytes(int K, int noe) {
+  if (K > MET_KMAX) return (long long)K * K / 8;  // fp_eval refuses it
+  const MetLayout L = met_layout(K, noe, MET_GRID_MAX);
+  return array_bytes((long long)sizeof(unsigned) * (long long)L.words) +
+         array_bytes((long long)sizeof(long long) * (6 + 5ll * K));
+}
+
 }  // namespace fpe
 
 using namespace fpe;

@@ -256,6 +256,10 @@ inline fp_status ensure_compact_tiles(fp_ctx* ctx, int R) {
   return FP_OK;
 }
 
+inline long long compact_tile_bytes(int R) {
+  return array_bytes((long long)sizeof(int2) * ((R + COMPACT_TILE - 1) / COMPACT_TILE));
+}
+
 template <bool WEIGHTS>
 inline void launch_round_compact(fp_ctx* ctx, const int* order, int r0, int nslots, int* slot_mi, int4* mv,
                                  int* mstat) {

@@ -89,23 +89,20 @@ fp_status sfail(fp_server* s, fp_status st, const char* fmt, ...) {
   return st;
 }
 
-// HBM a request needs beyond its resident hypergraph: the per-pass scratch of
-// its objective, an upper estimate that depends on the request alone (the
-// context keeps its scratch between requests, so this over-counts a
-// hypergraph that already served a request).
-long long scratch_bytes(const fp_server::Graph& g, fp_metric metric, int K, int R) {
-  const long long pins = g.pins, nov = g.nov;
-  const long long r = std::min<long long>(R > 0 ? R : nov, nov);
-  long long b = 8 * (long long)K * 8;  // sizes, frozen sizes, candidate totals, metric vectors
-  b += (long long)K * (long long)K / 8;  // message bitmap of the metric evaluation
+// HBM a request needs beyond its resident hypergraph: the arrays that its
+// calls allocate on a context that served none before (a context keeps its
+// scratch between requests, so this over-counts one that did).
+long long scratch_bytes(const fp_server::Graph& g, fp_metric metric, int K, const fp_schedule* sched) {
+  const fp_ctx* ctx = g.ctxs[0];  // what it counts by is the upload's, the same in every replica
+  const int R = sched && sched->round > 0 ? std::min(sched->round, g.nov) : g.nov;
+  const long long b = fpe::k_scratch_bytes(K) + fpe::eval_scratch_bytes(K, g.noe);
   switch (metric) {
-    case FP_METRIC_TV: b += 8 * r + 8 * (long long)K * ((r + 63) / 64); break;
-    case FP_METRIC_CN: b += 16 * pins + 40 * (long long)g.nov + 16 * pins; break;
+    case FP_METRIC_TV: return b + fpe::tv_scratch_bytes(K, R, sched && sched->kind == FP_SCHED_BAL);
+    case FP_METRIC_CN: return b + fpe::cn_scratch_bytes(ctx);
     case FP_METRIC_MSV:
-    case FP_METRIC_MSRV: b += 16 * pins + 24 * r; break;
-    default: b += 4 * (long long)K * K + 16 * (long long)K * ((K + 63) / 64) + 8 * 4 * pins + 24 * r; break;
+    case FP_METRIC_MSRV: return b + fpe::vol_scratch_bytes(ctx, K, R);
+    default: return b + fpe::conn_scratch_bytes(ctx, K, R, metric == FP_METRIC_MSM);
   }
-  return b;
 }
 
 // The nets' part masks of a request whose objective uses them. They are
@@ -319,7 +316,7 @@ fp_status fp_server_submit(fp_server* s, int graph_id, fp_metric metric, int K, 
     if (graph_id < 0 || graph_id >= (int)s->graphs.size()) return sfail(s, FP_ERR_ARG, "no hypergraph %d", graph_id);
     const fp_server::Graph& g = *s->graphs[(size_t)graph_id];
     q->part.assign(part, part + g.nov);
-    q->footprint = g.bytes + scratch_bytes(g, metric, K, sched ? sched->round : 0);
+    q->footprint = g.bytes + scratch_bytes(g, metric, K, sched);
     const long long extra = mask_bytes(g, metric, K);
     q->masks = q->footprint + extra <= s->budget;
     if (q->masks) q->footprint += extra;

@@ -1249,6 +1249,9 @@ fp_status ensure_round_scratch(fp_ctx* ctx, int R) {
   return FP_OK;
 }
 
+// of ensure_bal_scratch: an int and a long long per part and tile
+constexpr long long BAL_BYTES = sizeof(int) + sizeof(long long);
+
 fp_status ensure_bal_scratch(fp_ctx* ctx, int R) {
   const size_t ntiles = (size_t)(R + TILE - 1) / TILE;
   const size_t need = ntiles * (size_t)ctx->K;
@@ -1331,6 +1334,10 @@ EvalArgs make_eval_args(fp_ctx* ctx, const fp_schedule* s) {
 }
 
 }  // namespace
+
+long long tv_scratch_bytes(int K, int R, bool bal) {
+  return array_bytes(8ll * R, 2) + (bal ? array_bytes(BAL_BYTES * K * ((R + TILE - 1) / TILE), 2) : 0);
+}
 
 fp_status plan_tv(fp_ctx* ctx, RefinePlan& p) {
   const int K = ctx->K;

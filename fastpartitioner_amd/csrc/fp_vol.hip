@@ -1336,6 +1336,11 @@ fp_status ensure_vol_scratch(fp_ctx* ctx, int R) {
 
 }  // namespace
 
+long long vol_scratch_bytes(const fp_ctx* ctx, int K, int R) {
+  return array_bytes(4ll * K + 32, 2) + array_bytes(8ll * R + 20ll * (R + 1), 4) + compact_tile_bytes(R) +
+         array_bytes((long long)sizeof(int4) * std::max(ctx->pins, 1ll));
+}
+
 fp_status plan_vol(fp_ctx* ctx, RefinePlan& p) {
   const bool msrv = p.metric == FP_METRIC_MSRV;
   const int nov = ctx->nov, K = ctx->K;

@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 from fastpartitioner_amd import hypergraph as H
-from fastpartitioner_amd.engine import SCHED_REF, Engine, schedule
+from fastpartitioner_amd.engine import SCHED_BAL, SCHED_REF, Engine, Server, schedule
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +49,28 @@ def test_a_context_says_what_it_holds(nov):
             _refine(eng, hg, "TV", 16)
             eng.metrics()
             assert eng.device_bytes() == held
+
+
+@pytest.mark.parametrize("metric,K", [("TV", 3_000), ("CN", 2_000), ("TM", 3_200), ("MSM", 3_200), ("MSV", 3_200),
+                                      ("MSRV", 3_200), ("TM", 300), ("MSRV", 100)])
+def test_a_requests_footprint_covers_what_its_calls_allocate(metric, K):
+    # an engine of its own does the request's calls: of what it allocates, no
+    # more than the last two slabs can be unused
+    hg = H.colnet(4_200, H.DEG_FIXED, 1, seed=3)
+    C, max_pw, min_pw = H.ref_constants(hg.nov, K)
+    cap = H.balance_cap(hg.nov, K, 0.05)
+    sched = {"CN": None, "TV": schedule(SCHED_BAL, hg.nov, C, cap, 0, cap)}.get(
+        metric, schedule(SCHED_REF, hg.nov, C, max_pw, min_pw))
+    part = (np.arange(hg.nov) * K // hg.nov).astype(np.int32)
+    with Engine(0) as eng:
+        eng.upload(hg)
+        slab = eng.device_bytes()
+        eng.set_partition(K, part)
+        eng.refine(metric, 1, sched)
+        eng.metrics()
+        used = eng.device_bytes() - 2 * slab
+    with Server(0, hbm_budget=1 << 36, workers=1) as srv:
+        srv.add_graph(hg)
+        info, _ = srv.wait(srv.submit(0, metric, K, part, sched, 1))
+    print(f"footprint: {metric} K={K} slab {slab} used {used} footprint {info['footprint']}", flush=True)
+    assert used <= info["footprint"]
