@@ -102,17 +102,22 @@ fp_status dalloc_bytes(fp_ctx* ctx, void** p, size_t bytes) {
   return device_block(ctx, need, need, true, p);
 }
 
+bool dfree_own(fp_ctx* ctx, const void* p) {
+  const auto it = std::find_if(ctx->slabs.begin(), ctx->slabs.end(),
+                               [&](const fp_ctx::Slab& s) { return s.own && s.base == p; });
+  if (it == ctx->slabs.end()) return false;
+  (void)hipStreamSynchronize(ctx->stream);
+  (void)hipFree(it->base);
+  ctx->dev_bytes -= (long long)it->size;
+  ctx->gen++;
+  ctx->slabs.erase(it);
+  return true;
+}
+
 fp_status dgrow_bytes(fp_ctx* ctx, void** p, size_t bytes) {
-  const auto old = std::find_if(ctx->slabs.begin(), ctx->slabs.end(),
-                                [&](const fp_ctx::Slab& s) { return s.own && s.base == *p; });
+  if (*p) (void)dfree_own(ctx, *p);
   *p = nullptr;
   ctx->gen++;
-  if (old != ctx->slabs.end()) {
-    FP_HIP_OK(hipStreamSynchronize(ctx->stream));
-    (void)hipFree(old->base);
-    ctx->dev_bytes -= (long long)old->size;
-    ctx->slabs.erase(old);
-  }
   const size_t need = dalign(bytes);
   return device_block(ctx, need, need, true, p);
 }

@@ -896,6 +896,8 @@ fp_status dalloc_bytes(fp_ctx* ctx, void** p, size_t bytes);
 // A larger array in the place of *p (nullable), whose contents are given up: an
 // allocation of its own, freed in its turn when it is replaced. On failure *p is null.
 fp_status dgrow_bytes(fp_ctx* ctx, void** p, size_t bytes);
+// Frees array p if it is an allocation of its own; false if it is a slab's part.
+bool dfree_own(fp_ctx* ctx, const void* p);
 void dfree_all(fp_ctx* ctx);
 hipEvent_t pooled_event(fp_ctx* ctx, size_t i);
 

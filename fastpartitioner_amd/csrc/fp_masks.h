@@ -27,6 +27,10 @@ inline int mask_words(int K) { return K <= MASK_KMAX ? (K + 63) / 64 : 0; }
 // The context's mask array for its K, or nullptr when K is above MASK_KMAX or
 // the array cannot be allocated (the list evaluation then runs).
 unsigned long long* ensure_masks(fp_ctx* ctx);
+// Gives the array back, if it is an allocation of its own; the next
+// ensure_masks makes another.
+void drop_masks(fp_ctx* ctx);
+inline long long held_mask_bytes(const fp_ctx* ctx) { return (long long)(ctx->mask_cap * sizeof(unsigned long long)); }
 // Every record from the resident lists, on the context's stream.
 void build_masks(fp_ctx* ctx, unsigned long long* masks);
 

@@ -72,6 +72,13 @@ unsigned long long* ensure_masks(fp_ctx* ctx) {
   return ctx->masks;
 }
 
+void drop_masks(fp_ctx* ctx) {
+  if (ctx->masks && dfree_own(ctx, ctx->masks)) {
+    ctx->masks = nullptr;
+    ctx->mask_cap = 0;
+  }
+}
+
 void build_masks(fp_ctx* ctx, unsigned long long* masks) {
   const int grid = std::max(1, std::min((ctx->noe + MASK_BLOCK - 1) / MASK_BLOCK, 8192));
   k_build_masks<<<grid, MASK_BLOCK, 0, ctx->stream>>>(ctx->net_ptr, ctx->ent, ctx->noe, mask_words(ctx->K), ctx->pb,

@@ -50,8 +50,9 @@ struct fp_server {
     bool has_sched = false;
     fp_schedule sched{};
     std::vector<int> part;
-    long long footprint = 0;
-    bool masks = true;  // the footprint has room for the nets' part masks
+    long long footprint = 0;  // what the admission charges, the part masks included where it admits them
+    long long mask_bytes = 0;  // the nets' part masks that the request would use
+    bool masks = false;        // it is admitted with them
     // results
     bool done = false;
     fp_status status = FP_OK;
@@ -69,6 +70,7 @@ struct fp_server {
   std::unordered_map<long long, std::unique_ptr<Request>> reqs;
   long long next_id = 1;
   long long inflight_bytes = 0, peak_bytes = 0;
+  long long largest = 0;  // the largest footprint without masks of a request so far
   int inflight = 0, peak_inflight = 0;
   long long completed = 0;
   bool stop = false;
@@ -106,7 +108,7 @@ long long scratch_bytes(const fp_server::Graph& g, fp_metric metric, int K, cons
 }
 
 // The nets' part masks of a request whose objective uses them. They are
-// optional: a request that fits the budget only without them is evaluated
+// optional: where the budget has no room for them, the request is evaluated
 // through the lists.
 long long mask_bytes(const fp_server::Graph& g, fp_metric metric, int K) {
   return metric == FP_METRIC_CN ? 0 : 16ll * fpe::mask_words(K) * ((long long)g.noe + 1);
@@ -137,6 +139,7 @@ fp_status upload_replica(fp_server* s, const fp_server::Graph& g, fp_ctx** out) 
 
 void run_request(fp_server* s, fp_server::Request& q, fp_ctx* ctx) {
   ctx->use_masks = q.masks;
+  if (!q.masks) fpe::drop_masks(ctx);  // another request's, which this one's footprint does not hold
   fp_status st = fp_set_partition(ctx, q.K, q.part.data());
   fp_refine_stats stats{};
   if (st == FP_OK) st = fp_refine(ctx, q.metric, q.passes, q.has_sched ? &q.sched : nullptr, &stats);
@@ -170,6 +173,17 @@ void worker_loop(fp_server* s) {
           const bool grow = free_ci < 0 && (int)cg.ctxs.size() + cg.creating < s->max_replicas;
           if (free_ci < 0 && !grow) continue;
           if (s->inflight > 0 && s->inflight_bytes + c->footprint > s->budget) break;
+          // With the part masks (its own, or the larger ones that the context
+          // holds from another request) if the budget has room for them and
+          // for a request like the largest so far on every worker left: they
+          // never keep one waiting that would run beside this one without them.
+          const long long held = free_ci >= 0 ? fpe::held_mask_bytes(cg.ctxs[(size_t)free_ci]) : 0;
+          const long long masks = std::max(c->mask_bytes, held);
+          const long long idle = (long long)s->workers.size() - s->inflight - 1;
+          if (s->inflight_bytes + c->footprint + masks + idle * s->largest <= s->budget) {
+            c->masks = true;
+            c->footprint += masks;
+          }
           q = c;
           gi = c->graph;
           ci = free_ci;
@@ -317,9 +331,7 @@ fp_status fp_server_submit(fp_server* s, int graph_id, fp_metric metric, int K, 
     const fp_server::Graph& g = *s->graphs[(size_t)graph_id];
     q->part.assign(part, part + g.nov);
     q->footprint = g.bytes + scratch_bytes(g, metric, K, sched);
-    const long long extra = mask_bytes(g, metric, K);
-    q->masks = q->footprint + extra <= s->budget;
-    if (q->masks) q->footprint += extra;
+    q->mask_bytes = mask_bytes(g, metric, K);
     if (q->footprint > s->budget)
       return sfail(s, FP_ERR_BUDGET, "request needs %lld bytes, the budget is %lld", q->footprint, s->budget);
   }
@@ -331,6 +343,7 @@ fp_status fp_server_submit(fp_server* s, int graph_id, fp_metric metric, int K, 
   if (sched) q->sched = *sched;
   {
     std::lock_guard<std::mutex> lk(s->mu);
+    s->largest = std::max(s->largest, q->footprint);
     q->id = s->next_id++;
     q->submit_ms = s->now_ms();
     *request_id = q->id;
