@@ -1472,7 +1472,8 @@ fp_status pass_conn(fp_ctx* ctx, const RefinePlan& p) {
     if (p.masks) {
       a.ones = c.B + 2 * (size_t)K * (size_t)W;
       a.masks = p.masks;
-      const int egrid = mask_eval_grid(nslots, p.eval_grid, CONN_BLOCK / WAVE, a.per_wave);
+      a.per_wave = mask_eval_share(nslots, p.eval_grid, CONN_BLOCK / WAVE);
+      const int egrid = mask_eval_grid(nslots, p.eval_grid, CONN_BLOCK / WAVE);
       FP_TRY(launch_timed(ctx, msm ? conn_masks_kernel<true>(K) : conn_masks_kernel<false>(K), egrid, CONN_BLOCK, 0, a));
     } else {
       int egrid = std::max(1, std::min((nslots + waves - 1) / waves, 8192));

@@ -85,7 +85,6 @@ struct EvalArgs {
   const unsigned long long* masks;
   int noe;
   unsigned last_pin;  // the last element of vtx_nets
-  int per_wave;       // consecutive slots per wave (<= 64)
 };
 
 // slot decision of an unplaced vertex whose part the fallback assigns
@@ -446,7 +445,7 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
 // bit as the carry-in; the penalties and counts of a lane's parts stay in
 // registers, so the sweep and the LDG scan touch no LDS. The single bit of the
 // vertex's own part comes from one word per net, a net per lane.
-// A wave takes per_wave consecutive slots: their headers are loaded a slot per
+// A wave takes slots a round of the grid's waves apart: their headers are loaded a slot per
 // lane, their decisions written a slot per lane at the end. Both the vector
 // and the scalar unit are near their issue limit here, so addresses are 32-bit
 // offsets (the host checks the arrays' sizes) and everything per vertex that
@@ -459,15 +458,16 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
   __shared__ double s_pen[64 * P];
   __shared__ unsigned s_skey[64 * P];
   const int K = a.K;
-  const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
-  const int s0 = ((int)blockIdx.x * nw + wave) * a.per_wave;
-  const int ns = min(a.per_wave, a.nslots - s0);
+  const int lane = lane_id(), wave = wave_id();
+  int s0, stride, ns;
+  wave_slots(a.nslots, s0, stride, ns);
+  const int slot_l = s0 + lane * stride;
 
-  // lane i: slot s0 + i's vertex, its part and its net range
+  // lane i: the wave's slot i's vertex, its part and its net range
   int v_l = 0, own_l = 0;
   unsigned vb_l = 0, ve_l = 0;
   if (lane < ns) {
-    const int z = a.r0 + s0 + lane;
+    const int z = a.r0 + slot_l;
     v_l = a.order ? a.order[z] : z;
     own_l = a.part[v_l];
     vb_l = a.vtx_ptr[v_l];
@@ -498,7 +498,7 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
     pid[u] = (u * WAVE + lane) | (in ? 1 << 16 : 0);
   }
   const char* masks = reinterpret_cast<const char*>(a.masks);
-  // lane j: net j of slot s0 + i's vertex; past its last net some other net.
+  // lane j: net j of slot i's vertex; past its last net some other net.
   // Loaded a vertex ahead, by every lane (a load that a branch may skip could
   // only be waited for together with the ones after it).
   const char* nets = reinterpret_cast<const char*>(a.vtx_nets);
@@ -507,7 +507,7 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
     return *reinterpret_cast<const unsigned*>(nets + min(k, a.last_pin) * 4u);
   };
 
-  int dec_l = -1;  // lane i: slot s0 + i's decision: a part, -1 (none) or SLOT_FALLBACK
+  int dec_l = -1;  // lane i: slot i's decision: a part, -1 (none) or SLOT_FALLBACK
   // the headers have arrived before the loop (else its first wait would take in the loads of every turn)
   asm volatile("" ::"v"(own_l), "v"(vb_l), "v"(ve_l));
   unsigned id = ns > 0 ? load_nets(0) : 0u;
@@ -573,11 +573,11 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
     dec_l = lane == i ? dd : dec_l;
   }
   if (lane < ns) {
-    a.slot_own[s0 + lane] = own_l;
-    a.slot_dec[s0 + lane] = dec_l;
+    a.slot_own[slot_l] = own_l;
+    a.slot_dec[slot_l] = dec_l;
     if (dec_l >= 0 && a.hist) {
       const int w = a.vwgt ? a.vwgt[v_l] : 1;
-      atomicAdd(&a.hist[(size_t)dec_l * (size_t)a.ntiles + (size_t)((s0 + lane) / TILE)], w);
+      atomicAdd(&a.hist[(size_t)dec_l * (size_t)a.ntiles + (size_t)(slot_l / TILE)], w);
     }
   }
 }
@@ -1382,7 +1382,7 @@ fp_status pass_tv(fp_ctx* ctx, const RefinePlan& p) {
       a.masks = p.masks;
       a.noe = ctx->noe;
       a.last_pin = mask_last_pin(ctx);
-      const int grid = mask_eval_grid(nslots, p.eval_grid, EVAL_BLOCK / WAVE, a.per_wave);
+      const int grid = mask_eval_grid(nslots, p.eval_grid, EVAL_BLOCK / WAVE);
       FP_TRY(launch_timed(ctx, eval_masks_kernel<EVAL_REFINE>(K), grid, EVAL_BLOCK, 0, a));
     } else {
       int grid = eval_grid(nslots, waves);
@@ -1572,7 +1572,7 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
     a.masks = masks;
     a.noe = ctx->noe;
     a.last_pin = mask_last_pin(ctx);
-    const int grid = masks ? mask_eval_grid(nslots, 0, EVAL_BLOCK / WAVE, a.per_wave) : eval_grid(nslots, waves);
+    const int grid = masks ? mask_eval_grid(nslots, 0, EVAL_BLOCK / WAVE) : eval_grid(nslots, waves);
     if (masks)
       (eval_mode == EVAL_INIT_CN ? eval_masks_kernel<EVAL_INIT_CN>(K)
                                  : eval_masks_kernel<EVAL_INIT>(K))<<<grid, EVAL_BLOCK, 0, ctx->stream>>>(a);

@@ -107,7 +107,6 @@ struct VolEvalArgs {
   int* tcount;
   int* tcount_next;
   unsigned last_pin;  // the last element of vtx_nets and vtx_seg
-  int per_wave;       // consecutive slots per wave (<= 64)
   // k_vol_eval
   int shorts;        // the LDS has room for the short lists' rows
   unsigned pad_seg;  // the 64 zero words after the last segment: a list of length 0
@@ -247,7 +246,7 @@ __device__ int vol_long_choice(const VolEvalArgs& a, unsigned vb, int deg, int o
 // 262,144 vertices of 13 nets of 13 pins, K = 1024: 130 us, 100 of them vector
 // issue (375 us with a sweep and a scan of K counts for every vertex; 230 us
 // with the sources' parts gathered for every vertex).
-// A wave takes per_wave consecutive slots, their headers a slot per lane; a
+// A wave takes slots a round of the grid's waves apart, their headers a slot per lane; a
 // vertex's nets, segments and the sources' parts load while the one before it
 // is decided.
 __global__ void __launch_bounds__(VOL_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) k_vol_eval(VolEvalArgs a) {
@@ -312,19 +311,20 @@ __global__ void __launch_bounds__(VOL_BLOCK) __attribute__((amdgpu_waves_per_eu(
   }
   const int M = a.mstat[0], cntM = a.mstat[1];
 
-  const int s0 = ((int)blockIdx.x * nw + wave) * a.per_wave;
-  const int ns = min(a.per_wave, a.nslots - s0);
-  // lane i: slot s0 + i's vertex, its part and its net range
+  int s0, stride, ns;
+  wave_slots(a.nslots, s0, stride, ns);
+  const int slot_l = s0 + lane * stride;
+  // lane i: the wave's slot i's vertex, its part and its net range
   int v_l = 0, own_l = 0, dec_l = -1;
   unsigned vb_l = 0, ve_l = 0;
   if (lane < ns) {
-    const int z = a.r0 + s0 + lane;
+    const int z = a.r0 + slot_l;
     v_l = a.order ? a.order[z] : z;
     own_l = a.part[v_l];
     vb_l = a.vtx_ptr[v_l];
     ve_l = a.vtx_ptr[v_l + 1];
   }
-  // lane j: net j of slot s0 + i's vertex (past its last net that one again,
+  // lane j: net j of slot i's vertex (past its last net that one again,
   // which costs no cache line) and its segment offset, two vertices ahead; the
   // net's length, one. The sources and their parts are two gathers more, of a
   // cache line per net, and wait for a vertex whose choice is another part.
@@ -491,8 +491,8 @@ __global__ void __launch_bounds__(VOL_BLOCK) __attribute__((amdgpu_waves_per_eu(
     if (dec >= 0) wave_touch_nets(a.vtx_nets + vb, deg, a.tag, a.net_stamp, a.touched, a.tcount);
   }
   if (lane < ns) {
-    a.slot_own[s0 + lane] = own_l;
-    a.slot_dec[s0 + lane] = dec_l;
+    a.slot_own[slot_l] = own_l;
+    a.slot_dec[slot_l] = dec_l;
   }
 }
 
@@ -514,17 +514,18 @@ k_vol_eval_masks(VolEvalArgs a) {
   __shared__ int s_delta[VOL_MASK_BLOCK / WAVE][64 * P];    // losses - gains per part
   __shared__ unsigned s_hit[VOL_MASK_BLOCK / WAVE][2 * P];  // max parts the move affects (MSRV), one bit per part
   const int K = a.K;
-  const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
+  const int lane = lane_id(), wave = wave_id();
   int* delta = s_delta[wave];
   unsigned* hitb = s_hit[wave];
-  const int s0 = ((int)blockIdx.x * nw + wave) * a.per_wave;
-  const int ns = min(a.per_wave, a.nslots - s0);
+  int s0, stride, ns;
+  wave_slots(a.nslots, s0, stride, ns);
+  const int slot_l = s0 + lane * stride;
 
-  // lane i: slot s0 + i's vertex, its part and its net range
+  // lane i: the wave's slot i's vertex, its part and its net range
   int v_l = 0, own_l = 0;
   unsigned vb_l = 0, ve_l = 0;
   if (lane < ns) {
-    const int z = a.r0 + s0 + lane;
+    const int z = a.r0 + slot_l;
     v_l = a.order ? a.order[z] : z;
     own_l = a.part[v_l];
     vb_l = a.vtx_ptr[v_l];
@@ -552,13 +553,13 @@ k_vol_eval_masks(VolEvalArgs a) {
   const int M = a.mstat[0], cntM = a.mstat[1];
   const char* masks = reinterpret_cast<const char*>(a.masks);
   const char* nets = reinterpret_cast<const char*>(a.vtx_nets);
-  // lane j: net j of slot s0 + i's vertex; past its last net some other net
+  // lane j: net j of slot i's vertex; past its last net some other net
   auto load_nets = [&](int i) -> unsigned {
     const unsigned k = (unsigned)__builtin_amdgcn_readlane((int)vb_l, i) + (unsigned)lane;
     return *reinterpret_cast<const unsigned*>(nets + min(k, a.last_pin) * 4u);
   };
 
-  int dec_l = -1;  // lane i: slot s0 + i's decision
+  int dec_l = -1;  // lane i: slot i's decision
   // the headers have arrived before the loop (else its first wait would take in the loads of every turn)
   asm volatile("" ::"v"(v_l), "v"(own_l), "v"(vb_l), "v"(ve_l));
   unsigned id = ns > 0 ? load_nets(0) : 0u;
@@ -684,8 +685,8 @@ k_vol_eval_masks(VolEvalArgs a) {
     }
   }
   if (lane < ns) {
-    a.slot_own[s0 + lane] = own_l;
-    a.slot_dec[s0 + lane] = dec_l;
+    a.slot_own[slot_l] = own_l;
+    a.slot_dec[slot_l] = dec_l;
   }
 }
 
@@ -1427,7 +1428,7 @@ fp_status pass_vol(fp_ctx* ctx, const RefinePlan& p) {
     if (p.masks) {
       a.masks = p.masks;
       a.noe = ctx->noe;
-      const int egrid = mask_eval_grid(nslots, p.eval_grid, VOL_MASK_BLOCK / WAVE, a.per_wave);
+      const int egrid = mask_eval_grid(nslots, p.eval_grid, VOL_MASK_BLOCK / WAVE);
       FP_TRY(launch_timed(ctx, vol_masks_kernel(K), egrid, VOL_MASK_BLOCK, 0, a));
     } else {
       a.pad_seg = (unsigned)((size_t)ctx->pins + (size_t)ctx->noe);
@@ -1440,8 +1441,7 @@ fp_status pass_vol(fp_ctx* ctx, const RefinePlan& p) {
       a.shorts = shorts ? 1 : 0;
       // as many blocks as the 256 CUs hold: a few more would run alone at the end
       const int resident = 256 * std::max(1, vol_eval_per_cu(waves, lds_e));
-      const int egrid = mask_eval_grid(nslots, p.eval_grid > 0 ? std::min(p.eval_grid, resident) : resident, waves,
-                                       a.per_wave);
+      const int egrid = mask_eval_grid(nslots, p.eval_grid > 0 ? std::min(p.eval_grid, resident) : resident, waves);
       FP_TRY(launch_timed(ctx, k_vol_eval, egrid, waves * WAVE, lds_e, a));
     }
     launch_round_compact<false>(ctx, ctx->order, r0, nslots, vs.slot_mi, vs.mv, vs.mstat);
