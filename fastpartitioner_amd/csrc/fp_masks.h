@@ -67,15 +67,13 @@ __device__ __forceinline__ void wave_slots(int nslots, int& s0, int& stride, int
   ns = s0 < nslots ? min(WAVE, (nslots - s0 + stride - 1) / stride) : 0;
 }
 
-// c += this lane's bit of m (m wave-uniform): the bit is the add's carry-in
+// c += this lane's bit of m: the bit is the add's carry-in. m has to come from
+// scalar loads and scalar instructions: a mask that a vector instruction wrote
+// (a comparison, a ballot) may be read as a carry only two wait states later, and
+// the compiler, which keeps them for its own instructions, does not look into
+// this one. (For such a mask it makes the same instruction from c + (a == b).)
 __device__ __forceinline__ void add_lane_bit(unsigned& c, unsigned long long m) {
   asm("v_addc_co_u32_e64 %0, vcc, 0, %0, %1" : "+v"(c) : "s"(m) : "vcc");
-}
-// c - this lane's bit of m
-__device__ __forceinline__ unsigned sub_lane_bit(unsigned c, unsigned long long m) {
-  unsigned r;
-  asm("v_subbrev_co_u32_e64 %0, vcc, 0, %1, %2" : "=v"(r) : "v"(c), "s"(m) : "vcc");
-  return r;
 }
 
 // The counts start at MASK_BIAS: count_double turns a biased count, or one
@@ -162,7 +160,7 @@ __device__ __forceinline__ int mask_ldg(const unsigned long long* masks, const u
 #pragma unroll
   for (int u = 0; u < P; u++) {
     // a part in none of the nets scores 0, or (own) no more, and is no candidate
-    sc[u] = count_double(sub_lane_bit(cnt[u], __ballot(mine == u * WAVE))) * pen[u];
+    sc[u] = count_double(cnt[u] - (mine == u * WAVE ? 1u : 0u)) * pen[u];
     best = fmax(best, sc[u]);
   }
   // the wave's best: positive doubles order like their bit patterns, the

@@ -962,7 +962,7 @@ __device__ __forceinline__ void wave_replay_medium(const ApplyArgs& a, int n, un
     if (mp) {
       const int jp = __ffsll((long long)mp) - 1;
       if (__builtin_amdgcn_readlane((int)cnt, jp) > 1) {
-        cnt = sub_lane_bit(cnt, mp);
+        cnt -= key == p ? 1u : 0u;
       } else {
         // the last entry takes p's place
         L--;
@@ -974,7 +974,7 @@ __device__ __forceinline__ void wave_replay_medium(const ApplyArgs& a, int n, un
     }
     const unsigned long long mq = __ballot(key == q);
     if (mq) {
-      add_lane_bit(cnt, mq);
+      cnt += key == q ? 1u : 0u;
     } else {
       key = lane == L ? q : key;
       cnt = lane == L ? 1u : cnt;
