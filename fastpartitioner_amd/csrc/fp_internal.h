@@ -37,7 +37,7 @@ namespace fpe {
 constexpr int WAVE = 64;
 constexpr int LDS_BUDGET = 64 * 1024;
 constexpr int LDS_PER_CU = 160 * 1024;  // gfx950: LDS of a compute unit, shared by its workgroups
-constexpr int MAX_WAVES_PER_CU = 32;    // 8 wavefronts per SIMD
+constexpr unsigned XCDS = 8;            // gfx950: workgroups go to the dies in turn, each with an L2 of its own
 constexpr unsigned NOFIRST = 0xFFFFFFFFu;
 constexpr int ENT_PAD = 64;  // tail padding of the segment arrays
 constexpr unsigned EV_SINGLE = 0x8000u;  // evaluation view: the part has one pin in the net

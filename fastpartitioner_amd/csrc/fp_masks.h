@@ -53,16 +53,19 @@ inline unsigned mask_last_pin(const fp_ctx* ctx) { return (unsigned)std::max(ctx
 
 #ifdef __HIPCC__
 // A wave's slots s0, s0 + stride, ..., at most one per lane, and their number
-// ns: a whole round of the grid's waves apart. Vertices of many nets
-// often have neighbouring numbers, and a wave of neighbouring slots took several
-// of them one after another while the others were done: 60,000 vertices, the
-// first 8 in 15,000 nets each, two rounds of TV at K = 512 22.0 -> 2.9 ms, of
-// MSV at K = 1024 22.6 -> 5.3 ms. Without such vertices the strided headers
-// and decisions cost nothing (tens of slots a wave, 1,000,000 vertices:
-// 3.10 against 3.06 ms for 5 passes).
+// ns: a whole round of the grid's waves apart. Vertices of many nets often have
+// neighbouring numbers, and a wave of neighbouring slots took several of them
+// one after another while the others were done: 60,000 vertices, the first 8 in
+// 15,000 nets each, two rounds of TV at K = 512 22.0 -> 2.9 ms, of MSV at
+// K = 1024 22.6 -> 5.3 ms. The blocks of one die take neighbouring slots, so that
+// its L2 brings a line of headers once. Without such vertices 20 passes of
+// 1,000,000 slots in rounds of 262,144 take 13.82 ms so, 13.88 with the blocks in
+// launch order, and 13.71 with a wave's slots neighbouring.
 __device__ __forceinline__ void wave_slots(int nslots, int& s0, int& stride, int& ns) {
   const int nw = (int)(blockDim.x / WAVE);
-  s0 = (int)blockIdx.x * nw + wave_id();
+  const unsigned nb = gridDim.x, xcd = blockIdx.x % XCDS;
+  const int b = (int)(xcd * (nb / XCDS) + min(xcd, nb % XCDS) + blockIdx.x / XCDS);
+  s0 = b * nw + wave_id();
   stride = (int)gridDim.x * nw;
   ns = s0 < nslots ? min(WAVE, (nslots - s0 + stride - 1) / stride) : 0;
 }
