@@ -48,6 +48,9 @@ inline int mask_eval_grid(int nslots, int grid_cap, int waves_per_block) {
   const int per_block = mask_eval_share(nslots, grid_cap, waves_per_block) * waves_per_block;
   return std::max(1, (nslots + per_block - 1) / per_block);
 }
+// nets past which a vertex's records of more than 4 words are counted another way (mask_count_wide)
+constexpr int MASK_WIDE = 512;
+inline bool mask_wide(const fp_ctx* ctx) { return mask_words(ctx->K) > 4 && ctx->max_vdeg > (unsigned)MASK_WIDE; }
 // the last element of vtx_nets, which bounds its reads a vertex ahead
 inline unsigned mask_last_pin(const fp_ctx* ctx) { return (unsigned)std::max(ctx->pins - 1, 0ll); }
 
@@ -142,6 +145,72 @@ __device__ __forceinline__ void mask_count(const unsigned long long* masks, unsi
   int j0 = 0;
   for (; j0 + NB <= nn; j0 += NB) batch(j0, NB);
   if (j0 < nn) batch(j0, nn - j0);
+}
+
+// Past MASK_WIDE nets, for K > 256: of records of 5 to 8 words two or three in
+// flight are all that the scalar registers hold, and a vertex of thousands of
+// nets is a chain of their latencies. Here a load of the wave brings a dword
+// a lane, G records at once, MASK_WIDE_LOADS loads in flight; a lane counts the
+// bits of its dword in bytes (bit 8 i + k in byte i of word k), which go through
+// LDS (MASK_WIDE_WORDS words, the wave's own) to the lanes of their parts before
+// they can overflow. each(off) runs per 64 nets, lane j holding the byte offset of
+// net j's record (the zero record past the last net).
+// 60,000 vertices, the first 8 in 15,000 nets each, two rounds of 60,000 at
+// K = 512: TV 2.90 -> 1.21 ms, MSRV in rounds of 16,384 4.7 -> 1.32; with 512
+// nets each 0.24 -> 0.17 and 0.48 -> 0.36. The kernels that hold both ways of
+// counting are slower on ordinary vertices (200,000 Zipf vertices, K = 512, MSRV
+// 4.22 -> 4.42 ms; their registers spill), so they are instances of their own
+// for hypergraphs with such a vertex.
+constexpr int MASK_WIDE_LOADS = 4;
+constexpr int MASK_WIDE_WORDS = 8 * WAVE;
+
+template <int P, class Each>
+__device__ __forceinline__ void mask_count_wide(const char* masks, const char* vtx_nets, unsigned vb, int deg,
+                                                unsigned zero, unsigned* lds, unsigned (&cnt)[P], Each each) {
+  constexpr int D = 2 * P, G = WAVE / D, LOADS = (WAVE + G - 1) / G;  // dwords of a record; loads of 64 nets
+  const int lane = lane_id(), g = lane / D, t = lane - g * D;
+  unsigned bytes[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) bytes[k] = 0u;
+  auto flush = [&]() {
+#pragma unroll
+    for (int k = 0; k < 8; k++) lds[8 * lane + k] = bytes[k];
+    wave_lds_sync();
+    const int bit = lane & 31;
+#pragma unroll 1
+    for (int h = 0; h < G; h++)
+#pragma unroll
+      for (int u = 0; u < P; u++)
+        cnt[u] += (lds[8 * (h * D + 2 * u + (lane >> 5)) + (bit & 7)] >> (bit & 24)) & 255u;
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < 8; k++) bytes[k] = 0u;
+  };
+  int counted = 0;  // dwords a lane's bytes hold
+  for (int c0 = 0; c0 < deg; c0 += WAVE) {
+    const unsigned id = *reinterpret_cast<const unsigned*>(vtx_nets + (vb + (unsigned)min(c0 + lane, deg - 1)) * 4u);
+    const unsigned off = c0 + lane < deg ? id * (16u * P) : zero;
+    for (int i0 = 0; i0 < LOADS; i0 += MASK_WIDE_LOADS) {
+      unsigned x[MASK_WIDE_LOADS];
+#pragma unroll
+      for (int i = 0; i < MASK_WIDE_LOADS; i++) {
+        const int j = (i0 + i) * G + g;
+        const unsigned o = (unsigned)__shfl((int)off, j & (WAVE - 1));
+        x[i] = *reinterpret_cast<const unsigned*>(masks + ((g < G && j < WAVE ? o : zero) + 4u * (unsigned)t));
+      }
+#pragma unroll
+      for (int i = 0; i < MASK_WIDE_LOADS; i++)
+#pragma unroll
+        for (int k = 0; k < 8; k++) bytes[k] += (x[i] >> k) & 0x01010101u;
+    }
+    each(off);
+    counted += (LOADS + MASK_WIDE_LOADS - 1) / MASK_WIDE_LOADS * MASK_WIDE_LOADS;
+    if (counted > 255 - 2 * MASK_WIDE_LOADS - LOADS) {
+      flush();
+      counted = 0;
+    }
+  }
+  flush();
 }
 
 // The LDG choice of a vertex (its nets vtx_nets[vb .. vb + deg)) from its

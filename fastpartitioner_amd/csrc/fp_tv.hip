@@ -451,12 +451,15 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
 // offsets (the host checks the arrays' sizes) and everything per vertex that
 // a lane can hold is held by one.
 // The decision, the gain test and everything written are k_tv_eval's.
-template <int P, int MODE>
+// WIDE: for hypergraphs with a vertex of more than MASK_WIDE nets (mask_count_wide).
+template <int P, int MODE, bool WIDE>
 __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu(P <= 6 ? 7 : 6, P <= 6 ? 7 : 6))) k_tv_eval_masks(EvalArgs a) {
   constexpr int CH = mask_chunk<P>();
   constexpr unsigned ROW = 16u * P;  // bytes of a record
+  static_assert(!WIDE || MODE != EVAL_INIT_CN, "uncut nets only: not a count of whole records");
   __shared__ double s_pen[64 * P];
   __shared__ unsigned s_skey[64 * P];
+  __shared__ unsigned s_wide[WIDE ? EVAL_BLOCK / WAVE : 1][WIDE ? MASK_WIDE_WORDS : 1];
   const int K = a.K;
   const int lane = lane_id(), wave = wave_id();
   int s0, stride, ns;
@@ -490,13 +493,16 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
   double pen[P];
   unsigned skey[P];
   int pid[P];
+  auto load_parts = [&]() {
 #pragma unroll
-  for (int u = 0; u < P; u++) {
-    pen[u] = s_pen[u * WAVE + lane];
-    skey[u] = s_skey[u * WAVE + lane];
-    const bool in = skey[u] <= size_key(a.max_pw) && (MODE != EVAL_REFINE || skey[u] >= size_key(a.min_pw));
-    pid[u] = (u * WAVE + lane) | (in ? 1 << 16 : 0);
-  }
+    for (int u = 0; u < P; u++) {
+      pen[u] = s_pen[u * WAVE + lane];
+      skey[u] = s_skey[u * WAVE + lane];
+      const bool in = skey[u] <= size_key(a.max_pw) && (MODE != EVAL_REFINE || skey[u] >= size_key(a.min_pw));
+      pid[u] = (u * WAVE + lane) | (in ? 1 << 16 : 0);
+    }
+  };
+  load_parts();
   const char* masks = reinterpret_cast<const char*>(a.masks);
   // lane j: net j of slot i's vertex; past its last net some other net.
   // Loaded a vertex ahead, by every lane (a load that a branch may skip could
@@ -533,10 +539,19 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
       mask_count<P, MODE == EVAL_INIT_CN>(a.masks, off, nn, cnt);
       if (MODE == EVAL_REFINE) lg += (int)__popcll(__ballot(((sw >> (own & 31)) & 1u) != 0u));
     };
-    count_nets(id0, min(deg, CH));
-    for (int c0 = CH; c0 < deg; c0 += CH)
-      count_nets(*reinterpret_cast<const unsigned*>(nets + min(vb + (unsigned)(c0 + lane), a.last_pin) * 4u),
-                 min(deg - c0, CH));
+    if (WIDE && deg > MASK_WIDE) {
+      mask_count_wide<P>(masks, nets, vb, deg, (unsigned)a.noe * ROW, s_wide[WIDE ? wave : 0], cnt, [&](unsigned off) {
+        if (MODE != EVAL_REFINE) return;
+        const unsigned sw = *reinterpret_cast<const unsigned*>(masks + (8u * P + 4u * (unsigned)(own >> 5)) + off);
+        lg += (int)__popcll(__ballot(((sw >> (own & 31)) & 1u) != 0u));
+      });
+      load_parts();  // so that their registers are free above
+    } else {
+      count_nets(id0, min(deg, CH));
+      for (int c0 = CH; c0 < deg; c0 += CH)
+        count_nets(*reinterpret_cast<const unsigned*>(nets + min(vb + (unsigned)(c0 + lane), a.last_pin) * 4u),
+                   min(deg - c0, CH));
+    }
     unsigned craw = 0;
     const int pl = mask_ldg<P, MODE == EVAL_INIT_CN>(a.masks, a.vtx_nets, a.vtx_seg, a.ev, vb, deg,
                                                      MODE == EVAL_REFINE ? own : -1, cnt, pen, skey, pid, craw);
@@ -584,16 +599,24 @@ __global__ void __launch_bounds__(EVAL_BLOCK) __attribute__((amdgpu_waves_per_eu
 
 // the instance of k_tv_eval_masks for K parts
 template <int MODE>
-void (*eval_masks_kernel(int K))(EvalArgs) {
+void (*eval_masks_kernel(int K, bool wide))(EvalArgs) {
+  if constexpr (MODE != EVAL_INIT_CN) {
+    if (wide) switch (mask_words(K)) {
+        case 5: return k_tv_eval_masks<5, MODE, true>;
+        case 6: return k_tv_eval_masks<6, MODE, true>;
+        case 7: return k_tv_eval_masks<7, MODE, true>;
+        default: return k_tv_eval_masks<8, MODE, true>;
+      }
+  }
   switch (mask_words(K)) {
-    case 1: return k_tv_eval_masks<1, MODE>;
-    case 2: return k_tv_eval_masks<2, MODE>;
-    case 3: return k_tv_eval_masks<3, MODE>;
-    case 4: return k_tv_eval_masks<4, MODE>;
-    case 5: return k_tv_eval_masks<5, MODE>;
-    case 6: return k_tv_eval_masks<6, MODE>;
-    case 7: return k_tv_eval_masks<7, MODE>;
-    default: return k_tv_eval_masks<8, MODE>;
+    case 1: return k_tv_eval_masks<1, MODE, false>;
+    case 2: return k_tv_eval_masks<2, MODE, false>;
+    case 3: return k_tv_eval_masks<3, MODE, false>;
+    case 4: return k_tv_eval_masks<4, MODE, false>;
+    case 5: return k_tv_eval_masks<5, MODE, false>;
+    case 6: return k_tv_eval_masks<6, MODE, false>;
+    case 7: return k_tv_eval_masks<7, MODE, false>;
+    default: return k_tv_eval_masks<8, MODE, false>;
   }
 }
 
@@ -1383,7 +1406,7 @@ fp_status pass_tv(fp_ctx* ctx, const RefinePlan& p) {
       a.noe = ctx->noe;
       a.last_pin = mask_last_pin(ctx);
       const int grid = mask_eval_grid(nslots, p.eval_grid, EVAL_BLOCK / WAVE);
-      FP_TRY(launch_timed(ctx, eval_masks_kernel<EVAL_REFINE>(K), grid, EVAL_BLOCK, 0, a));
+      FP_TRY(launch_timed(ctx, eval_masks_kernel<EVAL_REFINE>(K, mask_wide(ctx)), grid, EVAL_BLOCK, 0, a));
     } else {
       int grid = eval_grid(nslots, waves);
       if (p.eval_grid > 0) grid = std::min(grid, p.eval_grid);
@@ -1574,8 +1597,8 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
     a.last_pin = mask_last_pin(ctx);
     const int grid = masks ? mask_eval_grid(nslots, 0, EVAL_BLOCK / WAVE) : eval_grid(nslots, waves);
     if (masks)
-      (eval_mode == EVAL_INIT_CN ? eval_masks_kernel<EVAL_INIT_CN>(K)
-                                 : eval_masks_kernel<EVAL_INIT>(K))<<<grid, EVAL_BLOCK, 0, ctx->stream>>>(a);
+      (eval_mode == EVAL_INIT_CN ? eval_masks_kernel<EVAL_INIT_CN>(K, false)
+                                 : eval_masks_kernel<EVAL_INIT>(K, mask_wide(ctx)))<<<grid, EVAL_BLOCK, 0, ctx->stream>>>(a);
     else if (eval_mode == EVAL_INIT_CN)
       k_tv_eval<EVAL_INIT_CN><<<grid, waves * WAVE, lds_e, ctx->stream>>>(a);
     else

@@ -504,7 +504,8 @@ __global__ void __launch_bounds__(VOL_BLOCK) __attribute__((amdgpu_waves_per_eu(
 // the lists a second time for them took as long as the first sweep.
 constexpr int VOL_MASK_BLOCK = 256;
 
-template <int P>
+// WIDE: for hypergraphs with a vertex of more than MASK_WIDE nets (mask_count_wide).
+template <int P, bool WIDE>
 __global__ void __launch_bounds__(VOL_MASK_BLOCK) __attribute__((amdgpu_waves_per_eu(P <= 6 ? 7 : 6, P <= 6 ? 7 : 6)))
 k_vol_eval_masks(VolEvalArgs a) {
   constexpr int CH = mask_chunk<P>();
@@ -513,6 +514,7 @@ k_vol_eval_masks(VolEvalArgs a) {
   __shared__ unsigned s_skey[64 * P];
   __shared__ int s_delta[VOL_MASK_BLOCK / WAVE][64 * P];    // losses - gains per part
   __shared__ unsigned s_hit[VOL_MASK_BLOCK / WAVE][2 * P];  // max parts the move affects (MSRV), one bit per part
+  __shared__ unsigned s_wide[WIDE ? VOL_MASK_BLOCK / WAVE : 1][WIDE ? MASK_WIDE_WORDS : 1];
   const int K = a.K;
   const int lane = lane_id(), wave = wave_id();
   int* delta = s_delta[wave];
@@ -544,12 +546,15 @@ k_vol_eval_masks(VolEvalArgs a) {
   double pen[P];
   unsigned skey[P];
   int pid[P];
+  auto load_parts = [&]() {
 #pragma unroll
-  for (int u = 0; u < P; u++) {
-    pen[u] = s_pen[u * WAVE + lane];
-    skey[u] = s_skey[u * WAVE + lane];
-    pid[u] = u * WAVE + lane;
-  }
+    for (int u = 0; u < P; u++) {
+      pen[u] = s_pen[u * WAVE + lane];
+      skey[u] = s_skey[u * WAVE + lane];
+      pid[u] = u * WAVE + lane;
+    }
+  };
+  load_parts();
   const int M = a.mstat[0], cntM = a.mstat[1];
   const char* masks = reinterpret_cast<const char*>(a.masks);
   const char* nets = reinterpret_cast<const char*>(a.vtx_nets);
@@ -593,11 +598,17 @@ k_vol_eval_masks(VolEvalArgs a) {
 #pragma unroll
     for (int u = 0; u < P; u++) cnt[u] = MASK_BIAS;
     Chunk c0 = load_chunk(id0, min(deg, CH));
-    mask_count<P, false>(a.masks, c0.off, min(deg, CH), cnt);
-    source_part(c0);
-    for (int b = CH; b < deg; b += CH) {
-      const int nn = min(deg - b, CH);
-      mask_count<P, false>(a.masks, (lane < nn ? net_ids(b) : (unsigned)a.noe) * ROW, nn, cnt);
+    if (WIDE && deg > MASK_WIDE) {
+      mask_count_wide<P>(masks, nets, vb, deg, (unsigned)a.noe * ROW, s_wide[WIDE ? wave : 0], cnt, [](unsigned) {});
+      load_parts();  // so that their registers are free above
+      source_part(c0);
+    } else {
+      mask_count<P, false>(a.masks, c0.off, min(deg, CH), cnt);
+      source_part(c0);
+      for (int b = CH; b < deg; b += CH) {
+        const int nn = min(deg - b, CH);
+        mask_count<P, false>(a.masks, (lane < nn ? net_ids(b) : (unsigned)a.noe) * ROW, nn, cnt);
+      }
     }
     unsigned craw = 0;
     int d = mask_ldg<P, false>(a.masks, a.vtx_nets, a.vtx_seg, a.ev, vb, deg, own, cnt, pen, skey, pid, craw);
@@ -642,43 +653,57 @@ k_vol_eval_masks(VolEvalArgs a) {
       atomicAdd(&delta[d], d_dec);
     }
     wave_lds_sync();
-    // the affected parts: own, d and every net's source part; every other part
-    // has gains = losses = 0. g(part) runs for every one of them
-    auto for_items = [&](auto g) {
-      if (lane < 2) g(lane == 0 ? own : d);
-      if (c0.ip >= 0) g(c0.ip);
-      for (int b = CH; b < deg; b += CH) {
-        const int nn = min(deg - b, CH);
-        if (lane < nn) {
-          const int s = a.src[net_ids(b)];
-          g(s == v ? own : a.part[s]);
-        }
-      }
-    };
-    // MSRV: max parts untouched by the move have gains = losses = 0 and fail
-    // the strict test, so every max part must be affected: maxhit counts the
-    // distinct max parts among the items
     bool bad = false;
     int maxhit = 0;
-    for_items([&](int p) {
-      const int dl = delta[p];
-      const int vv = a.vol[p];
-      if (vv == M) {
-        if (a.msrv ? dl >= 0 : dl > 0) bad = true;  // a max part must gain (MSRV: strictly)
-        const unsigned bit = 1u << (p & 31);
-        if (!(atomicOr(&hitb[p >> 5], bit) & bit)) maxhit++;
-      } else if (vv + dl >= M) {
-        bad = true;  // no other part may reach the max
+    if (WIDE && deg > MASK_WIDE) {
+      // Very many nets: all parts, instead of their sources' parts gathered again.
+      // A part that the move does not touch has gains = losses = 0, which fails
+      // the rule below for a max part of MSRV and no other.
+      for (int p = lane; p < K; p += WAVE) {
+        const int dl = delta[p];
+        const int vv = a.vol[p];
+        if (vv == M ? (a.msrv ? dl >= 0 : dl > 0) : vv + dl >= M) bad = true;
+        delta[p] = 0;
       }
-    });
+      maxhit = cntM;
+      wave_lds_sync();
+    } else {
+      // the affected parts: own, d and every net's source part; every other part
+      // has gains = losses = 0. g(part) runs for every one of them
+      auto for_items = [&](auto g) {
+        if (lane < 2) g(lane == 0 ? own : d);
+        if (c0.ip >= 0) g(c0.ip);
+        for (int b = CH; b < deg; b += CH) {
+          const int nn = min(deg - b, CH);
+          if (lane < nn) {
+            const int s = a.src[net_ids(b)];
+            g(s == v ? own : a.part[s]);
+          }
+        }
+      };
+      // MSRV: max parts untouched by the move have gains = losses = 0 and fail
+      // the strict test, so every max part must be affected: maxhit counts the
+      // distinct max parts among the items
+      for_items([&](int p) {
+        const int dl = delta[p];
+        const int vv = a.vol[p];
+        if (vv == M) {
+          if (a.msrv ? dl >= 0 : dl > 0) bad = true;  // a max part must gain (MSRV: strictly)
+          const unsigned bit = 1u << (p & 31);
+          if (!(atomicOr(&hitb[p >> 5], bit) & bit)) maxhit++;
+        } else if (vv + dl >= M) {
+          bad = true;  // no other part may reach the max
+        }
+      });
+      maxhit = wave_sum(maxhit);
+      wave_lds_sync();
+      for_items([&](int p) {
+        delta[p] = 0;
+        hitb[p >> 5] = 0u;
+      });
+      wave_lds_sync();
+    }
     bad = __ballot(bad) != 0;
-    maxhit = wave_sum(maxhit);
-    wave_lds_sync();
-    for_items([&](int p) {
-      delta[p] = 0;
-      hitb[p >> 5] = 0u;
-    });
-    wave_lds_sync();
     if (!bad && (!a.msrv || maxhit == cntM)) {
       dec_l = lane == i ? d : dec_l;
       wave_touch_nets(a.vtx_nets + vb, deg, a.tag, a.net_stamp, a.touched, a.tcount);
@@ -691,16 +716,22 @@ k_vol_eval_masks(VolEvalArgs a) {
 }
 
 // the instance of k_vol_eval_masks for K parts
-void (*vol_masks_kernel(int K))(VolEvalArgs) {
+void (*vol_masks_kernel(int K, bool wide))(VolEvalArgs) {
+  if (wide) switch (mask_words(K)) {
+      case 5: return k_vol_eval_masks<5, true>;
+      case 6: return k_vol_eval_masks<6, true>;
+      case 7: return k_vol_eval_masks<7, true>;
+      default: return k_vol_eval_masks<8, true>;
+    }
   switch (mask_words(K)) {
-    case 1: return k_vol_eval_masks<1>;
-    case 2: return k_vol_eval_masks<2>;
-    case 3: return k_vol_eval_masks<3>;
-    case 4: return k_vol_eval_masks<4>;
-    case 5: return k_vol_eval_masks<5>;
-    case 6: return k_vol_eval_masks<6>;
-    case 7: return k_vol_eval_masks<7>;
-    default: return k_vol_eval_masks<8>;
+    case 1: return k_vol_eval_masks<1, false>;
+    case 2: return k_vol_eval_masks<2, false>;
+    case 3: return k_vol_eval_masks<3, false>;
+    case 4: return k_vol_eval_masks<4, false>;
+    case 5: return k_vol_eval_masks<5, false>;
+    case 6: return k_vol_eval_masks<6, false>;
+    case 7: return k_vol_eval_masks<7, false>;
+    default: return k_vol_eval_masks<8, false>;
   }
 }
 
@@ -1429,7 +1460,7 @@ fp_status pass_vol(fp_ctx* ctx, const RefinePlan& p) {
       a.masks = p.masks;
       a.noe = ctx->noe;
       const int egrid = mask_eval_grid(nslots, p.eval_grid, VOL_MASK_BLOCK / WAVE);
-      FP_TRY(launch_timed(ctx, vol_masks_kernel(K), egrid, VOL_MASK_BLOCK, 0, a));
+      FP_TRY(launch_timed(ctx, vol_masks_kernel(K, mask_wide(ctx)), egrid, VOL_MASK_BLOCK, 0, a));
     } else {
       a.pad_seg = (unsigned)((size_t)ctx->pins + (size_t)ctx->noe);
       if (ctx->pins == 0) {
