@@ -40,23 +40,26 @@ constexpr int REPLAY_NET_BLOCKS = 2048;
 // sums in LDS. A lane per net, so that 64 nets' dependent reads (offset, length
 // and source, the source's part) go together; MSRV's lists of more than
 // VOL_INIT_SMALL entries are taken by the wavefront. A wavefront per net took
-// 582 us for 2,000,000 nets (MSV) and 77 us for 200,000 (MSRV).
+// 582 us for 2,000,000 nets (MSV) and 77 us for 200,000 (MSRV). Where the nets
+// are few, a wavefront takes per_wave < 64 of them: 2,000 nets of 1,500 pins
+// (MSRV, K = 1024) took 229 us on 32 wavefronts, now 25.
 constexpr int VOL_INIT_SMALL = 16;
+constexpr int VOL_INIT_WAVES = 4096;
 
 __global__ void __launch_bounds__(256) k_vol_init(const unsigned* __restrict__ net_ptr,
                                                   const unsigned* __restrict__ ent, const int* __restrict__ src,
-                                                  const int* __restrict__ part, int noe, unsigned pmask, int K,
-                                                  int msrv, int* __restrict__ vol) {
+                                                  const int* __restrict__ part, int noe, int per_wave, unsigned pmask,
+                                                  int K, int msrv, int* __restrict__ vol) {
   extern __shared__ int s_vol[];
   const int lane = lane_id();
   for (int q = (int)threadIdx.x; q < K; q += (int)blockDim.x) s_vol[q] = 0;
   __syncthreads();
   const int nw = (int)(gridDim.x * blockDim.x / WAVE);
-  for (int n0 = (int)((blockIdx.x * blockDim.x + threadIdx.x) / WAVE) * WAVE; n0 < noe; n0 += nw * WAVE) {
+  for (int n0 = (int)((blockIdx.x * blockDim.x + threadIdx.x) / WAVE) * per_wave; n0 < noe; n0 += nw * per_wave) {
     const int n = n0 + lane;
     unsigned seg = 0;
     int L = 0, sp = 0;
-    if (n < noe) {
+    if (lane < per_wave && n < noe) {
       seg = net_ptr[n] + (unsigned)n;
       L = (int)ent[seg];
       if (L > 0) sp = part[src[n]];
@@ -1398,9 +1401,11 @@ fp_status plan_vol(fp_ctx* ctx, RefinePlan& p) {
   // the volumes of the resident state, kept incrementally by the passes
   auto& vs = ctx->vol;
   fill_async<int>(ctx, vs.vol, (size_t)K, 0);
-  const int ngrid = std::max(1, std::min((ctx->noe + 255) / 256, 4096));
-  k_vol_init<<<std::min(ngrid * 8, 1024), 256, (size_t)K * sizeof(int), ctx->stream>>>(
-      ctx->net_ptr, ctx->ent, ctx->src, ctx->part, ctx->noe, ctx->pmask, K, msrv ? 1 : 0, vs.vol);
+  const int per_wave = std::max(1, std::min(WAVE, (ctx->noe + VOL_INIT_WAVES - 1) / VOL_INIT_WAVES));
+  const int per_block = per_wave * (256 / WAVE);
+  k_vol_init<<<std::max(1, std::min((ctx->noe + per_block - 1) / per_block, VOL_INIT_WAVES / (256 / WAVE))), 256,
+               (size_t)K * sizeof(int), ctx->stream>>>(ctx->net_ptr, ctx->ent, ctx->src, ctx->part, ctx->noe, per_wave,
+                                                       ctx->pmask, K, msrv ? 1 : 0, vs.vol);
   // the part masks of the resident lists, kept in step by the passes
   p.masks = ensure_masks(ctx);
   if (p.masks) build_masks(ctx, p.masks);
