@@ -591,9 +591,15 @@ fp_status fp_upload(fp_ctx* ctx, int nov, int noe, const unsigned* net_ptr, cons
   ctx->met_out_cap = 0;
   if (net_ptr[0] != 0) return fail(ctx, FP_ERR_ARG, "fp_upload: net_ptr[0] != 0");
   unsigned max_net = 0;
+  std::fill(std::begin(ctx->class_nets), std::end(ctx->class_nets), 0ll);
+  std::fill(std::begin(ctx->class_pins), std::end(ctx->class_pins), 0ll);
   for (int n = 0; n < noe; n++) {
     if (net_ptr[n + 1] < net_ptr[n]) return fail(ctx, FP_ERR_ARG, "fp_upload: net_ptr not monotone at %d", n);
-    max_net = std::max(max_net, net_ptr[n + 1] - net_ptr[n]);
+    const unsigned size = net_ptr[n + 1] - net_ptr[n];
+    max_net = std::max(max_net, size);
+    const int b = size ? std::min(31 - __builtin_clz(size), fp_ctx::SIZE_CLASSES - 1) : 0;
+    ctx->class_nets[b]++;
+    ctx->class_pins[b] += size;
   }
   {
     // the first pin out of range, on every host thread

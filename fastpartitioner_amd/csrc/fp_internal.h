@@ -742,6 +742,9 @@ struct fp_ctx {
   bool src_on_pins = false;  // every non-empty net's source is one of its pins
   long long total_weight = 0;
   unsigned max_net = 0, max_vdeg = 0;
+  // nets of 2^b to 2^(b + 1) - 1 pins (the last entry: and more), and their pins
+  static constexpr int SIZE_CLASSES = 20;
+  long long class_nets[SIZE_CLASSES] = {}, class_pins[SIZE_CLASSES] = {};
   unsigned long long max_src_pins = 0;  // max over vertices of the pins of the nets whose source it is
   unsigned long long sum_deg2 = 0;  // sum over vertices of degree^2 (bounds CN's per-pass edit list)
   std::vector<unsigned> h_net_ptr;

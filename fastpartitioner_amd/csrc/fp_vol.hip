@@ -1327,6 +1327,41 @@ size_t vol_eval_lds(int K, int waves, bool shorts) {
   return vol_short_at(K, waves) + (shorts ? (size_t)waves * VOL_SHORT_BYTES : 0);
 }
 
+// At most how many list entries the nets of a vertex have together, on average
+// over the vertices: a list has no more entries than its net has pins, nor than K.
+double vol_mean_entries(const fp_ctx* ctx, int K) {
+  double e = 0;
+  for (int b = 0; b < fp_ctx::SIZE_CLASSES; b++)
+    if (ctx->class_nets[b]) {
+      const double pins = (double)ctx->class_pins[b];
+      e += pins * std::min(pins / (double)ctx->class_nets[b], (double)K);
+    }
+  return e / ctx->nov;
+}
+
+// Blocks of k_vol_eval. In general a wave takes its share of the round, as many
+// waves as the 256 CUs hold: setting itself up takes as long as some vertices of
+// few entries. Shares of two or three vertices leave up to a third of the waves
+// idle, so a round of vertices of more entries, which take longer than the
+// setting up, is left to the order in which waves end, a vertex a wave, up
+// to a number of vertices per resident wave that grows with the entries.
+// us a launch, a vertex a wave against shares, rounds of 8,192 and 16,384 slots:
+//   169 entries a vertex (13 nets of 13 pins, K = 1024)    20   30      17   23
+//   1,024 (32 of 32, K = 600)                              54   76      58   78
+//   1,703 (Zipf, K = 600)                                  78  114      83  108
+//   16,384 (128 of 128, K = 600)                          377  562     435  620
+//   30,000 (50 of 1,500, K = 600)                         613  898     705  973
+// of 40,000 slots: 68 and 40, 147 and 133, 227 and 208, 958 and 953, 1,615 and 1,784.
+constexpr double VOL_LONG = 256;
+constexpr double VOL_PER_ROUND = 4096;
+
+int vol_eval_grid(const fp_ctx* ctx, int nslots, int waves, int resident, int grid_cap) {
+  const int cap = grid_cap > 0 ? std::min(grid_cap, resident) : resident;
+  const double e = vol_mean_entries(ctx, ctx->K);
+  if (e > VOL_LONG && nslots <= (2 + e / VOL_PER_ROUND) * cap * waves) return std::max(1, (nslots + waves - 1) / waves);
+  return mask_eval_grid(nslots, cap, waves);
+}
+
 // workgroups of that shape a CU holds (k_vol_eval's registers allow 6 waves per SIMD)
 int vol_eval_per_cu(int waves, size_t lds) { return std::min((int)((size_t)LDS_PER_CU / lds), VOL_CU_WAVES / waves); }
 
@@ -1475,9 +1510,8 @@ fp_status pass_vol(fp_ctx* ctx, const RefinePlan& p) {
         a.src = reinterpret_cast<const int*>(a.vtx_nets);
       }
       a.shorts = shorts ? 1 : 0;
-      // as many blocks as the 256 CUs hold: a few more would run alone at the end
       const int resident = 256 * std::max(1, vol_eval_per_cu(waves, lds_e));
-      const int egrid = mask_eval_grid(nslots, p.eval_grid > 0 ? std::min(p.eval_grid, resident) : resident, waves);
+      const int egrid = vol_eval_grid(ctx, nslots, waves, resident, p.eval_grid);
       FP_TRY(launch_timed(ctx, k_vol_eval, egrid, waves * WAVE, lds_e, a));
     }
     launch_round_compact<false>(ctx, ctx->order, r0, nslots, vs.slot_mi, vs.mv, vs.mstat);
