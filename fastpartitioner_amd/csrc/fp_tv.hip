@@ -50,6 +50,8 @@ constexpr int APPLY_BLOCK = 256;
 constexpr int SMALL_NET = 8;     // nets of at most this many pins are replayed one per lane
 constexpr int APPLY_NET_BLOCKS = 2048;  // all resident at 8 waves per SIMD (8,192 cost 8 to 18%)
 constexpr int APPLY_NETS = 512;    // nets per block of the apply at most
+constexpr int APPLY_LIST_NETS = 4;  // and at least, of a list
+constexpr int APPLY_LIST_NOE = 1 << 18, APPLY_LIST_RATIO = 32;  // apply_by_list
 constexpr unsigned HUGE_NET = 256;  // nets of at least this many pins are replayed first
 constexpr int APPLY_GROUP = 4;     // 64-rank windows of a net whose loads the apply issues together
 constexpr int APPLY_TOGETHER = 8;  // moves of a window tried together (wave_ilist_moves)
@@ -633,9 +635,10 @@ constexpr int SCAN_WAVE_TILES = 16 * WAVE;
 template <bool WAVE_ROWS>
 __global__ void __launch_bounds__(256) k_bal_scan(int* __restrict__ hist, long long* __restrict__ pref, int ntiles,
                                                   int K, const long long* __restrict__ sizes_frozen, long long cap,
-                                                  int* __restrict__ over) {
+                                                  int* __restrict__ over, int* __restrict__ tcount) {
   __shared__ long long s_wl[16];
   const int lane = lane_id();
+  if (blockIdx.x == 0 && threadIdx.x == 0) *tcount = 0;  // of the round's touched list (k_bal_admit)
   if (WAVE_ROWS) {
     const int nw = (int)(blockDim.x / WAVE);
     for (int d = (int)blockIdx.x * nw + wave_id(); d < K; d += (int)gridDim.x * nw) {
@@ -766,8 +769,10 @@ __global__ void __launch_bounds__(1024) k_init_fallback(int* __restrict__ slot_d
 // queue at one L2 slice: about 12 ns each, so the blocks are as large as they
 // can be).
 constexpr int ADMIT_BLOCK = 1024;
+constexpr int ADMIT_NETS = 4;
 
-template <bool AGG>
+// LIST: the touched nets go to a list, too (apply_by_list).
+template <bool AGG, bool LIST>
 __global__ void __launch_bounds__(ADMIT_BLOCK) k_bal_admit(int* __restrict__ slot_dec, const int* __restrict__ slot_own,
                                                    const int* __restrict__ order, const int* __restrict__ vwgt,
                                                    int r0, int nslots, int ntiles, int K,
@@ -778,7 +783,8 @@ __global__ void __launch_bounds__(ADMIT_BLOCK) k_bal_admit(int* __restrict__ slo
                                                    unsigned long long* __restrict__ moves,
                                                    const unsigned* __restrict__ vtx_ptr,
                                                    const unsigned* __restrict__ vtx_nets, unsigned tag,
-                                                   unsigned* __restrict__ net_stamp) {
+                                                   unsigned* __restrict__ net_stamp, int* __restrict__ touched,
+                                                   int* __restrict__ tcount) {
   const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
   // the block's admitted moves, added to the global count once per block
   // (same-address atomics from every wave would queue at one L2 slice)
@@ -794,11 +800,23 @@ __global__ void __launch_bounds__(ADMIT_BLOCK) k_bal_admit(int* __restrict__ slo
     const int slot = tile * TILE + lane;
     int d = -1, v = -1;
     long long w = 0;
+    unsigned vb = 0, ve = 0;
     if (slot < nslots) {
       d = slot_dec[slot];
       const int z = r0 + slot;
       v = order ? order[z] : z;
       w = vwgt ? vwgt[v] : 1;
+      if (LIST) {
+        // of the stream, whose candidates are nearly all admitted, and whose
+        // small launches are a chain of loads
+        vb = vtx_ptr[v];
+        ve = vtx_ptr[v + 1];
+      }
+    }
+    unsigned n[ADMIT_NETS];
+    if (LIST && d >= 0 && vb < ve) {
+#pragma unroll
+      for (int u = 0; u < ADMIT_NETS; u++) n[u] = vtx_nets[min(vb + (unsigned)u, ve - 1)];
     }
     const bool o = d >= 0 && over[d] != 0;
     bool adm = d >= 0;
@@ -827,26 +845,60 @@ __global__ void __launch_bounds__(ADMIT_BLOCK) k_bal_admit(int* __restrict__ slo
         atomic_add_i64(&sizes[d], w);
       }
     }
-    // the admitted moves' nets get the round's tag: by the move's lane, four
-    // at a time, or by the wave for a vertex of more than 64 nets
-    unsigned vb = 0, ve = 0;
-    if (adm) {
+    // the admitted moves' nets get the round's tag: by the move's lane,
+    // ADMIT_NETS at a time, or by the wave for a vertex of more than 64 nets
+    if (!LIST && adm) {
       vb = vtx_ptr[v];
       ve = vtx_ptr[v + 1];
     }
     const bool hub = adm && ve - vb > (unsigned)WAVE;
+    unsigned long long fresh = 0;  // LIST, bit j: the lane stamped its net j first
     if (adm && !hub)
-      for (unsigned j = vb; j < ve; j += 4) {
-        unsigned n[4];
+      for (unsigned j = vb; j < ve; j += ADMIT_NETS) {
+        // past the end the last net again (LIST: it has the tag by then)
+        if (!LIST || j != vb) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) n[u] = vtx_nets[min(j + (unsigned)u, ve - 1)];
+          for (int u = 0; u < ADMIT_NETS; u++) n[u] = vtx_nets[min(j + (unsigned)u, ve - 1)];
+        }
+        if (!LIST) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) net_stamp[n[u]] = tag;
+          for (int u = 0; u < ADMIT_NETS; u++) net_stamp[n[u]] = tag;
+        } else {
+          unsigned old[ADMIT_NETS];
+#pragma unroll
+          for (int u = 0; u < ADMIT_NETS; u++) old[u] = atomicExch(&net_stamp[n[u]], tag);
+#pragma unroll
+          for (int u = 0; u < ADMIT_NETS; u++) fresh |= old[u] != tag ? 1ull << (j - vb + (unsigned)u) : 0ull;
+        }
       }
+    if (LIST) {
+      const int mine = (int)__popcll(fresh), incl = wave_incl_scan(mine);
+      const int all = __builtin_amdgcn_readlane(incl, WAVE - 1);
+      int at = 0;
+      if (all && lane == 0) at = atomicAdd(tcount, all);
+      at = __builtin_amdgcn_readlane(at, 0) + incl - mine;
+      for (; fresh; fresh &= fresh - 1) touched[at++] = (int)vtx_nets[vb + (unsigned)__builtin_ctzll(fresh)];
+    }
     for (unsigned long long hm = __ballot(hub); hm; hm &= hm - 1) {
       const int l = __ffsll((long long)hm) - 1;
-      const unsigned b = (unsigned)__builtin_amdgcn_readlane((int)vb, l);
-      wave_stamp_nets(vtx_nets + b, (int)((unsigned)__builtin_amdgcn_readlane((int)ve, l) - b), tag, net_stamp);
+      const unsigned b = (unsigned)__builtin_amdgcn_readlane((int)vb, l), e = (unsigned)__builtin_amdgcn_readlane((int)ve, l);
+      if (!LIST) {
+        wave_stamp_nets(vtx_nets + b, (int)(e - b), tag, net_stamp);
+        continue;
+      }
+      for (unsigned j = b; j < e; j += (unsigned)WAVE) {
+        unsigned n = 0;
+        bool first = false;
+        if (j + (unsigned)lane < e) {
+          n = vtx_nets[j + (unsigned)lane];
+          first = atomicExch(&net_stamp[n], tag) != tag;
+        }
+        const unsigned long long fm = __ballot(first);
+        int at = 0;
+        if (fm && lane == 0) at = atomicAdd(tcount, (int)__popcll(fm));
+        at = __builtin_amdgcn_readlane(at, 0);
+        if (first) touched[at + (int)__popcll(fm & ((1ull << lane) - 1ull))] = (int)n;
+      }
     }
     const unsigned long long am = __ballot(adm);
     if (lane == 0 && am) atomicAdd(&s_moves, (unsigned long long)__popcll(am));
@@ -868,6 +920,8 @@ struct ApplyArgs {
   const unsigned* net_stamp;  // the nets stamped with the round's tag are touched
   unsigned tag;
   int noe, per_block;         // each block takes per_block consecutive nets
+  const int* touched;         // LIST: the touched nets, shared by the blocks
+  const int* tcount;
   int lane_words;             // LDS words per lane of the small nets' replay
   int wave_bytes;             // LDS bytes per wave
   unsigned* ent;
@@ -1020,11 +1074,13 @@ __device__ __forceinline__ void wave_replay_medium(const ApplyArgs& a, int n, un
 // The apply's LDS that does not depend on K: the block's touched nets (the
 // small ones from the front, the others from the back), the positions of the
 // huge ones, which are replayed first, and the waves' mask words.
+template <bool LIST>
 struct ApplyNets {
   int cnt[4];  // touched small nets, other nets, nets handed out, huge nets
   unsigned words[APPLY_BLOCK / WAVE][4 * MASK_PMAX];
   unsigned start[APPLY_NETS], len[APPLY_NETS];
-  unsigned short net[APPLY_NETS], huge[APPLY_NETS];
+  std::conditional_t<LIST, unsigned, unsigned short> net[APPLY_NETS];  // LIST: its number, else from the block's first net on
+  unsigned short huge[APPLY_NETS];
 };
 
 // Replays the round's moves on every touched net in ordering order
@@ -1034,7 +1090,9 @@ struct ApplyNets {
 // (TV/partition.cpp:818-830: the destination's size is left unchanged).
 // INDEXED: each wave keeps a part -> position index of its list in LDS (2
 // bytes per part after the list), for K where it fits.
-template <bool INDEXED>
+// LIST: the touched nets come as a list, else each block looks for them among
+// the stamps of its nets (apply_by_list).
+template <bool INDEXED, bool LIST>
 __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) k_apply(ApplyArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   const int lane = lane_id(), wave = wave_id(), nw = (int)(blockDim.x / WAVE);
@@ -1059,23 +1117,27 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
   unsigned* my = reinterpret_cast<unsigned*>(mem) + (size_t)lane * (size_t)a.lane_words;
   unsigned* list = reinterpret_cast<unsigned*>(mem);
   unsigned short* at = reinterpret_cast<unsigned short*>(list + a.K);
-  __shared__ ApplyNets s;
+  __shared__ ApplyNets<LIST> s;
   unsigned* words = s.words[wave];
 
   // the block's touched nets, the small ones and the others apart: a wave
   // then replays 64 small nets at a time, a lane each, and the big ones go
   // to whichever wave is free
-  const int n0 = (int)blockIdx.x * a.per_block;
-  const int nn = min(a.per_block, a.noe - n0);
+  const int total = LIST ? *a.tcount : a.noe;
+  const int per = LIST ? min(APPLY_NETS, max(APPLY_LIST_NETS, (total + a.net_blocks - 1) / a.net_blocks)) : a.per_block;
+  const int n0 = (int)blockIdx.x * per, net0 = LIST ? 0 : n0;
+  const int nn = min(per, total - n0);
+  if (LIST && nn <= 0) return;
   if (threadIdx.x < 4) s.cnt[threadIdx.x] = 0;
   __syncthreads();
   for (int i0 = 0; i0 < nn; i0 += APPLY_BLOCK) {
     const int i = i0 + (int)threadIdx.x;
-    const bool hit = i < nn && a.net_stamp[n0 + i] == a.tag;
-    unsigned st = 0, len = 0;
+    const bool hit = i < nn && (LIST || a.net_stamp[n0 + i] == a.tag);
+    unsigned n = 0, st = 0, len = 0;
     if (hit) {
-      st = a.net_ptr[n0 + i];
-      len = a.net_ptr[n0 + i + 1] - st;
+      n = LIST ? (unsigned)a.touched[n0 + i] : (unsigned)(n0 + i);
+      st = a.net_ptr[n];
+      len = a.net_ptr[n + 1] - st;
     }
     const bool sm = hit && len <= (unsigned)SMALL_NET;
     const unsigned long long ms = __ballot(sm), mb = __ballot(hit && !sm);
@@ -1090,7 +1152,7 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
     const unsigned long long lt = (1ull << lane) - 1ull;
     const int k = sm ? bs + (int)__popcll(ms & lt) : APPLY_NETS - 1 - (bb + (int)__popcll(mb & lt));
     if (hit) {
-      s.net[k] = (unsigned short)i;
+      s.net[k] = (decltype(s.net[0] + 0))(n - (unsigned)net0);
       s.start[k] = st;
       s.len[k] = len;
       if (len >= HUGE_NET) s.huge[atomicAdd(&s.cnt[3], 1)] = (unsigned short)k;
@@ -1101,7 +1163,7 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
   const int nhuge = __builtin_amdgcn_readfirstlane(s.cnt[3]);
 
   for (int b = wave * WAVE; b < nsmall; b += nw * WAVE)
-    if (b + lane < nsmall) lane_replay_small(a, n0 + s.net[b + lane], s.start[b + lane], s.len[b + lane], my);
+    if (b + lane < nsmall) lane_replay_small(a, net0 + (int)s.net[b + lane], s.start[b + lane], s.len[b + lane], my);
   if (nbig == 0) return;
   wave_lds_sync();
   if (INDEXED) wave_index_init(at, a.K);
@@ -1130,7 +1192,7 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
       if (lane == 0) k = atomicAdd(&s.cnt[2], 1);  // a huge one again: the next
       k = __builtin_amdgcn_readlane(k, 0);
     }
-    h.n = n0 + __builtin_amdgcn_readfirstlane((int)s.net[k]);
+    h.n = net0 + __builtin_amdgcn_readfirstlane((int)s.net[k]);
     h.s = (unsigned)__builtin_amdgcn_readfirstlane((int)s.start[k]);
     const unsigned np = (unsigned)__builtin_amdgcn_readfirstlane((int)s.len[k]);
     h.e = h.s + np;
@@ -1238,11 +1300,13 @@ size_t apply_wave_bytes(int K, bool indexed) {
   return (std::max(list, (size_t)WAVE * (size_t)apply_lane_words(K) * sizeof(unsigned)) + 15) & ~(size_t)15;
 }
 
-bool apply_indexed(int K) {
-  return (size_t)(APPLY_BLOCK / WAVE) * apply_wave_bytes(K, true) + sizeof(ApplyNets) <= (size_t)LDS_BUDGET;
+size_t apply_static(bool list) { return list ? sizeof(ApplyNets<true>) : sizeof(ApplyNets<false>); }
+
+bool apply_indexed(int K, bool list) {
+  return (size_t)(APPLY_BLOCK / WAVE) * apply_wave_bytes(K, true) + apply_static(list) <= (size_t)LDS_BUDGET;
 }
 
-size_t apply_lds(int K) { return (size_t)(APPLY_BLOCK / WAVE) * apply_wave_bytes(K, apply_indexed(K)); }
+size_t apply_lds(int K, bool list) { return (size_t)(APPLY_BLOCK / WAVE) * apply_wave_bytes(K, apply_indexed(K, list)); }
 
 size_t eval_lds(int K, int waves) {
   return (size_t)K * 12 + (size_t)waves * 8 * (size_t)(K + WAVE);
@@ -1294,15 +1358,59 @@ int apply_blocks(const fp_ctx* ctx, int& per_block) {
   return std::max(1, (ctx->noe + per_block - 1) / per_block);
 }
 
+// Whether a sub-round of the stream hands its touched nets to the apply as a list.
+// Looking for them among all nets' stamps costs a launch in proportion to the
+// nets, and leaves some blocks many of the few touched ones; a list costs the admission
+// an exchange a pin and an atomic per 64 slots on one counter. Whole streams,
+// K = 64 (16 for the first), stamps and list, ms:
+//   slots                 256          1,024        4,096       16,384      32,768
+//   1,000,000 Zipf     220  202      72.5 53.2    20.4 15.9    6.3  5.6    3.9  4.0
+//   2,000,000 of 13                   372  115    98.9 36.1   29.0 15.8   17.3 12.6
+//   600,000 of 9       211  115      67.9 30.6    18.0  9.0    5.3  3.6    3.2  2.8
+//   300,000 of 9        86   58      22.3 15.3     6.2  4.5    2.1  1.9    1.4  1.4
+//   200,000 Zipf      35.0 37.5       9.4 10.0     2.7  2.9    1.1  1.3
+// Passes of the balanced schedule, whose rounds move few vertices, take the stamps:
+// 300,000 nets, rounds of 256, 15.8 ms against 17.6; 1,000,000, of 16,384, 2.29 against 2.17.
+bool apply_by_list(const fp_ctx* ctx, int nslots) {
+  return ctx->noe >= APPLY_LIST_NOE && (long long)nslots * APPLY_LIST_RATIO <= ctx->noe;
+}
+
+void launch_apply(fp_ctx* ctx, ApplyArgs& ap, int extra_blocks, bool list) {
+  const int K = ctx->K;
+  const bool indexed = apply_indexed(K, list);
+  ap.noe = ctx->noe;
+  ap.net_ptr = ctx->net_ptr;
+  ap.apply_pins = ctx->apply_pins;
+  ap.slot_own = ctx->slot_own;
+  ap.slot_dec = ctx->slot_dec;
+  ap.net_stamp = ctx->net_stamp;
+  ap.touched = ctx->touched;
+  ap.tcount = ctx->counters;
+  ap.ent = ctx->ent;
+  ap.ev = ctx->ev;
+  ap.mask_words = mask_words(K);
+  ap.K = K;
+  ap.pb = ctx->pb;
+  ap.pmask = ctx->pmask;
+  ap.net_blocks = apply_blocks(ctx, ap.per_block);
+  ap.lane_words = apply_lane_words(K);
+  ap.wave_bytes = (int)apply_wave_bytes(K, indexed);
+  auto kernel = list ? (indexed ? k_apply<true, true> : k_apply<false, true>)
+                     : (indexed ? k_apply<true, false> : k_apply<false, false>);
+  kernel<<<ap.net_blocks + extra_blocks, APPLY_BLOCK, apply_lds(K, list), ctx->stream>>>(ap);
+}
+
 // the scan and the admission of a BAL round (first_free: of a sub-round of the stream)
-void launch_admission(fp_ctx* ctx, int r0, int nslots, int ntiles, long long cap, bool first_free, unsigned tag) {
+void launch_admission(fp_ctx* ctx, int r0, int nslots, int ntiles, long long cap, bool first_free, unsigned tag,
+                      bool list) {
   const int K = ctx->K;
   if (ntiles <= SCAN_WAVE_TILES)
     k_bal_scan<true><<<std::max(1, std::min((K + 3) / 4, 1024)), 256, 0, ctx->stream>>>(
-        ctx->hist, ctx->pref, ntiles, K, ctx->sizes_frozen, cap, ctx->over);
+        ctx->hist, ctx->pref, ntiles, K, ctx->sizes_frozen, cap, ctx->over, ctx->counters);
   else
     k_bal_scan<false><<<std::max(1, std::min(K, 1024)), 256, 0, ctx->stream>>>(ctx->hist, ctx->pref, ntiles, K,
-                                                                               ctx->sizes_frozen, cap, ctx->over);
+                                                                               ctx->sizes_frozen, cap, ctx->over,
+                                                                               ctx->counters);
   // the size changes are summed per block in LDS where K parts fit
   // large blocks where that still leaves many: every block adds to the K size
   // words, one after another (rounds of 262,144 slots: 16.4 -> 14.2 us with 16
@@ -1312,9 +1420,12 @@ void launch_admission(fp_ctx* ctx, int r0, int nslots, int ntiles, long long cap
   const int agrid = std::max(1, std::min((ntiles + tiles - 1) / tiles, 4096));
   const size_t lds = (size_t)K * sizeof(long long);
   const bool agg = lds <= (size_t)LDS_BUDGET;
-  (agg ? k_bal_admit<true> : k_bal_admit<false>)<<<agrid, ablock, agg ? lds : 0, ctx->stream>>>(
+  auto admit = list ? (agg ? k_bal_admit<true, true> : k_bal_admit<false, true>)
+                    : (agg ? k_bal_admit<true, false> : k_bal_admit<false, false>);
+  admit<<<agrid, ablock, agg ? lds : 0, ctx->stream>>>(
       ctx->slot_dec, ctx->slot_own, ctx->order, ctx->vwgt, r0, nslots, ntiles, K, ctx->sizes_frozen, cap, first_free,
-      ctx->over, ctx->pref, ctx->part, ctx->sizes, ctx->moves, ctx->vtx_ptr, ctx->vtx_nets, tag, ctx->net_stamp);
+      ctx->over, ctx->pref, ctx->part, ctx->sizes, ctx->moves, ctx->vtx_ptr, ctx->vtx_nets, tag, ctx->net_stamp,
+      ctx->touched, ctx->counters);
 }
 
 fp_status check_sched(fp_ctx* ctx, const fp_schedule* s) {
@@ -1367,7 +1478,7 @@ fp_status plan_tv(fp_ctx* ctx, RefinePlan& p) {
   const int waves = p.eval_waves > 0 ? std::min(p.eval_waves, eval_waves(K)) : eval_waves(K);
   if (waves == 0) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d needs more LDS than a workgroup has", K);
   p.eval_waves = waves;
-  if (apply_lds(K) + sizeof(ApplyNets) > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
+  if (apply_lds(K, true) + apply_static(true) > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
   p.R = std::min(p.sched.round, ctx->nov);
   FP_TRY(ensure_round_scratch(ctx, p.R));
   if (p.sched.kind == FP_SCHED_BAL) FP_TRY(ensure_bal_scratch(ctx, p.R));
@@ -1382,8 +1493,6 @@ fp_status pass_tv(fp_ctx* ctx, const RefinePlan& p) {
   const fp_schedule* sched = &p.sched;
   const bool bal = sched->kind == FP_SCHED_BAL;
   const size_t lds_e = eval_lds(K, waves);
-  const size_t lds_a = apply_lds(K);
-  auto apply = apply_indexed(K) ? k_apply<true> : k_apply<false>;
   // every pass restarts its round tags: clear the stamps
   pass_begin(ctx, nullptr, 0, nullptr);
   unsigned tag = 0;
@@ -1413,37 +1522,20 @@ fp_status pass_tv(fp_ctx* ctx, const RefinePlan& p) {
       FP_TRY(launch_timed(ctx, k_tv_eval<EVAL_REFINE>, grid, waves * WAVE, lds_e, a));
     }
     if (bal) {
-      launch_admission(ctx, r0, nslots, ntiles, sched->cap, false, tag);
+      launch_admission(ctx, r0, nslots, ntiles, sched->cap, false, tag, false);
     }
     ApplyArgs ap{};
-    ap.net_ptr = ctx->net_ptr;
-    ap.apply_pins = ctx->apply_pins;
-    ap.slot_own = ctx->slot_own;
-    ap.slot_dec = ctx->slot_dec;
-    ap.net_stamp = ctx->net_stamp;
     ap.tag = tag;
-    ap.noe = ctx->noe;
-    ap.ent = ctx->ent;
-    ap.ev = ctx->ev;
     ap.masks = p.masks;
-    ap.mask_words = mask_words(K);
-    ap.K = K;
-    ap.pb = ctx->pb;
-    ap.pmask = ctx->pmask;
     ap.r0 = r0;
     ap.r1 = r0 + nslots;
-    ap.net_blocks = apply_blocks(ctx, ap.per_block);
-    ap.lane_words = apply_lane_words(K);
-    ap.wave_bytes = (int)apply_wave_bytes(K, apply_indexed(K));
-    int grid_a = ap.net_blocks;
     if (!bal) {
       ap.order = ctx->order;
       ap.part = ctx->part;
       ap.sizes = ctx->sizes;
       ap.moves = ctx->moves;
-      grid_a += (nslots + APPLY_BLOCK - 1) / APPLY_BLOCK;
     }
-    apply<<<grid_a, APPLY_BLOCK, lds_a, ctx->stream>>>(ap);
+    launch_apply(ctx, ap, bal ? 0 : (nslots + APPLY_BLOCK - 1) / APPLY_BLOCK, false);
   }
   return FP_OK;
 }
@@ -1537,7 +1629,7 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
   FP_HIP_OK(hipSetDevice(ctx->device));
   FP_TRY(ensure_k(ctx, K));
   FP_TRY(check_envelope(ctx));
-  if (apply_lds(K) + sizeof(ApplyNets) > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
+  if (apply_lds(K, true) + apply_static(true) > (size_t)LDS_BUDGET) return fail(ctx, FP_ERR_UNSUPPORTED, "K = %d too large for the apply kernel", K);
   const int nov = ctx->nov;
   const int R = std::max(1, std::min(round, nov));
   const int waves = eval_waves(K);
@@ -1558,8 +1650,6 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
   FP_HIP_OK(hipEventRecord(e0, ctx->stream));
   const int eval_mode = mode == 2 ? EVAL_INIT_CN : EVAL_INIT;
   const size_t lds_e = eval_lds(K, waves);
-  const size_t lds_a = apply_lds(K);
-  auto apply = apply_indexed(K) ? k_apply<true> : k_apply<false>;
   int* fb = ctx->counters + 2;
   unsigned tag = 0;
   long long subrounds = 0, rounds = 0;
@@ -1605,28 +1695,14 @@ fp_status fp_initial_partition_device(fp_ctx* ctx, int mode, int K, int round, d
       k_tv_eval<EVAL_INIT><<<grid, waves * WAVE, lds_e, ctx->stream>>>(a);
     k_init_fallback<<<1, 1024, 0, ctx->stream>>>(ctx->slot_dec, ctx->order, ctx->vwgt, r0, nslots, ntiles, K, fb,
                                                  ctx->hist);
-    launch_admission(ctx, r0, nslots, ntiles, cap, true, tag);
+    const bool list = apply_by_list(ctx, nslots);
+    launch_admission(ctx, r0, nslots, ntiles, cap, true, tag, list);
     ApplyArgs ap{};
-    ap.net_ptr = ctx->net_ptr;
-    ap.apply_pins = ctx->apply_pins;
-    ap.slot_own = ctx->slot_own;
-    ap.slot_dec = ctx->slot_dec;
-    ap.net_stamp = ctx->net_stamp;
     ap.tag = tag;
-    ap.noe = ctx->noe;
-    ap.ent = ctx->ent;
-    ap.ev = ctx->ev;
     ap.masks = masks;
-    ap.mask_words = mask_words(K);
-    ap.K = K;
-    ap.pb = ctx->pb;
-    ap.pmask = ctx->pmask;
     ap.r0 = r0;
     ap.r1 = r0 + nslots;
-    ap.net_blocks = apply_blocks(ctx, ap.per_block);
-    ap.lane_words = apply_lane_words(K);
-    ap.wave_bytes = (int)apply_wave_bytes(K, apply_indexed(K));
-    apply<<<ap.net_blocks, APPLY_BLOCK, lds_a, ctx->stream>>>(ap);
+    launch_apply(ctx, ap, 0, list);
     FP_HIP_OK(hipGetLastError());
     subrounds++;
     return FP_OK;
