@@ -1130,15 +1130,29 @@ __global__ void __launch_bounds__(APPLY_BLOCK) __attribute__((amdgpu_waves_per_e
   if (LIST && nn <= 0) return;
   if (threadIdx.x < 4) s.cnt[threadIdx.x] = 0;
   __syncthreads();
-  for (int i0 = 0; i0 < nn; i0 += APPLY_BLOCK) {
-    const int i = i0 + (int)threadIdx.x;
-    const bool hit = i < nn && (LIST || a.net_stamp[n0 + i] == a.tag);
-    unsigned n = 0, st = 0, len = 0;
+  // the stamps (or numbers) of all the thread's nets load together, then their pin ranges
+  constexpr int OWN = APPLY_NETS / APPLY_BLOCK;
+  unsigned net[OWN], first[OWN], last[OWN];
+#pragma unroll
+  for (int u = 0; u < OWN; u++) {
+    const int i = u * APPLY_BLOCK + (int)threadIdx.x;
+    net[u] = i < nn ? (LIST ? (unsigned)a.touched[n0 + i] : a.net_stamp[n0 + i]) : ~0u;
+  }
+#pragma unroll
+  for (int u = 0; u < OWN; u++) {
+    const int i = u * APPLY_BLOCK + (int)threadIdx.x;
+    const bool hit = i < nn && (LIST || net[u] == a.tag);
+    net[u] = hit ? (LIST ? net[u] : (unsigned)(n0 + i)) : ~0u;
+    first[u] = last[u] = 0;
     if (hit) {
-      n = LIST ? (unsigned)a.touched[n0 + i] : (unsigned)(n0 + i);
-      st = a.net_ptr[n];
-      len = a.net_ptr[n + 1] - st;
+      first[u] = a.net_ptr[net[u]];
+      last[u] = a.net_ptr[net[u] + 1];
     }
+  }
+#pragma unroll
+  for (int u = 0; u < OWN; u++) {
+    const unsigned n = net[u], st = first[u], len = last[u] - first[u];
+    const bool hit = n != ~0u;
     const bool sm = hit && len <= (unsigned)SMALL_NET;
     const unsigned long long ms = __ballot(sm), mb = __ballot(hit && !sm);
     int bs = 0, bb = 0;
