@@ -92,10 +92,6 @@ struct EvalArgs {
 // slot decision of an unplaced vertex whose part the fallback assigns
 constexpr int SLOT_FALLBACK = -2;
 
-__device__ __forceinline__ bool better(double sc, long long sz, unsigned fi, double bsc, long long bsz, unsigned bfi) {
-  return sc > bsc || (sc == bsc && (sz < bsz || (sz == bsz && fi < bfi)));
-}
-
 // The LDG2 decision of one vertex with first-appearance ranks, for a vertex
 // whose best (score, size) two parts share: its lists are swept again into
 // pin counts and ranks (i << pb | t, i the net's index in the vertex's list,
@@ -766,9 +762,8 @@ __global__ void __launch_bounds__(1024) k_init_fallback(int* __restrict__ slot_d
 // vertex without a part, own -1, only adds to its new part's size). AGG:
 // the block sums its size changes per part in LDS first, so that sizes takes
 // one atomic per part and block (same-address atomics from every wave would
-// queue at one L2 slice: about 12 ns each, so the blocks are as large as they
-// can be).
-constexpr int ADMIT_BLOCK = 1024;
+// queue at one L2 slice, about 12 ns each).
+constexpr int ADMIT_BLOCK = 512;
 constexpr int ADMIT_NETS = 4;
 
 // LIST: the touched nets go to a list, too (apply_by_list).
@@ -1428,10 +1423,13 @@ void launch_admission(fp_ctx* ctx, int r0, int nslots, int ntiles, long long cap
     k_bal_scan<false><<<std::max(1, std::min(K, 1024)), 256, 0, ctx->stream>>>(ctx->hist, ctx->pref, ntiles, K,
                                                                                ctx->sizes_frozen, cap, ctx->over,
                                                                                ctx->counters);
-  // the size changes are summed per block in LDS where K parts fit
-  // large blocks where that still leaves many: every block adds to the K size
-  // words, one after another (rounds of 262,144 slots: 16.4 -> 14.2 us with 16
-  // waves; rounds of 16,384, whose blocks are few: 7.3 us with 4 waves, 13.4 with 16)
+  // the size changes are summed per block in LDS where K parts fit, and every
+  // block then adds to the K size words, one after another: larger blocks where
+  // that still leaves many. us with blocks of 256, 512 and 1,024, K = 16 and 256:
+  //   16,384 slots    5.0  5.4  6.4     7.5  8.7 11.3
+  //   65,536          8.0  7.8  9.7     8.5  8.7 11.4
+  //   131,072        12.6 10.9 12.9    10.7  9.5 11.8
+  //   262,144        17.7 13.7 13.5    15.8 12.8 13.0
   const int ablock = ntiles >= 2048 ? ADMIT_BLOCK : 256;
   const int tiles = ablock / WAVE;  // per block
   const int agrid = std::max(1, std::min((ntiles + tiles - 1) / tiles, 4096));
