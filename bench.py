@@ -575,13 +575,16 @@ def run_tv1m(args):
 
     # algorithmic bytes per pass of the evaluation step, each byte counted once
     # per use, no cache credit: 12 B per vertex and, per (vertex, net)
-    # incidence, the net's id and the words of its part mask that are read, one
-    # per 64 parts and the own part's (K <= 512); past that, in the reference
-    # layout, 12 B per incidence and 8 B per list entry visited (Lambda = sum
-    # over nets of |n| * lambda(n))
+    # incidence, the net's id and what is read of its part mask, 8 B per 64
+    # parts and the 4 B with the own part's single bit; where the engine
+    # evaluates through the lists (K > 512, or masks past their 32-bit offsets),
+    # in the reference layout, 12 B per incidence and 8 B per list entry visited
+    # (Lambda = sum over nets of |n| * lambda(n))
     lam_avg = 0.5 * (lam0 + lam1)
-    if K <= 512:
-        bytes_pass = 12 * hg.nov + (4 + 8 * ((K + 63) // 64 + 1)) * hg.pins
+    words = (K + 63) // 64
+    masks = K <= 512 and 16 * words * (hg.noe + 1) < 1 << 32 and hg.pins < 1 << 30
+    if masks:
+        bytes_pass = 12 * hg.nov + (4 + 8 * words + 4) * hg.pins
     else:
         bytes_pass = 12 * hg.nov + 12 * hg.pins + 8 * lam_avg
     avg_launch_ms = eval_ms / max(launches, 1)
@@ -590,7 +593,7 @@ def run_tv1m(args):
     traffic, traffic_detail = (None, {"skipped": "--no-traffic"}) if args.no_traffic else measure_traffic(args)
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-            "kernel": "k_tv_eval_masks" if K <= 512 else "k_tv_eval", "launches": launches, "avg_launch_us": round(avg_launch_ms * 1e3, 2),
+            "kernel": "k_tv_eval_masks" if masks else "k_tv_eval", "launches": launches, "avg_launch_us": round(avg_launch_ms * 1e3, 2),
             "bytes_per_launch": int(bytes_launch), "traffic_counters": traffic_detail,
             "pass_frac": round(bytes_pass / (secs / args.steps) / 1e9 / HBM_PEAK_GBS, 4)}
 
