@@ -19,7 +19,12 @@
 
 namespace fpe {
 
-constexpr int MASK_PMAX = 8;  // counts, penalties and size keys of 8 parts per lane fit 64 VGPRs
+// Counts, penalties, size keys and numbers of P parts take 5 P registers a lane, and
+// a record 2 P scalar registers: at P = 8 the evaluations use their whole budget
+// (80 vector registers at 6 waves per SIMD, 72 at 7 for P <= 6; two of them spill
+// 12 bytes) with two records in flight. Past that one of the two would have
+// to give; no larger P was measured.
+constexpr int MASK_PMAX = 8;
 constexpr int MASK_KMAX = 64 * MASK_PMAX;
 
 inline int mask_words(int K) { return K <= MASK_KMAX ? (K + 63) / 64 : 0; }

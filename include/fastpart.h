@@ -104,7 +104,9 @@ fp_status fp_device_count(int* count);
 fp_status fp_ctx_create(fp_ctx** ctx, int device);
 void fp_ctx_destroy(fp_ctx* ctx);
 const char* fp_ctx_last_error(const fp_ctx* ctx);
-/* bytes of device memory the context holds now */
+/* Bytes of device memory the context holds now: its allocations, of which a
+ * part may be unused (up to three times the arrays of a small hypergraph, some
+ * MiB of a large one's). */
 long long fp_ctx_device_bytes(const fp_ctx* ctx);
 
 /* ---- hypergraph --------------------------------------------------------- */
@@ -294,8 +296,10 @@ fp_status fp_batch_member(const fp_batch* batch, int i, long long* moves, int* e
  * uploaded once into a context of its own (CSR views and connectivity state
  * stay in HBM). Worker threads take requests in arrival order, skipping one
  * whose hypergraph is busy, and admit a request only while the HBM footprint
- * of the requests in flight plus its own stays within the budget; a request
- * sets its state from its part vector, refines and evaluates on its
+ * of the requests in flight plus its own stays within the budget. (Part masks,
+ * which speed a request up, are charged and used where the budget has room for
+ * them besides a request like the largest so far on every other idle worker.) A
+ * request sets its state from its part vector, refines and evaluates on its
  * hypergraph's stream, so requests on different hypergraphs overlap on the
  * device and new ones start as slots and memory free up. A request's result
  * depends only on the request. The reference has no counterpart. */
@@ -336,13 +340,14 @@ fp_status fp_server_submit(fp_server* server, int graph_id, fp_metric metric, in
 fp_status fp_server_wait(fp_server* server, long long request_id, fp_request_info* info, int* part_out);
 fp_status fp_server_stats(fp_server* server, long long* completed, int* peak_inflight, long long* peak_bytes);
 
-/* Event timing of the dominant refinement kernel in the last fp_refine (the
- * evaluation: TV k_tv_eval, MSV/MSRV k_vol_eval, TM/MSM k_conn_eval; CN has
- * none): launches, total device ms of those launches (HIP events around each
- * launch, on the context stream). */
+/* Timing of the dominant refinement kernel in the last fp_refine (the
+ * evaluation: for K <= 512 through the nets' part masks, TV k_tv_eval_masks,
+ * MSV/MSRV k_vol_eval_masks, TM/MSM k_conn_eval_masks; else through the lists,
+ * k_tv_eval, k_vol_eval, k_conn_eval; CN has none): launches, total device ms of
+ * those launches (the start and end stamps of each dispatch). */
 fp_status fp_last_kernel_timing(fp_ctx* ctx, long long* launches, double* total_ms);
-/* Enables (1) or disables (0) per-launch event timing of fp_refine's
- * dominant kernel (adds events around every launch). */
+/* Enables (1) or disables (0) per-launch timing of fp_refine's dominant
+ * kernel (its launches then carry start and end events). */
 fp_status fp_set_kernel_timing(fp_ctx* ctx, int enable);
 
 #ifdef __cplusplus
