@@ -1338,7 +1338,10 @@ fp_status ensure_incoff(fp_ctx* ctx) {
   off[(size_t)ctx->pins] = (unsigned)acc;
   const long long cap = (long long)std::max(acc, 1ull);
   if (cap > c.evcap) {
-    FP_TRY(dalloc(ctx, &c.evbuf, (size_t)cap));
+    // in the place of a smaller K's, which would stay until the next upload
+    const bool first = !c.evbuf;
+    c.evcap = 0;
+    FP_TRY(first ? dalloc(ctx, &c.evbuf, (size_t)cap) : dgrow(ctx, &c.evbuf, (size_t)cap));
     c.evcap = cap;
   }
   if (!c.incoff) FP_TRY(dalloc(ctx, &c.incoff, (size_t)ctx->pins + 1));

@@ -35,6 +35,27 @@ def test_part_masks_of_a_smaller_k_are_given_back():
     assert np.array_equal(state.part, again.part) and np.array_equal(state.ep_parts, again.ep_parts)
 
 
+def test_message_events_of_a_smaller_k_are_given_back():
+    # half a million pins: an event takes 8 bytes, a source's move has two for
+    # each part that its net can touch
+    hg = H.colnet(20_000, H.DEG_FIXED, 24, seed=3)
+    steps = (2, 5, 8, 11, 14, 17, 20, 23)
+    with Engine(0) as eng:
+        eng.upload(hg)
+        _refine(eng, hg, "MSM", steps[-1])
+        direct = eng.device_bytes()
+    with Engine(0) as eng:
+        eng.upload(hg)
+        for K in steps:
+            _refine(eng, hg, "MSM", K)
+        stepwise = eng.device_bytes()
+    # all eight arrays together are 93 MB, the last one 15; a slab or two
+    # of the small arrays may be left
+    last = 8 * (2 * (hg.pins - hg.noe) + 2 * steps[-1] * hg.noe)
+    print(f"message events: direct {direct} stepwise {stepwise} last {last}", flush=True)
+    assert stepwise - direct < 2 * last
+
+
 @pytest.mark.parametrize("nov", [1, 300, 1_000, 20_000])
 def test_a_context_says_what_it_holds(nov):
     # its slabs: a few times its arrays, and no more once a refinement's
